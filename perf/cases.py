@@ -78,7 +78,7 @@ def _widths(rng):
     if rng.random() < 0.5:
         return rng.choice(SHAPES)
     hidden = 256 * rng.randint(4, 32)
-    return hidden, 256 * max(4, round(hidden * rng.uniform(2.5, 3.0) / 256))
+    return hidden, 256 * min(70, max(4, round(hidden * rng.uniform(2.5, 3.0) / 256)))  # at most the 30B decoder's
 
 
 def _groupsize(rng, *ks):
