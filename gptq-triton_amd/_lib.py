@@ -1,5 +1,6 @@
 """ctypes binding of csrc/libgptq4.so (the C ABI declared in include/gptq4.h; tuning and test hooks in
-include/gptq4_experimental.h).
+include/gptq4_experimental.h), and _host.so (csrc/host/gptq4_host.cpp), the same library's calls for torch tensors, which
+the operators a decode step launches go through.
 
 The HIP library is the only compute path: if it is missing, load() raises, and every
 operator that needs it raises with it.  There is no CPU fallback.
@@ -13,6 +14,7 @@ from pathlib import Path
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "csrc" / "libgptq4.so"
+HOST_PATH = Path(__file__).resolve().parent / "_host.so"
 ABI_VERSION = 3
 WS_COUNTER_BYTES = 524288            # arrival counters
 WS_HEAD_BYTES = WS_COUNTER_BYTES + (16 << 20)  # GPTQ4_WS_HEAD_BYTES: counters + marked partial sums, zero between calls
@@ -84,16 +86,18 @@ class LibraryMissing(RuntimeError):
 
 
 _lib = None
+_native = None  # the _host extension
 
 
 def load() -> ctypes.CDLL:
     """Open the in-tree shared object and bind every entry point."""
-    global _lib
+    global _lib, _native
     if _lib is not None:
         return _lib
-    if not LIB_PATH.exists():
+    missing = [p for p in (LIB_PATH, HOST_PATH) if not p.exists()]
+    if missing:
         raise LibraryMissing(
-            f"{LIB_PATH} is not built; run `python -c 'import __graft_entry__ as g; g.build()'` "
+            f"{missing[0]} is not built; run `python -c 'import __graft_entry__ as g; g.build()'` "
             "or `python gptq-triton_amd/build.py` (needs hipcc)")
     lib = ctypes.CDLL(str(LIB_PATH))
     for name, (res, args) in SIGNATURES.items():
@@ -103,8 +107,18 @@ def load() -> ctypes.CDLL:
     got = lib.gptq4_abi_version()
     if got != ABI_VERSION:
         raise LibraryMissing(f"{LIB_PATH} has ABI version {got}, expected {ABI_VERSION}; rebuild it")
+    from . import _host
+    _host.init(_workspace_of_current_stream, check)
+    _native = _host
     _lib = lib
     return lib
+
+
+def host():
+    """The _host extension."""
+    if _native is None:
+        load()
+    return _native
 
 
 class Gptq4Error(RuntimeError):
@@ -117,6 +131,11 @@ class Gptq4Error(RuntimeError):
 def check(code: int, where: str) -> None:
     if code != 0:
         raise Gptq4Error(code, where)
+
+
+def refused(where: str) -> RuntimeError:
+    """For arguments the _host extension does not take though no check of the Python function found why."""
+    return RuntimeError(f"{where}: arguments of a kind or shape that the library does not take")
 
 
 def op_for(op: int, perm) -> int:
@@ -156,7 +175,14 @@ def workspace(device: torch.device, need: int):
             _outgrown.append(ws)
         ws = torch.zeros(max(need, _WS_BYTES, 2 * ws.numel() if ws is not None else 0), dtype=torch.uint8, device=device)
         _workspaces[key] = ws
+        host().set_workspace(*key, ws.data_ptr(), ws.numel())
     return ws
+
+
+def _workspace_of_current_stream(index: int, need: int) -> None:
+    """What the _host extension calls when it knows no workspace of `need` bytes for the stream it is about to launch on."""
+    ws = workspace(torch.device("cuda", index), need)
+    host().set_workspace(index, current_stream(ws.device), ws.data_ptr(), ws.numel())
 
 
 def exchange_errors() -> list:

@@ -1,6 +1,7 @@
 """Build recipe for the HIP library: hipcc cross-compiles every csrc/*.hip for gfx950
 and links one shared object next to the sources (in-tree, so it travels with the
-tree and is the file the loader opens)."""
+tree and is the file the loader opens), and for the CPython extension that calls it on
+torch tensors."""
 from __future__ import annotations
 
 import os
@@ -61,6 +62,28 @@ def build_library(verbose: bool = False, extra_flags=()) -> Path:
     return LIB_PATH
 
 
+HOST_SRC = CSRC / "host" / "gptq4_host.cpp"
+HOST_PATH = CSRC.parent / "_host.so"
+
+
+def build_host(verbose: bool = False) -> Path:
+    """Compile the CPython extension that calls libgptq4.so on torch tensors (host code only; build_library comes first)."""
+    import sysconfig
+
+    import torch
+    root = Path(torch.__file__).resolve().parent
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    tmp = HOST_PATH.with_suffix(".so.tmp")
+    _run([shutil.which("g++") or "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-sign-compare",
+          "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",  # what torch's and HIP's own headers ask of a compiler that is not hipcc
+          "-isystem", str(root / "include"), "-isystem", str(root / "include" / "torch" / "csrc" / "api" / "include"),
+          "-isystem", f"{rocm}/include", "-isystem", sysconfig.get_paths()["include"], str(HOST_SRC), "-o", str(tmp),
+          f"-L{root / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-ltorch",
+          f"-L{CSRC}", "-lgptq4", "-Wl,-rpath,$ORIGIN/csrc"], verbose)
+    os.replace(tmp, HOST_PATH)
+    return HOST_PATH
+
+
 PROBE_SRC = CSRC / "probe" / "floor_probe.hip"
 PROBE_PATH = CSRC / "probe" / "floor_probe"
 
@@ -75,4 +98,5 @@ def build_probe(verbose: bool = False) -> Path:
 if __name__ == "__main__":
     path = build_library(verbose=True, extra_flags=sys.argv[1:])
     print("built", path)
+    print("built", build_host(verbose=True))
     print("built", build_probe(verbose=True))

@@ -4,7 +4,6 @@ ops of the HF model it patches (LlamaRMSNorm; fused_attention.py:118-148); here 
 so that a whole decode step is a short chain of HIP launches that a graph can replay."""
 from __future__ import annotations
 
-import math
 import os
 
 import torch
@@ -33,7 +32,7 @@ def norm_fusion_pays(rows: int, hidden: int) -> bool:
 
 
 def check_norm_args(h: torch.Tensor, delta, weight: torch.Tensor):
-    """Validate (h, delta, norm weight) of a fused call; returns the [rows, hidden] views and the sum buffer."""
+    """Say what is wrong with (h, delta, norm weight) of a fused call."""
     for t, name in ((h, "h"), (delta, "delta"), (weight, "norm weight")):
         if t is None:
             continue
@@ -43,10 +42,11 @@ def check_norm_args(h: torch.Tensor, delta, weight: torch.Tensor):
     hidden = h.shape[-1]
     if weight.shape != (hidden,) or (delta is not None and delta.shape != h.shape):
         raise ValueError("h and delta must have one shape [..., H] and the norm weight [H]")
-    h2 = h.reshape(-1, hidden).contiguous()
-    d2 = None if delta is None else delta.reshape(-1, hidden).contiguous()
-    s = None if delta is None else torch.empty_like(h2)  # never aliases h or delta: other workgroups still read them
-    return h2, d2, s
+
+
+def contiguous_delta(delta):
+    """The residual of a fused call as the kernels read it (a strided one is copied; None stays None)."""
+    return delta if delta is None or delta.is_contiguous() else delta.contiguous()
 
 
 def _check_out_index(out_index, h: int) -> None:
@@ -59,6 +59,9 @@ def _check_out_index(out_index, h: int) -> None:
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float, out_index: torch.Tensor = None) -> torch.Tensor:
     """y = weight * fp16(x * rsqrt(mean(x^2, -1) + eps)) for fp16 x [..., H] on the GPU.  With out_index (int32
     [H], a permutation) value f of a row is stored at position out_index[f]."""
+    y = _lib.host().rms_norm(x, weight, eps, out_index)
+    if y is not None:
+        return y
     _lib.require_cuda(x, "x")
     _lib.require_cuda(weight, "weight")
     if x.dtype != torch.float16 or weight.dtype != torch.float16:
@@ -67,21 +70,17 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float, out_index: torch
     if weight.shape != (h,) or h % 8 != 0:
         raise ValueError(f"weight must be [{h}] and the hidden size a multiple of 8")
     _check_out_index(out_index, h)
-    x2 = x.reshape(-1, h)
-    if not x2.is_contiguous():
-        x2 = x2.contiguous()
-    y = torch.empty_like(x2)
-    if x2.shape[0] == 0:
-        return y.reshape(x.shape)
-    rc = _lib.load().gptq4_rmsnorm(x2.data_ptr(), weight.data_ptr(), y.data_ptr(), _lib.ptr(out_index), x2.shape[0], h,
-                                   float(eps), _lib.current_stream(x.device))
-    _lib.check(rc, "gptq4_rmsnorm")
-    return y.reshape(x.shape)
+    if x.is_contiguous() and weight.is_contiguous():
+        raise _lib.refused("rms_norm")
+    return rms_norm(x.contiguous(), weight.contiguous(), eps, out_index)
 
 
 def add_rms_norm(x: torch.Tensor, delta: torch.Tensor, weight: torch.Tensor, eps: float, out_index: torch.Tensor = None):
     """(x + delta, RMSNorm(x + delta)) in one launch; fp16 GPU tensors of equal shape [..., H].  out_index as in
     rms_norm (the sum keeps its order)."""
+    both = _lib.host().add_rms_norm(x, delta, weight, eps, out_index)
+    if both is not None:
+        return both
     for t, name in ((x, "x"), (delta, "delta"), (weight, "weight")):
         _lib.require_cuda(t, name)
         if t.dtype != torch.float16:
@@ -90,15 +89,9 @@ def add_rms_norm(x: torch.Tensor, delta: torch.Tensor, weight: torch.Tensor, eps
     if delta.shape != x.shape or weight.shape != (h,) or h % 8 != 0:
         raise ValueError("x and delta must have one shape [..., H], weight [H], H a multiple of 8")
     _check_out_index(out_index, h)
-    x2 = x.reshape(-1, h).contiguous()
-    d2 = delta.reshape(-1, h).contiguous()
-    s = torch.empty_like(x2)
-    y = torch.empty_like(x2)
-    if x2.shape[0]:
-        rc = _lib.load().gptq4_add_rmsnorm(x2.data_ptr(), d2.data_ptr(), weight.data_ptr(), s.data_ptr(), y.data_ptr(),
-                                           _lib.ptr(out_index), x2.shape[0], h, float(eps), _lib.current_stream(x.device))
-        _lib.check(rc, "gptq4_add_rmsnorm")
-    return s.reshape(x.shape), y.reshape(x.shape)
+    if x.is_contiguous() and delta.is_contiguous() and weight.is_contiguous():
+        raise _lib.refused("add_rms_norm")
+    return add_rms_norm(x.contiguous(), delta.contiguous(), weight.contiguous(), eps, out_index)
 
 
 HEAD_ARGMAX_K = (4096, 5120, 6656, 8192)  # row lengths gptq4_lm_head_argmax is built for
@@ -128,6 +121,9 @@ def prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
     """Causal attention of a prompt (or of a chunk behind `past` cached tokens): q fp16 [B, H, S, 128]; caches fp16
     [B, H, capacity, 128] holding the S new tokens in rows past .. past + S - 1 (for a plain prompt: the k and v the QKV
     projection returned); query i attends to rows 0 .. past + i.  Returns fp16 [B, S, H*128], what o_proj consumes."""
+    out = _lib.host().prefill_attention(q, k_cache, v_cache, past)
+    if out is not None:
+        return out
     for t, name in ((q, "q"), (k_cache, "k_cache"), (v_cache, "v_cache")):
         _lib.require_cuda(t, name)
         if t.dtype != torch.float16:
@@ -141,12 +137,7 @@ def prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
     cap = k_cache.shape[2]
     if past < 0 or past + q_len > cap:
         raise ValueError("the cache has no room for past + S rows")
-    out = torch.empty((bsz, q_len, heads * hd), dtype=torch.float16, device=q.device)
-    if q_len:
-        rc = _lib.load().gptq4_prefill_attention(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), bsz, heads, q_len,
-                                                 hd, cap, past, 1.0 / math.sqrt(hd), _lib.current_stream(q.device))
-        _lib.check(rc, "gptq4_prefill_attention")
-    return out
+    raise _lib.refused("prefill_attention")
 
 
 def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, positions: torch.Tensor,
@@ -154,6 +145,9 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     """q fp16 [B, H, 1, 128]; caches fp16 [B, H, capacity, 128]; positions int32 [B] or [B, 1]:
     sequence b attends to cache rows 0..positions[b].  Returns fp16 [B, 1, H*128]; with out_index
     (int32 [H*128], a permutation) feature f of a row is stored at position out_index[f]."""
+    out = _lib.host().decode_attention(q, k_cache, v_cache, positions, out_index)
+    if out is not None:
+        return out
     for t, name in ((q, "q"), (k_cache, "k_cache"), (v_cache, "v_cache"), (positions, "positions")):
         _lib.require_cuda(t, name)
     bsz, heads, q_len, hd = q.shape
@@ -164,18 +158,9 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
         raise ValueError("caches must be contiguous [B, H, capacity, 128] tensors matching q")
     if q.dtype != torch.float16 or k_cache.dtype != torch.float16 or v_cache.dtype != torch.float16:
         raise TypeError("decode_attention takes fp16 tensors")
-    pos = positions.reshape(-1)
-    if pos.dtype != torch.int32 or pos.numel() != bsz or not pos.is_contiguous():
-        pos = pos.to(torch.int32).contiguous()
-        if pos.numel() != bsz:
-            raise ValueError("one position per sequence")
+    if positions.numel() != bsz:
+        raise ValueError("one position per sequence")
     _check_out_index(out_index, heads * hd)
-    cap = k_cache.shape[2]
-    out = torch.empty((bsz, 1, heads * hd), dtype=torch.float16, device=q.device)
-    lib = _lib.load()
-    ws = _lib.workspace(q.device, lib.gptq4_workspace_bytes(_lib.OP_DECODE_ATTENTION, bsz * heads, cap, 0))
-    rc = lib.gptq4_decode_attention(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), pos.data_ptr(), out.data_ptr(),
-                                    _lib.ptr(out_index), bsz, heads, hd, cap, 1.0 / math.sqrt(hd), ws.data_ptr(), ws.numel(),
-                                    _lib.current_stream(q.device))
-    _lib.check(rc, "gptq4_decode_attention")
-    return out
+    if positions.dtype == torch.int32 and positions.is_contiguous():
+        raise _lib.refused("decode_attention")
+    return decode_attention(q, k_cache, v_cache, positions.to(torch.int32).contiguous(), out_index)

@@ -18,8 +18,8 @@ import torch
 import torch.nn as nn
 
 from . import _lib
-from .quant_linear import (QuantLinear, _check_device_tensors, _check_matmul_args, inverse_permutation, matmul4,
-                           tensor_key)
+from .decoder_ops import NORM_MAX_ROWS, check_norm_args, contiguous_delta, norm_fusable, norm_fusion_pays, prefill_attention
+from .quant_linear import QuantLinear, _check_device_tensors, _check_matmul_args, inverse_permutation, tensor_key
 
 
 @dataclass
@@ -75,55 +75,48 @@ def qkv_rotary(groupsize: int, hidden_states: torch.Tensor, qweight: torch.Tenso
     filled (kv_offset = KV_AT_POSITION: row position_ids[b, s] for token (b, s), so that a
     decode step has no host-side scalar that changes from token to token).
     position_ids int [B, S] index the cos/sin tables."""
-    k_in, n = _check_matmul_args(hidden_states, qweight, groupsize)
-    _check_device_tensors(hidden_states, qweight, scales, qzeros, perm, cos, sin)
+    kbuf, vbuf = (None, None) if kv_out is None else kv_out
+    delta, norm_weight, eps = (None, None, 0.0) if norm is None else norm
+    if norm is not None:
+        delta = contiguous_delta(delta)
+        if not norm_fusable(hidden_states.numel() // max(hidden_states.shape[-1], 1), hidden_states.shape[-1]):
+            _check_qkv_args(groupsize, hidden_states, qweight, (scales, qzeros, perm, cos, sin), num_heads, head_dim, kv_out, kv_offset)
+            raise ValueError("outside what the fused norm takes; run add_rms_norm and the plain call")
+    for pos in _positions(position_ids, hidden_states):
+        out = _lib.host().qkv_rotary(groupsize, hidden_states, qweight, scales, qzeros, pos, cos, sin, num_heads, head_dim, perm, kbuf, vbuf,
+                                     kv_offset if kv_out is not None else 0, delta, norm_weight, eps)
+        if out is not None:
+            return out
+    _check_qkv_args(groupsize, hidden_states, qweight, (scales, qzeros, perm, cos, sin), num_heads, head_dim, kv_out, kv_offset, norm)
+    raise _lib.refused("qkv_rotary")
+
+
+def _positions(position_ids: torch.Tensor, hidden_states: torch.Tensor):
+    """position_ids as they are, then - if the call does not take them so - as a contiguous int32 [B, S] tensor beside the
+    activations."""
+    yield position_ids
+    if hidden_states.dim() != 3:
+        return
+    bsz, q_len, _ = hidden_states.shape
+    yield position_ids.to(device=hidden_states.device, dtype=torch.int32).expand(bsz, q_len).contiguous()
+
+
+def _check_qkv_args(groupsize, hidden_states, words, others, num_heads, head_dim, kv_out, kv_offset, norm=None):
+    """Say what is wrong with the arguments of a fused QKV call."""
+    _, n = _check_matmul_args(hidden_states, words, groupsize)
+    _check_device_tensors(hidden_states, words, *others)
     if hidden_states.dim() != 3:
         raise ValueError(f"hidden_states must be [B, S, hidden], got {tuple(hidden_states.shape)}")
     bsz, q_len, _ = hidden_states.shape
     if n != 3 * num_heads * head_dim:
         raise ValueError(f"packed QKV has {n} columns, expected 3*{num_heads}*{head_dim}")
-    dev = hidden_states.device
-    pos = position_ids
-    if pos.dtype != torch.int32 or pos.device != dev or tuple(pos.shape) != (bsz, q_len) or not pos.is_contiguous():
-        pos = position_ids.to(device=dev, dtype=torch.int32).expand(bsz, q_len).contiguous()
-    q = torch.empty((bsz, num_heads, q_len, head_dim), dtype=torch.float16, device=dev)
-    if kv_out is None:
-        kk = torch.empty_like(q)
-        vv = torch.empty_like(q)
-        cap, off = q_len, 0
-    else:
+    if kv_out is not None:
         kk, vv = kv_out
-        cap, off = kk.shape[2], kv_offset
         if kk.shape != vv.shape or kk.shape[0] != bsz or kk.shape[1] != num_heads or kk.shape[3] != head_dim \
-                or not kk.is_contiguous() or not vv.is_contiguous() or off < KV_AT_POSITION or off + q_len > cap:
+                or not kk.is_contiguous() or not vv.is_contiguous() or kv_offset < KV_AT_POSITION or kv_offset + q_len > kk.shape[2]:
             raise ValueError("kv_out buffers must be contiguous [B, H, capacity, D] with room for the new rows")
     if norm is not None:
-        from .decoder_ops import check_norm_args, norm_fusable
-        delta, norm_weight, eps = norm
-        if not norm_fusable(bsz * q_len, k_in):
-            raise ValueError("outside what the fused norm takes; run add_rms_norm and the plain call")
-        h2, d2, s = check_norm_args(hidden_states, delta, norm_weight)
-        lib = _lib.load()
-        ws = _lib.workspace(dev, lib.gptq4_workspace_bytes(_lib.OP_QKV_ROTARY, bsz * q_len, k_in, n))
-        rc = lib.gptq4_norm_qkv_rotary(h2.data_ptr(), _lib.ptr(d2), norm_weight.data_ptr(), float(eps), _lib.ptr(s),
-                                       qweight.data_ptr(), qzeros.data_ptr(), scales.data_ptr(), _lib.ptr(perm), pos.data_ptr(),
-                                       cos.data_ptr(), sin.data_ptr(), cos.shape[0], q.data_ptr(), kk.data_ptr(),
-                                       vv.data_ptr(), bsz, q_len, num_heads, head_dim, k_in, groupsize, cap, off,
-                                       ws.data_ptr(), ws.numel(), _lib.current_stream(dev))
-        _lib.check(rc, "gptq4_norm_qkv_rotary")
-        return q, kk, vv, (hidden_states if s is None else s.view(hidden_states.shape))
-    if bsz * q_len == 0:
-        return q, kk, vv
-    lib = _lib.load()
-    need = lib.gptq4_workspace_bytes(_lib.op_for(_lib.OP_QKV_ROTARY, perm), bsz * q_len, k_in, n)
-    ws = _lib.workspace(dev, need)
-    x2d = hidden_states.view(-1, k_in)
-    rc = lib.gptq4_qkv_rotary(x2d.data_ptr(), qweight.data_ptr(), qzeros.data_ptr(), scales.data_ptr(),
-                              _lib.ptr(perm), pos.data_ptr(), cos.data_ptr(), sin.data_ptr(), cos.shape[0],
-                              q.data_ptr(), kk.data_ptr(), vv.data_ptr(), bsz, q_len, num_heads, head_dim, k_in,
-                              groupsize, cap, off, ws.data_ptr(), ws.numel(), _lib.current_stream(dev))
-    _lib.check(rc, "gptq4_qkv_rotary")
-    return q, kk, vv
+        check_norm_args(hidden_states, norm[0], norm[1])
 
 
 def qkv_rotary_stream(groupsize: int, hidden_states: torch.Tensor, sweight: torch.Tensor, smeta: torch.Tensor,
@@ -132,46 +125,16 @@ def qkv_rotary_stream(groupsize: int, hidden_states: torch.Tensor, sweight: torc
                       kv_offset: int = 0, norm=None):
     """qkv_rotary on a projection in streaming order (quant_linear.stream_pack), for up to stream_rows() tokens in all;
     same arguments otherwise, same results to the last bit of the fp32 sums' order."""
-    k_in, n = _check_matmul_args(hidden_states, sweight, groupsize)
-    _check_device_tensors(hidden_states, sweight, smeta, perm, cos, sin)
-    if hidden_states.dim() != 3:
-        raise ValueError(f"hidden_states must be [B, S, hidden], got {tuple(hidden_states.shape)}")
-    bsz, q_len, _ = hidden_states.shape
-    if n != 3 * num_heads * head_dim:
-        raise ValueError(f"packed QKV has {n} columns, expected 3*{num_heads}*{head_dim}")
-    dev = hidden_states.device
-    pos = position_ids
-    if pos.dtype != torch.int32 or pos.device != dev or tuple(pos.shape) != (bsz, q_len) or not pos.is_contiguous():
-        pos = position_ids.to(device=dev, dtype=torch.int32).expand(bsz, q_len).contiguous()
-    q = torch.empty((bsz, num_heads, q_len, head_dim), dtype=torch.float16, device=dev)
-    if kv_out is None:
-        kk, vv = torch.empty_like(q), torch.empty_like(q)
-        cap, off = q_len, 0
-    else:
-        kk, vv = kv_out
-        cap, off = kk.shape[2], kv_offset
-        if kk.shape != vv.shape or kk.shape[0] != bsz or kk.shape[1] != num_heads or kk.shape[3] != head_dim \
-                or not kk.is_contiguous() or not vv.is_contiguous() or off < KV_AT_POSITION or off + q_len > cap:
-            raise ValueError("kv_out buffers must be contiguous [B, H, capacity, D] with room for the new rows")
-    delta_p = nw_p = sum_p = None
-    eps, s = 0.0, None
-    x2d = hidden_states.view(-1, k_in)
-    if norm is not None:
-        from .decoder_ops import check_norm_args
-        delta, norm_weight, eps = norm
-        x2d, d2, s = check_norm_args(hidden_states, delta, norm_weight)
-        delta_p, nw_p, sum_p = _lib.ptr(d2), norm_weight.data_ptr(), _lib.ptr(s)
-    lib = _lib.load()
-    from .quant_linear import stream_workspace_bytes
-    ws = _lib.workspace(dev, stream_workspace_bytes(_lib.OP_QKV_ROTARY, bsz * q_len, k_in, n, perm is not None))
-    rc = lib.gptq4_stream_qkv_rotary(x2d.data_ptr(), delta_p, nw_p, float(eps), sum_p, sweight.data_ptr(), smeta.data_ptr(),
-                                     _lib.ptr(perm), pos.data_ptr(), cos.data_ptr(), sin.data_ptr(), cos.shape[0], q.data_ptr(),
-                                     kk.data_ptr(), vv.data_ptr(), bsz, q_len, num_heads, head_dim, k_in, groupsize, cap, off,
-                                     ws.data_ptr(), ws.numel(), _lib.current_stream(dev))
-    _lib.check(rc, "gptq4_stream_qkv_rotary")
-    if norm is None:
-        return q, kk, vv
-    return q, kk, vv, (hidden_states if s is None else s.view(hidden_states.shape))
+    kbuf, vbuf = (None, None) if kv_out is None else kv_out
+    delta, norm_weight, eps = (None, None, 0.0) if norm is None else norm
+    delta = contiguous_delta(delta)
+    for pos in _positions(position_ids, hidden_states):
+        out = _lib.host().stream_qkv_rotary(groupsize, hidden_states, sweight, smeta, pos, cos, sin, num_heads, head_dim, perm, kbuf, vbuf,
+                                            kv_offset if kv_out is not None else 0, delta, norm_weight, eps)
+        if out is not None:
+            return out
+    _check_qkv_args(groupsize, hidden_states, sweight, (smeta, perm, cos, sin), num_heads, head_dim, kv_out, kv_offset, norm)
+    raise _lib.refused("qkv_rotary_stream")
 
 
 def _fuse_qkv(q_proj: QuantLinear, k_proj: QuantLinear, v_proj: QuantLinear) -> QuantLinear:
@@ -268,14 +231,13 @@ class QuantLlamaAttention(nn.Module):
             need = max(kv_offset, 0) + hidden_states.shape[1]
         cos, sin = self.rope.get(hidden_states.device, max(need, self.max_position_embeddings))
         rows = hidden_states.shape[0] * hidden_states.shape[1]
-        sw = self.qkv_proj.stream_weights(rows)
-        from .decoder_ops import NORM_MAX_ROWS
+        qkv = self._modules['qkv_proj']
+        sw = qkv.stream_weights(rows)
         if sw is not None and (norm is None or rows <= NORM_MAX_ROWS):
-            return qkv_rotary_stream(self.qkv_proj.groupsize, hidden_states, sw[0], sw[1], position_ids, cos, sin, self.num_heads,
+            return qkv_rotary_stream(qkv.groupsize, hidden_states, sw[0], sw[1], position_ids, cos, sin, self.num_heads,
                                      self.head_dim, perm=None if ordered else sw[2], kv_out=kv_out, kv_offset=kv_offset, norm=norm)
-        qweight, perm = self.qkv_proj.kernel_weights()
-        return qkv_rotary(self.qkv_proj.groupsize, hidden_states, qweight, self.qkv_proj.scales,
-                          self.qkv_proj.qzeros, position_ids, cos, sin, self.num_heads, self.head_dim,
+        qweight, perm = qkv.kernel_weights()
+        return qkv_rotary(qkv.groupsize, hidden_states, qweight, qkv.scales, qkv.qzeros, position_ids, cos, sin, self.num_heads, self.head_dim,
                           perm=None if ordered else perm, kv_out=kv_out, kv_offset=kv_offset, norm=norm)
 
     def context_order(self):
@@ -305,7 +267,6 @@ class QuantLlamaAttention(nn.Module):
 
     def norm_fusable(self, rows: int) -> bool:
         """Whether project_qkv(norm=...) is the faster way for this many rows."""
-        from .decoder_ops import norm_fusion_pays
         return norm_fusion_pays(rows, self.hidden_size)
 
     def forward(
@@ -360,7 +321,6 @@ class QuantLlamaAttention(nn.Module):
                 f"Attention mask should be of size {(bsz, 1, q_len, kv_seq_len)}, but is {attention_mask.size()}")
 
         if causal and attention_mask is None and not output_attentions and q_len > 1 and self.head_dim == 128:
-            from .decoder_ops import prefill_attention
             attn_output = prefill_attention(query_states, key_states, value_states, past_len)  # [B, S, hidden]
             return self.o_proj(attn_output), None, past_key_value
         if causal and attention_mask is None and q_len > 1:
@@ -436,7 +396,6 @@ def _forward_with_cache(self, hidden_states, attention_mask, position_ids, cache
         attn_output = torch.matmul(attn_weights, value_states)
     elif attention_mask is None and q_len > 1 and self.head_dim == 128 and k_all.is_contiguous() and v_all.is_contiguous():
         # (the kernel reads cache rows 0 .. kv_len - 1 where they lie, whatever the capacity behind them)
-        from .decoder_ops import prefill_attention
         return self.o_proj(prefill_attention(query_states, k_all, v_all, kv_len - q_len)), None
     else:
         # as transformers' own scaled-dot-product path: a given mask is used as it is, none means causal for a prompt

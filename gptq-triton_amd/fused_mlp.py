@@ -13,8 +13,9 @@ import torch
 import torch.nn as nn
 
 from . import _lib
-from .quant_linear import (QuantLinear, _check_device_tensors, _check_matmul_args, matmul4, stream_pack, stream_rows, stream_workspace_bytes,
-                           stream_unpack, tensor_key)
+from .decoder_ops import NORM_MAX_ROWS, check_norm_args, contiguous_delta, norm_fusable, norm_fusion_pays
+from .quant_linear import (QuantLinear, _check_device_tensors, _check_matmul_args, matmul4, stream_pack, stream_rows, stream_unpack,
+                           tensor_key)
 
 
 def llama_mlp_4(groupsize: int, a: torch.Tensor,
@@ -26,22 +27,13 @@ def llama_mlp_4(groupsize: int, a: torch.Tensor,
     taken on the fp32 accumulators and rounded once."""
     assert (gate_qweight.shape == up_qweight.shape and gate_scales.shape == up_scales.shape
             and gate_qzeros.shape == up_qzeros.shape), "All weights must have the same shape"
-    k, n = _check_matmul_args(a, gate_qweight, groupsize)
-    _check_device_tensors(a, gate_qweight, gate_scales, gate_qzeros, up_qweight, up_scales, up_qzeros, perm)
-    lib = _lib.load()
-    x = a.view(-1, k)
-    m = x.shape[0]
-    c = torch.empty((m, n), device=a.device, dtype=torch.float16)
-    if m == 0:
-        return c.view(a.shape[:-1] + (n,))
-    need = lib.gptq4_workspace_bytes(_lib.op_for(_lib.OP_MLP_GATEUP, perm), m, k, n)
-    ws = _lib.workspace(a.device, need)
-    rc = lib.gptq4_mlp_gateup(x.data_ptr(), gate_qweight.data_ptr(), gate_qzeros.data_ptr(), gate_scales.data_ptr(),
-                              up_qweight.data_ptr(), up_qzeros.data_ptr(), up_scales.data_ptr(), _lib.ptr(perm),
-                              c.data_ptr(), m, k, n, groupsize, ws.data_ptr(), ws.numel(),
-                              _lib.current_stream(a.device))
-    _lib.check(rc, "gptq4_mlp_gateup")
-    return c.view(a.shape[:-1] + (n,))
+    c = _lib.host().mlp_gateup(groupsize, a, gate_qweight, gate_scales, gate_qzeros, up_qweight, up_scales, up_qzeros, perm,
+                               None, None, 0.0)
+    if c is None:
+        _check_matmul_args(a, gate_qweight, groupsize)
+        _check_device_tensors(a, gate_qweight, gate_scales, gate_qzeros, up_qweight, up_scales, up_qzeros, perm)
+        raise _lib.refused("llama_mlp_4")
+    return c
 
 
 triton_llama_mlp_4 = llama_mlp_4
@@ -54,24 +46,23 @@ def norm_llama_mlp_4(groupsize: int, h: torch.Tensor, delta: Optional[torch.Tens
     """(s, silu(gate(xn)) * up(xn)) with s = h + delta (h when delta is None) and xn = RMSNorm(s) * norm_weight,
     in ONE launch: the kernel normalises its own input.  Same bits as add_rms_norm followed by llama_mlp_4.
     Decode-sized inputs only (decoder_ops.norm_fusable)."""
-    from .decoder_ops import check_norm_args, norm_fusable
     assert (gate_qweight.shape == up_qweight.shape and gate_scales.shape == up_scales.shape
             and gate_qzeros.shape == up_qzeros.shape), "All weights must have the same shape"
-    k, n = _check_matmul_args(h, gate_qweight, groupsize)
-    _check_device_tensors(h, gate_qweight, gate_scales, gate_qzeros, up_qweight, up_scales, up_qzeros, perm)
-    h2, d2, s = check_norm_args(h, delta, norm_weight)
-    m = h2.shape[0]
-    if not norm_fusable(m, k):
-        raise ValueError(f"{m} rows of {k} values are outside what the fused norm takes; run add_rms_norm and llama_mlp_4")
-    lib = _lib.load()
-    c = torch.empty((m, n), device=h.device, dtype=torch.float16)
-    ws = _lib.workspace(h.device, lib.gptq4_workspace_bytes(_lib.OP_MLP_GATEUP, m, k, n))
-    rc = lib.gptq4_norm_mlp_gateup(h2.data_ptr(), _lib.ptr(d2), norm_weight.data_ptr(), float(eps), _lib.ptr(s),
-                                   gate_qweight.data_ptr(), gate_qzeros.data_ptr(), gate_scales.data_ptr(),
-                                   up_qweight.data_ptr(), up_qzeros.data_ptr(), up_scales.data_ptr(), _lib.ptr(perm),
-                                   c.data_ptr(), m, k, n, groupsize, ws.data_ptr(), ws.numel(), _lib.current_stream(h.device))
-    _lib.check(rc, "gptq4_norm_mlp_gateup")
-    return (h if s is None else s.view(h.shape)), c.view(h.shape[:-1] + (n,))
+    k = h.shape[-1]
+    rows = h.numel() // max(k, 1)
+    out = None
+    if norm_fusable(rows, k):
+        delta = contiguous_delta(delta)
+        out = _lib.host().mlp_gateup(groupsize, h, gate_qweight, gate_scales, gate_qzeros, up_qweight, up_scales, up_qzeros, perm,
+                                     delta, norm_weight, eps)
+    if out is None:
+        _check_matmul_args(h, gate_qweight, groupsize)
+        _check_device_tensors(h, gate_qweight, gate_scales, gate_qzeros, up_qweight, up_scales, up_qzeros, perm)
+        check_norm_args(h, delta, norm_weight)
+        if not norm_fusable(rows, k):
+            raise ValueError(f"{rows} rows of {k} values are outside what the fused norm takes; run add_rms_norm and llama_mlp_4")
+        raise _lib.refused("norm_llama_mlp_4")
+    return out
 
 
 def llama_mlp_4_stream(groupsize: int, a: torch.Tensor, gate_sweight: torch.Tensor, gate_smeta: torch.Tensor,
@@ -80,29 +71,19 @@ def llama_mlp_4_stream(groupsize: int, a: torch.Tensor, gate_sweight: torch.Tens
     norm = (delta or None, norm_weight, eps): `a` is the residual stream h and the kernel multiplies with
     RMSNorm(h + delta) * norm_weight; returns (h + delta, result) then."""
     assert gate_sweight.shape == up_sweight.shape and gate_smeta.shape == up_smeta.shape, "All weights must have the same shape"
-    k, n = _check_matmul_args(a, gate_sweight, groupsize)
-    _check_device_tensors(a, gate_sweight, gate_smeta, up_sweight, up_smeta, perm)
-    lib = _lib.load()
-    delta_p = nw_p = sum_p = None
+    delta = norm_weight = None
     eps = 0.0
-    x, s = a.view(-1, k), None
     if norm is not None:
-        from .decoder_ops import check_norm_args
         delta, norm_weight, eps = norm
-        x, d2, s = check_norm_args(a, delta, norm_weight)
-        delta_p, nw_p, sum_p = _lib.ptr(d2), norm_weight.data_ptr(), _lib.ptr(s)
-    m = x.shape[0]
-    c = torch.empty((m, n), device=a.device, dtype=torch.float16)
-    if m:
-        ws = _lib.workspace(a.device, stream_workspace_bytes(_lib.OP_MLP_GATEUP, m, k, n, perm is not None))
-        rc = lib.gptq4_stream_mlp_gateup(x.data_ptr(), delta_p, nw_p, float(eps), sum_p, gate_sweight.data_ptr(), gate_smeta.data_ptr(),
-                                         up_sweight.data_ptr(), up_smeta.data_ptr(), _lib.ptr(perm), c.data_ptr(), m, k, n, groupsize,
-                                         ws.data_ptr(), ws.numel(), _lib.current_stream(a.device))
-        _lib.check(rc, "gptq4_stream_mlp_gateup")
-    out = c.view(a.shape[:-1] + (n,))
-    if norm is None:
-        return out
-    return (a if s is None else s.view(a.shape)), out
+        delta = contiguous_delta(delta)
+    out = _lib.host().stream_mlp_gateup(groupsize, a, gate_sweight, gate_smeta, up_sweight, up_smeta, perm, delta, norm_weight, eps)
+    if out is None:
+        _check_matmul_args(a, gate_sweight, groupsize)
+        _check_device_tensors(a, gate_sweight, gate_smeta, up_sweight, up_smeta, perm)
+        if norm is not None:
+            check_norm_args(a, delta, norm_weight)
+        raise _lib.refused("llama_mlp_4_stream")
+    return out
 
 
 def _move_zero_columns(qzeros: torch.Tensor, cols: torch.Tensor) -> torch.Tensor:
@@ -324,28 +305,28 @@ class QuantLlamaMLP(nn.Module):
     def _stream_ready(self, x: torch.Tensor) -> bool:
         # (any number of rows: the decode kernels up to _stream_rows, the tiled kernel above 16)
         rows = x.numel() // max(self.infeatures, 1)
-        return self._gate_meta is not None and not (self._stream_rows < rows <= 16)
+        return self._buffers['_gate_meta'] is not None and not (self._stream_rows < rows <= 16)
 
     def forward(self, x: torch.Tensor, ordered: bool = False) -> torch.Tensor:
         if self._stream_ready(x):
-            mid = llama_mlp_4_stream(self.groupsize, x, self.gate_proj_qweight, self._gate_meta, self.up_proj_qweight, self._up_meta,
-                                     None if ordered else self._compact_rows)
-            return self.down_proj.multiply(mid, ordered=True)  # the columns of gate and up are laid out in the order down_proj reads
+            own = self._buffers
+            mid = llama_mlp_4_stream(self.groupsize, x, own['gate_proj_qweight'], own['_gate_meta'], own['up_proj_qweight'], own['_up_meta'],
+                                     None if ordered else own['_compact_rows'])
+            return self._modules['down_proj'].multiply(mid, ordered=True)  # the columns of gate and up are laid out in the order down_proj reads
         w, perm, down_q = self._chained_weights()
         return self._down(llama_mlp_4(self.groupsize, x, *w, None if ordered else perm), down_q)
 
     def norm_fusable(self, rows: int) -> bool:
         """Whether forward_normed is the faster way for this many rows."""
-        from .decoder_ops import norm_fusion_pays
         return norm_fusion_pays(rows, self.infeatures)
 
     def forward_normed(self, h: torch.Tensor, delta: Optional[torch.Tensor], norm_weight: torch.Tensor, eps: float):
         """(h + delta, forward(RMSNorm(h + delta))): the residual add and the norm run inside the gate/up launch."""
-        from .decoder_ops import NORM_MAX_ROWS
         if self._stream_ready(h) and h.numel() // self.infeatures <= NORM_MAX_ROWS:
-            s, mid = llama_mlp_4_stream(self.groupsize, h, self.gate_proj_qweight, self._gate_meta, self.up_proj_qweight, self._up_meta,
-                                        self._compact_rows, norm=(delta, norm_weight, eps))
-            return s, self.down_proj.multiply(mid, ordered=True)
+            own = self._buffers
+            s, mid = llama_mlp_4_stream(self.groupsize, h, own['gate_proj_qweight'], own['_gate_meta'], own['up_proj_qweight'], own['_up_meta'],
+                                        own['_compact_rows'], norm=(delta, norm_weight, eps))
+            return s, self._modules['down_proj'].multiply(mid, ordered=True)
         w, perm, down_q = self._chained_weights()
         s, mid = norm_llama_mlp_4(self.groupsize, h, delta, norm_weight, eps, *w, perm)
         return s, self._down(mid, down_q)

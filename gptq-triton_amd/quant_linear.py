@@ -53,21 +53,12 @@ def matmul4(groupsize: int, a: torch.Tensor, qweight: torch.Tensor, scales: torc
     of input features per group (K when there is one group).  `perm` is the row
     permutation from `prepare_act_order` (qweight must then be the sorted copy).
     """
-    k, n = _check_matmul_args(a, qweight, groupsize)
-    _check_device_tensors(a, qweight, scales, qzeros, bias, perm)
-    lib = _lib.load()
-    x = a.view(-1, k)
-    m = x.shape[0]
-    c = torch.empty((m, n), device=a.device, dtype=torch.float16)
-    if m == 0:
-        return c.view(a.shape[:-1] + (n,))
-    need = lib.gptq4_workspace_bytes(_lib.op_for(_lib.OP_MATMUL, perm), m, k, n)
-    ws = _lib.workspace(a.device, need)
-    rc = lib.gptq4_matmul(x.data_ptr(), qweight.data_ptr(), qzeros.data_ptr(), scales.data_ptr(),
-                          _lib.ptr(perm), _lib.ptr(bias), c.data_ptr(), m, k, n, groupsize,
-                          ws.data_ptr(), ws.numel(), _lib.current_stream(a.device))
-    _lib.check(rc, "gptq4_matmul")
-    return c.view(a.shape[:-1] + (n,))
+    c = _lib.host().matmul(groupsize, a, qweight, scales, qzeros, bias, perm)
+    if c is None:
+        _check_matmul_args(a, qweight, groupsize)
+        _check_device_tensors(a, qweight, scales, qzeros, bias, perm)
+        raise _lib.refused("matmul4")
+    return c
 
 
 # the reference's name for the same functional
@@ -139,14 +130,6 @@ def stream_rows(op: int, k: int, n: int, groupsize: int) -> int:
     return int(_lib.load().gptq4_stream_rows(op, k, n, groupsize))
 
 
-def stream_workspace_bytes(op: int, m: int, k: int, n: int, with_perm: bool) -> int:
-    """Workspace a streaming-order call needs: the zeroed head; for more than four rows of an act-order projection room for
-    the gathered rows; above 16 rows what the tiled kernel asks for (it reads the same words)."""
-    if m > 16:
-        return int(_lib.load().gptq4_workspace_bytes(op | (_lib.OP_WITH_PERM if with_perm else 0), m, k, n))
-    return _lib.WS_HEAD_BYTES + (2 * m * k if with_perm and m > 4 else 0)
-
-
 def _stream_source_index(k: int, n: int, device) -> torch.Tensor:
     """For every word o of the streaming order, its index kb * N + n in the checkpoint order (int64 [K/8 * N])."""
     nb = k // 128
@@ -196,19 +179,12 @@ def stream_unpack(sweight: torch.Tensor) -> torch.Tensor:
 def matmul4_stream(groupsize: int, a: torch.Tensor, sweight: torch.Tensor, smeta: torch.Tensor,
                    bias: Optional[torch.Tensor] = None, perm: Optional[torch.Tensor] = None) -> torch.Tensor:
     """matmul4 on a projection in streaming order (stream_pack): A (..., K) fp16 with at most stream_rows() rows."""
-    k, n = _check_matmul_args(a, sweight, groupsize)
-    _check_device_tensors(a, sweight, smeta, bias, perm)
-    lib = _lib.load()
-    x = a.view(-1, k)
-    m = x.shape[0]
-    c = torch.empty((m, n), device=a.device, dtype=torch.float16)
-    if m == 0:
-        return c.view(a.shape[:-1] + (n,))
-    ws = _lib.workspace(a.device, stream_workspace_bytes(_lib.OP_MATMUL, m, k, n, perm is not None))
-    rc = lib.gptq4_stream_matmul(x.data_ptr(), sweight.data_ptr(), smeta.data_ptr(), _lib.ptr(perm), _lib.ptr(bias), c.data_ptr(),
-                                 m, k, n, groupsize, ws.data_ptr(), ws.numel(), _lib.current_stream(a.device))
-    _lib.check(rc, "gptq4_stream_matmul")
-    return c.view(a.shape[:-1] + (n,))
+    c = _lib.host().stream_matmul(groupsize, a, sweight, smeta, bias, perm)
+    if c is None:
+        _check_matmul_args(a, sweight, groupsize)
+        _check_device_tensors(a, sweight, smeta, bias, perm)
+        raise _lib.refused("matmul4_stream")
+    return c
 
 
 def prepare_act_order(qweight: torch.Tensor, g_idx: torch.Tensor, groupsize: int):
@@ -357,18 +333,21 @@ class QuantLinear(nn.Module):
     def stream_weights(self, rows: int = 1):
         """(sweight, smeta, perm) if the module is in streaming order, else None (any number of rows: up to `_stream_rows`
         the decode kernels read these words, above that the tiled kernel does)."""
-        if self._stream_meta is None or self._stream_rows < rows <= 16:
+        own = self._buffers
+        meta = own['_stream_meta']
+        if meta is None or self._stream_rows < rows <= 16:
             return None
-        return self.qweight, self._stream_meta, self._compact_perm
+        return own['qweight'], meta, own['_compact_perm']
 
     def multiply(self, x: torch.Tensor, ordered: bool = False) -> torch.Tensor:
         """forward(x); ordered: x already is in the order of the sorted rows (act-order), no gather needed."""
-        rows = x.numel() // max(self.infeatures, 1)
-        sw = self.stream_weights(rows)
-        if sw is not None:
-            return matmul4_stream(self.groupsize, x, sw[0], sw[1], self.bias, None if ordered else sw[2])
+        own = self._buffers  # (looked up here and not through nn.Module's __getattr__: that costs half a microsecond each)
+        meta = own['_stream_meta']
+        bias = own['bias'] if 'bias' in own else self._parameters.get('bias')
+        if meta is not None and not self._stream_rows < x.numel() // max(self.infeatures, 1) <= 16:
+            return matmul4_stream(self.groupsize, x, own['qweight'], meta, bias, None if ordered else own['_compact_perm'])
         qweight, perm = self.kernel_weights()
-        return matmul4(self.groupsize, x, qweight, self.scales, self.qzeros, self.bias, None if ordered else perm)
+        return matmul4(self.groupsize, x, qweight, own['scales'], own['qzeros'], bias, None if ordered else perm)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         return self.multiply(x)
