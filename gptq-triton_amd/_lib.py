@@ -59,6 +59,7 @@ SIGNATURES = {
     "gptq4_rmsnorm": (c_int, [c_void_p] * 4 + [c_int, c_int, c_float, c_void_p]),
     "gptq4_add_rmsnorm": (c_int, [c_void_p] * 6 + [c_int, c_int, c_float, c_void_p]),
     "gptq4_decode_attention": (c_int, [c_void_p] * 6 + [c_int] * 4 + [c_float, c_void_p, c_size_t, c_void_p]),
+    "gptq4_extend_attention": (c_int, [c_void_p] * 7 + [c_int] * 4 + [c_float, c_void_p, c_size_t, c_void_p]),
     "gptq4_stream_rows": (c_int, [c_int, c_int, c_int, c_int]),
     "gptq4_stream_pack": (c_int, [c_void_p] * 5 + [c_int, c_int, c_int, c_void_p]),
     "gptq4_stream_unpack": (c_int, [c_void_p] * 5 + [c_int, c_int, c_int, c_void_p]),

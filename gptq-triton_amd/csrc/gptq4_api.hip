@@ -730,6 +730,21 @@ int gptq4_decode_attention(const void *q, const void *k_cache, const void *v_cac
                               reinterpret_cast<hipStream_t>(stream));
 }
 
+int gptq4_extend_attention(const void *q, const void *past_k, const void *past_v, void *k, void *v, void *out, const int32_t *out_index,
+                           int B, int H, int D, int past, float scale, void *workspace, size_t workspace_bytes, void *stream) {
+    if (!q || !k || !v || !out || (past > 0 && (!past_k || !past_v))) return -GPTQ4_E_NULL;
+    if (B < 1 || H < 1 || D != 128 || past < 0 || past >= 0x7fffffff - 64 || (long)B * H > SKINNY_MAX_TILES) return -GPTQ4_E_SHAPE;
+    if (past > 0 && (past_k == k || past_v == v)) return -GPTQ4_E_SHAPE;
+    if (misaligned16(q) || misaligned16(past_k) || misaligned16(past_v) || misaligned16(k) || misaligned16(v) || misaligned16(out))
+        return -GPTQ4_E_ALIGN;
+    if (workspace == nullptr || workspace_bytes < GPTQ4_WS_HEAD_BYTES + attn_decode_partial_bytes(B * H, past + 1)) return -GPTQ4_E_WORKSPACE;
+    float *partials = reinterpret_cast<float *>(reinterpret_cast<char *>(workspace) + GPTQ4_WS_HEAD_BYTES);
+    return launch_attn_extend(reinterpret_cast<const half_t *>(q), reinterpret_cast<const half_t *>(past_k),
+                              reinterpret_cast<const half_t *>(past_v), reinterpret_cast<half_t *>(k), reinterpret_cast<half_t *>(v),
+                              reinterpret_cast<half_t *>(out), out_index, B, H, past, scale, reinterpret_cast<int *>(workspace), partials,
+                              reinterpret_cast<hipStream_t>(stream));
+}
+
 int gptq4_lm_head_argmax(const void *x, const void *weight, int64_t *out, int B, int K, int V, void *workspace, size_t workspace_bytes,
                          void *stream) {
     if (!x || !weight || !out) return -GPTQ4_E_NULL;

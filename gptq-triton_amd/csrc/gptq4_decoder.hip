@@ -71,13 +71,20 @@ __global__ __launch_bounds__(256) void gptq4_rmsnorm_kernel(const half_t *x, con
 // in the matmul kernels); the last one merges the partials in split order and writes
 // out[b, h*128 + d] - or, with out_index, out[b, out_index[h*128 + d]]: the order in which an act-order
 // o_proj reads its input, so that it needs no gather.
+//
+// EXTEND: the cache is a (key, value) pair that grows by a row a call, as the reference's callers keep it: rows 0 .. past - 1
+// come from one pair of tensors and are stored to the next (capacity past + 1, whose last row the QKV launch wrote) on
+// their way to the arithmetic, and every sequence attends to all past + 1 rows.  Copying the pair first and attending after
+// that read everything twice: 2 x 8.2 us of copies beside 61 us of torch's attention for 32 heads x 1500 rows.
 constexpr int ATT_PART = 130;  // floats per partial: max, sum, 128 accumulators
 
-__global__ __launch_bounds__(256) void gptq4_attn_decode_kernel(const half_t *__restrict__ q, const half_t *__restrict__ kc,
-                                                                const half_t *__restrict__ vc, const int *__restrict__ positions,
+template <bool EXTEND>
+__global__ __launch_bounds__(256) void gptq4_attn_decode_kernel(const half_t *__restrict__ q, const half_t *kc, const half_t *vc,
+                                                                const int *__restrict__ positions,
                                                                 float *part, int *counters, half_t *__restrict__ out,
                                                                 const int32_t *__restrict__ out_index, int H,
-                                                                int capacity, int chunk, float scale) {
+                                                                int capacity, int chunk, float scale, const half_t *__restrict__ past_k,
+                                                                const half_t *__restrict__ past_v, half_t *kc_out, half_t *vc_out) {
     __shared__ float s_m[16], s_l[16];
     __shared__ float s_acc[16][128];
     __shared__ int s_is_last;
@@ -85,7 +92,7 @@ __global__ __launch_bounds__(256) void gptq4_attn_decode_kernel(const half_t *__
     const int slot = tid >> 4, sub = tid & 15;
     const int bh = blockIdx.y, split = blockIdx.x, nsplit = gridDim.x;
     const int b = bh / H;
-    const int len = min(max(positions[b], 0), capacity - 1) + 1;
+    const int len = EXTEND ? capacity : min(max(positions[b], 0), capacity - 1) + 1;
     // the valid prefix, not the capacity, is dealt to the splits (in multiples of the 16 rows of a pass): a short
     // context in a long cache still spreads over all of them
     const int mine = min(chunk, (((len + nsplit - 1) / nsplit) + 15) & ~15);
@@ -103,6 +110,9 @@ __global__ __launch_bounds__(256) void gptq4_attn_decode_kernel(const half_t *__
     }
     const half_t *kb = kc + (size_t)bh * capacity * 128 + 8 * sub;
     const half_t *vb = vc + (size_t)bh * capacity * 128 + 8 * sub;
+    const size_t old_rows = EXTEND ? (size_t)bh * (capacity - 1) * 128 + 8 * sub : 0;
+    const half_t *pk = EXTEND ? past_k + old_rows : nullptr, *pv = EXTEND ? past_v + old_rows : nullptr;
+    half_t *ko = EXTEND ? kc_out + (kb - kc) : nullptr, *vo = EXTEND ? vc_out + (vb - vc) : nullptr;
     float m = -INFINITY, l = 0.f, acc[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[i] = 0.f;
@@ -113,8 +123,19 @@ __global__ __launch_bounds__(256) void gptq4_attn_decode_kernel(const half_t *__
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int rr = min(r + 16 * u, r1 - 1);  // clamped: the load is always valid
-            kv[u] = *reinterpret_cast<const uint4 *>(kb + (size_t)rr * 128);
-            vv[u] = *reinterpret_cast<const uint4 *>(vb + (size_t)rr * 128);
+            const bool past = EXTEND && rr < capacity - 1;
+            kv[u] = *reinterpret_cast<const uint4 *>((past ? pk : kb) + (size_t)rr * 128);
+            vv[u] = *reinterpret_cast<const uint4 *>((past ? pv : vb) + (size_t)rr * 128);
+        }
+        if (EXTEND) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int rr = r + 16 * u;
+                if (rr < r1 && rr < capacity - 1) {
+                    *reinterpret_cast<uint4 *>(ko + (size_t)rr * 128) = kv[u];
+                    *reinterpret_cast<uint4 *>(vo + (size_t)rr * 128) = vv[u];
+                }
+            }
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -263,7 +284,17 @@ int launch_attn_decode(const half_t *q, const half_t *kc, const half_t *vc, cons
     const int nsplit = attn_decode_splits(BH, capacity);
     int chunk = (capacity + nsplit - 1) / nsplit;
     chunk = (chunk + 15) & ~15;
-    hipLaunchKernelGGL(gptq4_attn_decode_kernel, dim3((unsigned)nsplit, (unsigned)BH), dim3(256), 0, stream, q, kc, vc,
-                       positions, partials, counters, out, out_index, H, capacity, chunk, scale);
+    hipLaunchKernelGGL(gptq4_attn_decode_kernel<false>, dim3((unsigned)nsplit, (unsigned)BH), dim3(256), 0, stream, q, kc, vc,
+                       positions, partials, counters, out, out_index, H, capacity, chunk, scale, nullptr, nullptr, nullptr, nullptr);
+    return (int)hipGetLastError();
+}
+
+int launch_attn_extend(const half_t *q, const half_t *past_k, const half_t *past_v, half_t *k, half_t *v, half_t *out,
+                       const int32_t *out_index, int B, int H, int past, float scale, int *counters, float *partials, hipStream_t stream) {
+    const int BH = B * H, rows = past + 1;
+    const int nsplit = attn_decode_splits(BH, rows);
+    const int chunk = (((rows + nsplit - 1) / nsplit) + 15) & ~15;
+    hipLaunchKernelGGL(gptq4_attn_decode_kernel<true>, dim3((unsigned)nsplit, (unsigned)BH), dim3(256), 0, stream, q, k, v, nullptr,
+                       partials, counters, out, out_index, H, rows, chunk, scale, past_k, past_v, k, v);
     return (int)hipGetLastError();
 }

@@ -240,6 +240,9 @@ int launch_attn_prefill(const half_t *q, const half_t *kc, const half_t *vc, hal
 int launch_attn_decode(const half_t *q, const half_t *kc, const half_t *vc, const int *positions, half_t *out,
                        const int32_t *out_index, int B, int H, int capacity, float scale, int *counters, float *partials, hipStream_t stream);
 
+int launch_attn_extend(const half_t *q, const half_t *past_k, const half_t *past_v, half_t *k, half_t *v, half_t *out,
+                       const int32_t *out_index, int B, int H, int past, float scale, int *counters, float *partials, hipStream_t stream);
+
 // Compute units and XCDs of the current device, asked once per device (hipDeviceProp_t / hipDeviceAttributeNumberOfXccs).
 // Launch plans size their grids from it.  Where no device can be asked (plans made on a machine without a GPU, e.g.
 // gptq4_workspace_bytes in a host-only test) it answers with MI355X's 256 CUs in 8 XCDs.

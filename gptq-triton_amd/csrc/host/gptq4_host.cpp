@@ -128,11 +128,11 @@ bool projection_fits(const at::Tensor *x, const at::Tensor *words, long groupsiz
     return k == words->size(0) * 8 && k > 0 && k % 128 == 0 && n % 256 == 0 && groupsize % 128 == 0 && x->numel() / k < (1LL << 31);
 }
 
-// Bytes of workspace a streaming-order call needs: the zeroed head, the gathered rows of an act-order call above four
-// rows, and above 16 rows what the mid-M and tiled kernels ask for.
+// Bytes of workspace a streaming-order call needs: the zeroed head and room for the gathered rows of an act-order call (up to
+// four rows mostly gathered in the kernel), and above 16 rows what the mid-M and tiled kernels ask for.
 size_t stream_bytes(int op, long m, long k, long n, bool with_perm) {
     if (m > 16) return gptq4_workspace_bytes(op | (with_perm ? GPTQ4_OP_WITH_PERM : 0), (int)m, (int)k, (int)n);
-    return GPTQ4_WS_HEAD_BYTES + (with_perm && m > 4 ? (size_t)2 * m * k : 0);
+    return GPTQ4_WS_HEAD_BYTES + (with_perm ? (size_t)2 * m * k : 0);
 }
 
 size_t plain_bytes(int op, long m, long k, long n, bool with_perm) {
@@ -536,6 +536,32 @@ PyObject *decode_attention(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
+// extend_attention(q, past k, past v, k, v, out_index) -> [B, 1, H * 128]; past k and v None: no past
+PyObject *extend_attention(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    GPTQ4_TAKES(6)
+    Args a{v};
+    const at::Tensor *q = a.need(0), *pk = a.may(1), *pv = a.may(2), *kc = a.need(3), *vc = a.need(4), *index = a.may(5);
+    if (!a.fine || !caches_fit(q, kc, vc) || q->size(2) != 1 || (pk == nullptr) != (pv == nullptr)) Py_RETURN_NONE;
+    const at::Device dev = q->device();
+    const int64_t b = q->size(0), h = q->size(1), past = pk == nullptr ? 0 : pk->dim() == 4 ? pk->size(2) : -1;
+    if (past < 0 || (pk != nullptr && !caches_fit(q, pk, pv)) || kc->size(2) != past + 1 || !is_order(index, h * 128, dev)) Py_RETURN_NONE;
+    const int64_t size[3] = {b, 1, h * 128};
+    at::Tensor out = empty(size, dev);
+    const hipStream_t stream = stream_of(dev);
+    Workspace ws;
+    if (!workspace(dev.index(), stream, gptq4_workspace_bytes(GPTQ4_OP_DECODE_ATTENTION, (int)(b * h), (int)past + 1, 0), &ws)) return nullptr;
+    int rc;
+    {
+        NoGil unlocked;
+        rc = gptq4_extend_attention(data(q), data(pk), data(pv), data(kc), data(vc), out.data_ptr(), ints(index), (int)b, (int)h, 128,
+                                    (int)past, (float)(1.0 / std::sqrt(128.0)), ws.data, ws.bytes, stream);
+    }
+    if (rc) return failed(rc, "gptq4_extend_attention");
+    return THPVariable_Wrap(out);
+    END_HANDLE_TH_ERRORS
+}
+
 // set_workspace(device index, stream handle, address, bytes): what _lib.workspace() made for that stream
 PyObject *set_workspace(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
     GPTQ4_TAKES(4)
@@ -576,6 +602,7 @@ PyMethodDef g_methods[] = {GPTQ4_METHOD(init),
                            GPTQ4_METHOD(add_rms_norm),
                            GPTQ4_METHOD(prefill_attention),
                            GPTQ4_METHOD(decode_attention),
+                           GPTQ4_METHOD(extend_attention),
                            {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_host", "The package's calls of libgptq4 on torch tensors.", -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 

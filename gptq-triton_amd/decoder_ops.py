@@ -164,3 +164,20 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     if positions.dtype == torch.int32 and positions.is_contiguous():
         raise _lib.refused("decode_attention")
     return decode_attention(q, k_cache, v_cache, positions.to(torch.int32).contiguous(), out_index)
+
+
+ATTENTION_MAX_HEADS = 4096  # sequences x heads of one decode_attention / extend_attention call
+
+
+def extend_attention(q: torch.Tensor, past_k, past_v, k: torch.Tensor, v: torch.Tensor, out_index: torch.Tensor = None) -> torch.Tensor:
+    """One query token per sequence over a (key, value) pair that grows by a row: q fp16 [B, H, 1, 128]; past_k, past_v fp16
+    [B, H, past, 128] (None: no past); k, v [B, H, past + 1, 128], whose last row is in place already - the other rows are
+    copied from the past on the way.  Attends to all past + 1 rows; result and out_index as in decode_attention."""
+    out = _lib.host().extend_attention(q, past_k, past_v, k, v, out_index)
+    if out is not None:
+        return out
+    for t, name in ((q, "q"), (past_k, "past_k"), (past_v, "past_v"), (k, "k"), (v, "v")):
+        if t is not None:
+            _lib.require_cuda(t, name)
+    _check_out_index(out_index, q.shape[1] * q.shape[3])
+    raise ValueError("extend_attention takes contiguous fp16 tensors: q [B, H, 1, 128], past [B, H, P, 128], k and v [B, H, P + 1, 128]")

@@ -18,7 +18,8 @@ import torch
 import torch.nn as nn
 
 from . import _lib
-from .decoder_ops import NORM_MAX_ROWS, check_norm_args, contiguous_delta, norm_fusable, norm_fusion_pays, prefill_attention
+from .decoder_ops import (ATTENTION_MAX_HEADS, NORM_MAX_ROWS, check_norm_args, contiguous_delta, decode_attention, extend_attention,
+                          norm_fusable, norm_fusion_pays, prefill_attention)
 from .quant_linear import QuantLinear, _check_device_tensors, _check_matmul_args, inverse_permutation, tensor_key
 
 
@@ -43,6 +44,22 @@ class RotaryTable:
     def __init__(self, head_dim: int, max_pos: int = 2048, base: float = 10000.0):
         self.head_dim, self.max_pos, self.base = head_dim, max_pos, float(base)
         self._tables = {}
+        self._counts = {}
+
+    def positions(self, device: torch.device, start: int, bsz: int, q_len: int) -> torch.Tensor:
+        """position_ids of `q_len` tokens behind `start` others in every one of `bsz` sequences, int32 [B, S].  One sequence,
+        and one token of each of several, are a view of a table that is kept: no launch."""
+        if q_len > 1 and bsz > 1:
+            return torch.arange(start, start + q_len, dtype=torch.int32, device=device).expand(bsz, q_len).contiguous()
+        key = (device.index if device.index is not None else torch.cuda.current_device(), bsz)
+        tab = self._counts.get(key)
+        if tab is None or tab.shape[0] < start + q_len:
+            if len(self._counts) >= 16:
+                self._counts.clear()
+            rows = max(self.max_pos, start + q_len)
+            tab = torch.arange(rows, dtype=torch.int32, device=device).repeat_interleave(bsz).view(rows, bsz)
+            self._counts[key] = tab
+        return tab[start:start + q_len].view(bsz, q_len)
 
     def get(self, device: torch.device, need_pos: int):
         key = device.index if device.index is not None else torch.cuda.current_device()
@@ -244,7 +261,7 @@ class QuantLlamaAttention(nn.Module):
         """Where each feature of the attention output should be stored so that an act-order o_proj reads
         it in the order of its sorted rows (int32 [hidden], the inverse of o_proj's permutation), or
         None without act-order.  decode_attention(out_index=...) writes in that order."""
-        perm = self.o_proj.row_permutation()
+        perm = self._modules['o_proj'].row_permutation()
         if perm is None:
             return None
         if self._context_order is None or self._context_order[0] != tensor_key(perm):
@@ -261,9 +278,23 @@ class QuantLlamaAttention(nn.Module):
             self._input_order = (tensor_key(perm), inverse_permutation(perm))
         return self._input_order[1]
 
+    def attend_one(self, hidden_states: torch.Tensor, position_ids: torch.Tensor, past_key_value, norm=None):
+        """One token of each sequence behind a (key, value) pair (or None): (the arguments of project_out, the grown pair), and
+        with norm (see project_qkv) also the residual stream.  Two launches: the QKV projection stores its K and V as the
+        new pair's last row, the attention kernel copies the other rows while it attends to them."""
+        past_k, past_v = (None, None) if past_key_value is None else (t.contiguous() for t in past_key_value)
+        past = 0 if past_k is None else past_k.shape[2]
+        shape = (hidden_states.shape[0], self.num_heads, past + 1, self.head_dim)
+        pair = (torch.empty(shape, dtype=torch.float16, device=hidden_states.device),
+                torch.empty(shape, dtype=torch.float16, device=hidden_states.device))
+        q, _, _, *stream = self.project_qkv(hidden_states, position_ids, kv_out=pair, kv_offset=past, norm=norm)
+        order = self.context_order()
+        context = extend_attention(q, past_k, past_v, *pair, out_index=order), order is not None
+        return (context, pair, stream[0]) if norm is not None else (context, pair)
+
     def project_out(self, context: torch.Tensor, ordered: bool = False) -> torch.Tensor:
         """o_proj(context); ordered: the context already is in the order of context_order()."""
-        return self.o_proj.multiply(context, ordered=ordered)
+        return self._modules['o_proj'].multiply(context, ordered=ordered)
 
     def norm_fusable(self, rows: int) -> bool:
         """Whether project_qkv(norm=...) is the faster way for this many rows."""
@@ -301,8 +332,13 @@ class QuantLlamaAttention(nn.Module):
         past_len = 0 if past_key_value is None else past_key_value[0].shape[-2]
         kv_seq_len = past_len + q_len
         if position_ids is None:
-            position_ids = torch.arange(past_len, kv_seq_len, device=hidden_states.device).unsqueeze(0)
+            position_ids = self.rope.positions(hidden_states.device, past_len, bsz, q_len) if hidden_states.is_cuda \
+                else torch.arange(past_len, kv_seq_len, device=hidden_states.device).unsqueeze(0)
 
+        if q_len == 1 and attention_mask is None and not output_attentions and self.head_dim == 128 and hidden_states.is_cuda \
+                and bsz * self.num_heads <= ATTENTION_MAX_HEADS:
+            context, pair = self.attend_one(hidden_states, position_ids, past_key_value)
+            return self.project_out(*context), None, pair if use_cache else None
         if past_key_value is None:
             query_states, key_states, value_states = self.project_qkv(hidden_states, position_ids)
         else:
@@ -397,6 +433,11 @@ def _forward_with_cache(self, hidden_states, attention_mask, position_ids, cache
     elif attention_mask is None and q_len > 1 and self.head_dim == 128 and k_all.is_contiguous() and v_all.is_contiguous():
         # (the kernel reads cache rows 0 .. kv_len - 1 where they lie, whatever the capacity behind them)
         return self.o_proj(prefill_attention(query_states, k_all, v_all, kv_len - q_len)), None
+    elif attention_mask is None and q_len == 1 and self.head_dim == 128 and k_all.is_contiguous() and v_all.is_contiguous() \
+            and query_states.is_cuda and bsz * self.num_heads <= ATTENTION_MAX_HEADS:
+        last = self.rope.positions(query_states.device, kv_len - 1, bsz, 1)
+        order = self.context_order()
+        return self.project_out(decode_attention(query_states, k_all, v_all, last, out_index=order), order is not None), None
     else:
         # as transformers' own scaled-dot-product path: a given mask is used as it is, none means causal for a prompt
         # and full attention for a single token

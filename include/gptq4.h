@@ -222,6 +222,16 @@ int gptq4_decode_attention(const void *q, const void *k_cache, const void *v_cac
                            int kv_capacity, float scale, void *workspace,
                            size_t workspace_bytes, void *stream);
 
+/* The same for a (key, value) pair that grows by one row per call, as the reference's callers keep it
+ * (fused_attention.py:105-115: torch.cat of the past and the new row): past_k, past_v fp16 [B, H, past, D] (not read when
+ * past is 0), k, v fp16 [B, H, past + 1, D] whose row `past` the QKV call wrote (kv_capacity = past + 1, kv_offset = past).
+ * Rows 0 .. past - 1 of the old pair are stored to the new one while they are attended to, so the pair is read once; every
+ * sequence attends to all past + 1 rows.  The new pair may not overlap the old one.  Workspace: gptq4_workspace_bytes with
+ * GPTQ4_OP_DECODE_ATTENTION, B * H and past + 1. */
+int gptq4_extend_attention(const void *q, const void *past_k, const void *past_v, void *k, void *v,
+                           void *out, const int32_t *out_index, int B, int H, int D, int past,
+                           float scale, void *workspace, size_t workspace_bytes, void *stream);
+
 /* The end of a greedy decode step in one launch: out[b] = argmax over v of fp16(x[b] . weight[v]) - the fp16 lm_head
  * (weight fp16 [V, K], row-major as nn.Linear keeps it; no bias) and the argmax of its output, the lowest index among
  * equal logits.  x fp16 [B, K], B <= 16; out int64 [B]; K one of 4096, 5120, 6656, 8192 (else -GPTQ4_E_SHAPE: use a

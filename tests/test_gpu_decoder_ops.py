@@ -121,3 +121,27 @@ def test_decode_attention_peaked_scores_do_not_overflow():
     out = gptq().decode_attention(q.cuda(), k.cuda(), v.cuda(), torch.tensor([69], dtype=torch.int32).cuda())
     assert torch.isfinite(out).all()
     assert torch.equal(out.cpu().reshape(128), v[0, 0, 33])
+
+
+@pytest.mark.parametrize("bsz,heads,past", [(1, 32, 2047), (2, 8, 63), (3, 5, 64), (1, 2, 0), (8, 52, 15), (1, 1, 1)])
+def test_extend_attention(bsz, heads, past):
+    """The growing (key, value) pair: every old row arrives in the new pair bit for bit, the row the caller put there stays,
+    and the result is that of decode_attention on the grown pair (same splits, hence the same bits) and the oracle's."""
+    rng = np.random.default_rng(past + heads)
+    new = lambda rows: torch.from_numpy(rng.standard_normal((bsz, heads, rows, 128)).astype(np.float16)).cuda()
+    q, pk, pv, k, v = new(1), new(past), new(past), new(past + 1), new(past + 1)
+    k0, v0 = k.clone(), v.clone()
+    order = torch.from_numpy(rng.permutation(heads * 128).astype(np.int32)).cuda()
+    from gptq_triton_amd.decoder_ops import extend_attention
+    out = extend_attention(q, *((pk, pv) if past else (None, None)), k, v)
+    assert torch.equal(k[:, :, :past], pk) and torch.equal(v[:, :, :past], pv)
+    assert torch.equal(k[:, :, past], k0[:, :, past]) and torch.equal(v[:, :, past], v0[:, :, past])
+    assert torch.equal(out, gptq().decode_attention(q, k, v, torch.full((bsz,), past, dtype=torch.int32, device="cuda")))
+    ref = O.decode_attention_ref(q.cpu().numpy(), k.cpu().numpy(), v.cpu().numpy(), [past] * bsz)
+    assert np.abs(out.cpu().numpy().astype(np.float64) - ref).max() < 2e-3  # as test_decode_attention
+    moved = extend_attention(q, *((pk, pv) if past else (None, None)), k0, v0, out_index=order)
+    want = torch.empty_like(out)
+    want[..., order.long()] = out
+    assert torch.equal(moved, want)
+    with pytest.raises(ValueError):
+        extend_attention(q, pk, pv, k[:, :, 1:], v[:, :, 1:])
