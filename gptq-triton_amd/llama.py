@@ -18,8 +18,10 @@ import torch
 import torch.nn as nn
 
 from . import _lib
-from .decoder_ops import add_rms_norm, decode_attention, lm_head_argmax, rms_norm
-from .fused_attention import LlamaConfigLite
+from .decoder_ops import add_rms_norm, decode_attention, lm_head_argmax, norm_fusion_pays, rms_norm
+from .fused_attention import LlamaConfigLite, QuantLlamaAttention
+from .fused_mlp import llama_mlp_4_stream
+from .quant_linear import QuantLinear, stream_rows, tensor_key
 
 # up to this many rows the decoder's norms write act-order inputs in their consumer's order
 ORDERED_NORM_ROWS = 16
@@ -77,9 +79,51 @@ class LlamaMLP(nn.Module):
         self.gate_proj = nn.Linear(h, i, bias=False)
         self.down_proj = nn.Linear(i, h, bias=False)
         self.up_proj = nn.Linear(h, i, bias=False)
+        self._same_rows = self._most_rows = None
 
-    def forward(self, x):  # unfused path: three QuantLinear calls + torch silu*mul
+    def _pair(self, rows: int):
+        """(groupsize, gate words and {scale, zero} words, up's, row permutation) where one launch can compute
+        silu(gate) * up from the two modules' own tensors in streaming order, else None."""
+        gate, up = self._modules['gate_proj'], self._modules['up_proj']
+        if not (isinstance(gate, QuantLinear) and isinstance(up, QuantLinear)):
+            return None
+        g, u = gate.stream_weights(rows), up.stream_weights(rows)
+        if g is None or u is None or gate.groupsize != up.groupsize or g[0].shape != u[0].shape \
+                or gate.bias_tensor() is not None or up.bias_tensor() is not None or rows <= 16 and self._pair_rows(gate) < rows:
+            return None
+        if (g[2] is None) != (u[2] is None):
+            return None
+        if g[2] is not None:
+            key = tensor_key(g[2], u[2])
+            if self._same_rows is None or self._same_rows[0] != key:
+                self._same_rows = (key, torch.equal(g[2], u[2]))  # (once: the only synchronisation here)
+            if not self._same_rows[1]:
+                return None
+        return gate.groupsize, g[0], g[1], u[0], u[1], g[2]
+
+    def _pair_rows(self, gate) -> int:
+        if self._most_rows is None:
+            self._most_rows = stream_rows(_lib.OP_MLP_GATEUP, gate.infeatures, gate.outfeatures, gate.groupsize)
+        return self._most_rows
+
+    def forward(self, x):
+        # without make_fused_mlp the three projections stay modules of their own; on the GPU gate and up still are one
+        # launch, with SiLU and the product on the fp32 sums (two launches and two elementwise ones otherwise)
+        pair = self._pair(x.numel() // max(x.shape[-1], 1)) if x.is_cuda else None
+        if pair is not None:
+            groupsize, gw, gm, uw, um, perm = pair
+            return self._modules['down_proj'](llama_mlp_4_stream(groupsize, x, gw, gm, uw, um, perm))
         return self.down_proj(torch.nn.functional.silu(self.gate_proj(x)) * self.up_proj(x))
+
+    def norm_fusable(self, rows: int) -> bool:
+        """Whether forward_normed is the faster way for this many rows."""
+        return self._pair(rows) is not None and norm_fusion_pays(rows, self.gate_proj.infeatures)
+
+    def forward_normed(self, h, delta, norm_weight, eps):
+        """(h + delta, forward(RMSNorm(h + delta))) with the residual add and the norm inside the gate/up launch."""
+        groupsize, gw, gm, uw, um, perm = self._pair(h.numel() // h.shape[-1])
+        s, mid = llama_mlp_4_stream(groupsize, h, gw, gm, uw, um, perm, norm=(delta, norm_weight, eps))
+        return s, self._modules['down_proj'](mid)
 
 
 class LlamaDecoderLayer(nn.Module):
@@ -133,8 +177,14 @@ class LlamaForCausalLM(nn.Module):
         """input_ids [B, S] -> (logits [B, S or 1, vocab], past_key_values or None)."""
         bsz, q_len = input_ids.shape
         past_len = 0 if past_key_values is None else past_key_values[0][0].shape[2]
-        position_ids = torch.arange(past_len, past_len + q_len, device=input_ids.device).unsqueeze(0)
         h = self.model.embed_tokens(input_ids)
+        layers = self.model.layers
+        if h.is_cuda and h.dtype == torch.float16 and len(layers) and all(isinstance(l.self_attn, QuantLlamaAttention) for l in layers):
+            h, presents = self._layers_fused(h, past_len, past_key_values, use_cache)
+            if last_token_only:
+                h = h[:, -1:, :]
+            return self.lm_head(h), (presents if use_cache else None)
+        position_ids = torch.arange(past_len, past_len + q_len, device=input_ids.device).unsqueeze(0)
         presents = []
         for i, layer in enumerate(self.model.layers):
             # (causal: the attention block masks by position itself - on the GPU inside the attention kernel)
@@ -146,6 +196,33 @@ class LlamaForCausalLM(nn.Module):
         if last_token_only:
             h = h[:, -1:, :]
         return self.lm_head(h), (presents if use_cache else None)
+
+    def _layers_fused(self, h, past_len, past_key_values, use_cache):
+        """The stack and the final norm with every residual add in the launch of the norm behind it, and with one token in all
+        both of them in the projection's launch."""
+        layers = self.model.layers
+        bsz, q_len, _ = h.shape
+        position_ids = layers[0].self_attn.rope.positions(h.device, past_len, bsz, q_len)
+        inside = q_len == 1 and all(l.self_attn.norm_fusable(bsz) and getattr(l.mlp, "norm_fusable", lambda r: False)(bsz) for l in layers)
+        presents = []
+        delta = None
+        for i, layer in enumerate(layers):
+            attn, n1, n2 = layer.self_attn, layer.input_layernorm, layer.post_attention_layernorm
+            past = None if past_key_values is None else past_key_values[i]
+            if inside:
+                context, present, h = attn.attend_one(h, position_ids, past, norm=(delta, n1.weight, n1.variance_epsilon))
+                h, delta = layer.mlp.forward_normed(h, attn.project_out(*context), n2.weight, n2.variance_epsilon)
+            else:
+                if delta is None:
+                    x = rms_norm(h, n1.weight, n1.variance_epsilon)
+                else:
+                    h, x = add_rms_norm(h, delta, n1.weight, n1.variance_epsilon)
+                out, _, present = attn(hidden_states=x, position_ids=position_ids, past_key_value=past, use_cache=use_cache, causal=True)
+                h, x = add_rms_norm(h, out, n2.weight, n2.variance_epsilon)
+                delta = layer.mlp(x)
+            presents.append(present)
+        norm = self.model.norm
+        return add_rms_norm(h, delta, norm.weight, norm.variance_epsilon)[1], presents
 
     @torch.no_grad()
     def generate_greedy(self, input_ids: torch.Tensor, max_new_tokens: int, use_graph: bool = False) -> torch.Tensor:

@@ -328,7 +328,8 @@ class QuantLinear(nn.Module):
         """perm of kernel_weights() alone (None without act-order)."""
         if self.g_idx is None:
             return None
-        return self._compact_perm if self._compact_perm is not None else self._act_order()[1]
+        own = self._buffers
+        return own['_compact_perm'] if own['_compact_perm'] is not None else self._act_order()[1]
 
     def stream_weights(self, rows: int = 1):
         """(sweight, smeta, perm) if the module is in streaming order, else None (any number of rows: up to `_stream_rows`
@@ -339,11 +340,14 @@ class QuantLinear(nn.Module):
             return None
         return own['qweight'], meta, own['_compact_perm']
 
+    def bias_tensor(self):
+        return self._buffers['bias'] if 'bias' in self._buffers else self._parameters.get('bias')
+
     def multiply(self, x: torch.Tensor, ordered: bool = False) -> torch.Tensor:
         """forward(x); ordered: x already is in the order of the sorted rows (act-order), no gather needed."""
         own = self._buffers  # (looked up here and not through nn.Module's __getattr__: that costs half a microsecond each)
         meta = own['_stream_meta']
-        bias = own['bias'] if 'bias' in own else self._parameters.get('bias')
+        bias = self.bias_tensor()
         if meta is not None and not self._stream_rows < x.numel() // max(self.infeatures, 1) <= 16:
             return matmul4_stream(self.groupsize, x, own['qweight'], meta, bias, None if ordered else own['_compact_perm'])
         qweight, perm = self.kernel_weights()
