@@ -883,7 +883,7 @@ uint32_t smagic(int d) { return d > 1 ? (uint32_t)(0x100000000ull / (unsigned)d 
 
 StreamTuning g_stream_tuning = {0, 0};
 
-static StreamPlan stream_plan_with(int epi, int M, int N, int K, bool norm, int strips);
+static StreamPlan stream_plan_with(int epi, int M, int N, int K, bool norm, int strips, bool tall);
 
 StreamPlan stream_plan(int epi, int M, int N, int K, bool norm) {
     // 8 .. 16 rows: a unit is the 128 input rows of TWO adjacent tiles, so that the rows' chunks - twice the bytes of a
@@ -895,13 +895,15 @@ StreamPlan stream_plan(int epi, int M, int N, int K, bool norm) {
     const int tiles = (epi == EPI_ROPE) ? N / 32 : N / 16;
     const int mode = g_stream_tuning.depth / 10;
     if (M > STREAM_MAX_M && (tiles % 2) == 0 && mode != 1) {
-        const StreamPlan two = stream_plan_with(epi, M, N, K, norm, 2);
+        const StreamPlan two = stream_plan_with(epi, M, N, K, norm, 2, true);
         if (two.ok && (mode == 2 || (M >= 8 && two.q >= 40))) return two;
     }
-    return stream_plan_with(epi, M, N, K, norm, 1);
+    const StreamPlan pl = stream_plan_with(epi, M, N, K, norm, 1, M > STREAM_MAX_M);
+    // rows that with all of K do not fit the LDS (four of more than about 18000 values) are fetched with the units
+    return !pl.ok && !pl.tall && !norm ? stream_plan_with(epi, M, N, K, norm, 1, true) : pl;
 }
 
-static StreamPlan stream_plan_with(int epi, int M, int N, int K, bool norm, int strips) {
+static StreamPlan stream_plan_with(int epi, int M, int N, int K, bool norm, int strips, bool tall) {
     StreamPlan pl = {};
     const int tuned_depth = g_stream_tuning.depth % 10;
     pl.depth = tuned_depth ? tuned_depth : 2;
@@ -922,7 +924,7 @@ static StreamPlan stream_plan_with(int epi, int M, int N, int K, bool norm, int 
     if (!g_stream_tuning.waves && pl.nb < pl.waves) pl.waves = 8;
     if (pl.waves == 16 && pl.depth > 2) pl.depth = 2;
     pl.pieces = (pl.q + 1 + pl.nb - 1) / pl.nb + 1;
-    if (M > STREAM_MAX_M) {
+    if (tall) {
         // the A operand comes from memory with every unit, LDS holds the waves' partial sums (1 KiB per wave, matrix and
         // tile) and the rotary table rows of the tokens
         pl.tall = true;
@@ -936,7 +938,7 @@ static StreamPlan stream_plan_with(int epi, int M, int N, int K, bool norm, int 
         size_t lds = ((size_t)pl.nat_off + (size_t)pl.waves * 16 * 17) * 16;
         if (lds < (size_t)81 * 1024) lds = (size_t)81 * 1024;
         pl.lds_bytes = lds;
-        pl.ok = M <= STREAM_TALL_MAX_M && !norm && lds <= STREAM_LDS_BUDGET && (long)K * N < (1L << 32) && (long)M * K < (1L << 30) &&
+        pl.ok = M >= 1 && M <= STREAM_TALL_MAX_M && !norm && lds <= STREAM_LDS_BUDGET && (long)K * N < (1L << 32) && (long)M * K < (1L << 30) &&
                 units < (1L << 24) && units * (pl.nb > pl.q + 1 ? pl.nb : pl.q + 1) < (1L << 32) &&
                 (size_t)pl.workgroups * nv2 * 16 * M * sizeof(uint64_t) <= GPTQ4_WS_TAGGED_BYTES && pl.nb >= pl.waves &&
                 pl.pieces * pl.strips * M < 1024 && (epi != EPI_ROPE || (N % 128) == 0);

@@ -568,6 +568,55 @@ def test_fused_mlp_in_streaming_order(act):
     assert mlp._gate_meta is None and torch.equal(mlp.gate_proj_qweight, before["gate_proj_qweight"])
 
 
+@pytest.mark.parametrize("act", [None, "shared", "own"])
+@pytest.mark.parametrize("rows", [1, 4, 5, 16, 17])
+def test_unfused_mlp_runs_gate_and_up_in_one_launch(act, rows):
+    """LlamaMLP with three quantised projections of its own: gate and up go through one launch where they read their rows in one
+    order, through two where each has its own; either way within the tolerance of the composed oracle."""
+    G = gptq()
+    from gptq_triton_amd.llama import LlamaMLP
+    k, inter, g = 1024, 2816, 128
+    (gate, Lg), (up, Lu), (down, Ld) = (_quant_linear(*s, g, 1950 + i, act is not None) for i, s in enumerate(((k, inter), (k, inter), (inter, k))))
+    if act == "shared":
+        up.g_idx.copy_(gate.g_idx)
+        Lu["g_idx"] = Lg["g_idx"]
+    block = LlamaMLP(G.LlamaConfigLite(hidden_size=k, intermediate_size=inter))
+    block.gate_proj, block.up_proj, block.down_proj = gate.cuda(), up.cuda(), down.cuda()
+    G.set_layout(block, "stream")
+    x = O.make_x(rows, k, seed=rows)
+    y = block(torch.from_numpy(x).cuda())
+    assert (block._pair(rows) is not None) == (act != "own")
+    order = lambda d: d["g_idx"] if act else None
+    parts = [O.quant_matmul_ref(x, d["qweight"], d["qzeros"], d["scales"], g, g_idx=order(d)) for d in (Lg, Lu)]
+    mid = (parts[0] / (1 + np.exp(-parts[0])) * parts[1]).astype(np.float16)
+    ref = O.quant_matmul_ref(mid, Ld["qweight"], Ld["qzeros"], Ld["scales"], g, g_idx=order(Ld))
+    # the intermediate rounds to fp16 once (one launch) or three times (two): relative 2^-11 each, over `inter` terms of random
+    # sign a relative error of the sum no larger in the 2-norm
+    err = np.linalg.norm(y.float().cpu().numpy() - ref) / np.linalg.norm(ref)
+    assert err < 4 * 2.0 ** -11, err
+    h = torch.from_numpy(O.make_x(rows, k, seed=50)).cuda()
+    if block.norm_fusable(rows):
+        w = torch.ones(k, dtype=torch.float16, device="cuda")
+        s, out = block.forward_normed(h, None, w, 1e-6)
+        assert torch.equal(s, h) and torch.equal(out, block(G.rms_norm(h, w, 1e-6)))
+
+
+@pytest.mark.parametrize("act", [False, True])
+def test_four_rows_of_a_projection_too_long_for_the_lds(act):
+    """Four rows of 20480 values do not fit a workgroup's LDS: they take the kernel that fetches its rows with every unit."""
+    G = gptq()
+    k, n, g = 20480, 512, 128
+    q, L = _quant_linear(k, n, g, 1960, act)
+    q = q.cuda()
+    assert q.to_stream() and q._stream_rows == 16
+    for rows in (3, 4):
+        x = O.make_x(rows, k, seed=rows)
+        y = q(torch.from_numpy(x).cuda())
+        ref = O.quant_matmul_ref(x, L["qweight"], L["qzeros"], L["scales"], g, g_idx=L["g_idx"] if act else None)
+        ok, max_abs, _ = O.within_tolerance(y.cpu().numpy(), ref)
+        assert ok, max_abs
+
+
 def random_quant_model(hidden, inter, heads, layers, groupsize, seed, act_order=False):
     """A random-init decoder of the given shape on the GPU, attention and MLP blocks fused."""
     G = gptq()
