@@ -59,6 +59,7 @@ SIGNATURES = {
     "gptq4_rmsnorm": (c_int, [c_void_p] * 4 + [c_int, c_int, c_float, c_void_p]),
     "gptq4_add_rmsnorm": (c_int, [c_void_p] * 6 + [c_int, c_int, c_float, c_void_p]),
     "gptq4_decode_attention": (c_int, [c_void_p] * 6 + [c_int] * 4 + [c_float, c_void_p, c_size_t, c_void_p]),
+    "gptq4_greedy_step_end": (c_int, [c_void_p] * 3 + [c_float, c_void_p] + [c_int] * 3 + [c_void_p] * 3 + [c_int] + [c_void_p] * 3 + [c_size_t, c_void_p]),
     "gptq4_extend_attention": (c_int, [c_void_p] * 7 + [c_int] * 4 + [c_float, c_void_p, c_size_t, c_void_p]),
     "gptq4_stream_rows": (c_int, [c_int, c_int, c_int, c_int]),
     "gptq4_stream_pack": (c_int, [c_void_p] * 5 + [c_int, c_int, c_int, c_void_p]),
@@ -189,10 +190,14 @@ def _workspace_of_current_stream(index: int, need: int) -> None:
 def exchange_errors() -> list:
     """(device, stream) keys of the workspaces whose error word is set: a kernel's bounded wait for another
     workgroup's partial sums ran out there, and the results of that call are not valid.  Synchronises."""
-    bad = []
+    by_device: dict = {}
     for key, ws in list(_workspaces.items()) + [(None, w) for w in _outgrown]:
-        if int(ws[4 * WS_ERROR_WORD:4 * WS_ERROR_WORD + 4].view(torch.int32).item()) != 0:
-            bad.append(key)
+        word = ws[4 * WS_ERROR_WORD:4 * WS_ERROR_WORD + 4].view(torch.int32)
+        by_device.setdefault(ws.device, []).append((key, word))
+    bad = []
+    for words in by_device.values():  # (one read back per device)
+        values = (words[0][1] if len(words) == 1 else torch.cat([w for _, w in words])).tolist()
+        bad += [key for (key, _), value in zip(words, values) if value != 0]
     return bad
 
 

@@ -369,9 +369,9 @@ void gptq4_set_midm_tuning(int mode, int mt, int splitk) {
     g_kslice_tuning.waves = (mt >= 200) ? 8 : (mt >= 100) ? 4 : 0;
     mt %= 100;
     // 10 + mt: 128-column strips for plain projections; a plain 1 or 2 also pins the 64-column strips
-    g_kslice_tuning.wide = (mt >= 10) ? 1 : ((mt == 1 || mt == 2) ? -1 : 0);
+    g_kslice_tuning.wide = (mt >= 10) ? 1 : ((mt >= 1 && mt <= 4) ? -1 : 0);
     if (mt >= 10) mt -= 10;
-    g_kslice_tuning.mt = (mt == 1 || mt == 2) ? mt : 0;
+    g_kslice_tuning.mt = (mt >= 1 && mt <= 4) ? mt : 0;
     g_kslice_tuning.splitk = splitk > 0 ? splitk : 0;
 }
 
@@ -745,14 +745,54 @@ int gptq4_extend_attention(const void *q, const void *past_k, const void *past_v
                               reinterpret_cast<hipStream_t>(stream));
 }
 
+static int head_argmax(HeadArgs &a, void *workspace, size_t workspace_bytes, void *stream) {
+    if (!head_argmax_fits(a.B, a.K, a.V)) return -GPTQ4_E_SHAPE;
+    if (workspace == nullptr || workspace_bytes < GPTQ4_WS_HEAD_BYTES + head_argmax_partial_bytes()) return -GPTQ4_E_WORKSPACE;
+    a.part = reinterpret_cast<float *>(reinterpret_cast<char *>(workspace) + GPTQ4_WS_HEAD_BYTES);
+    a.counters = reinterpret_cast<int *>(workspace);
+    return launch_head_argmax(a, reinterpret_cast<hipStream_t>(stream));
+}
+
 int gptq4_lm_head_argmax(const void *x, const void *weight, int64_t *out, int B, int K, int V, void *workspace, size_t workspace_bytes,
                          void *stream) {
     if (!x || !weight || !out) return -GPTQ4_E_NULL;
     if (misaligned16(x) || misaligned16(weight) || (reinterpret_cast<uintptr_t>(out) & 7)) return -GPTQ4_E_ALIGN;
-    if (workspace == nullptr || workspace_bytes < GPTQ4_WS_HEAD_BYTES + head_argmax_partial_bytes()) return -GPTQ4_E_WORKSPACE;
-    float *part = reinterpret_cast<float *>(reinterpret_cast<char *>(workspace) + GPTQ4_WS_HEAD_BYTES);
-    return launch_head_argmax(reinterpret_cast<const half_t *>(x), reinterpret_cast<const half_t *>(weight), reinterpret_cast<long long *>(out),
-                              part, reinterpret_cast<int *>(workspace), B, K, V, reinterpret_cast<hipStream_t>(stream));
+    HeadArgs a = {};
+    a.x = reinterpret_cast<const half_t *>(x);
+    a.w = reinterpret_cast<const half_t *>(weight);
+    a.tokens = reinterpret_cast<long long *>(out);
+    a.B = B;
+    a.K = K;
+    a.V = V;
+    return head_argmax(a, workspace, workspace_bytes, stream);
+}
+
+int gptq4_greedy_step_end(const void *x, const void *delta, const void *norm_weight, float eps, const void *weight, int B, int K, int V,
+                          int64_t *tokens, int32_t *positions, int64_t *history, int history_capacity, const void *embed,
+                          void *next_hidden, void *workspace, size_t workspace_bytes, void *stream) {
+    if (!x || !weight || !tokens || !positions || !history || !embed || !next_hidden) return -GPTQ4_E_NULL;
+    if (history_capacity < 1 || (!norm_weight && delta) || (norm_weight && (B != 1 || K > NORM_MAX_H || !(eps >= 0.f)))) return -GPTQ4_E_SHAPE;
+    // (the workgroups that are still reading x and delta must not see the next step's row)
+    if (next_hidden == x || (delta && next_hidden == delta)) return -GPTQ4_E_SHAPE;
+    if (misaligned16(x) || misaligned16(weight) || misaligned16(embed) || misaligned16(next_hidden) || misaligned16(delta) ||
+        misaligned16(norm_weight) || ((reinterpret_cast<uintptr_t>(tokens) | reinterpret_cast<uintptr_t>(history)) & 7))
+        return -GPTQ4_E_ALIGN;
+    HeadArgs a = {};
+    a.x = reinterpret_cast<const half_t *>(x);
+    a.w = reinterpret_cast<const half_t *>(weight);
+    a.tokens = reinterpret_cast<long long *>(tokens);
+    a.B = B;
+    a.K = K;
+    a.V = V;
+    a.positions = positions;
+    a.history = reinterpret_cast<long long *>(history);
+    a.history_capacity = history_capacity;
+    a.embed = reinterpret_cast<const half_t *>(embed);
+    a.next_hidden = reinterpret_cast<half_t *>(next_hidden);
+    a.delta = reinterpret_cast<const half_t *>(delta);
+    a.nrm_weight = reinterpret_cast<const half_t *>(norm_weight);
+    a.eps = eps;
+    return head_argmax(a, workspace, workspace_bytes, stream);
 }
 
 int gptq4_prefill_attention(const void *q, const void *k_cache, const void *v_cache, void *out, int B, int H, int S, int D,

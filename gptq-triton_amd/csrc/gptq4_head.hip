@@ -1,105 +1,142 @@
 // The last step of a greedy decode token: logits = x . W^T with the fp16 lm_head weight W [V, K] and the index of the
-// largest logit per row, in one launch.  (The reference's scripts call the model's lm_head - a dense fp16 linear -
-// and take the argmax of its output, generate.py; the vendor's GEMV plus torch's argmax are 59 + 15 us of a 1.6 ms
-// LLaMA-7B step.)  A memory-bound stream over V x K x 2 bytes: the rows of W are dealt to the workgroups in contiguous
-// ranges, inside a workgroup to the waves one by one; a wave has the next row's loads in flight while it multiplies
-// one (64 lanes x KCH 16-byte chunks, the x rows out of LDS), rounds the sum to fp16 as the linear layer's output
-// would be, and keeps the best (value, index) per x row - the lower index among equal values, as torch.argmax does.
-// Workgroup bests go through the workspace; the last workgroup to arrive picks the winners.
+// largest logit per row, in one launch - and, for a decoding loop, what the next step starts from: the token and its place in
+// the sequence, the position, and the token's embedding row.  (The reference's scripts call the model's lm_head - a dense
+// fp16 linear - and take the argmax of its output, generate.py.)
+//
+// A memory-bound stream over V x K x 2 bytes.  The rows of W are dealt to the workgroups in contiguous ranges and inside a
+// workgroup to its eight waves; a wave multiplies up to 16 of its rows at a time, as the A operand of
+// v_mfma_f32_16x16x32_f16 (lane (r, c): 16 bytes of row c), with the x rows as B out of LDS, so that one to sixteen
+// sequences cost the same: 8 KiB of W per wave are in flight while the 8 KiB before are multiplied.  Rows are dealt evenly,
+// not in sixteens: lanes past a tile's rows load nothing.  Sums are rounded to fp16 as the linear layer's output would be;
+// the best (value, index) per x row is kept in registers - the lower index among equal values, as torch.argmax does -, the
+// workgroups' bests go through the workspace and the last workgroup to arrive picks the winners, one wave per x row.
 #include "../../include/gptq4.h"
 #include "gptq4_internal.h"
+#include "gptq4_norm.h"
 
 namespace {
 
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 constexpr int HEAD_WAVES = 8;
 constexpr int HEAD_MAX_B = 16;
+constexpr int HEAD_STEPS = 8;  // matrix steps (32 values of every row) per group of loads
 
 __device__ __forceinline__ bool better(float v, int i, float bv, int bi) { return v > bv || (v == bv && i < bi); }
 
-template <int KCH>
-__global__ __launch_bounds__(64 * HEAD_WAVES) void gptq4_head_argmax_kernel(const half_t *__restrict__ x, const half_t *__restrict__ w,
-                                                                            long long *__restrict__ out, float *part, int *counters,
-                                                                            int B, int V, int rows_per_wg) {
-    constexpr int K = KCH * 512;
-    constexpr int CHUNKS = K / 8;
-    extern __shared__ uint4 head_xs[];  // [B][CHUNKS]
+// NORM: 0 x as it is, 1 its RMSNorm, 2 the RMSNorm of x + delta
+template <int NORM>
+__global__ __launch_bounds__(64 * HEAD_WAVES) void gptq4_head_argmax_kernel(HeadArgs p) {
+    extern __shared__ uint4 head_xs[];  // [B][K / 8 + 1] chunks of 16 bytes: rows a chunk apart, conflict-free for 16 rows
     __shared__ float s_val[HEAD_WAVES][HEAD_MAX_B];
     __shared__ int s_idx[HEAD_WAVES][HEAD_MAX_B];
+    __shared__ float s_part[4];
     __shared__ int s_last;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    for (int c = tid; c < B * CHUNKS; c += 64 * HEAD_WAVES) head_xs[c] = reinterpret_cast<const uint4 *>(x)[c];
-    if (lane < HEAD_MAX_B) {
-        s_val[wave][lane] = -INFINITY;
-        s_idx[wave][lane] = 0x7fffffff;
+    const int r = lane >> 4, c = lane & 15;
+    const int B = p.B, K = p.K, chunks = K >> 3, pitch = chunks + 1;
+
+    // this wave's rows, in ntile tiles of `step` rows (16 at most)
+    const int wg0 = blockIdx.x * p.rows_per_wg, wg1 = min(wg0 + p.rows_per_wg, p.V);
+    const int per_wave = (p.rows_per_wg + HEAD_WAVES - 1) / HEAD_WAVES;
+    const int r0 = wg0 + wave * per_wave, r1 = min(r0 + per_wave, wg1);
+    const int ntile = (per_wave + 15) / 16, step = (per_wave + ntile - 1) / ntile;
+    const int groups = K / (32 * HEAD_STEPS);
+    // (rows of 4096 or 8192 values are a power of two apart: waves that all started at the beginning of their rows would ask
+    // the same few memory channels at a time, so every wave starts at a group of its own and goes round)
+    const int g_first = (int)((blockIdx.x * HEAD_WAVES + wave) * 7u % (unsigned)groups);
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(p.w), 0, (int)0x7FFFFFF0, 0x00020000);
+    u32x4_t cur[HEAD_STEPS], nxt[HEAD_STEPS];
+    auto fetch = [&](u32x4_t (&dst)[HEAD_STEPS], int row0, int g) {
+        const int row = row0 + c;
+        // (a row past the tile: an offset the buffer rejects - zeros, no memory touched)
+        const uint32_t off = (c < step && row < r1) ? (uint32_t)row * (uint32_t)(K * 2) + 16u * r : 0x80000000u;
+#pragma unroll
+        for (int j = 0; j < HEAD_STEPS; ++j) dst[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, off, (uint32_t)(g * HEAD_STEPS + j) * 64u, 0);
+    };
+    if constexpr (NORM == 0) {
+        fetch(cur, r0, g_first);
+        for (int i = tid; i < B * chunks; i += 64 * HEAD_WAVES) {
+            const int b = i / chunks;
+            head_xs[i + b] = reinterpret_cast<const uint4 *>(p.x)[i];
+        }
+    } else {
+        NormLoads<NORM_KEEP> row;
+        norm_issue_row0<NORM == 2, NORM_KEEP>(p.x, p.delta, p.nrm_weight, K, tid & 255, row);
+        fetch(cur, r0, g_first);
+        norm_rows_put<NORM == 2, NORM_KEEP>(p.x, p.delta, p.nrm_weight, nullptr, [&](int, int at, uint4 v) { head_xs[at] = v; }, s_part, 1, K,
+                                            p.eps, tid & 255, row, tid < 256);
     }
     __syncthreads();
 
-    const int r0 = blockIdx.x * rows_per_wg, r1 = min(r0 + rows_per_wg, V);
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(w), 0, (int)0x7FFFFFF0, 0x00020000);
-    u32x4_t cur[KCH], nxt[KCH];
-    auto fetch = [&](u32x4_t (&dst)[KCH], int row) {
-        // (rows past the range: a lane offset the buffer rejects - zeros, no memory touched)
-        const uint32_t off = row < r1 ? (uint32_t)lane * 16u : 0x80000000u;
+    const uint4 *const xb = head_xs + min(c, B - 1) * pitch + r;
+    float bv = -INFINITY;
+    int bi = 0x7fffffff;
+    f4_t acc = {0.f, 0.f, 0.f, 0.f};
+    int row0 = r0, g = g_first, left = groups;
+    for (int t = ntile * groups; t > 0; --t) {
+        const bool tile_ends = left == 1;
+        const int row_n = tile_ends ? row0 + step : row0, g_n = g + 1 == groups ? 0 : g + 1;
+        left = tile_ends ? groups : left - 1;
+        fetch(nxt, t > 1 ? row_n : r1, g_n);
 #pragma unroll
-        for (int j = 0; j < KCH; ++j) dst[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, off, (uint32_t)row * (uint32_t)(K * 2) + 1024u * j, 0);
-    };
-    fetch(cur, r0 + wave);
-    for (int row = r0 + wave; row < r1; row += HEAD_WAVES) {
-        fetch(nxt, row + HEAD_WAVES);
-        for (int b = 0; b < B; ++b) {
-            const uint4 *xb = head_xs + b * CHUNKS + lane;
-            float acc = 0.f;
+        for (int j = 0; j < HEAD_STEPS; ++j)
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, cur[j]), __builtin_bit_cast(h8_t, xb[4 * (g * HEAD_STEPS + j)]), acc,
+                                                         0, 0, 0);
+        if (tile_ends) {
 #pragma unroll
-            for (int j = 0; j < KCH; ++j) {
-                const uint4 xv = xb[64 * j];
-                acc = __builtin_amdgcn_fdot2(as_h2(cur[j].x), as_h2(xv.x), acc, false);
-                acc = __builtin_amdgcn_fdot2(as_h2(cur[j].y), as_h2(xv.y), acc, false);
-                acc = __builtin_amdgcn_fdot2(as_h2(cur[j].z), as_h2(xv.z), acc, false);
-                acc = __builtin_amdgcn_fdot2(as_h2(cur[j].w), as_h2(xv.w), acc, false);
+            for (int i = 0; i < 4; ++i) {
+                const int at = 4 * r + i, row = row0 + at;
+                const float v = (float)(half_t)acc[i];  // the linear layer's fp16 output
+                if (at < step && row < r1 && better(v, row, bv, bi)) bv = v, bi = row;
             }
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) acc += __shfl_xor(acc, o);
-            const float v = (float)(half_t)acc;  // the linear layer's fp16 output
-            if (lane == 0 && better(v, row, s_val[wave][b], s_idx[wave][b])) {
-                s_val[wave][b] = v;
-                s_idx[wave][b] = row;
-            }
+            acc = f4_t{0.f, 0.f, 0.f, 0.f};
         }
+        row0 = row_n, g = g_n;
 #pragma unroll
-        for (int j = 0; j < KCH; ++j) cur[j] = nxt[j];
+        for (int j = 0; j < HEAD_STEPS; ++j) cur[j] = nxt[j];
+    }
+    // lanes c, c + 16, c + 32, c + 48 hold bests of x row c
+#pragma unroll
+    for (int o = 16; o <= 32; o <<= 1) {
+        const float ov = __shfl_xor(bv, o);
+        const int oi = __shfl_xor(bi, o);
+        if (better(ov, oi, bv, bi)) bv = ov, bi = oi;
+    }
+    if (lane < HEAD_MAX_B) {
+        s_val[wave][lane] = bv;
+        s_idx[wave][lane] = bi;
     }
     __syncthreads();
 
     // ---- the workgroup's best per x row -> workspace; the last workgroup to arrive reduces them
     const int nwg = gridDim.x;
     if (tid < B) {
-        float bv = -INFINITY;
-        int bi = 0x7fffffff;
+        bv = -INFINITY;
+        bi = 0x7fffffff;
 #pragma unroll
         for (int wv = 0; wv < HEAD_WAVES; ++wv)
             if (better(s_val[wv][tid], s_idx[wv][tid], bv, bi)) bv = s_val[wv][tid], bi = s_idx[wv][tid];
-        float *dst = part + ((size_t)blockIdx.x * HEAD_MAX_B + tid) * 2;
+        float *dst = p.part + ((size_t)blockIdx.x * HEAD_MAX_B + tid) * 2;
         __hip_atomic_store(dst, bv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(reinterpret_cast<int *>(dst) + 1, bi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (tid == 0) {
-        const int old = __hip_atomic_fetch_add(&counters[0], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int old = __hip_atomic_fetch_add(&p.counters[0], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         s_last = (old == nwg - 1);
     }
     __syncthreads();
     if (!s_last) return;
-    if (tid == 0) __hip_atomic_store(&counters[0], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (int b = 0; b < B; ++b) {
-        float bv = -INFINITY;
-        int bi = 0x7fffffff;
-        for (int g = tid; g < nwg; g += 64 * HEAD_WAVES) {
-            const float *src = part + ((size_t)g * HEAD_MAX_B + b) * 2;
+    if (tid == 0) __hip_atomic_store(&p.counters[0], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int b = wave; b < B; b += HEAD_WAVES) {
+        bv = -INFINITY;
+        bi = 0x7fffffff;
+        for (int i = lane; i < nwg; i += 64) {
+            const float *src = p.part + ((size_t)i * HEAD_MAX_B + b) * 2;
             const float v = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const int i = __hip_atomic_load(reinterpret_cast<const int *>(src) + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (better(v, i, bv, bi)) bv = v, bi = i;
+            const int at = __hip_atomic_load(reinterpret_cast<const int *>(src) + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (better(v, at, bv, bi)) bv = v, bi = at;
         }
 #pragma unroll
         for (int o = 32; o >= 1; o >>= 1) {
@@ -107,39 +144,38 @@ __global__ __launch_bounds__(64 * HEAD_WAVES) void gptq4_head_argmax_kernel(cons
             const int oi = __shfl_xor(bi, o);
             if (better(ov, oi, bv, bi)) bv = ov, bi = oi;
         }
-        __syncthreads();  // (the slots of the row before have been read)
-        if (lane == 0) {
-            s_val[wave][0] = bv;
-            s_idx[wave][0] = bi;
-        }
-        __syncthreads();
-        if (tid == 0) {
-#pragma unroll
-            for (int wv = 1; wv < HEAD_WAVES; ++wv)
-                if (better(s_val[wv][0], s_idx[wv][0], bv, bi)) bv = s_val[wv][0], bi = s_idx[wv][0];
-            out[b] = (long long)bi;
+        const int token = __builtin_amdgcn_readfirstlane(min(bi, p.V - 1));  // (all logits NaN: no winner)
+        if (lane == 0) p.tokens[b] = (long long)token;
+        if (p.positions != nullptr) {
+            if (lane == 0) {
+                const int at = p.positions[b] + 1;
+                p.positions[b] = at;
+                if (at >= 0 && at < p.history_capacity) p.history[(size_t)b * p.history_capacity + at] = (long long)token;
+            }
+            const uint4 *src = reinterpret_cast<const uint4 *>(p.embed + (size_t)token * K);
+            uint4 *dst = reinterpret_cast<uint4 *>(p.next_hidden + (size_t)b * K);
+            for (int i = lane; i < chunks; i += 64) dst[i] = src[i];
         }
     }
 }
 
-template <int KCH>
-int launch_kch(const half_t *x, const half_t *w, long long *out, float *part, int *counters, int B, int V, hipStream_t stream) {
+template <int NORM>
+int launch_norm(HeadArgs &a, hipStream_t stream) {
     const int cus = device_shape().cus;
-    const int nwg = V < cus ? V : cus;
-    const int rows_per_wg = (V + nwg - 1) / nwg;
-    const int grid = (V + rows_per_wg - 1) / rows_per_wg;
-    const size_t lds = (size_t)B * KCH * 512 * sizeof(half_t);
+    const int nwg = a.V < cus ? a.V : cus;
+    a.rows_per_wg = (a.V + nwg - 1) / nwg;
+    const int grid = (a.V + a.rows_per_wg - 1) / a.rows_per_wg;
+    const size_t lds = (size_t)a.B * (a.K / 8 + 1) * 16;
     if (lds > 48 * 1024) {
         static bool allowed = false;
         if (!allowed) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gptq4_head_argmax_kernel<KCH>),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 2048);
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gptq4_head_argmax_kernel<NORM>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, HEAD_LDS_BYTES);
             if (e != hipSuccess) return (int)e;
             allowed = true;
         }
     }
-    hipLaunchKernelGGL((gptq4_head_argmax_kernel<KCH>), dim3((unsigned)grid), dim3(64 * HEAD_WAVES), lds, stream, x, w, out, part, counters, B, V,
-                       rows_per_wg);
+    hipLaunchKernelGGL((gptq4_head_argmax_kernel<NORM>), dim3((unsigned)grid), dim3(64 * HEAD_WAVES), lds, stream, a);
     return (int)hipGetLastError();
 }
 
@@ -147,14 +183,12 @@ int launch_kch(const half_t *x, const half_t *w, long long *out, float *part, in
 
 size_t head_argmax_partial_bytes() { return (size_t)device_shape().cus * HEAD_MAX_B * 2 * sizeof(float); }
 
-// -GPTQ4_E_SHAPE for row lengths without an instantiation
-int launch_head_argmax(const half_t *x, const half_t *w, long long *out, float *part, int *counters, int B, int K, int V, hipStream_t stream) {
-    if (B < 1 || B > HEAD_MAX_B || V < 1 || (size_t)V * K * 2 >= 0x7FFFFFF0ull || (size_t)B * K * 2 > 160 * 1024 - 2048) return -GPTQ4_E_SHAPE;
-    switch (K) {
-        case 4096: return launch_kch<8>(x, w, out, part, counters, B, V, stream);
-        case 5120: return launch_kch<10>(x, w, out, part, counters, B, V, stream);
-        case 6656: return launch_kch<13>(x, w, out, part, counters, B, V, stream);
-        case 8192: return launch_kch<16>(x, w, out, part, counters, B, V, stream);
-        default: return -GPTQ4_E_SHAPE;
-    }
+bool head_argmax_fits(int B, int K, int V) {
+    return B >= 1 && B <= HEAD_MAX_B && V >= 1 && K >= 256 && (K % 256) == 0 && (size_t)V * K * 2 < 0x7FFFFFF0ull &&
+           (size_t)B * (K / 8 + 1) * 16 <= (size_t)HEAD_LDS_BYTES;
+}
+
+int launch_head_argmax(HeadArgs &a, hipStream_t stream) {
+    if (a.nrm_weight == nullptr) return launch_norm<0>(a, stream);
+    return a.delta == nullptr ? launch_norm<1>(a, stream) : launch_norm<2>(a, stream);
 }

@@ -234,7 +234,27 @@ int launch_rmsnorm(const half_t *x, const half_t *delta, const half_t *w, half_t
                    int M, int H, float eps, hipStream_t stream);
 size_t attn_decode_partial_bytes(int BH, int capacity);
 size_t head_argmax_partial_bytes();
-int launch_head_argmax(const half_t *x, const half_t *w, long long *out, float *part, int *counters, int B, int K, int V, hipStream_t stream);
+constexpr int HEAD_LDS_BYTES = 160 * 1024 - 2048;
+struct HeadArgs {
+    const half_t *x;  // [B, K]
+    const half_t *w;  // [V, K]
+    long long *tokens;
+    float *part;
+    int *counters;
+    int B, K, V, rows_per_wg;
+    // a decoding loop's state (positions null: tokens only): positions[b] moves on by one, the token is stored at that place
+    // of history [B, history_capacity] and its row of embed [V, K] goes to next_hidden [B, K]
+    int *positions;
+    long long *history;
+    int history_capacity;
+    const half_t *embed;
+    half_t *next_hidden;
+    // one row: the kernel multiplies with nrm_weight * rmsnorm(x (+ delta)); nrm_weight null: with x
+    const half_t *delta, *nrm_weight;
+    float eps;
+};
+bool head_argmax_fits(int B, int K, int V);
+int launch_head_argmax(HeadArgs &a, hipStream_t stream);
 int launch_attn_prefill(const half_t *q, const half_t *kc, const half_t *vc, half_t *out, int B, int H, int S, int capacity, int past,
                         float scale, hipStream_t stream);
 int launch_attn_decode(const half_t *q, const half_t *kc, const half_t *vc, const int *positions, half_t *out,

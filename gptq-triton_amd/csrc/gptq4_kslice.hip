@@ -39,7 +39,6 @@
 namespace {
 
 constexpr int BK = 64;
-
 // WIDE (plain epilogue only): two adjacent 64-column blocks per wave tile, like a rotary head.
 // KS: waves of the workgroup, each with its own slice of K (4 or 8).  A wave spends about half of its life
 // waiting (first loads, the exchanges at the end) and the other half issuing ~20 instructions per MFMA, one wave
@@ -54,8 +53,9 @@ constexpr int BK = 64;
 // multiplies packed row 4 * (ks / 2) + 2 * lhi + ks % 2 of the tile.
 template <int EPI, int MT, bool WIDE, int KS, bool PAIRED = false, bool SB = false>
 // (eight waves: one workgroup per CU - all its registers - wherever the wave tile has two column blocks or two row blocks)
-__global__ __launch_bounds__(64 * KS, KS == 8 && (MT == 2 || (EPI != EPI_PLAIN && !PAIRED) || WIDE) ? 1 : 2) void gptq4_kslice_kernel(MatmulArgs p) {
+__global__ __launch_bounds__(64 * KS, MT > 2 || (KS == 8 && (MT == 2 || (EPI != EPI_PLAIN && !PAIRED) || WIDE)) ? 1 : 2) void gptq4_kslice_kernel(MatmulArgs p) {
     static_assert(KS == 4 || KS == 8, "four or eight waves");
+    static_assert(MT <= 2 || KS == 4, "the activation tiles of eight waves of 96 rows do not fit the LDS");
     static_assert(!WIDE || EPI == EPI_PLAIN, "the other epilogues have two blocks already");
     static_assert(!PAIRED || EPI == EPI_ROPE, "paired columns are a rotary head's");
     constexpr bool ADJ = (EPI == EPI_ROPE && !PAIRED) || WIDE;  // the second block is columns + 64 of the same matrix
@@ -618,6 +618,18 @@ int launch_one(const MatmulArgs &a, int tiles, hipStream_t stream) {
     return (int)hipGetLastError();
 }
 
+// 96- and 128-row tiles: four waves, one workgroup per CU
+template <int EPI, int MT>
+int launch_tall(const MatmulArgs &a, const KslicePlan &pl, hipStream_t stream) {
+    if constexpr (EPI == EPI_ROPE) {
+        if (pl.paired) return launch_one<EPI_ROPE, MT, false, 4, true>(a, pl.tiles, stream);
+    }
+    if constexpr (EPI == EPI_PLAIN) {
+        if (pl.wide) return launch_one<EPI_PLAIN, MT, true, 4>(a, pl.tiles, stream);
+    }
+    return launch_one<EPI, MT, false, 4>(a, pl.tiles, stream);
+}
+
 template <int EPI, int KS>
 int launch_waves(const MatmulArgs &a, const KslicePlan &pl, hipStream_t stream) {
     if constexpr (EPI == EPI_ROPE) {
@@ -641,6 +653,8 @@ int launch_waves(const MatmulArgs &a, const KslicePlan &pl, hipStream_t stream) 
 
 template <int EPI>
 int launch_epi(const MatmulArgs &a, const KslicePlan &pl, hipStream_t stream) {
+    if (pl.mt == 3) return launch_tall<EPI, 3>(a, pl, stream);
+    if (pl.mt == 4) return launch_tall<EPI, 4>(a, pl, stream);
     return pl.waves == 8 ? launch_waves<EPI, 8>(a, pl, stream) : launch_waves<EPI, 4>(a, pl, stream);
 }
 
@@ -672,6 +686,7 @@ static KslicePlan plan_variant(int epi, int M, int N, int K, bool has_perm, bool
     const int bn = ((epi == EPI_ROPE && !pl.paired) || pl.wide) ? 128 : 64;
     const int nk = K / 64;
     pl.mt = g_kslice_tuning.mt ? g_kslice_tuning.mt : (M <= 32 ? 1 : 2);
+    if (pl.mt > 2) pl.waves = ks = 4;
     int bm = 32 * pl.mt;
     pl.tiles = ((M + bm - 1) / bm) * (N / bn);
     const long cus = device_shape().cus;  // 256 on MI355X

@@ -562,6 +562,66 @@ PyObject *extend_attention(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
+constexpr size_t HEAD_BYTES = GPTQ4_WS_HEAD_BYTES + (64 << 10);
+
+// the fp16 lm_head weight [V, K] and an embedding of the same shape
+bool is_table(const at::Tensor *w, int64_t k, at::Device dev) { return is_rows(w) && w->dim() == 2 && w->size(1) == k && w->device() == dev; }
+
+// lm_head_argmax(x, weight) -> int64 tokens of x's shape without the last dimension
+PyObject *lm_head_argmax(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    GPTQ4_TAKES(2)
+    Args a{v};
+    const at::Tensor *x = a.need(0), *w = a.need(1);
+    if (!a.fine || !is_rows(x) || x->size(-1) == 0 || !is_table(w, x->size(-1), x->device())) Py_RETURN_NONE;
+    const int64_t k = x->size(-1), b = x->numel() / k;
+    at::Tensor out = empty(x->sizes().slice(0, x->dim() - 1), x->device(), at::kLong);
+    const hipStream_t stream = stream_of(x->device());
+    Workspace ws;
+    if (!workspace(x->device().index(), stream, HEAD_BYTES, &ws)) return nullptr;
+    int rc;
+    {
+        NoGil unlocked;
+        rc = gptq4_lm_head_argmax(data(x), data(w), out.data_ptr<int64_t>(), (int)b, (int)k, (int)w->size(0), ws.data, ws.bytes, stream);
+    }
+    if (rc) return failed(rc, "gptq4_lm_head_argmax");
+    return THPVariable_Wrap(out);
+    END_HANDLE_TH_ERRORS
+}
+
+// greedy_step_end(x, delta, norm weight, eps, lm_head weight, tokens, positions, history, embedding, next hidden) -> True
+PyObject *greedy_step_end(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    GPTQ4_TAKES(10)
+    Args a{v};
+    const at::Tensor *x = a.need(0);
+    Norm norm;
+    norm.delta = a.may(1), norm.weight = a.may(2), norm.eps = (float)a.real(3);
+    const at::Tensor *w = a.need(4), *tokens = a.need(5), *pos = a.need(6), *history = a.need(7), *embed = a.need(8), *next = a.need(9);
+    if (!a.fine || !is_rows(x) || x->size(-1) == 0 || !norm.fits(x)) Py_RETURN_NONE;
+    const at::Device dev = x->device();
+    const int64_t k = x->size(-1), b = x->numel() / k;
+    if (!is_table(w, k, dev) || !is_table(embed, k, dev) || embed->size(0) < w->size(0)) Py_RETURN_NONE;
+    for (const at::Tensor *t : {tokens, pos, history, next, norm.delta, norm.weight})
+        if (!beside(t, dev)) Py_RETURN_NONE;
+    if (tokens->scalar_type() != at::kLong || tokens->numel() != b || pos->scalar_type() != at::kInt || pos->numel() != b ||
+        history->scalar_type() != at::kLong || history->dim() != 2 || history->size(0) != b || !is_rows(next) || next->numel() != b * k)
+        Py_RETURN_NONE;
+    const hipStream_t stream = stream_of(dev);
+    Workspace ws;
+    if (!workspace(dev.index(), stream, HEAD_BYTES, &ws)) return nullptr;
+    int rc;
+    {
+        NoGil unlocked;
+        rc = gptq4_greedy_step_end(data(x), data(norm.delta), data(norm.weight), norm.eps, data(w), (int)b, (int)k, (int)w->size(0),
+                                   tokens->data_ptr<int64_t>(), pos->data_ptr<int32_t>(), history->data_ptr<int64_t>(), (int)history->size(1),
+                                   data(embed), data(next), ws.data, ws.bytes, stream);
+    }
+    if (rc) return failed(rc, "gptq4_greedy_step_end");
+    Py_RETURN_TRUE;
+    END_HANDLE_TH_ERRORS
+}
+
 // set_workspace(device index, stream handle, address, bytes): what _lib.workspace() made for that stream
 PyObject *set_workspace(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
     GPTQ4_TAKES(4)
@@ -603,6 +663,8 @@ PyMethodDef g_methods[] = {GPTQ4_METHOD(init),
                            GPTQ4_METHOD(prefill_attention),
                            GPTQ4_METHOD(decode_attention),
                            GPTQ4_METHOD(extend_attention),
+                           GPTQ4_METHOD(lm_head_argmax),
+                           GPTQ4_METHOD(greedy_step_end),
                            {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_host", "The package's calls of libgptq4 on torch tensors.", -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -94,27 +94,37 @@ def add_rms_norm(x: torch.Tensor, delta: torch.Tensor, weight: torch.Tensor, eps
     return add_rms_norm(x.contiguous(), delta.contiguous(), weight.contiguous(), eps, out_index)
 
 
-HEAD_ARGMAX_K = (4096, 5120, 6656, 8192)  # row lengths gptq4_lm_head_argmax is built for
+HEAD_MAX_ROWS = 16
 
 
-def lm_head_argmax(x: torch.Tensor, weight: torch.Tensor, max_rows: int = 4) -> torch.Tensor:
+def head_argmax_takes(rows: int, weight: torch.Tensor) -> bool:
+    """Whether the lm_head kernels take this many rows of an fp16 weight [V, K]."""
+    k = weight.shape[1]
+    return weight.is_cuda and weight.dtype == torch.float16 and weight.is_contiguous() and k % 256 == 0 and 0 < rows <= HEAD_MAX_ROWS \
+        and rows * (k + 8) * 2 <= 160 * 1024 - 2048 and weight.numel() * 2 < 0x7FFFFFF0
+
+
+def lm_head_argmax(x: torch.Tensor, weight: torch.Tensor, max_rows: int = HEAD_MAX_ROWS) -> torch.Tensor:
     """Greedy next tokens: argmax(x @ weight.T, -1) in one launch, for x fp16 [..., K] and an fp16 lm_head weight [V, K].
-    Returns int64 of x's shape without the last dimension.  The kernel takes up to 16 rows but pays up to `max_rows`
-    (one row of 4096: 52 us against 77 for the library's GEMV + argmax; eight rows: 97 against 83); more rows, and shapes
-    it is not built for, go through torch."""
+    Returns int64 of x's shape without the last dimension.  More than `max_rows` rows, and shapes the kernel does not take
+    (head_argmax_takes), go through torch."""
     k = x.shape[-1]
     rows = x.numel() // max(k, 1)
-    if not (x.is_cuda and x.dtype == torch.float16 and weight.dtype == torch.float16 and weight.is_contiguous() and weight.dim() == 2
-            and weight.shape[1] == k and k in HEAD_ARGMAX_K and 0 < rows <= min(max_rows, 16) and rows * k * 2 <= 160 * 1024 - 2048
-            and weight.numel() * 2 < 0x7FFFFFF0):
+    if rows > max_rows or weight.dim() != 2 or weight.shape[1] != k or not x.is_cuda or x.dtype != torch.float16 or not head_argmax_takes(rows, weight):
         return torch.nn.functional.linear(x, weight).argmax(-1)
-    xc = x.reshape(rows, k).contiguous()
-    out = torch.empty(rows, dtype=torch.int64, device=x.device)
-    ws = _lib.workspace(x.device, _lib.WS_HEAD_BYTES + (64 << 10))
-    rc = _lib.load().gptq4_lm_head_argmax(xc.data_ptr(), weight.data_ptr(), out.data_ptr(), rows, k, weight.shape[0], ws.data_ptr(), ws.numel(),
-                                          _lib.current_stream(x.device))
-    _lib.check(rc, "gptq4_lm_head_argmax")
-    return out.view(x.shape[:-1])
+    out = _lib.host().lm_head_argmax(x.contiguous(), weight)
+    if out is None:
+        raise _lib.refused("lm_head_argmax")
+    return out
+
+
+def greedy_step_end(x, delta, norm_weight, eps, weight, tokens, positions, history, embed, next_hidden) -> None:
+    """The end of a greedy decode step in one launch: tokens (int64) become the argmax of the logits, positions (int32) go up by
+    one, the tokens are stored at those places of history (int64 [B, capacity]) and their rows of the embedding in next_hidden.
+    norm_weight None: x is what the lm_head reads; else (one row) x is the residual stream and the logits are those of
+    RMSNorm(x + delta) * norm_weight, as add_rms_norm gives it."""
+    if _lib.host().greedy_step_end(x, delta, norm_weight, eps, weight, tokens, positions, history, embed, next_hidden) is None:
+        raise _lib.refused("greedy_step_end")
 
 
 def prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, past: int = 0) -> torch.Tensor:

@@ -18,8 +18,9 @@ import torch
 import torch.nn as nn
 
 from . import _lib
-from .decoder_ops import add_rms_norm, decode_attention, lm_head_argmax, norm_fusion_pays, rms_norm
-from .fused_attention import LlamaConfigLite, QuantLlamaAttention
+from .decoder_ops import (NORM_MAX_HIDDEN, add_rms_norm, decode_attention, greedy_step_end, head_argmax_takes, lm_head_argmax,
+                          norm_fusion_pays, prefill_attention, rms_norm)
+from .fused_attention import KV_AT_POSITION, LlamaConfigLite, QuantLlamaAttention
 from .fused_mlp import llama_mlp_4_stream
 from .quant_linear import QuantLinear, stream_rows, tensor_key
 
@@ -262,16 +263,25 @@ class GreedyDecoder:
                        for _ in model.model.layers]
         self.tokens = torch.zeros((bsz, 1), dtype=torch.long, device=dev)
         self.position = torch.zeros((bsz, 1), dtype=torch.int32, device=dev)
+        # with one_launch_end a decode step ends in one launch that picks the tokens, moves the positions on, keeps the tokens at
+        # their places in the sequence and fetches their embedding rows for the next step
+        head, embed = model.lm_head.weight, model.model.embed_tokens.weight
+        self.one_launch_end = head_argmax_takes(bsz, head) and embed.is_cuda and embed.dtype == torch.float16 and embed.is_contiguous() \
+            and embed.shape[0] >= head.shape[0] and model.lm_head.bias is None
+        self.history = torch.zeros((bsz, capacity + 1), dtype=torch.long, device=dev)
+        self.hidden = torch.zeros((bsz, 1, cfg.hidden_size), dtype=torch.float16, device=dev)
+        self._at = None  # (version of the position tensor, the one position of every sequence) as this object left it
         self.graph = None
 
-    def _layers(self, h, position_ids, kv_offset, attend):
-        """The decoder stack on hidden states h [B, S, hidden]; every residual add is fused
-        with the RMSNorm that follows it.  Returns the greedy next token [B, 1]."""
+    def _layers(self, h, position_ids, kv_offset, attend, end):
+        """The decoder stack on hidden states h [B, S, hidden]; every residual add is fused with the RMSNorm that follows it.
+        Returns end(residual stream, its last addend, norm, None), or end(None, None, norm, normed hidden states) where the
+        final norm has run: the greedy next tokens, for a decode step in place."""
         layers = self.model.model.layers
         rows = h.shape[0] * h.shape[1]
         if all(getattr(l.self_attn, "norm_fusable", lambda r: False)(rows) and getattr(l.mlp, "norm_fusable", lambda r: False)(rows)
                for l in layers):
-            return self._layers_norm_in_matmul(h, position_ids, kv_offset, attend)
+            return self._layers_norm_in_matmul(h, position_ids, kv_offset, attend, end)
         # act-order and a handful of rows: every norm writes in the order its consumer's sorted rows read, so the
         # consumer needs no gather launch (tall inputs leave the gather to the consumer: there the norm's
         # scattered 2-byte stores would cost more than the copy)
@@ -294,9 +304,9 @@ class GreedyDecoder:
             oq = None if last else order_of(layers[i + 1].self_attn)
             y = layer.mlp(x, ordered=True) if om is not None else layer.mlp(x)
             h, x = add_rms_norm(h, y, norm.weight, norm.variance_epsilon, out_index=oq)
-        return lm_head_argmax(x[:, -1:, :], self.model.lm_head.weight)
+        return end(None, None, norm, x)
 
-    def _layers_norm_in_matmul(self, h, position_ids, kv_offset, attend):
+    def _layers_norm_in_matmul(self, h, position_ids, kv_offset, attend, end):
         """The same stack for a handful of rows: the QKV and the gate/up launch each do the residual
         add and the RMSNorm of their own input (same bits as _layers' separate launches), so a
         layer is 5 launches instead of 7."""
@@ -307,9 +317,30 @@ class GreedyDecoder:
             q, _, _, h = attn.project_qkv(h, position_ids, kv_out=(kc, vc), kv_offset=kv_offset,
                                           norm=(delta, n1.weight, n1.variance_epsilon))
             h, delta = layer.mlp.forward_normed(h, attn.project_out(*attend(q, kc, vc, attn)), n2.weight, n2.variance_epsilon)
-        norm = self.model.model.norm
-        h, x = add_rms_norm(h, delta, norm.weight, norm.variance_epsilon)
+        return end(h, delta, self.model.model.norm, None)
+
+    def _last_tokens(self, h, delta, norm, x):
+        """Greedy tokens behind the last position [B, 1]."""
+        if x is None:
+            _, x = add_rms_norm(h, delta, norm.weight, norm.variance_epsilon)
         return lm_head_argmax(x[:, -1:, :], self.model.lm_head.weight)
+
+    def _end_step(self, h, delta, norm, x):
+        """The end of a decode step: tokens and position move on, in place."""
+        model = self.model
+        if not self.one_launch_end:
+            self.tokens.copy_(self._last_tokens(h, delta, norm, x))
+            self.position.add_(1)
+            return
+        w = norm.weight
+        if x is None and self.bsz == 1 and w.numel() <= NORM_MAX_HIDDEN:
+            x = h  # (the launch normalises its row itself)
+        else:
+            if x is None:
+                _, x = add_rms_norm(h, delta, w, norm.variance_epsilon)
+            delta = w = None
+        greedy_step_end(x, delta, w, norm.variance_epsilon, model.lm_head.weight, self.tokens, self.position, self.history,
+                        model.model.embed_tokens.weight, self.hidden)
 
     @torch.no_grad()
     def prefill(self, input_ids: torch.Tensor) -> torch.Tensor:
@@ -319,52 +350,74 @@ class GreedyDecoder:
             raise ValueError("prompt does not fit this decoder's batch size / capacity")
         dev = input_ids.device
         position_ids = torch.arange(prompt, device=dev, dtype=torch.int32).unsqueeze(0).expand(bsz, prompt).contiguous()
-        from .decoder_ops import prefill_attention
-
         def attend(q, kc, vc, attn):
             # the prompt's K and V are in cache rows 0 .. prompt - 1 already; the result comes in o_proj's input layout
             return prefill_attention(q, kc, vc, 0), False
 
-        nxt = self._layers(self.model.model.embed_tokens(input_ids), position_ids, 0, attend)
+        nxt = self._layers(self.model.model.embed_tokens(input_ids), position_ids, 0, attend, self._last_tokens)
         self.tokens.copy_(nxt)
         self.position.fill_(prompt)
+        self._moved_to(prompt)
         return nxt
 
     def _step(self):
-        """One decode token from the static buffers: reads tokens/position, writes them back."""
-        from .fused_attention import KV_AT_POSITION
+        """One decode token from the static buffers: reads tokens (or their embedding rows) and position, writes them back."""
 
         def attend(q, kc, vc, attn):  # rows 0..position of the cache; act-order o_proj: written in the order it reads
             order = attn.context_order()
             return decode_attention(q, kc, vc, self.position, out_index=order), order is not None
 
-        nxt = self._layers(self.model.model.embed_tokens(self.tokens), self.position, KV_AT_POSITION, attend)
-        self.tokens.copy_(nxt)
-        self.position.add_(1)
+        self._layers(self.hidden if self.one_launch_end else self.model.model.embed_tokens(self.tokens), self.position, KV_AT_POSITION,
+                     attend, self._end_step)
 
     @torch.no_grad()
     def decode(self, steps: int, use_graph: bool = False) -> torch.Tensor:
         """`steps` more greedy tokens after prefill -> [B, steps]."""
-        out = torch.empty((self.bsz, steps), dtype=torch.long, device=self.tokens.device)
-        if int(self.position.max()) + steps > self.capacity:
+        # where the sequences stand: known if this object moved them there, else (someone wrote to `position`) read back
+        at = self._known_position()
+        if (int(self.position.max()) if at is None else at) + steps > self.capacity:
             raise ValueError("decode would run past the cache capacity")
+        if self.one_launch_end:
+            self.hidden.copy_(self.model.model.embed_tokens(self.tokens))
         if use_graph and self.graph is None and steps > 0:
             self._capture()
+        # the tokens are at their places in `history` afterwards; where the positions are not known on the host, or the step
+        # does not keep them there, they are collected one by one
+        kept = self.one_launch_end and at is not None
+        out = None if kept else torch.empty((self.bsz, steps), dtype=torch.long, device=self.tokens.device)
         for i in range(steps):
             if use_graph:
                 self.graph.replay()
             else:
                 self._step()
-            out[:, i:i + 1].copy_(self.tokens)
+            if not kept:
+                out[:, i:i + 1].copy_(self.tokens)
+        self._moved_to(None if at is None else at + steps)
+        if kept:
+            out = self.history[:, at + 1:at + 1 + steps].clone()
         # one 4-byte read per workspace: a bounded wait of the small-M kernels that ran out would have made tokens wrong silently
         _lib.check_exchange_errors()
         return out
+
+    def _refetch(self, at):
+        """The embedding rows and the host's idea of the position for tokens and positions that were put back."""
+        if self.one_launch_end:
+            self.hidden.copy_(self.model.model.embed_tokens(self.tokens))
+        self._moved_to(at)
+
+    def _moved_to(self, at) -> None:
+        # (tensors made in inference mode have no version: their positions are read back)
+        self._at = None if at is None or self.position.is_inference() else (self.position._version, at)
+
+    def _known_position(self):
+        return self._at[1] if self._at is not None and self._at[0] == self.position._version else None
 
     def _capture(self):
         """Capture _step as a graph.  The warm-up steps run on the capture stream first, so
         workspaces and tables exist before capture; their effect on tokens, position and the
         cache rows they wrote is undone (the rows lie beyond the current position and are
         rewritten before any later step attends to them)."""
+        at = self._known_position()
         tokens0, position0 = self.tokens.clone(), self.position.clone()
         side = torch.cuda.Stream(device=self.tokens.device)
         side.wait_stream(torch.cuda.current_stream())
@@ -372,6 +425,7 @@ class GreedyDecoder:
             self._step()
             self.tokens.copy_(tokens0)
             self.position.copy_(position0)
+            self._refetch(at)
         torch.cuda.current_stream().wait_stream(side)
         torch.cuda.synchronize()
         self.graph = torch.cuda.CUDAGraph()
@@ -379,4 +433,5 @@ class GreedyDecoder:
             self._step()
         self.tokens.copy_(tokens0)
         self.position.copy_(position0)
+        self._refetch(at)
         torch.cuda.synchronize()

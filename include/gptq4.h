@@ -234,13 +234,24 @@ int gptq4_extend_attention(const void *q, const void *past_k, const void *past_v
 
 /* The end of a greedy decode step in one launch: out[b] = argmax over v of fp16(x[b] . weight[v]) - the fp16 lm_head
  * (weight fp16 [V, K], row-major as nn.Linear keeps it; no bias) and the argmax of its output, the lowest index among
- * equal logits.  x fp16 [B, K], B <= 16; out int64 [B]; K one of 4096, 5120, 6656, 8192 (else -GPTQ4_E_SHAPE: use a
- * dense GEMV and an argmax).  workspace: the zeroed head + 32 KiB behind it (gptq4_workspace_bytes of any operator
+ * equal logits.  x fp16 [B, K], B <= 16; out int64 [B]; K a multiple of 256 whose B rows fit the LDS (B * (K + 8) * 2 <=
+ * 161792 bytes) and V * K * 2 < 2^31 - 16 (else -GPTQ4_E_SHAPE: use a dense GEMV and an argmax).  workspace: the zeroed head + 32 KiB behind it (gptq4_workspace_bytes of any operator
  * covers it).  The sums are fp32 and rounded to fp16 once, so a logit can differ from a library GEMV's by an fp16
  * ulp and the index with it where two logits are that close.  Replaces `model.lm_head(h).argmax(-1)` of a greedy
  * decoding loop (the reference's generate.py leaves both to transformers). */
 int gptq4_lm_head_argmax(const void *x, const void *weight, int64_t *out, int B, int K, int V, void *workspace,
                          size_t workspace_bytes, void *stream);
+
+/* The same launch also moves a decoding loop on to its next step: tokens[b] = the argmax; positions[b] (int32) goes up by
+ * one, tokens[b] is stored at that place of history int64 [B, history_capacity] (if it has room), and its row of the
+ * embedding embed fp16 [V, K] is copied to next_hidden fp16 [B, K], which may not be x or delta.  With norm_weight fp16
+ * [K] (B == 1, K <= 8192) x is the residual stream and the logits are those of
+ * norm_weight * rmsnorm(x + delta) (delta nullable), the same bits as gptq4_add_rmsnorm / gptq4_rmsnorm and
+ * gptq4_lm_head_argmax one after the other.  No reference counterpart (transformers' generate loop there). */
+int gptq4_greedy_step_end(const void *x, const void *delta, const void *norm_weight, float eps,
+                          const void *weight, int B, int K, int V, int64_t *tokens, int32_t *positions,
+                          int64_t *history, int history_capacity, const void *embed,
+                          void *next_hidden, void *workspace, size_t workspace_bytes, void *stream);
 
 /* Causal attention of S query tokens per sequence (a prompt, or a chunk of one behind `past` cached tokens): query i
  * attends to cache rows 0 .. past + i; softmax in fp32, output fp16 out [B, S, H*D] - the layout o_proj consumes, no

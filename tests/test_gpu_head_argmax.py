@@ -64,3 +64,43 @@ def test_other_shapes_go_through_torch():
     assert lib.gptq4_lm_head_argmax(fake, fake, fake, 17, 4096, 32000, fake, _lib.WS_HEAD_BYTES + (64 << 10), None) == -2
     assert lib.gptq4_lm_head_argmax(fake, fake, fake, 1, 4096, 32000, fake, 64, None) == -4
     assert lib.gptq4_lm_head_argmax(None, fake, fake, 1, 4096, 32000, fake, _lib.WS_HEAD_BYTES + (64 << 10), None) == -1
+
+
+@pytest.mark.parametrize("b,k,v", [(1, 256, 16), (5, 1280, 333), (1, 7680, 2001), (16, 4864, 257), (9, 2048, 50257)])
+def test_any_multiple_of_256(b, k, v):
+    """Row lengths and vocabularies of no particular size, against torch on the same tensors: logits are fp32 sums rounded to
+    fp16 on both sides, so the chosen logit is within two fp16 ulps of the largest."""
+    gen = torch.Generator(device="cuda").manual_seed(b * k + v)
+    x = torch.randn((b, k), device="cuda", generator=gen).half()
+    w = (0.02 * torch.randn((v, k), device="cuda", generator=gen)).half()
+    out = ops().lm_head_argmax(x, w)
+    logits = x.double() @ w.double().t()
+    top = logits.max(1).values
+    got = logits.gather(1, out[:, None])[:, 0]
+    assert ((top - got) <= 2 * 2.0 ** -10 * top.abs()).all(), (top - got).max()
+    assert head_is_zero()
+
+
+@pytest.mark.parametrize("b,k,norm", [(1, 1024, "add"), (1, 8192, "plain"), (1, 1280, None), (6, 4096, None)])
+def test_step_end_moves_the_loop_on(b, k, norm):
+    """One launch = the norm launch, the argmax launch and the bookkeeping of a greedy loop, bit for bit."""
+    gen = torch.Generator(device="cuda").manual_seed(k + b)
+    new = lambda *s: torch.randn(s, device="cuda", generator=gen).half()
+    v, cap = 1003, 9
+    x, delta, nw = new(b, 1, k), new(b, 1, k), (1 + 0.1 * new(k)).half()
+    w, embed = (0.02 * new(v, k)).half(), new(v, k)
+    tokens = torch.zeros((b, 1), dtype=torch.int64, device="cuda")
+    pos = torch.arange(b, dtype=torch.int32, device="cuda")[:, None].contiguous() + 3
+    history = torch.full((b, cap), -1, dtype=torch.int64, device="cuda")
+    hidden = torch.zeros((b, 1, k), dtype=torch.float16, device="cuda")
+    normed = x if norm is None else ops().add_rms_norm(x, delta, nw, 1e-6)[1] if norm == "add" else ops().rms_norm(x, nw, 1e-6)
+    want = ops().lm_head_argmax(normed, w)
+    ops().greedy_step_end(x, delta if norm == "add" else None, None if norm is None else nw, 1e-6, w, tokens, pos, history, embed, hidden)
+    assert torch.equal(tokens, want)
+    assert pos[:, 0].tolist() == [4 + i for i in range(b)]
+    assert torch.equal(hidden[:, 0], embed[want[:, 0]])
+    expect = torch.full_like(history, -1)
+    for i in range(b):
+        if 4 + i < cap:   # (a place past the end is not written)
+            expect[i, 4 + i] = want[i, 0]
+    assert torch.equal(history, expect) and head_is_zero()
