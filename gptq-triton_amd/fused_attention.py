@@ -278,7 +278,7 @@ class QuantLlamaAttention(nn.Module):
             self._input_order = (tensor_key(perm), inverse_permutation(perm))
         return self._input_order[1]
 
-    def attend_one(self, hidden_states: torch.Tensor, position_ids: torch.Tensor, past_key_value, norm=None):
+    def attend_one(self, hidden_states: torch.Tensor, position_ids: torch.Tensor, past_key_value, norm=None, ordered: bool = False):
         """One token of each sequence behind a (key, value) pair (or None): (the arguments of project_out, the grown pair), and
         with norm (see project_qkv) also the residual stream.  Two launches: the QKV projection stores its K and V as the
         new pair's last row, the attention kernel copies the other rows while it attends to them."""
@@ -287,7 +287,7 @@ class QuantLlamaAttention(nn.Module):
         shape = (hidden_states.shape[0], self.num_heads, past + 1, self.head_dim)
         pair = (torch.empty(shape, dtype=torch.float16, device=hidden_states.device),
                 torch.empty(shape, dtype=torch.float16, device=hidden_states.device))
-        q, _, _, *stream = self.project_qkv(hidden_states, position_ids, kv_out=pair, kv_offset=past, norm=norm)
+        q, _, _, *stream = self.project_qkv(hidden_states, position_ids, kv_out=pair, kv_offset=past, norm=norm, ordered=ordered)
         order = self.context_order()
         context = extend_attention(q, past_k, past_v, *pair, out_index=order), order is not None
         return (context, pair, stream[0]) if norm is not None else (context, pair)
@@ -311,6 +311,7 @@ class QuantLlamaAttention(nn.Module):
         past_key_values=None,
         position_embeddings=None,
         causal: bool = False,
+        ordered: bool = False,
         **kwargs,
     ) -> Tuple[torch.Tensor, Optional[torch.Tensor], Optional[Tuple[torch.Tensor]]]:
         """Input shape: Batch x Time x Channel.
@@ -323,11 +324,13 @@ class QuantLlamaAttention(nn.Module):
 
         causal (not in the reference, whose callers hand over an additive mask): with no attention_mask, query i attends to
         the past and to the new tokens up to itself - the prompt pass of this package's own decoder, which runs on the
-        library's attention kernel instead of a materialised mask."""
+        library's attention kernel instead of a materialised mask.
+
+        ordered (act-order): hidden_states already are in the order of input_order()."""
         if past_key_values is not None or position_embeddings is not None:
             return self._forward_with_cache(hidden_states, attention_mask, position_ids, past_key_values,
                                             output_attentions or bool(kwargs.get('output_attentions', False)),
-                                            kwargs.get('cache_position'))
+                                            kwargs.get('cache_position'), ordered)
         bsz, q_len, _ = hidden_states.size()
         past_len = 0 if past_key_value is None else past_key_value[0].shape[-2]
         kv_seq_len = past_len + q_len
@@ -337,10 +340,10 @@ class QuantLlamaAttention(nn.Module):
 
         if q_len == 1 and attention_mask is None and not output_attentions and self.head_dim == 128 and hidden_states.is_cuda \
                 and bsz * self.num_heads <= ATTENTION_MAX_HEADS:
-            context, pair = self.attend_one(hidden_states, position_ids, past_key_value)
+            context, pair = self.attend_one(hidden_states, position_ids, past_key_value, ordered=ordered)
             return self.project_out(*context), None, pair if use_cache else None
         if past_key_value is None:
-            query_states, key_states, value_states = self.project_qkv(hidden_states, position_ids)
+            query_states, key_states, value_states = self.project_qkv(hidden_states, position_ids, ordered=ordered)
         else:
             # new K/V rows are written by the kernel behind the copied past: no separate cat
             shape = (bsz, self.num_heads, kv_seq_len, self.head_dim)
@@ -349,7 +352,7 @@ class QuantLlamaAttention(nn.Module):
             key_states[:, :, :past_len].copy_(past_key_value[0])
             value_states[:, :, :past_len].copy_(past_key_value[1])
             query_states, _, _ = self.project_qkv(hidden_states, position_ids,
-                                                  kv_out=(key_states, value_states), kv_offset=past_len)
+                                                  kv_out=(key_states, value_states), kv_offset=past_len, ordered=ordered)
         past_key_value = (key_states, value_states) if use_cache else None
 
         if attention_mask is not None and attention_mask.size() != (bsz, 1, q_len, kv_seq_len):
@@ -389,7 +392,7 @@ class QuantLlamaAttention(nn.Module):
         return attn_output, attn_weights, past_key_value
 
 
-def _forward_with_cache(self, hidden_states, attention_mask, position_ids, cache, output_attentions, cache_position):
+def _forward_with_cache(self, hidden_states, attention_mask, position_ids, cache, output_attentions, cache_position, ordered=False):
     """The call of a current transformers decoder layer (see QuantLlamaAttention.forward)."""
     bsz, q_len, _ = hidden_states.size()
     if position_ids is None:
@@ -404,7 +407,7 @@ def _forward_with_cache(self, hidden_states, attention_mask, position_ids, cache
         raise ValueError("this attention block does not know its layer index and cannot update a Cache")
     # tokens the cache holds before this call; read only when no mask says what to attend to
     past = int(cache.get_seq_length(self.layer_idx)) if cache is not None and attention_mask is None else 0
-    query_states, key_states, value_states = self.project_qkv(hidden_states, position_ids.contiguous())
+    query_states, key_states, value_states = self.project_qkv(hidden_states, position_ids.contiguous(), ordered=ordered)
     if cache is not None:
         key_states, value_states = cache.update(key_states, value_states, self.layer_idx)
     kv_len = key_states.shape[-2]

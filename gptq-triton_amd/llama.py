@@ -24,8 +24,6 @@ from .fused_attention import KV_AT_POSITION, LlamaConfigLite, QuantLlamaAttentio
 from .fused_mlp import llama_mlp_4_stream
 from .quant_linear import QuantLinear, stream_rows, tensor_key
 
-# up to this many rows the decoder's norms write act-order inputs in their consumer's order
-ORDERED_NORM_ROWS = 16
 # the rows the decode kernels built on the streaming-order weight layout take (more rows: the mid-M and tiled kernels)
 STREAM_BATCH = 16
 
@@ -214,13 +212,16 @@ class LlamaForCausalLM(nn.Module):
                 context, present, h = attn.attend_one(h, position_ids, past, norm=(delta, n1.weight, n1.variance_epsilon))
                 h, delta = layer.mlp.forward_normed(h, attn.project_out(*context), n2.weight, n2.variance_epsilon)
             else:
+                order = order_of(attn)
                 if delta is None:
-                    x = rms_norm(h, n1.weight, n1.variance_epsilon)
+                    x = rms_norm(h, n1.weight, n1.variance_epsilon, out_index=order)
                 else:
-                    h, x = add_rms_norm(h, delta, n1.weight, n1.variance_epsilon)
-                out, _, present = attn(hidden_states=x, position_ids=position_ids, past_key_value=past, use_cache=use_cache, causal=True)
-                h, x = add_rms_norm(h, out, n2.weight, n2.variance_epsilon)
-                delta = layer.mlp(x)
+                    h, x = add_rms_norm(h, delta, n1.weight, n1.variance_epsilon, out_index=order)
+                out, _, present = attn(hidden_states=x, position_ids=position_ids, past_key_value=past, use_cache=use_cache, causal=True,
+                                       ordered=order is not None)
+                order = order_of(layer.mlp)
+                h, x = add_rms_norm(h, out, n2.weight, n2.variance_epsilon, out_index=order)
+                delta = layer.mlp(x, ordered=True) if order is not None else layer.mlp(x)
             presents.append(present)
         norm = self.model.norm
         return add_rms_norm(h, delta, norm.weight, norm.variance_epsilon)[1], presents
@@ -236,6 +237,12 @@ class LlamaForCausalLM(nn.Module):
         first = dec.prefill(input_ids)
         rest = dec.decode(max_new_tokens - 1, use_graph=use_graph) if max_new_tokens > 1 else first[:, :0]
         return torch.cat([input_ids, first, rest], dim=1)
+
+
+def order_of(block):
+    """Where the norm in front of an act-order block should store each feature (None: no act-order, or gathered by the block)."""
+    fn = getattr(block, "input_order", None)
+    return fn() if fn is not None else None
 
 
 class GreedyDecoder:
@@ -282,13 +289,7 @@ class GreedyDecoder:
         if all(getattr(l.self_attn, "norm_fusable", lambda r: False)(rows) and getattr(l.mlp, "norm_fusable", lambda r: False)(rows)
                for l in layers):
             return self._layers_norm_in_matmul(h, position_ids, kv_offset, attend, end)
-        # act-order and a handful of rows: every norm writes in the order its consumer's sorted rows read, so the
-        # consumer needs no gather launch (tall inputs leave the gather to the consumer: there the norm's
-        # scattered 2-byte stores would cost more than the copy)
-        def order_of(block):
-            fn = getattr(block, "input_order", None)
-            return fn() if fn is not None and rows <= ORDERED_NORM_ROWS else None
-
+        # act-order: every norm writes in the order its consumer's sorted rows read, so the consumer needs no gather launch
         n0 = layers[0].input_layernorm
         oq = order_of(layers[0].self_attn)
         x = rms_norm(h, n0.weight, n0.variance_epsilon, out_index=oq)

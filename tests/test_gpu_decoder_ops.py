@@ -45,7 +45,7 @@ def test_add_rmsnorm(m, h):
     assert torch.equal(y, y2)
 
 
-@pytest.mark.parametrize("m,h", [(1, 4096), (8, 5120), (16, 13824), (40, 6656), (2, 8200)])
+@pytest.mark.parametrize("m,h", [(1, 4096), (8, 5120), (16, 13824), (40, 6656), (2, 8200), (3, 24576), (2, 24584), (1, 8)])
 def test_norms_store_in_a_given_order(m, h):
     """With out_index, value f of every row lands at position out_index[f]: the same bits, moved (rows longer
     than the 8192 values held in registers included); the sum keeps its order."""
