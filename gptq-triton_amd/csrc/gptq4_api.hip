@@ -164,7 +164,7 @@ int setup_norm(MatmulArgs &a, const void *delta, const void *norm_weight, void *
 // 640 rows 110.4 against 123.4.)
 bool prefer_kslice(const KslicePlan &kp, int epi, int M, int N, int K) {
     if (!kp.ok || g_kslice_tuning.mode == 0) return false;
-    if (g_kslice_tuning.mode == 2) return true;
+    if (g_kslice_tuning.mode == 2 || kp.one_round) return true;
     if (M > 768) return false;
     const int wide_bn = (epi == EPI_SILU_MUL) ? 128 : 256;
     const long wide = (long)((M + 127) / 128) * (N / wide_bn);
@@ -250,35 +250,55 @@ TiledChoice choose_part(int epi, int M, int K, const ColumnParts &parts, int i, 
     return choose_tiled(epi, M, parts.cols[i], K, kernel_gathers, allow_streamed);
 }
 
+// A call's whole plan.  Making one weighs up to a hundred launch shapes (5 - 20 us of host time, as much as a small call
+// takes on the GPU), so every thread keeps its last ones: 64 slots by the call's sizes, good for one set of tuning values.
+struct TiledPlan {
+    int epi, M, N, K, cus;
+    bool kernel_gathers, allow_streamed;
+    unsigned generation;  // of the tuning values; 0: an empty slot
+    ColumnParts parts;
+    TiledChoice choice[2];
+    size_t partial;  // the largest partial-sum region of the parts
+};
+unsigned g_tuning_generation = 1;
+
+const TiledPlan &tiled_plan(int epi, int M, int N, int K, bool kernel_gathers, bool allow_streamed) {
+    static thread_local TiledPlan kept[64];
+    const int cus = device_shape().cus;
+    TiledPlan &t = kept[((unsigned)M * 2654435761u ^ (unsigned)N * 40503u ^ (unsigned)K * 97u ^ (unsigned)epi * 7u) >> 7 & 63u];
+    if (t.generation == g_tuning_generation && t.epi == epi && t.M == M && t.N == N && t.K == K && t.cus == cus &&
+        t.kernel_gathers == kernel_gathers && t.allow_streamed == allow_streamed)
+        return t;
+    t = TiledPlan{epi, M, N, K, cus, kernel_gathers, allow_streamed, g_tuning_generation, {}, {}, 0};
+    t.parts = tiled_parts(epi, M, N, K, kernel_gathers);
+    for (int i = 0; i < t.parts.count; ++i) {
+        t.choice[i] = choose_part(epi, M, K, t.parts, i, kernel_gathers, allow_streamed);
+        if (t.choice[i].partial > t.partial) t.partial = t.choice[i].partial;
+    }
+    return t;
+}
+
 int run_tiled(int epi, MatmulArgs &a, void *workspace, size_t workspace_bytes, hipStream_t s) {
     // act-order: staged activations wherever they fit the staging limit and the workspace (then the mid-M
     // kernel can run too); else the tiled kernel gathers by itself
     const size_t rows_bytes = (size_t)a.M * a.K * sizeof(half_t);
     bool stage = a.perm != nullptr && !g_gemm_tuning.own_gather && rows_bytes <= ACT_ORDER_STAGE_MAX;
-    ColumnParts parts;
-    TiledChoice choice[2];
-    size_t partial = 0;
     bool allow_streamed = true;
-    auto plan_all = [&]() {
-        const bool kernel_gathers = a.perm != nullptr && !stage;
-        parts = tiled_parts(epi, a.M, a.N, a.K, kernel_gathers);
-        partial = 0;
-        for (int i = 0; i < parts.count; ++i) {
-            choice[i] = choose_part(epi, a.M, a.K, parts, i, kernel_gathers, allow_streamed);
-            if (choice[i].partial > partial) partial = choice[i].partial;
-        }
-    };
-    plan_all();
+    auto plan_all = [&]() { return tiled_plan(epi, a.M, a.N, a.K, a.perm != nullptr && !stage, allow_streamed); };
+    TiledPlan pl = plan_all();
     // the streamed schedule keeps 128 MiB of partial sums: without the room for them, the unstreamed plan
-    if (parts.count == 1 && !choice[0].kslice && choice[0].gp.streamed &&
-        (workspace == nullptr || workspace_bytes < GPTQ4_WS_HEAD_BYTES + partial + (stage ? rows_bytes : 0))) {
+    if (pl.parts.count == 1 && !pl.choice[0].kslice && pl.choice[0].gp.streamed &&
+        (workspace == nullptr || workspace_bytes < GPTQ4_WS_HEAD_BYTES + pl.partial + (stage ? rows_bytes : 0))) {
         allow_streamed = false;
-        plan_all();
+        pl = plan_all();
     }
-    if (stage && (workspace == nullptr || workspace_bytes < GPTQ4_WS_HEAD_BYTES + partial + rows_bytes)) {
+    if (stage && (workspace == nullptr || workspace_bytes < GPTQ4_WS_HEAD_BYTES + pl.partial + rows_bytes)) {
         stage = false;
-        plan_all();
+        pl = plan_all();
     }
+    const ColumnParts &parts = pl.parts;
+    const TiledChoice *choice = pl.choice;
+    const size_t partial = pl.partial;
     if (partial > 0 && (workspace == nullptr || workspace_bytes < GPTQ4_WS_HEAD_BYTES + partial)) return -GPTQ4_E_WORKSPACE;
     if (stage) {
         // once, behind the largest partial-sum region any part uses
@@ -346,6 +366,7 @@ const char *gptq4_strerror(int code) {
 }
 
 void gptq4_set_gemm_tuning(int mt, int splitk) {
+    ++g_tuning_generation;
     // 100: never the streamed schedule, 200: the streamed schedule wherever it can run (both with automatic tile and split);
     // 300: never two launches over column ranges (automatic otherwise)
     g_gemm_tuning.streamed = (mt == 100) ? 1 : (mt == 200) ? 2 : 0;
@@ -361,6 +382,7 @@ void gptq4_set_gemm_tuning(int mt, int splitk) {
 }
 
 void gptq4_set_midm_tuning(int mode, int mt, int splitk) {
+    ++g_tuning_generation;
     g_kslice_tuning.mode = (mode >= 0 && mode <= 2) ? mode : 1;
     // 1000 + mt: the rotary epilogue on tiles of 32 + 32 paired columns wherever the mid-M kernel runs, 2000 + mt: never
     g_kslice_tuning.paired = (mt >= 2000) ? 2 : (mt >= 1000) ? 1 : 0;
@@ -369,9 +391,9 @@ void gptq4_set_midm_tuning(int mode, int mt, int splitk) {
     g_kslice_tuning.waves = (mt >= 200) ? 8 : (mt >= 100) ? 4 : 0;
     mt %= 100;
     // 10 + mt: 128-column strips for plain projections; a plain 1 or 2 also pins the 64-column strips
-    g_kslice_tuning.wide = (mt >= 10) ? 1 : ((mt >= 1 && mt <= 4) ? -1 : 0);
+    g_kslice_tuning.wide = (mt >= 10) ? 1 : ((mt >= 1 && mt <= 3) ? -1 : 0);
     if (mt >= 10) mt -= 10;
-    g_kslice_tuning.mt = (mt >= 1 && mt <= 4) ? mt : 0;
+    g_kslice_tuning.mt = (mt >= 1 && mt <= 3) ? mt : 0;
     g_kslice_tuning.splitk = splitk > 0 ? splitk : 0;
 }
 
@@ -408,6 +430,20 @@ static size_t workspace_need(int op, int M, int K, int N, bool allow_streamed) {
         size_t need = partial_bytes(SKINNY_MAX_SPLITK, M, cols);
         bytes += need + (with_perm ? (size_t)M * K * 2 : 0);  // + the rows gathered for an act-order call
     } else if ((K % 64) == 0) {
+        // (kept like the plans it is made of)
+        struct Need {
+            int op, M, K, N, cus;
+            bool allow_streamed;
+            unsigned generation;
+            size_t need;
+        };
+        static thread_local Need kept[64];
+        const int cus = device_shape().cus;
+        Need &slot = kept[((unsigned)M * 2654435761u ^ (unsigned)N * 40503u ^ (unsigned)K * 97u ^ (unsigned)op * 7u) >> 7 & 63u];
+        const size_t rows = with_perm && (size_t)M * K * 2 <= ACT_ORDER_STAGE_MAX ? (size_t)M * K * 2 : 0;  // gathered for an act-order call
+        if (slot.generation == g_tuning_generation && slot.op == op && slot.M == M && slot.K == K && slot.N == N && slot.cus == cus &&
+            slot.allow_streamed == allow_streamed)
+            return bytes + slot.need + rows;
         const int epi = (op == GPTQ4_OP_MLP_GATEUP) ? EPI_SILU_MUL : (op == GPTQ4_OP_QKV_ROTARY ? EPI_ROPE : EPI_PLAIN);
         // whichever kernel the current (automatic or forced) plans pick, with or without act-order, for the whole
         // matrix and for each of the column ranges a call may be cut into
@@ -421,9 +457,8 @@ static size_t workspace_need(int op, int M, int K, int N, bool allow_streamed) {
             const KslicePlan pk = kslice_plan(epi, M, parts.cols[i], K, false);
             if (pk.ok && kslice_partial_bytes(epi, pk) > need) need = kslice_partial_bytes(epi, pk);
         }
-        bytes += need;
-        // + the rows gathered for an act-order call
-        if (with_perm && (size_t)M * K * 2 <= ACT_ORDER_STAGE_MAX) bytes += (size_t)M * K * 2;
+        slot = Need{op, M, K, N, cus, allow_streamed, g_tuning_generation, need};
+        bytes += need + rows;
     }
     return bytes;
 }

@@ -132,13 +132,14 @@ int launch_gemm(int epi, const MatmulArgs &a, const GemmPlan &plan, hipStream_t 
 
 // Launch shape of the mid-M kernel (K split across the waves of a workgroup).
 struct KslicePlan {
-    int mt;      // 32-row blocks per row tile (1 or 2)
+    int mt;      // 32-row blocks per row tile (1 to 3)
     int splitk;  // workgroups sharing one tile along K, on top of the split inside the workgroup
     int tiles;
     bool wide;   // plain epilogue: 128-column strips (two blocks per wave tile) instead of 64
     int waves;   // waves per workgroup, each with its own slice of K (4 or 8)
     bool paired; // rotary epilogue: tiles of 32 columns of a head plus their 32 rotation partners instead of whole heads
     bool ok;     // false: the shape needs another kernel
+    bool one_round;  // planned by its estimated time, which also was ahead of the tiled kernel's
     // tail_split > 1 (only with splitk == 1): tiles [0, tail_first) whole, every later one - the last column strips
     // of the launch, all their row tiles - shared by tail_split workgroups along K
     int tail_first, tail_split;

@@ -55,7 +55,7 @@ template <int EPI, int MT, bool WIDE, int KS, bool PAIRED = false, bool SB = fal
 // (eight waves: one workgroup per CU - all its registers - wherever the wave tile has two column blocks or two row blocks)
 __global__ __launch_bounds__(64 * KS, MT > 2 || (KS == 8 && (MT == 2 || (EPI != EPI_PLAIN && !PAIRED) || WIDE)) ? 1 : 2) void gptq4_kslice_kernel(MatmulArgs p) {
     static_assert(KS == 4 || KS == 8, "four or eight waves");
-    static_assert(MT <= 2 || KS == 4, "the activation tiles of eight waves of 96 rows do not fit the LDS");
+    static_assert(MT <= 3 && (MT <= 2 || KS == 4), "the activation tiles of eight waves of 96 rows do not fit the LDS");
     static_assert(!WIDE || EPI == EPI_PLAIN, "the other epilogues have two blocks already");
     static_assert(!PAIRED || EPI == EPI_ROPE, "paired columns are a rotary head's");
     constexpr bool ADJ = (EPI == EPI_ROPE && !PAIRED) || WIDE;  // the second block is columns + 64 of the same matrix
@@ -618,7 +618,7 @@ int launch_one(const MatmulArgs &a, int tiles, hipStream_t stream) {
     return (int)hipGetLastError();
 }
 
-// 96- and 128-row tiles: four waves, one workgroup per CU
+// 96-row tiles: four waves, one workgroup per CU
 template <int EPI, int MT>
 int launch_tall(const MatmulArgs &a, const KslicePlan &pl, hipStream_t stream) {
     if constexpr (EPI == EPI_ROPE) {
@@ -654,7 +654,6 @@ int launch_waves(const MatmulArgs &a, const KslicePlan &pl, hipStream_t stream) 
 template <int EPI>
 int launch_epi(const MatmulArgs &a, const KslicePlan &pl, hipStream_t stream) {
     if (pl.mt == 3) return launch_tall<EPI, 3>(a, pl, stream);
-    if (pl.mt == 4) return launch_tall<EPI, 4>(a, pl, stream);
     return pl.waves == 8 ? launch_waves<EPI, 8>(a, pl, stream) : launch_waves<EPI, 4>(a, pl, stream);
 }
 
@@ -785,8 +784,8 @@ static KslicePlan plan_variant(int epi, int M, int N, int K, bool has_perm, bool
 // many MFMAs per activation fragment (priced at 0.85 of the rate).  Each variant is planned by itself and the better
 // split score wins (never with a larger split than whole heads take).  LLaMA-7B QKV: 15.7 -> 13.0 us at 17 rows, 16.2 -> 13.4 at 32 (16 rows: 12.4), 21.1 -> 16.9 at 64,
 // 42.4 -> 37.0 at 192; 13B 18.7 -> 16.2 at 32, 24.6 -> 20.6 at 64; 30B 60 -> 54 at 96 rows and whole heads below that
-// (312 paired tiles do not fit one round of 256 CUs).
-KslicePlan kslice_plan(int epi, int M, int N, int K, bool has_perm) {
+// (312 paired tiles do not fit one round of 256 CUs).  The plan for launches of more than one round (and for forced shapes).
+static KslicePlan rounds_plan(int epi, int M, int N, int K, bool has_perm) {
     double score = 0.0;
     if (epi != EPI_ROPE || g_kslice_tuning.paired == 2) return plan_variant(epi, M, N, K, has_perm, false, &score);
     if (g_kslice_tuning.paired == 1) return plan_variant(epi, M, N, K, has_perm, true, &score);
@@ -798,6 +797,98 @@ KslicePlan kslice_plan(int epi, int M, int N, int K, bool has_perm) {
     // tiles 87.8)
     const bool few = (long)heads.tiles < 2 * device_shape().cus;
     return (pairs.ok && few && score > 0.0 && pairs.splitk <= heads.splitk && 0.85 * score_p > score + 1e-9) ? pairs : heads;
+}
+
+// ---- launches of at most one round: every workgroup resident at once, so that the time is that of one workgroup:
+//   t0 + steps * (step + load * workgroups / CUs) + exchange
+// with steps = K tiles of the longest wave, `step` that of one workgroup or of two to a CU, `load` what the others' traffic
+// adds to a step, and the cost of splitting K across workgroups (the first split, then every further one).  One line per
+// kernel variant, in us, fitted to 3500 timings over 20 projections (K and N from 2048 to 19968) at 24 to 768 rows with the
+// weights from HBM: 3 - 7 % off per variant.
+struct RoundCost {
+    float t0, one, two, load, split, more;  // two = 0: one workgroup to a CU
+};
+static const RoundCost round_cost[3][2][2] = {
+    // [row tile / 32 - 1][eight waves][two column blocks]
+    {{{4.2f, 0.480f, 0.751f, 0.065f, 1.98f, 0.40f}, {6.1f, 0.665f, 1.265f, 0.178f, 2.59f, 0.67f}},
+     {{4.8f, 0.632f, 1.375f, 0.168f, 1.62f, 0.40f}, {5.7f, 1.327f, 0.f, 0.364f, 3.00f, 0.50f}}},
+    {{{5.2f, 0.579f, 0.890f, 0.215f, 2.22f, 0.43f}, {8.1f, 0.681f, 1.432f, 0.404f, 3.18f, 0.64f}},
+     {{5.6f, 0.823f, 0.f, 0.458f, 1.65f, 0.47f}, {9.1f, 1.210f, 0.f, 0.903f, 1.81f, 0.55f}}},
+    {{{5.0f, 0.760f, 0.f, 0.279f, 2.27f, 0.49f}, {8.2f, 1.024f, 0.f, 0.491f, 3.44f, 0.85f}}, {}}};
+
+// us, or 0 for a launch of more than one round
+static double one_round_estimate(int epi, int K, const KslicePlan &pl, long cus) {
+    const bool two_blocks = !((epi == EPI_PLAIN && !pl.wide) || pl.paired);
+    const RoundCost &c = round_cost[pl.mt - 1][pl.waves == 8][two_blocks];
+    const long wgs = (long)pl.tiles * pl.splitk;
+    if (wgs > (c.two > 0.f ? 2 : 1) * cus) return 0.0;
+    const int steps = ((K / 64 + pl.splitk - 1) / pl.splitk + pl.waves - 1) / pl.waves;
+    return c.t0 + steps * ((wgs <= cus ? c.one : c.two) + c.load * (double)wgs / (double)cus) +
+           (pl.splitk > 1 ? c.split + c.more * (pl.splitk - 2) : 0.0);
+}
+
+// What the tiled kernel takes, whatever plan it chooses (us; fitted to the same timings, 10 % off).
+static double tiled_estimate(int epi, int M, int N, int K) {
+    const double tiles = (double)((M + 127) / 128) * (N / (epi == EPI_SILU_MUL ? 128 : 256)) / device_shape().cus, nk = K / 64;
+    const double t0 = epi == EPI_PLAIN ? 12.9 : epi == EPI_SILU_MUL ? 8.5 : 19.0;
+    const double flat = epi == EPI_PLAIN ? 0.122 : epi == EPI_SILU_MUL ? 0.568 : 0.155;
+    const double knee = epi == EPI_PLAIN ? 0.028 : epi == EPI_SILU_MUL ? 0.44 : 0.078;
+    return t0 + nk * (flat + (tiles > knee ? 0.86 * (tiles - knee) : 0.0));
+}
+
+// The fastest launch of at most one round by that estimate, if it is 5 % ahead of the tiled kernel (ok = false otherwise).
+// 96-row tiles exist for this: one row tile for 65 .. 96 rows, two for 129 .. 192, where 64- and 128-row tiles pad a third
+// to a half, each weight decoded once per 96 rows: LLaMA-7B gate/up at 96 rows 35.3 -> 30.1 us, 13B 47.9 -> 38.2; QKV
+// (plain) at 192 rows 37.2 -> 29.5; 4096 x 4096 at 640 rows 37.7 -> 31.0.  (128-row tiles never were the fastest: with two
+// column blocks they spill, with one they halve the workgroups of 64-row tiles.)
+static KslicePlan one_round_plan(int epi, int M, int N, int K) {
+    KslicePlan best = {};
+    const int cus = device_shape().cus, nk = K / 64;
+    double best_us = 0.95 * tiled_estimate(epi, M, N, K);
+    for (int mt = 1; mt <= 3; ++mt)
+        for (int waves = 4; waves <= 8; waves += 4)
+            for (int form = 0; form < (epi == EPI_SILU_MUL ? 1 : 2); ++form) {
+                KslicePlan pl = {};
+                pl.mt = mt;
+                pl.waves = waves;
+                pl.wide = epi == EPI_PLAIN && form == 1;
+                pl.paired = epi == EPI_ROPE && form == 1;
+                pl.tail_split = 1;
+                pl.ok = pl.one_round = true;
+                const int bn = (pl.wide || (epi == EPI_ROPE && !pl.paired)) ? 128 : 64;
+                // (variants that are not built: the activation tiles do not fit, or were never the faster ones)
+                if ((N % bn) != 0 || (waves == 8 && (mt == 3 || (mt == 1 && pl.wide)))) continue;
+                pl.tiles = ((M + 32 * mt - 1) / (32 * mt)) * (N / bn);
+                for (pl.splitk = 1; pl.splitk <= 8; ++pl.splitk) {
+                    // (two K tiles a wave at least; below a quarter of the CUs the estimate was not fitted)
+                    if (nk / pl.splitk < 2 * waves) break;
+                    const double us = one_round_estimate(epi, K, pl, cus);
+                    if (us <= 0.0) break;
+                    if (4L * pl.tiles * pl.splitk < cus) continue;
+                    if (us < best_us) {
+                        best_us = us;
+                        best = pl;
+                    }
+                }
+            }
+    return best;
+}
+
+KslicePlan kslice_plan(int epi, int M, int N, int K, bool has_perm) {
+    const KsliceTuning &t = g_kslice_tuning;
+    KslicePlan pl = rounds_plan(epi, M, N, K, has_perm);
+    if (t.mode != 1 || t.mt != 0 || t.splitk != 0 || t.wide != 0 || t.waves != 0 || t.paired != 0 || has_perm) return pl;
+    const KslicePlan one = one_round_plan(epi, M, N, K);
+    if (!one.ok) return pl;
+    // the plan by scores stays where the estimates do not tell the two apart; with its last strips shared along K it takes
+    // some 6 % less than the estimate for whole tiles
+    const int cus = device_shape().cus;
+    const double us = (pl.ok ? one_round_estimate(epi, K, pl, cus) : 0.0) * (pl.tail_split > 1 ? 0.94 : 1.0);
+    if (us > 0.0 && us <= 1.07 * one_round_estimate(epi, K, one, cus)) {
+        pl.one_round = true;
+        return pl;
+    }
+    return one;
 }
 
 size_t kslice_partial_bytes(int epi, const KslicePlan &pl) {

@@ -22,7 +22,7 @@ from .decoder_ops import (NORM_MAX_HIDDEN, add_rms_norm, decode_attention, greed
                           norm_fusion_pays, prefill_attention, rms_norm)
 from .fused_attention import KV_AT_POSITION, LlamaConfigLite, QuantLlamaAttention
 from .fused_mlp import llama_mlp_4_stream
-from .quant_linear import QuantLinear, stream_rows, tensor_key
+from .quant_linear import QuantLinear, inverse_permutation, stream_rows, tensor_key
 
 # the rows the decode kernels built on the streaming-order weight layout take (more rows: the mid-M and tiled kernels)
 STREAM_BATCH = 16
@@ -90,28 +90,39 @@ class LlamaMLP(nn.Module):
         if g is None or u is None or gate.groupsize != up.groupsize or g[0].shape != u[0].shape \
                 or gate.bias_tensor() is not None or up.bias_tensor() is not None or rows <= 16 and self._pair_rows(gate) < rows:
             return None
-        if (g[2] is None) != (u[2] is None):
+        if (g[2] is None) != (u[2] is None) or g[2] is not None and self._shared_order(g[2], u[2]) is None:
             return None
-        if g[2] is not None:
-            key = tensor_key(g[2], u[2])
-            if self._same_rows is None or self._same_rows[0] != key:
-                self._same_rows = (key, torch.equal(g[2], u[2]))  # (once: the only synchronisation here)
-            if not self._same_rows[1]:
-                return None
         return gate.groupsize, g[0], g[1], u[0], u[1], g[2]
+
+    def _shared_order(self, perm, other):
+        """The inverse of the row permutation of gate and up where it is one, else None.  (Compared once per pair of
+        permutations: the only synchronisation here.)"""
+        key = tensor_key(perm, other)
+        if self._same_rows is None or self._same_rows[0] != key:
+            self._same_rows = (key, inverse_permutation(perm) if torch.equal(perm, other) else None)
+        return self._same_rows[1]
+
+    def input_order(self):
+        """As QuantLlamaMLP.input_order: None without act-order, or where gate and up each have an order of their own."""
+        gate, up = self._modules['gate_proj'], self._modules['up_proj']
+        if not (isinstance(gate, QuantLinear) and isinstance(up, QuantLinear)) or gate.g_idx is None or up.g_idx is None:
+            return None
+        return self._shared_order(gate.row_permutation(), up.row_permutation())
 
     def _pair_rows(self, gate) -> int:
         if self._most_rows is None:
             self._most_rows = stream_rows(_lib.OP_MLP_GATEUP, gate.infeatures, gate.outfeatures, gate.groupsize)
         return self._most_rows
 
-    def forward(self, x):
+    def forward(self, x, ordered: bool = False):
         # without make_fused_mlp the three projections stay modules of their own; on the GPU gate and up still are one
         # launch, with SiLU and the product on the fp32 sums (two launches and two elementwise ones otherwise)
         pair = self._pair(x.numel() // max(x.shape[-1], 1)) if x.is_cuda else None
         if pair is not None:
             groupsize, gw, gm, uw, um, perm = pair
-            return self._modules['down_proj'](llama_mlp_4_stream(groupsize, x, gw, gm, uw, um, perm))
+            return self._modules['down_proj'](llama_mlp_4_stream(groupsize, x, gw, gm, uw, um, None if ordered else perm))
+        if ordered:
+            return self.down_proj(torch.nn.functional.silu(self.gate_proj.multiply(x, ordered=True)) * self.up_proj.multiply(x, ordered=True))
         return self.down_proj(torch.nn.functional.silu(self.gate_proj(x)) * self.up_proj(x))
 
     def norm_fusable(self, rows: int) -> bool:

@@ -40,6 +40,7 @@ enum gptq4_midm_shape {
     GPTQ4_MIDM_AUTO = 0,
     GPTQ4_MIDM_ROWS_32 = 1,
     GPTQ4_MIDM_ROWS_64 = 2,
+    GPTQ4_MIDM_ROWS_96 = 3, /* four waves */
     GPTQ4_MIDM_WIDE_STRIPS = 10, /* 128-column strips for plain projections */
     GPTQ4_MIDM_WAVES_4 = 100,
     GPTQ4_MIDM_WAVES_8 = 200,

@@ -20,7 +20,8 @@ pytestmark = pytest.mark.gpu
 CONFIGS = [(0, 0), (1, 1), (2, 1), (1, 2), (2, 3), (10, 0), (11, 1), (12, 3),
            (100, 0), (101, 1), (102, 1), (101, 3), (102, 2), (111, 2), (112, 1),
            (200, 0), (201, 1), (202, 1), (201, 2), (202, 2), (211, 1), (212, 1),
-           (1000, 0), (1001, 1), (1002, 2), (1101, 2), (1102, 1), (1201, 1), (1202, 1), (2000, 0)]
+           (1000, 0), (1001, 1), (1002, 2), (1101, 2), (1102, 1), (1201, 1), (1202, 1), (2000, 0),
+           (3, 1), (3, 2), (13, 1), (1003, 1), (2003, 2)]  # (96-row tiles: four waves)
 
 @pytest.fixture(params=CONFIGS, ids=lambda c: "mt%d_s%d" % c)
 def forced_midm(request):
@@ -129,6 +130,36 @@ def test_midm_places_cache_rows_by_position(forced_midm):
         untouched = torch.ones(cap, dtype=torch.bool)
         untouched[pos[bi]] = False
         assert bool((kc[bi][:, untouched] == 7.0).all()) and bool((vc[bi][:, untouched] == 7.0).all())
+
+
+@pytest.mark.parametrize("m", [65, 96, 97, 193])
+def test_96_row_tiles_on_streaming_order_words(m):
+    """The three epilogues with 96-row tiles on streaming-order words against the same on the checkpoint's.  The two number a
+    tile's K steps differently: fp32 sums of the same 1024 products in two orders, apart by at most 1024 * 2^-24 times the sum
+    of their sizes (~ 50 here: 3e-3, typically 1e-5), then one fp16 rounding each, 2^-10 of the value apart at most; the gate /
+    up product has two such factors."""
+    def close(got, want):
+        got, want = got.float(), want.float()
+        return bool(((got - want).abs() <= 3e-3 + 2 * 2.0 ** -10 * want.abs()).all())
+
+    from gptq_triton_amd import _lib
+    G, lib = gptq(), _lib.load()
+    k, n, g, H = 1024, 3072, 128, 8
+    A, B = to_dev(O.make_layer(k, n, g, seed=700)), to_dev(O.make_layer(k, n, g, seed=701))
+    x = torch.from_numpy(O.make_x(m, k, seed=m)).cuda()
+    pos = torch.arange(m, dtype=torch.int32, device="cuda")[None]
+    cos, sin = G.RotaryTable(128, 2048).get(torch.device("cuda"), 2048)
+    sa, sb = (G.stream_pack(D["qweight"], D["qzeros"], D["scales"], g) for D in (A, B))
+    flat = lambda D: (D["qweight"], D["scales"], D["qzeros"])
+    try:
+        for code, split in ((3, 1), (3, 2), (13, 1), (1003, 1), (2003, 1)):
+            lib.gptq4_set_midm_tuning(2, code, split)
+            assert close(G.matmul4_stream(g, x, *sa), G.matmul4(g, x, *flat(A)))
+            assert close(G.llama_mlp_4_stream(g, x, *sa, *sb), G.llama_mlp_4(g, x, *flat(A), *flat(B)))
+            for got, want in zip(G.qkv_rotary_stream(g, x[None], *sa, pos, cos, sin, H), G.qkv_rotary(g, x[None], *flat(A), pos, cos, sin, H)):
+                assert close(got, want)
+    finally:
+        lib.gptq4_set_midm_tuning(1, 0, 0)
 
 
 def test_midm_and_tiled_kernels_agree_within_rounding():

@@ -594,6 +594,13 @@ def test_unfused_mlp_runs_gate_and_up_in_one_launch(act, rows):
     # sign a relative error of the sum no larger in the 2-norm
     err = np.linalg.norm(y.float().cpu().numpy() - ref) / np.linalg.norm(ref)
     assert err < 4 * 2.0 ** -11, err
+    if act == "shared":
+        inv = block.input_order()
+        moved = torch.empty_like(torch.from_numpy(x)).cuda()
+        moved[:, inv.long()] = torch.from_numpy(x).cuda()
+        assert torch.equal(block(moved, ordered=True), y)   # the same gate and up sums: the gather only moves values
+    else:
+        assert block.input_order() is None
     h = torch.from_numpy(O.make_x(rows, k, seed=50)).cuda()
     if block.norm_fusable(rows):
         w = torch.ones(k, dtype=torch.float16, device="cuda")
