@@ -886,17 +886,22 @@ StreamTuning g_stream_tuning = {0, 0};
 static StreamPlan stream_plan_with(int epi, int M, int N, int K, bool norm, int strips, bool tall);
 
 StreamPlan stream_plan(int epi, int M, int N, int K, bool norm) {
-    // 8 .. 16 rows: a unit is the 128 input rows of TWO adjacent tiles, so that the rows' chunks - twice the bytes of a
-    // tile's weights at 16 rows - are fetched and turned once for both; only where a workgroup's range stays long (LLaMA-7B at
-    // 16 rows: gate/up 16.8 against 17.7 us, down_proj 10.7 against 11.3 with 43 units to a workgroup; QKV 13.2 against
-    // 11.4 and o_proj 7.3 against 5.9 with 24 and 16, where the ranges stop lining up with the tiles), where the tile
-    // count is even and the partial sums of two tiles fit the LDS.  (depth + 10 in the tuning call: never; + 20: wherever
-    // it can run.)
+    // 5 .. 16 rows: a unit is the 128 input rows of TWO adjacent tiles, so that the rows' chunks - twice the bytes of a
+    // tile's weights at 16 rows - are fetched and turned once for both; only where the tile count is even, the partial sums
+    // of two tiles fit the LDS and a workgroup's range stays long, or takes in whole tiles: with shorter ranges the cuts stop
+    // lining up with the tiles.  From a sweep of both over the projections of hidden sizes 2048 to 8192 (us, one tile / two;
+    // q = units of two tiles to a workgroup, nb = units of a tile):
+    //   plain, q >= 40:  5120 x 15360 at 5 rows 16.9 / 14.1, 17920 x 6656 23.2 / 18.5, 11008 x 4096 10.2 / 9.7, 16 rows 11.7 / 11.0
+    //   plain, q >= nb (K from 1536 on: 1024 x 17920 at 16 rows 7.5 / 7.7):  3072 x 8192 (q 24, nb 24) at 16 rows 7.6 / 7.1; below both: 8192 x 3072 (24, 64) 8.5 / 9.2, 4096 x 4096 6.4 / 7.6
+    //   rotary, q >= 40: 6656 at 5 rows 21.2 / 19.9, 16 rows 25.5 / 23.3; below: 5120 (q 37) 14.7 / 15.6, 17.3 / 17.9
+    //   gate/up, whose unit is two matrices already: from 9 rows on, 5120 at 8 rows 20.9 / 21.5, 10 rows 22.7 / 22.3, 13 rows 24.0 / 23.1
+    // (depth + 10 in the tuning call: never; + 20: wherever it can run.)
     const int tiles = (epi == EPI_ROPE) ? N / 32 : N / 16;
     const int mode = g_stream_tuning.depth / 10;
     if (M > STREAM_MAX_M && (tiles % 2) == 0 && mode != 1) {
         const StreamPlan two = stream_plan_with(epi, M, N, K, norm, 2, true);
-        if (two.ok && (mode == 2 || (M >= 8 && two.q >= 40))) return two;
+        const bool longer = two.q >= 40 || (epi == EPI_PLAIN && two.nb >= 12 && two.q >= two.nb);
+        if (two.ok && (mode == 2 || (longer && (epi != EPI_SILU_MUL || M >= 9)))) return two;
     }
     const StreamPlan pl = stream_plan_with(epi, M, N, K, norm, 1, M > STREAM_MAX_M);
     // rows that with all of K do not fit the LDS (four of more than about 18000 values) are fetched with the units
