@@ -98,6 +98,17 @@ __global__ __launch_bounds__(256) void gptq4_rmsnorm_kernel(const half_t *x, con
 // that read everything twice: 2 x 8.2 us of copies beside 61 us of torch's attention for 32 heads x 1500 rows.
 constexpr int ATT_PART = 130;  // floats per partial: max, sum, 128 accumulators
 
+// Sum over the 16 lanes of a DPP row, in every lane: the same additions as four butterfly exchanges, without their trips
+// through the LDS (after the quads have met, the mirrored lane holds the sum of the other quad, then of the other half).  32 heads over
+// 2040 rows 11.2 -> 10.95 us, 52 heads 16.4 -> 15.95, 8 x 40 heads over 110 rows 7.7 -> 7.3.
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+    return v + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float row16_sum(float v) {
+    return dpp_add<0x140>(dpp_add<0x141>(dpp_add<0x4E>(dpp_add<0xB1>(v))));  // quad_perm 1032, 2301, row_half_mirror, row_mirror
+}
+
 template <bool EXTEND>
 __global__ __launch_bounds__(256) void gptq4_attn_decode_kernel(const half_t *__restrict__ q, const half_t *kc, const half_t *vc,
                                                                 const int *__restrict__ positions,
@@ -163,10 +174,7 @@ __global__ __launch_bounds__(256) void gptq4_attn_decode_kernel(const half_t *__
             float s = 0.f;
 #pragma unroll
             for (int i = 0; i < 4; ++i) s += qf[2 * i] * (float)kp[i].x + qf[2 * i + 1] * (float)kp[i].y;
-            s += __shfl_xor(s, 1);
-            s += __shfl_xor(s, 2);
-            s += __shfl_xor(s, 4);
-            s += __shfl_xor(s, 8);
+            s = row16_sum(s);
             if (r + 16 * u < r1) {  // uniform over the 16 lanes of a row
                 const float mn = fmaxf(m, s);
                 const float corr = __expf(m - mn), pw = __expf(s - mn);
