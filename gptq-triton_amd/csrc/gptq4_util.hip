@@ -79,28 +79,50 @@ __global__ __launch_bounds__(256) void gptq4_gather_cols_kernel(const half_t *__
     *reinterpret_cast<uint4 *>(out + (size_t)blockIdx.y * K + 8 * c) = o;
 }
 
-// The same for many rows: one workgroup per row first copies the row into LDS (whole 16-byte chunks), then
-// gathers from there - single 2-byte reads of global memory cost a cache line each.
-__global__ __launch_bounds__(256) void gptq4_gather_cols_lds_kernel(const half_t *__restrict__ x,
-                                                                    const int32_t *__restrict__ perm,
-                                                                    half_t *__restrict__ out, int K) {
+// The same through LDS, for rows that fit: one workgroup per row copies the row there in whole 16-byte chunks and gathers
+// from it - single 2-byte reads of global memory cost a cache line each.  KEEP: chunks a thread holds (longer rows loop), with
+// the permutation asked for together with the row - one round trip to memory instead of two, which is what few long rows
+// wait for.  With the streaming-order projection behind it (us, KEEP 0 in 256 threads / 4 in 512): 13824 x 5120 at 20 rows
+// 25.9 / 23.5, 100 rows 41.5 / 39.6, 17920 x 6656 at 20 rows 34.8 / 32.0; short rows and many rows lose by the larger
+// workgroups: 1024 x 1024 at 20 rows 7.9 / 8.0, 13824 x 5120 at 400 rows 91.7 / 93.3.
+template <int NT, int KEEP>
+__global__ __launch_bounds__(NT) void gptq4_gather_cols_lds_kernel(const half_t *__restrict__ x,
+                                                                   const int32_t *__restrict__ perm,
+                                                                   half_t *__restrict__ out, int K) {
     extern __shared__ uint4 row_chunks[];  // K / 8
-    const int chunks = K >> 3;
+    const int chunks = K >> 3, tid = threadIdx.x;
     const uint4 *src = reinterpret_cast<const uint4 *>(x + (size_t)blockIdx.x * K);
-    for (int c = threadIdx.x; c < chunks; c += 256) row_chunks[c] = src[c];
+    const int4 *order = reinterpret_cast<const int4 *>(perm);
+    uint4 held[KEEP ? KEEP : 1];
+    int4 idx[KEEP ? KEEP : 1][2];
+#pragma unroll
+    for (int n = 0; n < KEEP; ++n) {
+        const int c = tid + NT * n;
+        if (c < chunks) {
+            held[n] = src[c];
+            idx[n][0] = order[2 * c];
+            idx[n][1] = order[2 * c + 1];
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < KEEP; ++n)
+        if (tid + NT * n < chunks) row_chunks[tid + NT * n] = held[n];
+    for (int c = tid + NT * KEEP; c < chunks; c += NT) row_chunks[c] = src[c];
     __syncthreads();
     const uint16_t *row = reinterpret_cast<const uint16_t *>(row_chunks);
     uint4 *dst = reinterpret_cast<uint4 *>(out + (size_t)blockIdx.x * K);
-    for (int c = threadIdx.x; c < chunks; c += 256) {
-        const int4 i0 = *reinterpret_cast<const int4 *>(perm + 8 * c);
-        const int4 i1 = *reinterpret_cast<const int4 *>(perm + 8 * c + 4);
+    auto put = [&](int c, int4 i0, int4 i1) {
         uint4 o;
         o.x = (uint32_t)row[i0.x] | ((uint32_t)row[i0.y] << 16);
         o.y = (uint32_t)row[i0.z] | ((uint32_t)row[i0.w] << 16);
         o.z = (uint32_t)row[i1.x] | ((uint32_t)row[i1.y] << 16);
         o.w = (uint32_t)row[i1.z] | ((uint32_t)row[i1.w] << 16);
         dst[c] = o;
-    }
+    };
+#pragma unroll
+    for (int n = 0; n < KEEP; ++n)
+        if (tid + NT * n < chunks) put(tid + NT * n, idx[n][0], idx[n][1]);
+    for (int c = tid + NT * KEEP; c < chunks; c += NT) put(c, order[2 * c], order[2 * c + 1]);
 }
 
 __global__ __launch_bounds__(256) void gptq4_rope_table_kernel(float *__restrict__ cos_out,
@@ -159,8 +181,11 @@ int launch_sort_rows(const uint32_t *qweight, const int32_t *perm, uint32_t *out
 
 int launch_gather_cols(const half_t *x, const int32_t *perm, half_t *out, int M, int K, hipStream_t stream) {
     if (M > 16 && (size_t)K * sizeof(half_t) <= 65536) {
-        hipLaunchKernelGGL(gptq4_gather_cols_lds_kernel, dim3((unsigned)M), dim3(256), (size_t)K * sizeof(half_t), stream, x,
-                           perm, out, K);
+        const size_t lds = (size_t)K * sizeof(half_t);
+        if (M <= 128 && K > 4096)
+            hipLaunchKernelGGL((gptq4_gather_cols_lds_kernel<512, 4>), dim3((unsigned)M), dim3(512), lds, stream, x, perm, out, K);
+        else
+            hipLaunchKernelGGL((gptq4_gather_cols_lds_kernel<256, 0>), dim3((unsigned)M), dim3(256), lds, stream, x, perm, out, K);
         return (int)hipGetLastError();
     }
     const int threads = (K / 8 >= 256) ? 256 : 64;

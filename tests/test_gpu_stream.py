@@ -331,6 +331,20 @@ def test_matmul_act_order(k, n, g, m):
     assert_close(y.cpu().numpy(), ref, f"act-order stream matmul {k}x{n} M={m}")
 
 
+@pytest.mark.parametrize("k", [4096, 4224, 16384, 16512])  # 4096: the shortest rows' kernel; past 16384: chunks beyond the held ones
+@pytest.mark.parametrize("m", [17, 128, 129])
+def test_act_order_rows_gathered_ahead_are_the_rows_in_that_order(k, m):
+    """Above 16 rows a launch gathers the rows first: the very bits of the same call on rows gathered by torch."""
+    G = gptq()
+    D = to_dev(O.make_layer(k, 512, 128, seed=1400 + k, act_order=True))
+    qs, perm = G.prepare_act_order(D["qweight"], D["g_idx"], 128)
+    sw, meta = G.stream_pack(qs, D["qzeros"], D["scales"], 128)
+    x = torch.from_numpy(O.make_x(m, k, seed=m + 41)).cuda()
+    y = G.matmul4_stream(128, x, sw, meta, None, perm)
+    want = G.matmul4_stream(128, x[:, perm.long()].contiguous(), sw, meta)
+    assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+
+
 @pytest.mark.parametrize("k,inter,g", [(1024, 2816, 128), (4096, 11008, 128), (5120, 13824, 128), (6656, 17920, 512)])
 @pytest.mark.parametrize("m", [1, 2, 4, 5, 11, 16])
 def test_mlp_gateup(k, inter, g, m):
