@@ -288,7 +288,6 @@ class GreedyDecoder:
             and embed.shape[0] >= head.shape[0] and model.lm_head.bias is None
         self.history = torch.zeros((bsz, capacity + 1), dtype=torch.long, device=dev)
         self.hidden = torch.zeros((bsz, 1, cfg.hidden_size), dtype=torch.float16, device=dev)
-        self._at = None  # (version of the position tensor, the one position of every sequence) as this object left it
         self.graph = None
 
     def _layers(self, h, position_ids, kv_offset, attend, end):
@@ -369,7 +368,6 @@ class GreedyDecoder:
         nxt = self._layers(self.model.model.embed_tokens(input_ids), position_ids, 0, attend, self._last_tokens)
         self.tokens.copy_(nxt)
         self.position.fill_(prompt)
-        self._moved_to(prompt)
         return nxt
 
     def _step(self):
@@ -385,17 +383,19 @@ class GreedyDecoder:
     @torch.no_grad()
     def decode(self, steps: int, use_graph: bool = False) -> torch.Tensor:
         """`steps` more greedy tokens after prefill -> [B, steps]."""
-        # where the sequences stand: known if this object moved them there, else (someone wrote to `position`) read back
-        at = self._known_position()
-        if (int(self.position.max()) if at is None else at) + steps > self.capacity:
+        # where the sequences stand is read back: the kernels move `position` on, also in a step that is interrupted on the host
+        # and in a replay of `graph` by the caller, and the caller may write to it
+        stand = self.position.flatten().tolist()
+        if max(stand) + steps > self.capacity:
             raise ValueError("decode would run past the cache capacity")
         if self.one_launch_end:
             self.hidden.copy_(self.model.model.embed_tokens(self.tokens))
         if use_graph and self.graph is None and steps > 0:
             self._capture()
-        # the tokens are at their places in `history` afterwards; where the positions are not known on the host, or the step
+        # the tokens are at their places in `history` afterwards; where the sequences stand at different places, or the step
         # does not keep them there, they are collected one by one
-        kept = self.one_launch_end and at is not None
+        at = stand[0]
+        kept = self.one_launch_end and at >= 0 and min(stand) == max(stand)
         out = None if kept else torch.empty((self.bsz, steps), dtype=torch.long, device=self.tokens.device)
         for i in range(steps):
             if use_graph:
@@ -404,32 +404,22 @@ class GreedyDecoder:
                 self._step()
             if not kept:
                 out[:, i:i + 1].copy_(self.tokens)
-        self._moved_to(None if at is None else at + steps)
         if kept:
             out = self.history[:, at + 1:at + 1 + steps].clone()
         # one 4-byte read per workspace: a bounded wait of the small-M kernels that ran out would have made tokens wrong silently
         _lib.check_exchange_errors()
         return out
 
-    def _refetch(self, at):
-        """The embedding rows and the host's idea of the position for tokens and positions that were put back."""
+    def _refetch(self):
+        """The embedding rows for tokens that were put back."""
         if self.one_launch_end:
             self.hidden.copy_(self.model.model.embed_tokens(self.tokens))
-        self._moved_to(at)
-
-    def _moved_to(self, at) -> None:
-        # (tensors made in inference mode have no version: their positions are read back)
-        self._at = None if at is None or self.position.is_inference() else (self.position._version, at)
-
-    def _known_position(self):
-        return self._at[1] if self._at is not None and self._at[0] == self.position._version else None
 
     def _capture(self):
         """Capture _step as a graph.  The warm-up steps run on the capture stream first, so
         workspaces and tables exist before capture; their effect on tokens, position and the
         cache rows they wrote is undone (the rows lie beyond the current position and are
         rewritten before any later step attends to them)."""
-        at = self._known_position()
         tokens0, position0 = self.tokens.clone(), self.position.clone()
         side = torch.cuda.Stream(device=self.tokens.device)
         side.wait_stream(torch.cuda.current_stream())
@@ -437,7 +427,7 @@ class GreedyDecoder:
             self._step()
             self.tokens.copy_(tokens0)
             self.position.copy_(position0)
-            self._refetch(at)
+            self._refetch()
         torch.cuda.current_stream().wait_stream(side)
         torch.cuda.synchronize()
         self.graph = torch.cuda.CUDAGraph()
@@ -445,5 +435,5 @@ class GreedyDecoder:
             self._step()
         self.tokens.copy_(tokens0)
         self.position.copy_(position0)
-        self._refetch(at)
+        self._refetch()
         torch.cuda.synchronize()
