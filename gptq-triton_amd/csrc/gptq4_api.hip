@@ -805,7 +805,7 @@ int gptq4_lm_head_argmax(const void *x, const void *weight, int64_t *out, int B,
 int gptq4_greedy_step_end(const void *x, const void *delta, const void *norm_weight, float eps, const void *weight, int B, int K, int V,
                           int64_t *tokens, int32_t *positions, int64_t *history, int history_capacity, const void *embed,
                           void *next_hidden, void *workspace, size_t workspace_bytes, void *stream) {
-    if (!x || !weight || !tokens || !positions || !history || !embed || !next_hidden) return -GPTQ4_E_NULL;
+    if (!x || !weight || !tokens || !positions || !history || (embed == nullptr) != (next_hidden == nullptr)) return -GPTQ4_E_NULL;
     if (history_capacity < 1 || (!norm_weight && delta) || (norm_weight && (B != 1 || K > NORM_MAX_H || !(eps >= 0.f)))) return -GPTQ4_E_SHAPE;
     // (the workgroups that are still reading x and delta must not see the next step's row)
     if (next_hidden == x || (delta && next_hidden == delta)) return -GPTQ4_E_SHAPE;

@@ -1,6 +1,6 @@
 // The last step of a greedy decode token: logits = x . W^T with the fp16 lm_head weight W [V, K] and the index of the
 // largest logit per row, in one launch - and, for a decoding loop, what the next step starts from: the token and its place in
-// the sequence, the position, and the token's embedding row.  (The reference's scripts call the model's lm_head - a dense
+// the sequence, the position, and on request the token's embedding row.  (The reference's scripts call the model's lm_head - a dense
 // fp16 linear - and take the argmax of its output, generate.py.)
 //
 // A memory-bound stream over V x K x 2 bytes.  The rows of W are dealt to the workgroups in contiguous ranges and inside a
@@ -152,6 +152,7 @@ __global__ __launch_bounds__(64 * HEAD_WAVES) void gptq4_head_argmax_kernel(Head
                 p.positions[b] = at;
                 if (at >= 0 && at < p.history_capacity) p.history[(size_t)b * p.history_capacity + at] = (long long)token;
             }
+            if (p.embed == nullptr) continue;
             const uint4 *src = reinterpret_cast<const uint4 *>(p.embed + (size_t)token * K);
             uint4 *dst = reinterpret_cast<uint4 *>(p.next_hidden + (size_t)b * K);
             for (int i = lane; i < chunks; i += 64) dst[i] = src[i];

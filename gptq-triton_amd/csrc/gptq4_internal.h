@@ -244,7 +244,7 @@ struct HeadArgs {
     int *counters;
     int B, K, V, rows_per_wg;
     // a decoding loop's state (positions null: tokens only): positions[b] moves on by one, the token is stored at that place
-    // of history [B, history_capacity] and its row of embed [V, K] goes to next_hidden [B, K]
+    // of history [B, history_capacity] and (embed not null) its row of embed [V, K] goes to next_hidden [B, K]
     int *positions;
     long long *history;
     int history_capacity;

@@ -589,7 +589,8 @@ PyObject *lm_head_argmax(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
-// greedy_step_end(x, delta, norm weight, eps, lm_head weight, tokens, positions, history, embedding, next hidden) -> True
+// greedy_step_end(x, delta, norm weight, eps, lm_head weight, tokens, positions, history, embedding, next hidden) -> True;
+// embedding and next hidden None: not fetched
 PyObject *greedy_step_end(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
     GPTQ4_TAKES(10)
@@ -597,15 +598,16 @@ PyObject *greedy_step_end(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
     const at::Tensor *x = a.need(0);
     Norm norm;
     norm.delta = a.may(1), norm.weight = a.may(2), norm.eps = (float)a.real(3);
-    const at::Tensor *w = a.need(4), *tokens = a.need(5), *pos = a.need(6), *history = a.need(7), *embed = a.need(8), *next = a.need(9);
+    const at::Tensor *w = a.need(4), *tokens = a.need(5), *pos = a.need(6), *history = a.need(7), *embed = a.may(8), *next = a.may(9);
     if (!a.fine || !is_rows(x) || x->size(-1) == 0 || !norm.fits(x)) Py_RETURN_NONE;
     const at::Device dev = x->device();
     const int64_t k = x->size(-1), b = x->numel() / k;
-    if (!is_table(w, k, dev) || !is_table(embed, k, dev) || embed->size(0) < w->size(0)) Py_RETURN_NONE;
+    if (!is_table(w, k, dev) || (embed == nullptr) != (next == nullptr)) Py_RETURN_NONE;
+    if (embed != nullptr && (!is_table(embed, k, dev) || embed->size(0) < w->size(0) || !is_rows(next) || next->numel() != b * k)) Py_RETURN_NONE;
     for (const at::Tensor *t : {tokens, pos, history, next, norm.delta, norm.weight})
         if (!beside(t, dev)) Py_RETURN_NONE;
     if (tokens->scalar_type() != at::kLong || tokens->numel() != b || pos->scalar_type() != at::kInt || pos->numel() != b ||
-        history->scalar_type() != at::kLong || history->dim() != 2 || history->size(0) != b || !is_rows(next) || next->numel() != b * k)
+        history->scalar_type() != at::kLong || history->dim() != 2 || history->size(0) != b)
         Py_RETURN_NONE;
     const hipStream_t stream = stream_of(dev);
     Workspace ws;

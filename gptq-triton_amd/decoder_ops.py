@@ -118,9 +118,10 @@ def lm_head_argmax(x: torch.Tensor, weight: torch.Tensor, max_rows: int = HEAD_M
     return out
 
 
-def greedy_step_end(x, delta, norm_weight, eps, weight, tokens, positions, history, embed, next_hidden) -> None:
+def greedy_step_end(x, delta, norm_weight, eps, weight, tokens, positions, history, embed=None, next_hidden=None) -> None:
     """The end of a greedy decode step in one launch: tokens (int64) become the argmax of the logits, positions (int32) go up by
-    one, the tokens are stored at those places of history (int64 [B, capacity]) and their rows of the embedding in next_hidden.
+    one, the tokens are stored at those places of history (int64 [B, capacity]) and, if given, their rows of the embedding in
+    next_hidden.
     norm_weight None: x is what the lm_head reads; else (one row) x is the residual stream and the logits are those of
     RMSNorm(x + delta) * norm_weight, as add_rms_norm gives it."""
     if _lib.host().greedy_step_end(x, delta, norm_weight, eps, weight, tokens, positions, history, embed, next_hidden) is None:

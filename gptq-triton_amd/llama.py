@@ -281,13 +281,11 @@ class GreedyDecoder:
                        for _ in model.model.layers]
         self.tokens = torch.zeros((bsz, 1), dtype=torch.long, device=dev)
         self.position = torch.zeros((bsz, 1), dtype=torch.int32, device=dev)
-        # with one_launch_end a decode step ends in one launch that picks the tokens, moves the positions on, keeps the tokens at
-        # their places in the sequence and fetches their embedding rows for the next step
-        head, embed = model.lm_head.weight, model.model.embed_tokens.weight
-        self.one_launch_end = head_argmax_takes(bsz, head) and embed.is_cuda and embed.dtype == torch.float16 and embed.is_contiguous() \
-            and embed.shape[0] >= head.shape[0] and model.lm_head.bias is None
+        # with one_launch_end a decode step ends in one launch that picks the tokens, moves the positions on and keeps the tokens
+        # at their places in the sequence.  (It can fetch their embedding rows for the next step too, but a step starts from
+        # `tokens`, which the caller may write to between two steps or two replays of `graph`.)
+        self.one_launch_end = head_argmax_takes(bsz, model.lm_head.weight) and model.lm_head.bias is None
         self.history = torch.zeros((bsz, capacity + 1), dtype=torch.long, device=dev)
-        self.hidden = torch.zeros((bsz, 1, cfg.hidden_size), dtype=torch.float16, device=dev)
         self.graph = None
 
     def _layers(self, h, position_ids, kv_offset, attend, end):
@@ -350,8 +348,7 @@ class GreedyDecoder:
             if x is None:
                 _, x = add_rms_norm(h, delta, w, norm.variance_epsilon)
             delta = w = None
-        greedy_step_end(x, delta, w, norm.variance_epsilon, model.lm_head.weight, self.tokens, self.position, self.history,
-                        model.model.embed_tokens.weight, self.hidden)
+        greedy_step_end(x, delta, w, norm.variance_epsilon, model.lm_head.weight, self.tokens, self.position, self.history)
 
     @torch.no_grad()
     def prefill(self, input_ids: torch.Tensor) -> torch.Tensor:
@@ -371,14 +368,13 @@ class GreedyDecoder:
         return nxt
 
     def _step(self):
-        """One decode token from the static buffers: reads tokens (or their embedding rows) and position, writes them back."""
+        """One decode token from the static buffers: reads tokens and position, writes them back."""
 
         def attend(q, kc, vc, attn):  # rows 0..position of the cache; act-order o_proj: written in the order it reads
             order = attn.context_order()
             return decode_attention(q, kc, vc, self.position, out_index=order), order is not None
 
-        self._layers(self.hidden if self.one_launch_end else self.model.model.embed_tokens(self.tokens), self.position, KV_AT_POSITION,
-                     attend, self._end_step)
+        self._layers(self.model.model.embed_tokens(self.tokens), self.position, KV_AT_POSITION, attend, self._end_step)
 
     @torch.no_grad()
     def decode(self, steps: int, use_graph: bool = False) -> torch.Tensor:
@@ -388,8 +384,6 @@ class GreedyDecoder:
         stand = self.position.flatten().tolist()
         if max(stand) + steps > self.capacity:
             raise ValueError("decode would run past the cache capacity")
-        if self.one_launch_end:
-            self.hidden.copy_(self.model.model.embed_tokens(self.tokens))
         if use_graph and self.graph is None and steps > 0:
             self._capture()
         # the tokens are at their places in `history` afterwards; where the sequences stand at different places, or the step
@@ -410,11 +404,6 @@ class GreedyDecoder:
         _lib.check_exchange_errors()
         return out
 
-    def _refetch(self):
-        """The embedding rows for tokens that were put back."""
-        if self.one_launch_end:
-            self.hidden.copy_(self.model.model.embed_tokens(self.tokens))
-
     def _capture(self):
         """Capture _step as a graph.  The warm-up steps run on the capture stream first, so
         workspaces and tables exist before capture; their effect on tokens, position and the
@@ -427,7 +416,6 @@ class GreedyDecoder:
             self._step()
             self.tokens.copy_(tokens0)
             self.position.copy_(position0)
-            self._refetch()
         torch.cuda.current_stream().wait_stream(side)
         torch.cuda.synchronize()
         self.graph = torch.cuda.CUDAGraph()
@@ -435,5 +423,4 @@ class GreedyDecoder:
             self._step()
         self.tokens.copy_(tokens0)
         self.position.copy_(position0)
-        self._refetch()
         torch.cuda.synchronize()

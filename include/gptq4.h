@@ -243,9 +243,9 @@ int gptq4_lm_head_argmax(const void *x, const void *weight, int64_t *out, int B,
                          size_t workspace_bytes, void *stream);
 
 /* The same launch also moves a decoding loop on to its next step: tokens[b] = the argmax; positions[b] (int32) goes up by
- * one, tokens[b] is stored at that place of history int64 [B, history_capacity] (if it has room), and its row of the
- * embedding embed fp16 [V, K] is copied to next_hidden fp16 [B, K], which may not be x or delta.  With norm_weight fp16
- * [K] (B == 1, K <= 8192) x is the residual stream and the logits are those of
+ * one, tokens[b] is stored at that place of history int64 [B, history_capacity] (if it has room), and, with
+ * embed and next_hidden (both or neither), its row of the embedding embed fp16 [V, K] is copied to next_hidden fp16 [B, K],
+ * which may not be x or delta.  With norm_weight fp16 [K] (B == 1, K <= 8192) x is the residual stream and the logits are those of
  * norm_weight * rmsnorm(x + delta) (delta nullable), the same bits as gptq4_add_rmsnorm / gptq4_rmsnorm and
  * gptq4_lm_head_argmax one after the other.  No reference counterpart (transformers' generate loop there). */
 int gptq4_greedy_step_end(const void *x, const void *delta, const void *norm_weight, float eps,

@@ -1,5 +1,5 @@
-"""GreedyDecoder keeps the right place whoever moved its state: decode() after a step that was interrupted on the host, after the
-caller replayed the captured graph, and after the caller wrote to the position buffer."""
+"""GreedyDecoder goes on from its state buffers whoever moved them: decode() after a step that was interrupted on the host, after the
+caller replayed the captured graph, and after the caller wrote to the position or the tokens."""
 import pytest
 import torch
 
@@ -79,6 +79,40 @@ def test_decode_of_sequences_at_different_places(monkeypatch):
     assert got.tolist() == [[token_at(5 + i, 0) for i in range(3)], [token_at(10 + i, 1) for i in range(3)]]
     with pytest.raises(ValueError):
         dec.decode(CAPACITY - 12 + 1)
+
+
+def test_a_step_starts_from_the_tokens_buffer(monkeypatch):
+    monkeypatch.setattr(GreedyDecoder, "one_launch_end", True, raising=False)
+    cfg = LlamaConfigLite(hidden_size=64, num_attention_heads=2, intermediate_size=64, num_hidden_layers=1, vocab_size=512)
+    model = LlamaForCausalLM(cfg)
+    dec = GreedyDecoder(model, 2, CAPACITY)
+    if not dec.one_launch_end:
+        dec.one_launch_end = True
+    seen = []
+    monkeypatch.setattr(dec, "_layers", lambda h, *a, **k: seen.append(h.clone()))
+    dec.tokens.copy_(torch.tensor([[17], [400]]))
+    dec._step()
+    assert torch.equal(seen[0], model.model.embed_tokens(dec.tokens))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bsz", [1, 3])
+def test_replays_follow_tokens_and_prompts_written_between_them(tmp_path, bsz):
+    """decoder.graph after another prefill, and after the caller put other tokens in place (a sampling loop on the graph)."""
+    cfg = make_checkpoint(tmp_path, 128, seed=32)
+    model = G.load_quant(str(tmp_path), device="cuda", fuse_mlp=True)
+    torch.manual_seed(8)
+    ids, other = torch.randint(0, cfg.vocab_size, (2, bsz, 6)).cuda()
+    forced = torch.randint(0, cfg.vocab_size, (bsz, 1)).cuda()
+    graph, eager = GreedyDecoder(model, bsz, 24), GreedyDecoder(model, bsz, 24)
+    graph.prefill(ids)
+    graph.decode(3, use_graph=True)
+    graph.prefill(other), eager.prefill(other)
+    for _ in range(3):
+        graph.graph.replay(), eager.decode(1)
+        assert torch.equal(graph.tokens, eager.tokens) and torch.equal(graph.position, eager.position)
+        graph.tokens.copy_(forced), eager.tokens.copy_(forced)
+    assert torch.equal(graph.decode(2, use_graph=True), eager.decode(2))
 
 
 @pytest.mark.gpu
