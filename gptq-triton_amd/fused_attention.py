@@ -48,15 +48,19 @@ class RotaryTable:
 
     def positions(self, device: torch.device, start: int, bsz: int, q_len: int) -> torch.Tensor:
         """position_ids of `q_len` tokens behind `start` others in every one of `bsz` sequences, int32 [B, S].  One sequence,
-        and one token of each of several, are a view of a table that is kept: no launch."""
-        if q_len > 1 and bsz > 1:
+        and one token of each of several, are a view of a table that is kept: no launch.
+
+        A table belongs to the stream it was filled on (no other stream reads it, and what it gives back is reused in that
+        stream's order), and a call that is being captured makes its own positions inside the graph: a graph holds bare
+        addresses, and a table filled by a graph would be empty until the first replay."""
+        if (q_len > 1 and bsz > 1) or torch.cuda.is_current_stream_capturing():
             return torch.arange(start, start + q_len, dtype=torch.int32, device=device).expand(bsz, q_len).contiguous()
-        key = (device.index if device.index is not None else torch.cuda.current_device(), bsz)
+        key = (device.index if device.index is not None else torch.cuda.current_device(), _lib.current_stream(device), bsz)
         tab = self._counts.get(key)
         if tab is None or tab.shape[0] < start + q_len:
             if len(self._counts) >= 16:
                 self._counts.clear()
-            rows = max(self.max_pos, start + q_len)
+            rows = max(self.max_pos, 2 * (start + q_len) if tab is not None else start + q_len)
             tab = torch.arange(rows, dtype=torch.int32, device=device).repeat_interleave(bsz).view(rows, bsz)
             self._counts[key] = tab
         return tab[start:start + q_len].view(bsz, q_len)
