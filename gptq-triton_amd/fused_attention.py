@@ -20,7 +20,7 @@ import torch.nn as nn
 from . import _lib
 from .decoder_ops import (ATTENTION_MAX_HEADS, NORM_MAX_ROWS, check_norm_args, contiguous_delta, decode_attention, extend_attention,
                           norm_fusable, norm_fusion_pays, prefill_attention)
-from .quant_linear import QuantLinear, _check_device_tensors, _check_matmul_args, inverse_permutation, tensor_key
+from .quant_linear import QuantLinear, _check_device_tensors, _check_matmul_args, inverse_permutation, only_itself, tensor_key
 
 
 @dataclass
@@ -264,8 +264,9 @@ class QuantLlamaAttention(nn.Module):
     def context_order(self):
         """Where each feature of the attention output should be stored so that an act-order o_proj reads
         it in the order of its sorted rows (int32 [hidden], the inverse of o_proj's permutation), or
-        None without act-order.  decode_attention(out_index=...) writes in that order."""
-        perm = self._modules['o_proj'].row_permutation()
+        None without act-order and where o_proj is to be called as a module (only_itself).
+        decode_attention(out_index=...) writes in that order."""
+        perm = self.o_proj.row_permutation() if only_itself(self.o_proj, QuantLinear) else None
         if perm is None:
             return None
         if self._context_order is None or self._context_order[0] != tensor_key(perm):
@@ -298,7 +299,7 @@ class QuantLlamaAttention(nn.Module):
 
     def project_out(self, context: torch.Tensor, ordered: bool = False) -> torch.Tensor:
         """o_proj(context); ordered: the context already is in the order of context_order()."""
-        return self._modules['o_proj'].multiply(context, ordered=ordered)
+        return self.o_proj.multiply(context, ordered=True) if ordered else self.o_proj(context)
 
     def norm_fusable(self, rows: int) -> bool:
         """Whether project_qkv(norm=...) is the faster way for this many rows."""
@@ -394,6 +395,8 @@ class QuantLlamaAttention(nn.Module):
         attn_output = attn_output.transpose(1, 2).reshape(bsz, q_len, self.hidden_size)
         attn_output = self.o_proj(attn_output)
         return attn_output, attn_weights, past_key_value
+
+    own_forward = forward
 
 
 def _forward_with_cache(self, hidden_states, attention_mask, position_ids, cache, output_attentions, cache_position, ordered=False):

@@ -316,6 +316,8 @@ class QuantLlamaMLP(nn.Module):
         w, perm, down_q = self._chained_weights()
         return self._down(llama_mlp_4(self.groupsize, x, *w, None if ordered else perm), down_q)
 
+    own_forward = forward
+
     def norm_fusable(self, rows: int) -> bool:
         """Whether forward_normed is the faster way for this many rows."""
         return norm_fusion_pays(rows, self.infeatures)

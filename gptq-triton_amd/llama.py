@@ -21,8 +21,8 @@ from . import _lib
 from .decoder_ops import (NORM_MAX_HIDDEN, add_rms_norm, decode_attention, greedy_step_end, head_argmax_takes, lm_head_argmax,
                           norm_fusion_pays, prefill_attention, rms_norm)
 from .fused_attention import KV_AT_POSITION, LlamaConfigLite, QuantLlamaAttention
-from .fused_mlp import llama_mlp_4_stream
-from .quant_linear import QuantLinear, inverse_permutation, stream_rows, tensor_key
+from .fused_mlp import QuantLlamaMLP, llama_mlp_4_stream
+from .quant_linear import QuantLinear, inverse_permutation, only_itself, stream_rows, tensor_key
 
 # the rows the decode kernels built on the streaming-order weight layout take (more rows: the mid-M and tiled kernels)
 STREAM_BATCH = 16
@@ -55,6 +55,8 @@ class LlamaRMSNorm(nn.Module):
         xf = xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + self.variance_epsilon)
         return self.weight * xf.to(x.dtype)
 
+    own_forward = forward
+
 
 class LlamaAttention(nn.Module):
     """Skeleton attention block: four linears to be replaced by make_quant / make_quant_attn."""
@@ -83,8 +85,8 @@ class LlamaMLP(nn.Module):
     def _pair(self, rows: int):
         """(groupsize, gate words and {scale, zero} words, up's, row permutation) where one launch can compute
         silu(gate) * up from the two modules' own tensors in streaming order, else None."""
-        gate, up = self._modules['gate_proj'], self._modules['up_proj']
-        if not (isinstance(gate, QuantLinear) and isinstance(up, QuantLinear)):
+        gate, up = self.gate_proj, self.up_proj
+        if not (only_itself(gate, QuantLinear) and only_itself(up, QuantLinear)):
             return None
         g, u = gate.stream_weights(rows), up.stream_weights(rows)
         if g is None or u is None or gate.groupsize != up.groupsize or g[0].shape != u[0].shape \
@@ -103,9 +105,11 @@ class LlamaMLP(nn.Module):
         return self._same_rows[1]
 
     def input_order(self):
-        """As QuantLlamaMLP.input_order: None without act-order, or where gate and up each have an order of their own."""
-        gate, up = self._modules['gate_proj'], self._modules['up_proj']
-        if not (isinstance(gate, QuantLinear) and isinstance(up, QuantLinear)) or gate.g_idx is None or up.g_idx is None:
+        """As QuantLlamaMLP.input_order: None without act-order, where gate and up each have an order of their own, and where
+        this block, gate or up is to be called as a module (only_itself)."""
+        gate, up = self.gate_proj, self.up_proj
+        if not (only_itself(self, LlamaMLP) and only_itself(gate, QuantLinear) and only_itself(up, QuantLinear)) \
+                or gate.g_idx is None or up.g_idx is None:
             return None
         return self._shared_order(gate.row_permutation(), up.row_permutation())
 
@@ -120,20 +124,22 @@ class LlamaMLP(nn.Module):
         pair = self._pair(x.numel() // max(x.shape[-1], 1)) if x.is_cuda else None
         if pair is not None:
             groupsize, gw, gm, uw, um, perm = pair
-            return self._modules['down_proj'](llama_mlp_4_stream(groupsize, x, gw, gm, uw, um, None if ordered else perm))
+            return self.down_proj(llama_mlp_4_stream(groupsize, x, gw, gm, uw, um, None if ordered else perm))
         if ordered:
             return self.down_proj(torch.nn.functional.silu(self.gate_proj.multiply(x, ordered=True)) * self.up_proj.multiply(x, ordered=True))
         return self.down_proj(torch.nn.functional.silu(self.gate_proj(x)) * self.up_proj(x))
 
+    own_forward = forward
+
     def norm_fusable(self, rows: int) -> bool:
         """Whether forward_normed is the faster way for this many rows."""
-        return self._pair(rows) is not None and norm_fusion_pays(rows, self.gate_proj.infeatures)
+        return only_itself(self, LlamaMLP) and self._pair(rows) is not None and norm_fusion_pays(rows, self.gate_proj.infeatures)
 
     def forward_normed(self, h, delta, norm_weight, eps):
         """(h + delta, forward(RMSNorm(h + delta))) with the residual add and the norm inside the gate/up launch."""
         groupsize, gw, gm, uw, um, perm = self._pair(h.numel() // h.shape[-1])
         s, mid = llama_mlp_4_stream(groupsize, h, gw, gm, uw, um, perm, norm=(delta, norm_weight, eps))
-        return s, self._modules['down_proj'](mid)
+        return s, self.down_proj(mid)
 
 
 class LlamaDecoderLayer(nn.Module):
@@ -151,6 +157,15 @@ class LlamaDecoderLayer(nn.Module):
         hidden_states = hidden_states + attn_out
         hidden_states = hidden_states + self.mlp(self.post_attention_layernorm(hidden_states))
         return hidden_states, present
+
+    own_forward = forward
+
+    def only_themselves(self) -> bool:
+        """Whether the layer and the blocks it calls are this package's own and nothing else would run with them."""
+        attn, mlp = self.self_attn, self.mlp
+        return only_itself(self, LlamaDecoderLayer) and only_itself(attn, QuantLlamaAttention) \
+            and only_itself(mlp, QuantLlamaMLP if type(mlp) is QuantLlamaMLP else LlamaMLP) \
+            and only_itself(self.input_layernorm, LlamaRMSNorm) and only_itself(self.post_attention_layernorm, LlamaRMSNorm)
 
 
 class LlamaModel(nn.Module):
@@ -189,7 +204,8 @@ class LlamaForCausalLM(nn.Module):
         past_len = 0 if past_key_values is None else past_key_values[0][0].shape[2]
         h = self.model.embed_tokens(input_ids)
         layers = self.model.layers
-        if h.is_cuda and h.dtype == torch.float16 and len(layers) and all(isinstance(l.self_attn, QuantLlamaAttention) for l in layers):
+        if h.is_cuda and h.dtype == torch.float16 and len(layers) and only_itself(self.model.norm, LlamaRMSNorm) \
+                and all(type(l) is LlamaDecoderLayer and l.only_themselves() for l in layers):
             h, presents = self._layers_fused(h, past_len, past_key_values, use_cache)
             if last_token_only:
                 h = h[:, -1:, :]
@@ -213,7 +229,7 @@ class LlamaForCausalLM(nn.Module):
         layers = self.model.layers
         bsz, q_len, _ = h.shape
         position_ids = layers[0].self_attn.rope.positions(h.device, past_len, bsz, q_len)
-        inside = q_len == 1 and all(l.self_attn.norm_fusable(bsz) and getattr(l.mlp, "norm_fusable", lambda r: False)(bsz) for l in layers)
+        inside = q_len == 1 and all(l.self_attn.norm_fusable(bsz) and l.mlp.norm_fusable(bsz) for l in layers)
         presents = []
         delta = None
         for i, layer in enumerate(layers):

@@ -16,8 +16,21 @@ from typing import Optional
 
 import torch
 import torch.nn as nn
+from torch.nn.modules import module as _nn_module
 
 from . import _lib
+
+
+def only_itself(m, cls) -> bool:
+    """Whether calling `m` runs the forward that `cls` came with and nothing else: no subclass, no hook on it or on all modules,
+    no forward put in the place of the instance's or the class's.  What computes a module's result without calling it asks
+    this first.  (cls.own_forward: the forward a class of this package was defined with.)"""
+    if type(m) is not cls or cls.forward is not cls.own_forward:
+        return False
+    d = m.__dict__
+    return not (d['_forward_hooks'] or d['_forward_pre_hooks'] or d['_backward_hooks'] or d['_backward_pre_hooks'] or 'forward' in d
+                or _nn_module._global_forward_hooks or _nn_module._global_forward_pre_hooks
+                or _nn_module._global_backward_hooks or _nn_module._global_backward_pre_hooks)
 
 
 def _check_matmul_args(a: torch.Tensor, qweight: torch.Tensor, groupsize: int):
@@ -355,6 +368,8 @@ class QuantLinear(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         return self.multiply(x)
+
+    own_forward = forward
 
     def dequantize(self) -> torch.Tensor:
         return dequantize(self.checkpoint_qweight(), self.qzeros, self.scales, self.groupsize, self.g_idx)
