@@ -215,6 +215,15 @@ def make_quant_attn(model: nn.Module):
         setattr(parent, child, attn)
 
 
+def _past_rows(t: torch.Tensor, shape, device) -> torch.Tensor:
+    """A past key or value tensor as the attention kernel reads it.  What a copy into the new pair would take is taken: another
+    float type or device, any strides, one sequence for all of them."""
+    if t.dtype == torch.float16 and t.shape == shape and t.device == device and t.is_contiguous() and t.data_ptr() % 16 == 0:
+        return t
+    t = t.to(device=device, dtype=torch.float16).expand(shape).contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 class QuantLlamaAttention(nn.Module):
     """LLaMA self-attention with the q, k, v projections and the rotary embedding fused
     into one kernel call.  Signature and return values follow the reference module."""
@@ -287,9 +296,10 @@ class QuantLlamaAttention(nn.Module):
         """One token of each sequence behind a (key, value) pair (or None): (the arguments of project_out, the grown pair), and
         with norm (see project_qkv) also the residual stream.  Two launches: the QKV projection stores its K and V as the
         new pair's last row, the attention kernel copies the other rows while it attends to them."""
-        past_k, past_v = (None, None) if past_key_value is None else (t.contiguous() for t in past_key_value)
-        past = 0 if past_k is None else past_k.shape[2]
-        shape = (hidden_states.shape[0], self.num_heads, past + 1, self.head_dim)
+        past = 0 if past_key_value is None else past_key_value[0].shape[-2]
+        rows = (hidden_states.shape[0], self.num_heads, past, self.head_dim)
+        past_k, past_v = (None, None) if past_key_value is None else (_past_rows(t, rows, hidden_states.device) for t in past_key_value)
+        shape = rows[:2] + (past + 1, self.head_dim)
         pair = (torch.empty(shape, dtype=torch.float16, device=hidden_states.device),
                 torch.empty(shape, dtype=torch.float16, device=hidden_states.device))
         q, _, _, *stream = self.project_qkv(hidden_states, position_ids, kv_out=pair, kv_offset=past, norm=norm, ordered=ordered)
@@ -343,8 +353,10 @@ class QuantLlamaAttention(nn.Module):
             position_ids = self.rope.positions(hidden_states.device, past_len, bsz, q_len) if hidden_states.is_cuda \
                 else torch.arange(past_len, kv_seq_len, device=hidden_states.device).unsqueeze(0)
 
+        # (a past that is part of a gradient's graph stays in it by the copies below)
+        traced = past_key_value is not None and torch.is_grad_enabled() and any(t.requires_grad for t in past_key_value)
         if q_len == 1 and attention_mask is None and not output_attentions and self.head_dim == 128 and hidden_states.is_cuda \
-                and bsz * self.num_heads <= ATTENTION_MAX_HEADS:
+                and bsz * self.num_heads <= ATTENTION_MAX_HEADS and not traced:
             context, pair = self.attend_one(hidden_states, position_ids, past_key_value, ordered=ordered)
             return self.project_out(*context), None, pair if use_cache else None
         if past_key_value is None:

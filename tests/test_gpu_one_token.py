@@ -1,0 +1,76 @@
+"""One token behind a (key, value) pair: every past the block took when it copied it into the new pair."""
+import pytest
+import torch
+
+import gptq_triton_amd as G
+from test_gpu_stream import random_quant_model
+
+pytestmark = pytest.mark.gpu
+HEADS, PAST = 8, 37
+
+
+def strided(t):
+    return t.transpose(1, 2).contiguous().transpose(1, 2)
+
+
+def misaligned(t):
+    flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:]
+    return flat.copy_(t.flatten()).view(t.shape)
+
+
+def halves_of_a_longer_one(t):
+    return torch.cat([t, t], dim=2)[:, :, :t.shape[2]]
+
+
+FORMS = {"float32": lambda t: t.float(), "bfloat16": lambda t: t.bfloat16(), "host": lambda t: t.cpu(), "host float32": lambda t: t.cpu().float(),
+         "one for all": lambda t: t[:1], "expanded": lambda t: t[:1].expand(t.shape), "no batch": lambda t: t[0], "strided": strided,
+         "misaligned": misaligned, "part": halves_of_a_longer_one}
+
+
+@pytest.fixture(scope="module")
+def model():
+    return random_quant_model(hidden=1024, inter=2816, heads=HEADS, layers=2, groupsize=128, seed=61)
+
+
+def pairs(bsz, past=PAST, layers=2):
+    gen = torch.Generator(device="cuda").manual_seed(past)
+    # (values that bfloat16 holds as well, the same in every sequence: every form below has the same contents)
+    new = lambda: torch.randn((1, HEADS, past, 128), device="cuda", generator=gen).bfloat16().half().expand(bsz, -1, -1, -1).contiguous()
+    return [(new(), new()) for _ in range(layers)]
+
+
+@pytest.mark.parametrize("form", list(FORMS))
+@pytest.mark.parametrize("bsz", [1, 2])
+def test_forms_of_the_past(model, form, bsz):
+    attn = model.model.layers[0].self_attn
+    x = torch.randn((bsz, 1, 1024), device="cuda", generator=torch.Generator(device="cuda").manual_seed(5)).half()
+    past = pairs(bsz)
+    as_form = [tuple(FORMS[form](t) for t in p) for p in past]
+    want, _, (wk, wv) = attn(hidden_states=x, past_key_value=past[0], use_cache=True)
+    got, _, (gk, gv) = attn(hidden_states=x, past_key_value=as_form[0], use_cache=True)
+    assert torch.equal(got, want) and torch.equal(gk, wk) and torch.equal(gv, wv)
+    assert torch.equal(gk[:, :, :PAST], past[0][0]) and torch.equal(gv[:, :, :PAST], past[0][1])
+    if form != "no batch":   # (the model reads the length of its past from the third dimension)
+        ids = torch.arange(bsz, device="cuda").view(bsz, 1)
+        want, new = model(ids, past_key_values=past, use_cache=True)
+        got, got_new = model(ids, past_key_values=as_form, use_cache=True)
+        assert torch.equal(got, want)
+        for a, b in zip(new, got_new):
+            assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
+def test_a_past_that_takes_a_gradient_stays_in_its_graph(model):
+    attn = model.model.layers[0].self_attn
+    x = torch.randn((1, 1, 1024), device="cuda").half()
+    k, v = (t.requires_grad_() for t in pairs(1)[0])
+    _, _, (pk, pv) = attn(hidden_states=x, past_key_value=(k, v), use_cache=True)
+    pk.sum().backward()
+    assert torch.equal(k.grad, torch.ones_like(k))
+
+
+def test_an_empty_past_is_no_past(model):
+    attn = model.model.layers[0].self_attn
+    x = torch.randn((1, 1, 1024), device="cuda").half()
+    empty = tuple(torch.empty((1, HEADS, 0, 128), dtype=torch.float16, device="cuda") for _ in range(2))
+    want = attn(hidden_states=x)[0]
+    assert torch.equal(attn(hidden_states=x, past_key_value=empty)[0], want)
