@@ -249,7 +249,8 @@ class LlamaForCausalLM(nn.Module):
                 order = order_of(layer.mlp)
                 h, x = add_rms_norm(h, out, n2.weight, n2.variance_epsilon, out_index=order)
                 delta = layer.mlp(x, ordered=True) if order is not None else layer.mlp(x)
-            presents.append(present)
+            presents.append(present if use_cache else None)
+            del present  # (without use_cache a layer's pair is given back before the next one's is made)
         norm = self.model.norm
         return add_rms_norm(h, delta, norm.weight, norm.variance_epsilon)[1], presents
 

@@ -74,3 +74,21 @@ def test_an_empty_past_is_no_past(model):
     empty = tuple(torch.empty((1, HEADS, 0, 128), dtype=torch.float16, device="cuda") for _ in range(2))
     want = attn(hidden_states=x)[0]
     assert torch.equal(attn(hidden_states=x, past_key_value=empty)[0], want)
+
+
+def test_nothing_is_kept_without_use_cache(model):
+    """The pairs of all layers are not alive together when the caller does not ask for them."""
+    ids = torch.zeros((1, 1), dtype=torch.long, device="cuda")
+    past = pairs(1, past=4000)
+    model(ids, past_key_values=past), model(ids, past_key_values=past, use_cache=True)   # (tables and workspaces exist)
+
+    def peak(use_cache):
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        out = model(ids, past_key_values=past, use_cache=use_cache)
+        del out
+        return torch.cuda.max_memory_allocated() - before
+
+    one_layer = 2 * HEADS * 4001 * 128 * 2
+    assert peak(False) + one_layer // 2 < peak(True)
