@@ -298,12 +298,18 @@ class GreedyDecoder:
                        for _ in model.model.layers]
         self.tokens = torch.zeros((bsz, 1), dtype=torch.long, device=dev)
         self.position = torch.zeros((bsz, 1), dtype=torch.int32, device=dev)
-        # with one_launch_end a decode step ends in one launch that picks the tokens, moves the positions on and keeps the tokens
-        # at their places in the sequence.  (It can fetch their embedding rows for the next step too, but a step starts from
-        # `tokens`, which the caller may write to between two steps or two replays of `graph`.)
-        self.one_launch_end = head_argmax_takes(bsz, model.lm_head.weight) and model.lm_head.bias is None
         self.history = torch.zeros((bsz, capacity + 1), dtype=torch.long, device=dev)
         self.graph = None
+        self._graph_keeps_history = False  # whether the captured step is one with one_launch_end
+
+    @property
+    def one_launch_end(self) -> bool:
+        """Whether a decode step ends in one launch that picks the tokens, moves the positions on and keeps the tokens at their
+        places in `history`.  Asked for every step: the caller may replace or convert the lm_head of a decoder that is kept.
+        (The launch can fetch the embedding rows of the next step too, but a step starts from `tokens`, which the caller may
+        write to between two steps or two replays of `graph`.)"""
+        head = self.model.lm_head
+        return head_argmax_takes(self.bsz, head.weight) and head.bias is None
 
     def _layers(self, h, position_ids, kv_offset, attend, end):
         """The decoder stack on hidden states h [B, S, hidden]; every residual add is fused with the RMSNorm that follows it.
@@ -406,7 +412,7 @@ class GreedyDecoder:
         # the tokens are at their places in `history` afterwards; where the sequences stand at different places, or the step
         # does not keep them there, they are collected one by one
         at = stand[0]
-        kept = self.one_launch_end and at >= 0 and min(stand) == max(stand)
+        kept = (self._graph_keeps_history if use_graph else self.one_launch_end) and at >= 0 and min(stand) == max(stand)
         out = None if kept else torch.empty((self.bsz, steps), dtype=torch.long, device=self.tokens.device)
         for i in range(steps):
             if use_graph:
@@ -435,6 +441,7 @@ class GreedyDecoder:
             self.position.copy_(position0)
         torch.cuda.current_stream().wait_stream(side)
         torch.cuda.synchronize()
+        self._graph_keeps_history = self.one_launch_end
         self.graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(self.graph, stream=side):
             self._step()

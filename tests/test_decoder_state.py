@@ -95,6 +95,45 @@ def test_a_step_starts_from_the_tokens_buffer(monkeypatch):
     assert torch.equal(seen[0], model.model.embed_tokens(dec.tokens))
 
 
+def test_an_lm_head_replaced_later(monkeypatch):
+    """The one-launch end is chosen by the lm_head there is at the step, not by the one the decoder was made with."""
+    from gptq_triton_amd import llama
+    cfg = LlamaConfigLite(hidden_size=64, num_attention_heads=2, intermediate_size=64, num_hidden_layers=1, vocab_size=512)
+    model = LlamaForCausalLM(cfg)
+    launches = []
+    monkeypatch.setattr(llama, "head_argmax_takes", lambda rows, weight: weight.shape[0] == 512)
+    monkeypatch.setattr(llama, "greedy_step_end", lambda *a: launches.append(a))
+    dec = GreedyDecoder(model, 2, CAPACITY)
+    x = torch.randn(2, 1, 64)
+    dec._end_step(None, None, model.model.norm, x)
+    assert len(launches) == 1
+    model.lm_head = torch.nn.Linear(64, 300, bias=False)
+    dec._end_step(None, None, model.model.norm, x)
+    assert len(launches) == 1 and torch.equal(dec.tokens, model.lm_head(x).argmax(-1)) and dec.position.tolist() == [[1], [1]]
+    model.lm_head = torch.nn.Linear(64, 512, bias=False)
+    dec._end_step(None, None, model.model.norm, x)
+    assert len(launches) == 2
+
+
+@pytest.mark.gpu
+def test_decoder_whose_lm_head_is_replaced(tmp_path):
+    """An lm_head the launch does not take (a strided weight) after a few steps: the decoder goes on, with the same tokens."""
+    cfg = make_checkpoint(tmp_path, 128, seed=33)
+    model = G.load_quant(str(tmp_path), device="cuda", fuse_mlp=True)
+    ids = torch.arange(6, device="cuda").view(1, 6)
+    want = model.generate_greedy(ids, 13)[:, 6:]
+    dec = GreedyDecoder(model, 1, 24)
+    got = [dec.prefill(ids), dec.decode(4)]
+    assert dec.one_launch_end
+    weight = model.lm_head.weight
+    model.lm_head.weight = torch.nn.Parameter(weight.t().contiguous().t(), requires_grad=False)
+    assert not dec.one_launch_end
+    got += [dec.decode(4), dec.decode(2, use_graph=True)]
+    model.lm_head.weight = weight
+    got.append(dec.decode(2))
+    assert torch.equal(torch.cat(got, dim=1), want)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("bsz", [1, 3])
 def test_replays_follow_tokens_and_prompts_written_between_them(tmp_path, bsz):
