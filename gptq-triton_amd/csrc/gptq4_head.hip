@@ -8,7 +8,7 @@
 // v_mfma_f32_16x16x32_f16 (lane (r, c): 16 bytes of row c), with the x rows as B out of LDS, so that one to sixteen
 // sequences cost the same: 8 KiB of W per wave are in flight while the 8 KiB before are multiplied.  Rows are dealt evenly,
 // not in sixteens: lanes past a tile's rows load nothing.  Sums are rounded to fp16 as the linear layer's output would be;
-// the best (value, index) per x row is kept in registers - the lower index among equal values, as torch.argmax does -, the
+// the best (value, index) per x row is kept in registers - torch.argmax's choice among equal values and NaN -, the
 // workgroups' bests go through the workspace and the last workgroup to arrive picks the winners, one wave per x row.
 #include "../../include/gptq4.h"
 #include "gptq4_internal.h"
@@ -21,7 +21,11 @@ constexpr int HEAD_WAVES = 8;
 constexpr int HEAD_MAX_B = 16;
 constexpr int HEAD_STEPS = 8;  // matrix steps (32 values of every row) per group of loads
 
-__device__ __forceinline__ bool better(float v, int i, float bv, int bi) { return v > bv || (v == bv && i < bi); }
+// torch.argmax's order: NaN above every number, the lower index among equal values.
+__device__ __forceinline__ bool better(float v, int i, float bv, int bi) {
+    if (v != v || bv != bv) return v != v && (bv == bv || i < bi);
+    return v > bv || (v == bv && i < bi);
+}
 
 // NORM: 0 x as it is, 1 its RMSNorm, 2 the RMSNorm of x + delta
 template <int NORM>
@@ -144,7 +148,7 @@ __global__ __launch_bounds__(64 * HEAD_WAVES) void gptq4_head_argmax_kernel(Head
             const int oi = __shfl_xor(bi, o);
             if (better(ov, oi, bv, bi)) bv = ov, bi = oi;
         }
-        const int token = __builtin_amdgcn_readfirstlane(min(bi, p.V - 1));  // (all logits NaN: no winner)
+        const int token = __builtin_amdgcn_readfirstlane(min(bi, p.V - 1));  // (whatever happens, a row of the table)
         if (lane == 0) p.tokens[b] = (long long)token;
         if (p.positions != nullptr) {
             if (lane == 0) {

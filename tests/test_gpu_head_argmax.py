@@ -104,3 +104,37 @@ def test_step_end_moves_the_loop_on(b, k, norm):
         if 4 + i < cap:   # (a place past the end is not written)
             expect[i, 4 + i] = want[i, 0]
     assert torch.equal(history, expect) and head_is_zero()
+
+
+@pytest.mark.parametrize("b,k,v", [(1, 4096, 32000), (3, 1024, 700), (16, 512, 1003)])
+def test_nan_and_infinite_logits(b, k, v):
+    """NaN counts as the largest logit, infinities as numbers, the lowest index among equals: torch.argmax of the same logits."""
+    gen = torch.Generator(device="cuda").manual_seed(b + k)
+    x = (0.5 + torch.rand((b, k), device="cuda", generator=gen)).half()   # positive: a row of one sign has a logit of that sign
+    w = (0.02 * torch.randn((v, k), device="cuda", generator=gen)).half()
+    nan, inf = float("nan"), float("inf")
+
+    def check(expect, x=x):
+        assert ops().lm_head_argmax(x, w).tolist() == expect
+        tokens = torch.zeros((b, 1), dtype=torch.int64, device="cuda")
+        pos = torch.zeros((b, 1), dtype=torch.int32, device="cuda")
+        ops().greedy_step_end(x.view(b, 1, k), None, None, 1e-6, w, tokens, pos, torch.zeros((b, 4), dtype=torch.int64, device="cuda"))
+        assert tokens[:, 0].tolist() == expect
+        assert torch.nn.functional.linear(x, w).argmax(-1).tolist() == expect
+
+    w[v - 3, k // 2] = inf
+    check([v - 3] * b)
+    w[5, 1] = inf
+    check([5] * b)
+    w[v // 2, 7] = nan
+    check([v // 2] * b)
+    w[v - 1, 0] = nan
+    check([v // 2] * b)
+    w[2, k - 1] = nan
+    check([2] * b)
+    bad = x.clone()
+    bad[b - 1, 3] = nan        # every logit of the last row
+    check([2] * (b - 1) + [0], bad)
+    w.fill_(-inf)
+    check([0] * b)
+    assert head_is_zero()
