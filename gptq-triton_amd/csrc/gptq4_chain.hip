@@ -733,17 +733,8 @@ int device_info(DeviceInfo *out) {
 constexpr size_t CHAIN_LDS_BUDGET = 160 * 1024 - 1024;  // dynamic LDS a workgroup may ask for (the rest: the kernel's static words)
 
 int launch_chain(const ChainArgs &a, int grid, size_t lds, hipStream_t stream) {
-    static bool prepared = false;
-    static std::mutex lock;
-    {
-        std::lock_guard<std::mutex> guard(lock);
-        if (!prepared) {
-            const void *fn = reinterpret_cast<const void *>(&gptq4_chain_kernel);
-            hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)CHAIN_LDS_BUDGET);
-            if (e != hipSuccess) return (int)e;
-            prepared = true;
-        }
-    }
+    static LdsGrant grant;
+    if (const int rc = allow_lds(grant, reinterpret_cast<const void *>(&gptq4_chain_kernel), CHAIN_LDS_BUDGET)) return rc;
     // the grid must be resident as a whole (workgroups wait for each other's sums): one workgroup per CU
     int per_cu = 0;
     hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gptq4_chain_kernel, 64 * (CHAIN_NS + CHAIN_NH), lds);

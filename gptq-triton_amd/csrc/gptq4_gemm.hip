@@ -832,20 +832,16 @@ int launch_one(const MatmulArgs &a, int tiles, hipStream_t stream) {
     dim3 grid((unsigned)tiles, (unsigned)a.splitk), block(256);
     const bool perm = a.perm != nullptr;
     // the wide rotary tile stages its cos / sin rows in 32 KiB of LDS on top of the activation tiles: more than
-    // the 64 KiB a launch may ask for unless the kernel is marked for it (once per variant)
+    // the 64 KiB a launch may ask for unless the kernel is marked for it
     const size_t lds = (EPI == EPI_ROPE && MT == 4) ? 2 * 2 * 32 * 64 * sizeof(float) : 0;
     if (a.stream_b && perm) return (int)hipErrorInvalidValue;  // (the entry points gather beforehand)
     const int variant = a.stream_b ? 2 : (perm ? 1 : 0);
     if (lds) {
-        static bool allowed[3] = {false, false, false};
-        if (!allowed[variant]) {
-            const void *fn = variant == 2   ? reinterpret_cast<const void *>(&gptq4_gemm_kernel<EPI, MT, false, false, true>)
-                             : variant == 1 ? reinterpret_cast<const void *>(&gptq4_gemm_kernel<EPI, MT, true>)
-                                            : reinterpret_cast<const void *>(&gptq4_gemm_kernel<EPI, MT, false>);
-            const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return (int)e;
-            allowed[variant] = true;
-        }
+        static LdsGrant grant[3];
+        const void *fn = variant == 2   ? reinterpret_cast<const void *>(&gptq4_gemm_kernel<EPI, MT, false, false, true>)
+                         : variant == 1 ? reinterpret_cast<const void *>(&gptq4_gemm_kernel<EPI, MT, true>)
+                                        : reinterpret_cast<const void *>(&gptq4_gemm_kernel<EPI, MT, false>);
+        if (const int rc = allow_lds(grant[variant], fn, lds)) return rc;
     }
     if (variant == 2)
         hipLaunchKernelGGL((gptq4_gemm_kernel<EPI, MT, false, false, true>), grid, block, lds, stream, a);
@@ -863,13 +859,8 @@ int launch_streamed(const MatmulArgs &a, int workgroups, hipStream_t stream) {
     const size_t lds = (EPI == EPI_ROPE) ? 2 * 2 * 32 * 64 * sizeof(float) : 0;
     if (a.perm != nullptr) return (int)hipErrorInvalidValue;
     if (lds) {
-        static bool allowed = false;
-        if (!allowed) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gptq4_gemm_kernel<EPI, 4, false, true>),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return (int)e;
-            allowed = true;
-        }
+        static LdsGrant grant;
+        if (const int rc = allow_lds(grant, reinterpret_cast<const void *>(&gptq4_gemm_kernel<EPI, 4, false, true>), lds)) return rc;
     }
     hipLaunchKernelGGL((gptq4_gemm_kernel<EPI, 4, false, true>), grid, block, lds, stream, a);
     return (int)hipGetLastError();

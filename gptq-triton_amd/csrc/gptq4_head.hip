@@ -172,13 +172,8 @@ int launch_norm(HeadArgs &a, hipStream_t stream) {
     const int grid = (a.V + a.rows_per_wg - 1) / a.rows_per_wg;
     const size_t lds = (size_t)a.B * (a.K / 8 + 1) * 16;
     if (lds > 48 * 1024) {
-        static bool allowed = false;
-        if (!allowed) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gptq4_head_argmax_kernel<NORM>),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, HEAD_LDS_BYTES);
-            if (e != hipSuccess) return (int)e;
-            allowed = true;
-        }
+        static LdsGrant grant;
+        if (const int rc = allow_lds(grant, reinterpret_cast<const void *>(&gptq4_head_argmax_kernel<NORM>), HEAD_LDS_BYTES)) return rc;
     }
     hipLaunchKernelGGL((gptq4_head_argmax_kernel<NORM>), dim3((unsigned)grid), dim3(64 * HEAD_WAVES), lds, stream, a);
     return (int)hipGetLastError();

@@ -2,6 +2,7 @@
 #pragma once
 
 #include "gptq4_common.h"
+#include "gptq4_lds.h"
 
 // Kernel arguments are fetched with scalar loads where the compiler first needs them, and an early exit or a loop
 // between two uses turns that into two or three dependent round trips to memory at the very start of a launch

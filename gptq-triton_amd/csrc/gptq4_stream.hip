@@ -30,8 +30,6 @@
 #include "gptq4_internal.h"
 #include "gptq4_norm.h"
 
-#include <mutex>
-
 namespace {
 
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
@@ -804,17 +802,8 @@ constexpr size_t STREAM_LDS_BUDGET = 160 * 1024 - 512;  // dynamic LDS a workgro
 
 template <int EPI, int NW, int DEPTH, bool PERM, int NORM, bool NOMATH>
 int launch_kernel(const StreamArgs &a, const StreamPlan &pl, hipStream_t stream) {
-    static bool prepared = false;
-    static std::mutex lock;
-    {
-        std::lock_guard<std::mutex> guard(lock);
-        if (!prepared) {
-            const void *fn = reinterpret_cast<const void *>(&gptq4_stream_kernel<EPI, NW, DEPTH, PERM, NORM, NOMATH>);
-            const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)STREAM_LDS_BUDGET);
-            if (e != hipSuccess) return (int)e;
-            prepared = true;
-        }
-    }
+    static LdsGrant grant;
+    if (const int rc = allow_lds(grant, reinterpret_cast<const void *>(&gptq4_stream_kernel<EPI, NW, DEPTH, PERM, NORM, NOMATH>), STREAM_LDS_BUDGET)) return rc;
     hipLaunchKernelGGL((gptq4_stream_kernel<EPI, NW, DEPTH, PERM, NORM, NOMATH>), dim3((unsigned)pl.workgroups), dim3(64 * NW), pl.lds_bytes,
                        stream, STREAM_HOT_ARGS(a), a);
     return (int)hipGetLastError();
@@ -835,17 +824,8 @@ int launch_shape(const StreamArgs &a, const StreamPlan &pl, bool nomath, hipStre
 
 template <int EPI, int NW, int DEPTH, int NS>
 int launch_tall(const StreamArgs &a, const StreamPlan &pl, hipStream_t stream) {
-    static bool prepared = false;
-    static std::mutex lock;
-    {
-        std::lock_guard<std::mutex> guard(lock);
-        if (!prepared) {
-            const void *fn = reinterpret_cast<const void *>(&gptq4_stream_tall_kernel<EPI, NW, DEPTH, NS>);
-            const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)STREAM_LDS_BUDGET);
-            if (e != hipSuccess) return (int)e;
-            prepared = true;
-        }
-    }
+    static LdsGrant grant;
+    if (const int rc = allow_lds(grant, reinterpret_cast<const void *>(&gptq4_stream_tall_kernel<EPI, NW, DEPTH, NS>), STREAM_LDS_BUDGET)) return rc;
     hipLaunchKernelGGL((gptq4_stream_tall_kernel<EPI, NW, DEPTH, NS>), dim3((unsigned)pl.workgroups), dim3(64 * NW), pl.lds_bytes, stream,
                        STREAM_HOT_ARGS(a), a);
     return (int)hipGetLastError();
