@@ -481,6 +481,14 @@ int gptq4_column_parts(int op, int M, int K, int N, int *begin, int *cols) {
     return parts.count;
 }
 
+int gptq4_planned_kernel(int op, int M, int K, int N) {
+    op &= ~GPTQ4_OP_WITH_PERM;
+    if (M <= SKINNY_MAX_M || N <= 0 || K <= 0 || (K % 64) != 0 || (N % 256) != 0 || op < GPTQ4_OP_MATMUL || op > GPTQ4_OP_QKV_ROTARY) return -GPTQ4_E_SHAPE;
+    const int epi = (op == GPTQ4_OP_MLP_GATEUP) ? EPI_SILU_MUL : (op == GPTQ4_OP_QKV_ROTARY ? EPI_ROPE : EPI_PLAIN);
+    const TiledChoice c = choose_tiled(epi, M, N, K, false);
+    return !c.kslice ? 0 : c.kp.one_round ? 2 : 1;
+}
+
 int gptq4_dequant(const int32_t *qweight, const int32_t *qzeros, const void *scales, const int32_t *g_idx,
                   void *W_out, int K, int N, int groupsize, void *stream) {
     if (!qweight || !qzeros || !scales || !W_out) return -GPTQ4_E_NULL;

@@ -140,7 +140,7 @@ struct KslicePlan {
     int waves;   // waves per workgroup, each with its own slice of K (4 or 8)
     bool paired; // rotary epilogue: tiles of 32 columns of a head plus their 32 rotation partners instead of whole heads
     bool ok;     // false: the shape needs another kernel
-    bool one_round;  // planned by its estimated time, which also was ahead of the tiled kernel's
+    bool one_round;  // planned by its estimated time, or within 7 % of the plan that is: not weighed against the tiled kernel again
     // tail_split > 1 (only with splitk == 1): tiles [0, tail_first) whole, every later one - the last column strips
     // of the launch, all their row tiles - shared by tail_split workgroups along K
     int tail_first, tail_split;

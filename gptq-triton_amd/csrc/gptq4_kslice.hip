@@ -827,7 +827,7 @@ static double one_round_estimate(int epi, int K, const KslicePlan &pl, long cus)
            (pl.splitk > 1 ? c.split + c.more * (pl.splitk - 2) : 0.0);
 }
 
-// What the tiled kernel takes, whatever plan it chooses (us; fitted to the same timings, 10 % off).
+// What the tiled kernel takes, whatever plan it chooses (us; fitted to the same timings, 10 % off; see one_round_margin).
 static double tiled_estimate(int epi, int M, int N, int K) {
     const double tiles = (double)((M + 127) / 128) * (N / (epi == EPI_SILU_MUL ? 128 : 256)) / device_shape().cus, nk = K / 64;
     const double t0 = epi == EPI_PLAIN ? 12.9 : epi == EPI_SILU_MUL ? 8.5 : 19.0;
@@ -836,7 +836,20 @@ static double tiled_estimate(int epi, int M, int N, int K) {
     return t0 + nk * (flat + (tiles > knee ? 0.86 * (tiles - knee) : 0.0));
 }
 
-// The fastest launch of at most one round by that estimate, if it is 5 % ahead of the tiled kernel (ok = false otherwise).
+// How far a launch of one round has to be ahead of the tiled kernel's estimate to be planned (0: never), so that the two
+// estimates' errors do not choose the slower one.  Both were fitted at 24 to 768 rows; against the plan by scores and the tiled
+// kernel they were then timed on 1800 calls outside the fit (17 to 8192 rows, K from 512 to 32768, N from 256 to 32000):
+//   up to 768 rows, 5 % ahead:     on average 11 % (plain, gate/up) and 20 % (rotary) faster; 11 of 871 calls slower, by 5 - 11 %
+//   769 .. 2048 rows, 15 % ahead:  on average 27 % and 29 % faster, 3 of 405 slower (12 % at most); at 5 % ahead 21 were, up to 24 %
+//   2049 .. 8192 rows, 30 % ahead: 40 of 99 calls still go there, 17 % faster, 1 slower; at 5 % ahead 17 were, up to 38 %
+//   K below 1024, over 64 rows:    the tiled kernel takes half of what its line says (512 x 6144 at 512 rows 8.9 us, estimated
+//                                  16.3): 98 of 291 plain and gate/up calls were slower, up to 79 %; no rotary call was
+static double one_round_margin(int epi, int M, int K) {
+    if (K < 1024 && M > 64 && epi != EPI_ROPE) return 0.0;
+    return M <= 768 ? 0.95 : M <= 2048 ? 0.85 : M <= 8192 ? 0.70 : 0.0;
+}
+
+// The fastest launch of at most one round by that estimate, if it is ahead of the tiled kernel by that margin (ok = false otherwise).
 // 96-row tiles exist for this: one row tile for 65 .. 96 rows, two for 129 .. 192, where 64- and 128-row tiles pad a third
 // to a half, each weight decoded once per 96 rows: LLaMA-7B gate/up at 96 rows 35.3 -> 30.1 us, 13B 47.9 -> 38.2; QKV
 // (plain) at 192 rows 37.2 -> 29.5; 4096 x 4096 at 640 rows 37.7 -> 31.0.  (128-row tiles never were the fastest: with two
@@ -844,7 +857,7 @@ static double tiled_estimate(int epi, int M, int N, int K) {
 static KslicePlan one_round_plan(int epi, int M, int N, int K) {
     KslicePlan best = {};
     const int cus = device_shape().cus, nk = K / 64;
-    double best_us = 0.95 * tiled_estimate(epi, M, N, K);
+    double best_us = one_round_margin(epi, M, K) * tiled_estimate(epi, M, N, K);
     for (int mt = 1; mt <= 3; ++mt)
         for (int waves = 4; waves <= 8; waves += 4)
             for (int form = 0; form < (epi == EPI_SILU_MUL ? 1 : 2); ++form) {
@@ -880,8 +893,8 @@ KslicePlan kslice_plan(int epi, int M, int N, int K, bool has_perm) {
     if (t.mode != 1 || t.mt != 0 || t.splitk != 0 || t.wide != 0 || t.waves != 0 || t.paired != 0 || has_perm) return pl;
     const KslicePlan one = one_round_plan(epi, M, N, K);
     if (!one.ok) return pl;
-    // the plan by scores stays where the estimates do not tell the two apart; with its last strips shared along K it takes
-    // some 6 % less than the estimate for whole tiles
+    // the plan by scores stays where the estimates do not tell the two apart (7 %: it may then be level with the tiled kernel's
+    // estimate instead of ahead of it); with its last strips shared along K it takes some 6 % less than the estimate for whole tiles
     const int cus = device_shape().cus;
     const double us = (pl.ok ? one_round_estimate(epi, K, pl, cus) : 0.0) * (pl.tail_split > 1 ? 0.94 : 1.0);
     if (us > 0.0 && us <= 1.07 * one_round_estimate(epi, K, one, cus)) {

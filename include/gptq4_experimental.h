@@ -162,6 +162,10 @@ void gptq4_set_gemv_tuning(int mode /* enum gptq4_kernel_mode */, int depth, int
  * own.  `op` is a GPTQ4_OP_* selector (N of one matrix for the gate/up pair); begin and cols have room for two
  * values (or are NULL).  For diagnostics and tests; no reference counterpart. */
 int gptq4_column_parts(int op, int M, int K, int N, int *begin, int *cols);
+/* Which kernel a call with more than 16 rows is planned for: 0 the tiled one (or, cut into column ranges, one of its own for
+ * every range), 1 the mid-M kernel by its split scores, 2 the mid-M kernel in at most one round of workgroups by its estimated
+ * time; -GPTQ4_E_SHAPE for other calls.  For diagnostics and tests; no reference counterpart. */
+int gptq4_planned_kernel(int op, int M, int K, int N);
 
 /* How often a finishing wave of the small-M kernels polls for another wave's marked partial sums before it gives up
  * and sets GPTQ4_WS_ERROR_WORD (0 = the default, about four million polls).  0xFFFFFFFF is the hook for tests of
