@@ -261,7 +261,7 @@ class QuantLlamaAttention(nn.Module):
             need = max(kv_offset, 0) + hidden_states.shape[1]
         cos, sin = self.rope.get(hidden_states.device, max(need, self.max_position_embeddings))
         rows = hidden_states.shape[0] * hidden_states.shape[1]
-        qkv = self._modules['qkv_proj']
+        qkv = self.qkv_proj
         sw = qkv.stream_weights(rows)
         if sw is not None and (norm is None or rows <= NORM_MAX_ROWS):
             return qkv_rotary_stream(qkv.groupsize, hidden_states, sw[0], sw[1], position_ids, cos, sin, self.num_heads,

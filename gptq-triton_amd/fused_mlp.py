@@ -14,7 +14,7 @@ import torch.nn as nn
 
 from . import _lib
 from .decoder_ops import NORM_MAX_ROWS, check_norm_args, contiguous_delta, norm_fusable, norm_fusion_pays
-from .quant_linear import (QuantLinear, _check_device_tensors, _check_matmul_args, matmul4, stream_pack, stream_rows, stream_unpack,
+from .quant_linear import (QuantLinear, _check_device_tensors, _check_matmul_args, held, matmul4, stream_pack, stream_rows, stream_unpack,
                            tensor_key)
 
 
@@ -305,14 +305,15 @@ class QuantLlamaMLP(nn.Module):
     def _stream_ready(self, x: torch.Tensor) -> bool:
         # (any number of rows: the decode kernels up to _stream_rows, the tiled kernel above 16)
         rows = x.numel() // max(self.infeatures, 1)
-        return self._buffers['_gate_meta'] is not None and not (self._stream_rows < rows <= 16)
+        return held(self, '_gate_meta') is not None and not (self._stream_rows < rows <= 16)
+
+    def _stream_words(self):
+        return held(self, 'gate_proj_qweight'), held(self, '_gate_meta'), held(self, 'up_proj_qweight'), held(self, '_up_meta')
 
     def forward(self, x: torch.Tensor, ordered: bool = False) -> torch.Tensor:
         if self._stream_ready(x):
-            own = self._buffers
-            mid = llama_mlp_4_stream(self.groupsize, x, own['gate_proj_qweight'], own['_gate_meta'], own['up_proj_qweight'], own['_up_meta'],
-                                     None if ordered else own['_compact_rows'])
-            return self._modules['down_proj'].multiply(mid, ordered=True)  # the columns of gate and up are laid out in the order down_proj reads
+            mid = llama_mlp_4_stream(self.groupsize, x, *self._stream_words(), None if ordered else held(self, '_compact_rows'))
+            return self.down_proj.multiply(mid, ordered=True)  # the columns of gate and up are laid out in the order down_proj reads
         w, perm, down_q = self._chained_weights()
         return self._down(llama_mlp_4(self.groupsize, x, *w, None if ordered else perm), down_q)
 
@@ -325,10 +326,8 @@ class QuantLlamaMLP(nn.Module):
     def forward_normed(self, h: torch.Tensor, delta: Optional[torch.Tensor], norm_weight: torch.Tensor, eps: float):
         """(h + delta, forward(RMSNorm(h + delta))): the residual add and the norm run inside the gate/up launch."""
         if self._stream_ready(h) and h.numel() // self.infeatures <= NORM_MAX_ROWS:
-            own = self._buffers
-            s, mid = llama_mlp_4_stream(self.groupsize, h, own['gate_proj_qweight'], own['_gate_meta'], own['up_proj_qweight'], own['_up_meta'],
-                                        own['_compact_rows'], norm=(delta, norm_weight, eps))
-            return s, self._modules['down_proj'].multiply(mid, ordered=True)
+            s, mid = llama_mlp_4_stream(self.groupsize, h, *self._stream_words(), held(self, '_compact_rows'), norm=(delta, norm_weight, eps))
+            return s, self.down_proj.multiply(mid, ordered=True)
         w, perm, down_q = self._chained_weights()
         s, mid = norm_llama_mlp_4(self.groupsize, h, delta, norm_weight, eps, *w, perm)
         return s, self._down(mid, down_q)

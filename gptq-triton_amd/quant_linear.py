@@ -33,6 +33,13 @@ def only_itself(m, cls) -> bool:
                 or _nn_module._global_backward_hooks or _nn_module._global_backward_pre_hooks)
 
 
+def held(m: nn.Module, name: str):
+    """m.<name> of what usually is a buffer, without the half microsecond that nn.Module's __getattr__ takes; a loader may have
+    made it a parameter or something else."""
+    own = m._buffers
+    return own[name] if name in own else getattr(m, name)
+
+
 def _check_matmul_args(a: torch.Tensor, qweight: torch.Tensor, groupsize: int):
     # the reference's host-side contract (quant_linear.py:244-257)
     assert a.shape[-1] == qweight.shape[0] * 8, "A must be a multiple of 8 in the last dimension"
@@ -341,30 +348,28 @@ class QuantLinear(nn.Module):
         """perm of kernel_weights() alone (None without act-order)."""
         if self.g_idx is None:
             return None
-        own = self._buffers
-        return own['_compact_perm'] if own['_compact_perm'] is not None else self._act_order()[1]
+        perm = held(self, '_compact_perm')
+        return perm if perm is not None else self._act_order()[1]
 
     def stream_weights(self, rows: int = 1):
         """(sweight, smeta, perm) if the module is in streaming order, else None (any number of rows: up to `_stream_rows`
         the decode kernels read these words, above that the tiled kernel does)."""
-        own = self._buffers
-        meta = own['_stream_meta']
+        meta = held(self, '_stream_meta')
         if meta is None or self._stream_rows < rows <= 16:
             return None
-        return own['qweight'], meta, own['_compact_perm']
+        return held(self, 'qweight'), meta, held(self, '_compact_perm')
 
     def bias_tensor(self):
-        return self._buffers['bias'] if 'bias' in self._buffers else self._parameters.get('bias')
+        return self._parameters['bias'] if 'bias' in self._parameters else held(self, 'bias')
 
     def multiply(self, x: torch.Tensor, ordered: bool = False) -> torch.Tensor:
         """forward(x); ordered: x already is in the order of the sorted rows (act-order), no gather needed."""
-        own = self._buffers  # (looked up here and not through nn.Module's __getattr__: that costs half a microsecond each)
-        meta = own['_stream_meta']
+        meta = held(self, '_stream_meta')
         bias = self.bias_tensor()
         if meta is not None and not self._stream_rows < x.numel() // max(self.infeatures, 1) <= 16:
-            return matmul4_stream(self.groupsize, x, own['qweight'], meta, bias, None if ordered else own['_compact_perm'])
+            return matmul4_stream(self.groupsize, x, held(self, 'qweight'), meta, bias, None if ordered else held(self, '_compact_perm'))
         qweight, perm = self.kernel_weights()
-        return matmul4(self.groupsize, x, qweight, own['scales'], own['qzeros'], bias, None if ordered else perm)
+        return matmul4(self.groupsize, x, qweight, held(self, 'scales'), held(self, 'qzeros'), bias, None if ordered else perm)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         return self.multiply(x)
