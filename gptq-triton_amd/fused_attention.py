@@ -20,7 +20,7 @@ import torch.nn as nn
 from . import _lib
 from .decoder_ops import (ATTENTION_MAX_HEADS, NORM_MAX_ROWS, check_norm_args, contiguous_delta, decode_attention, extend_attention,
                           norm_fusable, norm_fusion_pays, prefill_attention)
-from .quant_linear import QuantLinear, _check_device_tensors, _check_matmul_args, inverse_permutation, only_itself, tensor_key
+from .quant_linear import QuantLinear, _check_device_tensors, _check_matmul_args, InverseOrder, only_itself
 
 
 @dataclass
@@ -246,8 +246,8 @@ class QuantLlamaAttention(nn.Module):
         self.rotary_emb = rotary_emb
         self.rope = RotaryTable(self.head_dim, self.max_position_embeddings, _rope_base(config))
         self.layer_idx = None
-        self._context_order = None
-        self._input_order = None
+        self._context_order = InverseOrder()
+        self._input_order = InverseOrder()
 
     def project_qkv(self, hidden_states: torch.Tensor, position_ids: torch.Tensor,
                     kv_out=None, kv_offset: int = 0, norm=None, ordered: bool = False):
@@ -276,21 +276,13 @@ class QuantLlamaAttention(nn.Module):
         None without act-order and where o_proj is to be called as a module (only_itself).
         decode_attention(out_index=...) writes in that order."""
         perm = self.o_proj.row_permutation() if only_itself(self.o_proj, QuantLinear) else None
-        if perm is None:
-            return None
-        if self._context_order is None or self._context_order[0] != tensor_key(perm):
-            self._context_order = (tensor_key(perm), inverse_permutation(perm))
-        return self._context_order[1]
+        return None if perm is None else self._context_order.of(perm)
 
     def input_order(self):
         """The same for the input of the fused QKV projection: rms_norm / add_rms_norm(out_index=...) write in
         that order, and project_qkv(ordered=True) then runs without a gather.  None without act-order."""
         perm = self.qkv_proj.row_permutation()
-        if perm is None:
-            return None
-        if self._input_order is None or self._input_order[0] != tensor_key(perm):
-            self._input_order = (tensor_key(perm), inverse_permutation(perm))
-        return self._input_order[1]
+        return None if perm is None else self._input_order.of(perm)
 
     def attend_one(self, hidden_states: torch.Tensor, position_ids: torch.Tensor, past_key_value, norm=None, ordered: bool = False):
         """One token of each sequence behind a (key, value) pair (or None): (the arguments of project_out, the grown pair), and

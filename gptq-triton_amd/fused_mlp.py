@@ -14,7 +14,7 @@ import torch.nn as nn
 
 from . import _lib
 from .decoder_ops import NORM_MAX_ROWS, check_norm_args, contiguous_delta, norm_fusable, norm_fusion_pays
-from .quant_linear import (QuantLinear, _check_device_tensors, _check_matmul_args, held, matmul4, stream_pack, stream_rows, stream_unpack,
+from .quant_linear import (InverseOrder, QuantLinear, _check_device_tensors, _check_matmul_args, held, matmul4, stream_pack, stream_rows, stream_unpack,
                            tensor_key)
 
 
@@ -126,7 +126,7 @@ class QuantLlamaMLP(nn.Module):
             self.g_idx = None
         self._sorted = None
         self._chained = None
-        self._input_order = None
+        self._input_order = InverseOrder()
         # compact(): the six gate / up buffers hold the layout forward() multiplies with; these say how it was made
         self._is_compact = False
         self.register_buffer('_compact_rows', None, persistent=False)   # row permutation (act-order input), or None
@@ -295,12 +295,7 @@ class QuantLlamaMLP(nn.Module):
         rms_norm / add_rms_norm(out_index=...) write in that order and forward(x, ordered=True) runs
         without a gather."""
         perm = self._compact_rows if (self._is_compact or self._gate_meta is not None) else self._chained_weights()[1]
-        if perm is None:
-            return None
-        if self._input_order is None or self._input_order[0] != tensor_key(perm):
-            from .quant_linear import inverse_permutation
-            self._input_order = (tensor_key(perm), inverse_permutation(perm))
-        return self._input_order[1]
+        return None if perm is None else self._input_order.of(perm)
 
     def _stream_ready(self, x: torch.Tensor) -> bool:
         # (any number of rows: the decode kernels up to _stream_rows, the tiled kernel above 16)

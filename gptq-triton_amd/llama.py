@@ -22,7 +22,7 @@ from .decoder_ops import (NORM_MAX_HIDDEN, add_rms_norm, decode_attention, greed
                           norm_fusion_pays, prefill_attention, rms_norm)
 from .fused_attention import KV_AT_POSITION, LlamaConfigLite, QuantLlamaAttention
 from .fused_mlp import QuantLlamaMLP, llama_mlp_4_stream
-from .quant_linear import QuantLinear, inverse_permutation, only_itself, stream_rows, tensor_key
+from .quant_linear import InverseOrder, QuantLinear, only_itself, stream_rows
 
 # the rows the decode kernels built on the streaming-order weight layout take (more rows: the mid-M and tiled kernels)
 STREAM_BATCH = 16
@@ -80,7 +80,8 @@ class LlamaMLP(nn.Module):
         self.gate_proj = nn.Linear(h, i, bias=False)
         self.down_proj = nn.Linear(i, h, bias=False)
         self.up_proj = nn.Linear(h, i, bias=False)
-        self._same_rows = self._most_rows = None
+        self._same_rows = InverseOrder()  # of gate's and up's permutation, where it is one
+        self._most_rows = None
 
     def _pair(self, rows: int):
         """(groupsize, gate words and {scale, zero} words, up's, row permutation) where one launch can compute
@@ -92,17 +93,9 @@ class LlamaMLP(nn.Module):
         if g is None or u is None or gate.groupsize != up.groupsize or g[0].shape != u[0].shape \
                 or gate.bias_tensor() is not None or up.bias_tensor() is not None or rows <= 16 and self._pair_rows(gate) < rows:
             return None
-        if (g[2] is None) != (u[2] is None) or g[2] is not None and self._shared_order(g[2], u[2]) is None:
+        if (g[2] is None) != (u[2] is None) or g[2] is not None and self._same_rows.of(g[2], u[2]) is None:
             return None
         return gate.groupsize, g[0], g[1], u[0], u[1], g[2]
-
-    def _shared_order(self, perm, other):
-        """The inverse of the row permutation of gate and up where it is one, else None.  (Compared once per pair of
-        permutations: the only synchronisation here.)"""
-        key = tensor_key(perm, other)
-        if self._same_rows is None or self._same_rows[0] != key:
-            self._same_rows = (key, inverse_permutation(perm) if torch.equal(perm, other) else None)
-        return self._same_rows[1]
 
     def input_order(self):
         """As QuantLlamaMLP.input_order: None without act-order, where gate and up each have an order of their own, and where
@@ -111,7 +104,7 @@ class LlamaMLP(nn.Module):
         if not (only_itself(self, LlamaMLP) and only_itself(gate, QuantLinear) and only_itself(up, QuantLinear)) \
                 or gate.g_idx is None or up.g_idx is None:
             return None
-        return self._shared_order(gate.row_permutation(), up.row_permutation())
+        return self._same_rows.of(gate.row_permutation(), up.row_permutation())
 
     def _pair_rows(self, gate) -> int:
         if self._most_rows is None:

@@ -112,6 +112,25 @@ def inverse_permutation(perm: torch.Tensor) -> torch.Tensor:
     return inv
 
 
+class InverseOrder:
+    """inverse_permutation() of a module's row permutation, worked out once per permutation.  The permutation is kept with it:
+    what tensor_key() names cannot come back as another tensor's address then."""
+
+    def __init__(self):
+        self._kept = None  # (key, the permutations, the inverse)
+
+    def of(self, *perms):
+        """The inverse of the permutation that all of `perms` are; None where they differ (looking at them synchronises, once), and
+        in a call that is being captured before the first one that is not."""
+        key = tensor_key(*perms)
+        if self._kept is None or self._kept[0] != key:
+            if perms[0].is_cuda and torch.cuda.is_current_stream_capturing():
+                return None
+            same = all(torch.equal(perms[0], p) for p in perms[1:])
+            self._kept = (key, perms, inverse_permutation(perms[0]) if same else None)
+        return self._kept[2]
+
+
 def _nibble_rows(qweight: torch.Tensor) -> torch.Tensor:
     """[K/8, N] packed words -> [K, N] nibbles (int64), plain torch."""
     shifts = torch.arange(0, 32, 4, device=qweight.device, dtype=torch.int64).view(1, 8, 1)
