@@ -626,6 +626,7 @@ PyObject *greedy_step_end(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
 
 // set_workspace(device index, stream handle, address, bytes): what _lib.workspace() made for that stream
 PyObject *set_workspace(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
     GPTQ4_TAKES(4)
     Workspace w;
     w.device = (int)PyLong_AsLong(v[0]);
@@ -640,6 +641,7 @@ PyObject *set_workspace(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
         }
     g_workspaces.push_back(w);
     Py_RETURN_NONE;
+    END_HANDLE_TH_ERRORS
 }
 
 // init(workspace hook, error hook)
