@@ -108,7 +108,10 @@ def assemblies(tmp_path_factory):
     return {name: _assembly(CSRC / name, tmp) for name in ("gptq4_gemm.hip", "gptq4_kslice.hip")}
 
 
-@pytest.mark.parametrize("source,variants", [("gptq4_gemm.hip", 9), ("gptq4_kslice.hip", 19)])
+ACT_ORDER_GEMM = re.compile(r"gptq4_gemm_kernelILi\dELi\dELb1E")  # <EPI, MT, PERM = true, ..>
+
+
+@pytest.mark.parametrize("source,variants", [("gptq4_gemm.hip", 15), ("gptq4_kslice.hip", 48)])
 def test_hand_written_wait_counts_match_the_loads_behind_the_lds_direct_loads(assemblies, source, variants):
     with_waits = 0
     for name, lines in _kernels(assemblies[source]):
@@ -116,9 +119,16 @@ def test_hand_written_wait_counts_match_the_loads_behind_the_lds_direct_loads(as
         for n, behind, at in found:
             assert behind >= n, (f"{name}: a path reaches `{lines[at][0]}` with only {behind} vector-memory instructions "
                                  f"behind the activation tile's LDS-direct loads: the tile may not have landed")
+        # (the act-order variants of the tiled kernel stage their tiles through registers and have no such wait)
+        assert bool(found) != bool(ACT_ORDER_GEMM.search(name)), f"{name}: the scan sees {len(found)} paths to such a wait"
         with_waits += bool(found)
-    # (the act-order variants of the tiled kernel stage their tiles through registers and have no such wait)
-    assert with_waits >= variants, f"only {with_waits} kernel variants of {source} show such waits: the scan no longer sees them"
+    assert with_waits == variants, f"{with_waits} kernel variants of {source} show such waits"
+
+
+def test_the_scan_covers_the_96_row_tiles(assemblies):
+    """Five variants (plain, wide strips, gate/up, whole and paired rotary heads) on both weight layouts."""
+    tall = {name for name, lines in _kernels(assemblies["gptq4_kslice.hip"]) if re.search(r"kslice_kernelILi\dELi3E", name) and _paths_to_waits(lines)}
+    assert len(tall) == 10
 
 
 def test_the_scan_sees_a_missing_load():
