@@ -156,7 +156,8 @@ int setup_norm(MatmulArgs &a, const void *delta, const void *norm_weight, void *
     return 0;
 }
 
-// M > 16: the mid-M kernel where it is the faster one, else the tiled kernel.  Measured at LLaMA-7B /
+// M > 16: the mid-M kernel where it is the faster one, else the tiled kernel.  (A plan of one round was weighed against the tiled
+// kernel when it was made: one_round_margin in gptq4_kslice.hip.)  The crossovers of the plan by scores, measured at LLaMA-7B /
 // 13B / 30B shapes, 256..768 rows: the tiled kernel takes over once it has enough wide tiles (72 for a plain
 // projection, 160 for the gate/up pair, more than 192 with the rotary epilogue: LLaMA-7B QKV at 512 rows, 192 tiles, 75 -> 68 us).
 // (Tile counts just over one per CU used to stay with the mid-M kernel for the rotary epilogue; since the tiled kernel
@@ -858,7 +859,7 @@ static int stream_fill(StreamArgs &a, int epi, int groupsize, void *workspace, s
     if (!pl.ok) return -GPTQ4_E_SHAPE;
     if (workspace == nullptr || workspace_bytes < GPTQ4_WS_HEAD_BYTES) return -GPTQ4_E_WORKSPACE;
     if (pl.tall && a.perm != nullptr) {
-        // the kernel for more than STREAM_MAX_M rows does not gather: one small launch does, into the workspace behind the head
+        // the kernel that fetches its rows with the units does not gather: one small launch does, into the workspace behind the head
         const size_t bytes = (size_t)a.M * a.K * sizeof(half_t);
         if (workspace_bytes < GPTQ4_WS_HEAD_BYTES + bytes) return -GPTQ4_E_WORKSPACE;
         half_t *xg = reinterpret_cast<half_t *>(reinterpret_cast<char *>(workspace) + GPTQ4_WS_HEAD_BYTES);

@@ -207,7 +207,7 @@ struct StreamPlan {
     int xrow, red_off, nat_off;
     size_t lds_bytes;
     bool ok;
-    bool tall;  // 5 .. 16 rows: the kernel that fetches its A operand with every unit
+    bool tall;  // the kernel that fetches its A operand with every unit: 5 .. 16 rows, and fewer that with all of K do not fit the LDS
 };
 struct StreamTuning {
     int waves, depth;  // 0 = automatic

@@ -1,14 +1,14 @@
-// Dequant-fused matmul for mid-sized M (17 .. a few hundred rows) on gfx950.
+// Dequant-fused matmul for mid-sized M (17 .. a few hundred rows, a few thousand of a narrow matrix) on gfx950.
 //
 // With so few rows there is one row tile (or a handful), so the tiled kernel's tile count
 // - N / 256 - leaves most CUs idle unless K is split across workgroups, and every split
 // costs a round trip of fp32 partial sums through memory.  Here the split along K happens
 // inside the workgroup: a workgroup owns a strip of only 64 output columns (128 for a
-// rotary head), and its four waves each run the tiled kernel's wave loop over their own
-// contiguous quarter of K.  The waves share nothing while they stream: each has its own
+// rotary head), and its four or eight waves each run the tiled kernel's wave loop over their own
+// contiguous part of K.  The waves share nothing while they stream: each has its own
 // double-buffered activation tile in LDS, filled by its own LDS-direct loads, so the loop
-// has no barrier at all.  At the end the four accumulator sets meet in LDS: row block mt
-// is summed and finished by wave mt.
+// has no barrier at all.  At the end the accumulator sets meet in LDS, where the waves share the
+// row blocks among them.
 //
 // Wave tile: (32*MT) rows x NB blocks of 64 columns.
 //   plain   : NB = 1, one 64-column strip; or (WIDE, long K and many rows) NB = 2, two adjacent strips.
@@ -39,6 +39,7 @@
 namespace {
 
 constexpr int BK = 64;
+
 // WIDE (plain epilogue only): two adjacent 64-column blocks per wave tile, like a rotary head.
 // KS: waves of the workgroup, each with its own slice of K (4 or 8).  A wave spends about half of its life
 // waiting (first loads, the exchanges at the end) and the other half issuing ~20 instructions per MFMA, one wave
@@ -638,10 +639,9 @@ int launch_waves(const MatmulArgs &a, const KslicePlan &pl, hipStream_t stream) 
                               : launch_one<EPI_ROPE, 2, false, KS, true>(a, pl.tiles, stream);
     }
     if constexpr (KS == 8) {
-        // 32-row tiles with two column blocks per wave tile are never planned with eight waves (kslice_plan)
         if (EPI == EPI_PLAIN && !pl.wide)
             return pl.mt == 1 ? launch_one<EPI_PLAIN, 1, false, 8>(a, pl.tiles, stream) : launch_one<EPI_PLAIN, 2, false, 8>(a, pl.tiles, stream);
-        // (128-column strips of a plain projection on 32-row tiles are never planned with eight waves)
+        // (128-column strips of a plain projection on 32-row tiles are not built for eight waves; neither plan asks for them)
         if (EPI == EPI_PLAIN) return pl.mt == 1 ? (int)hipErrorInvalidValue : launch_one<EPI_PLAIN, 2, true, 8>(a, pl.tiles, stream);
         return pl.mt == 1 ? launch_one<EPI, 1, false, 8>(a, pl.tiles, stream) : launch_one<EPI, 2, false, 8>(a, pl.tiles, stream);
     } else {
@@ -661,18 +661,17 @@ int launch_epi(const MatmulArgs &a, const KslicePlan &pl, hipStream_t stream) {
 
 KsliceTuning g_kslice_tuning = {1, 0, 0, 0, 0, 0};
 
-// Row tile: 32 rows up to M = 32, else 64 - or 32 for plain projections where that scores higher, see below.  (128-row tiles decode each weight once instead of twice at M = 128 and
-// halve the instructions per MFMA, but came out no faster: 17.3 against 15.1 us on 4096 x 4096, level on
-// 11008 x 4096.  Four activation tiles per wave instead of two - the tile three K tiles on requested while one is
-// multiplied - gained nothing that eight waves do not gain as well.)  How far K is split across workgroups on top is
-// scored below.
-// One variant of the plan: the rotary epilogue on whole heads or on paired quarter heads.  *score: that of the split it
+// The plan by scores, for launches of more than one round, forced shapes, and calls outside one_round_margin's range.
+// Row tile: 32 rows up to M = 32, else 64 - or 32 for plain projections where that scores higher, see below.  (Four
+// activation tiles per wave instead of two - the tile three K tiles on requested while one is multiplied - gained nothing
+// that eight waves do not gain as well.)  How far K is split across workgroups on top is scored below.
+// One variant of it: the rotary epilogue on whole heads or on paired quarter heads.  *score: that of the split it
 // chose (0 with a forced split).
 static KslicePlan plan_variant(int epi, int M, int N, int K, bool has_perm, bool paired, double *score) {
     KslicePlan pl = {};
     // eight waves for plain projections wherever they fit (checked below): ahead of four waves by 4 - 18 % at
-    // LLaMA-7B / 30B shapes from 17 to 256 rows, level at 512; the gate/up pair and the rotary epilogue take eight up to
-    // 32 rows (one workgroup per CU then: two column blocks per wave tile need the registers of a whole SIMD; 7B QKV
+    // LLaMA-7B / 30B shapes from 17 to 256 rows with the same tiles, level at 512; the gate/up pair and the rotary epilogue
+    // take eight up to 32 rows (one workgroup per CU then: two column blocks per wave tile need the registers of a whole SIMD; 7B QKV
     // 16.9 -> 15.6 us, gate/up 19.6 -> 18.6, 13B QKV 19.3 -> 18.0) and stay at four beyond (level or 3 % behind)
     // (paired quarter heads: one column block per wave tile like a plain strip, so eight waves fit as they do there)
     pl.paired = paired;
@@ -804,7 +803,7 @@ static KslicePlan rounds_plan(int epi, int M, int N, int K, bool has_perm) {
 // with steps = K tiles of the longest wave, `step` that of one workgroup or of two to a CU, `load` what the others' traffic
 // adds to a step, and the cost of splitting K across workgroups (the first split, then every further one).  One line per
 // kernel variant, in us, fitted to 3500 timings over 20 projections (K and N from 2048 to 19968) at 24 to 768 rows with the
-// weights from HBM: 3 - 7 % off per variant.
+// weights from HBM: 3 - 7 % off per variant.  (Where it may decide: one_round_margin.)
 struct RoundCost {
     float t0, one, two, load, split, more;  // two = 0: one workgroup to a CU
 };
