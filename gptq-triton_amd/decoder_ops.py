@@ -98,9 +98,10 @@ HEAD_MAX_ROWS = 16
 
 
 def head_argmax_takes(rows: int, weight: torch.Tensor) -> bool:
-    """Whether the lm_head kernels take this many rows of an fp16 weight [V, K]."""
+    """Whether the lm_head kernels take this many rows of an fp16 weight [V, K] (which they read 16 bytes at a time)."""
     k = weight.shape[1]
-    return weight.is_cuda and weight.dtype == torch.float16 and weight.is_contiguous() and k % 256 == 0 and 0 < rows <= HEAD_MAX_ROWS \
+    return weight.is_cuda and weight.dtype == torch.float16 and weight.is_contiguous() and weight.data_ptr() % 16 == 0 \
+        and k % 256 == 0 and 0 < rows <= HEAD_MAX_ROWS \
         and rows * (k + 8) * 2 <= 160 * 1024 - 2048 and weight.numel() * 2 < 0x7FFFFFF0
 
 
@@ -112,7 +113,8 @@ def lm_head_argmax(x: torch.Tensor, weight: torch.Tensor, max_rows: int = HEAD_M
     rows = x.numel() // max(k, 1)
     if rows > max_rows or weight.dim() != 2 or weight.shape[1] != k or not x.is_cuda or x.dtype != torch.float16 or not head_argmax_takes(rows, weight):
         return torch.nn.functional.linear(x, weight).argmax(-1)
-    out = _lib.host().lm_head_argmax(x.contiguous(), weight)
+    x = x.contiguous()
+    out = _lib.host().lm_head_argmax(x if x.data_ptr() % 16 == 0 else x.clone(), weight)
     if out is None:
         raise _lib.refused("lm_head_argmax")
     return out

@@ -138,3 +138,21 @@ def test_nan_and_infinite_logits(b, k, v):
     w.fill_(-inf)
     check([0] * b)
     assert head_is_zero()
+
+
+def off_by_one(t):
+    flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:]
+    return flat.copy_(t.flatten()).view(t.shape)
+
+
+@pytest.mark.parametrize("b", [1, 5, 16])
+@pytest.mark.parametrize("which", ["x", "weight", "both"])
+def test_operands_off_the_16_byte_grid(b, which):
+    """Views into a flat buffer: the library reads 16 bytes at a time and refuses them, the function does not."""
+    gen = torch.Generator(device="cuda").manual_seed(b)
+    x = torch.randn((b, 1, 2048), device="cuda", generator=gen).half()
+    w = 0.02 * torch.randn((1000, 2048), device="cuda", generator=gen).half()
+    best = torch.arange(b, device="cuda") * 7 + 3
+    w[best] = 0.05 * x[:, 0]   # row `best` wins by far: its logit is about 100 where the others' spread is about 1
+    got = ops().lm_head_argmax(off_by_one(x) if which != "weight" else x, off_by_one(w) if which != "x" else w)
+    assert torch.equal(got.view(-1), best)
