@@ -39,6 +39,20 @@ def pairs(bsz, past=PAST, layers=2):
     return [(new(), new()) for _ in range(layers)]
 
 
+class KeptPair:
+    """A transformers Cache of one layer, as far as the attention block asks."""
+
+    def __init__(self, k, v, form=lambda t: t):
+        self.k, self.v, self.form = k, v, form
+
+    def get_seq_length(self, layer):
+        return self.k.shape[2]
+
+    def update(self, k, v, layer):
+        self.k, self.v = (self.form(torch.cat([a, b], dim=2)) for a, b in ((self.k, k), (self.v, v)))
+        return self.k, self.v
+
+
 @pytest.mark.parametrize("form", list(FORMS))
 @pytest.mark.parametrize("bsz", [1, 2])
 def test_forms_of_the_past(model, form, bsz):
@@ -92,3 +106,21 @@ def test_nothing_is_kept_without_use_cache(model):
 
     one_layer = 2 * HEADS * 4001 * 128 * 2
     assert peak(False) + one_layer // 2 < peak(True)
+
+
+@pytest.mark.parametrize("past", [None, PAST])
+def test_no_sequences(model, past, monkeypatch):
+    """A batch that has run empty: no rows in, none out."""
+    ids = torch.zeros((0, 1), dtype=torch.long, device="cuda")
+    pair = None if past is None else pairs(0, past)
+    rows = 1 if past is None else past + 1
+    logits, new = model(ids, past_key_values=pair, use_cache=True)
+    assert logits.shape == (0, 1, 320) and all(t.shape == (0, HEADS, rows, 128) for p in new for t in p)
+    x = torch.zeros((0, 1, 1024), dtype=torch.float16, device="cuda")
+    attn = model.model.layers[0].self_attn
+    out, _, (k, v) = attn(hidden_states=x, past_key_value=None if pair is None else pair[0], use_cache=True)
+    assert out.shape == x.shape and k.shape == v.shape == (0, HEADS, rows, 128)
+    held = None if pair is None else KeptPair(*pair[0])
+    monkeypatch.setattr(attn, "layer_idx", 0)
+    out, _ = attn(hidden_states=x, position_ids=ids, past_key_values=held, position_embeddings=())
+    assert out.shape == x.shape
