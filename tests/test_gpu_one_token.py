@@ -124,3 +124,29 @@ def test_no_sequences(model, past, monkeypatch):
     monkeypatch.setattr(attn, "layer_idx", 0)
     out, _ = attn(hidden_states=x, position_ids=ids, past_key_values=held, position_embeddings=())
     assert out.shape == x.shape
+
+
+@pytest.mark.parametrize("bsz", [1, 2])
+@pytest.mark.parametrize("form", ["misaligned", "strided", "part"])
+def test_forms_of_a_cache(model, form, bsz, monkeypatch):
+    """One token with a Cache that hands back its rows in other forms than a contiguous aligned tensor (those may take torch's
+    attention, which rounds the probabilities to fp16: 2^-11 of a value each, and the result once more)."""
+    attn = model.model.layers[0].self_attn
+    monkeypatch.setattr(attn, "layer_idx", 0)
+    x = torch.randn((bsz, 1, 1024), device="cuda", generator=torch.Generator(device="cuda").manual_seed(6)).half()
+    ids = torch.full((bsz, 1), PAST, dtype=torch.long, device="cuda")
+    step = lambda cache: attn(hidden_states=x, position_ids=ids, past_key_values=cache, position_embeddings=())[0]
+    want, got = step(KeptPair(*pairs(bsz)[0])), step(KeptPair(*pairs(bsz)[0], form=FORMS[form]))
+    assert (got - want).float().norm() <= 2 ** -9 * want.float().norm()
+
+
+def test_a_cache_that_takes_a_gradient_stays_in_its_graph(model, monkeypatch):
+    attn = model.model.layers[0].self_attn
+    monkeypatch.setattr(attn, "layer_idx", 0)
+    x = torch.randn((1, 1, 1024), device="cuda").half()
+    k, v = (t.requires_grad_() for t in pairs(1)[0])
+    seen = []
+    hook = attn.o_proj.register_forward_pre_hook(lambda m, args: seen.append(args[0]))
+    attn(hidden_states=x, position_ids=torch.full((1, 1), PAST, device="cuda"), past_key_values=KeptPair(k, v), position_embeddings=())
+    hook.remove()
+    assert seen[0].requires_grad
