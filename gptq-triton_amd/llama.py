@@ -223,6 +223,7 @@ class LlamaForCausalLM(nn.Module):
         bsz, q_len, _ = h.shape
         position_ids = layers[0].self_attn.rope.positions(h.device, past_len, bsz, q_len)
         inside = q_len == 1 and all(l.self_attn.norm_fusable(bsz) and l.mlp.norm_fusable(bsz) for l in layers)
+        h = h.contiguous()  # (the projections that normalise their own input take no strides)
         presents = []
         delta = None
         for i, layer in enumerate(layers):

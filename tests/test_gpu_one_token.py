@@ -150,3 +150,14 @@ def test_a_cache_that_takes_a_gradient_stays_in_its_graph(model, monkeypatch):
     attn(hidden_states=x, position_ids=torch.full((1, 1), PAST, device="cuda"), past_key_values=KeptPair(k, v), position_embeddings=())
     hook.remove()
     assert seen[0].requires_grad
+
+
+def test_embedding_rows_with_a_stride(model):
+    ids = torch.full((1, 1), 11, dtype=torch.long, device="cuda")
+    want = model(ids, past_key_values=pairs(1))[0]
+    hook = model.model.embed_tokens.register_forward_hook(lambda m, args, rows: torch.stack([rows, rows], -1)[..., 0])
+    try:
+        got = model(ids, past_key_values=pairs(1))[0]
+    finally:
+        hook.remove()
+    assert torch.equal(got, want)
