@@ -353,7 +353,7 @@ class QuantLlamaAttention(nn.Module):
         # (a past that is part of a gradient's graph stays in it by the copies below)
         traced = past_key_value is not None and torch.is_grad_enabled() and any(t.requires_grad for t in past_key_value)
         if q_len == 1 and attention_mask is None and not output_attentions and self.head_dim == 128 and hidden_states.is_cuda \
-                and 0 < bsz * self.num_heads <= ATTENTION_MAX_HEADS and not traced:
+                and bsz * self.num_heads <= ATTENTION_MAX_HEADS and not traced:
             context, pair = self.attend_one(hidden_states, position_ids, past_key_value, ordered=ordered)
             return self.project_out(*context), None, pair if use_cache else None
         if past_key_value is None:
@@ -453,7 +453,7 @@ def _forward_with_cache(self, hidden_states, attention_mask, position_ids, cache
         # (the kernel reads cache rows 0 .. kv_len - 1 where they lie, whatever the capacity behind them)
         return self.o_proj(prefill_attention(query_states, k_all, v_all, kv_len - q_len)), None
     elif attention_mask is None and q_len == 1 and self.head_dim == 128 and _readable(k_all) and _readable(v_all) \
-            and query_states.is_cuda and 0 < bsz * self.num_heads <= ATTENTION_MAX_HEADS:
+            and query_states.is_cuda and bsz * self.num_heads <= ATTENTION_MAX_HEADS:
         last = self.rope.positions(query_states.device, kv_len - 1, bsz, 1)
         order = self.context_order()
         return self.project_out(decode_attention(query_states, k_all, v_all, last, out_index=order), order is not None), None

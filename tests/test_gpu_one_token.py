@@ -108,24 +108,6 @@ def test_nothing_is_kept_without_use_cache(model):
     assert peak(False) + one_layer // 2 < peak(True)
 
 
-@pytest.mark.parametrize("past", [None, PAST])
-def test_no_sequences(model, past, monkeypatch):
-    """A batch that has run empty: no rows in, none out."""
-    ids = torch.zeros((0, 1), dtype=torch.long, device="cuda")
-    pair = None if past is None else pairs(0, past)
-    rows = 1 if past is None else past + 1
-    logits, new = model(ids, past_key_values=pair, use_cache=True)
-    assert logits.shape == (0, 1, 320) and all(t.shape == (0, HEADS, rows, 128) for p in new for t in p)
-    x = torch.zeros((0, 1, 1024), dtype=torch.float16, device="cuda")
-    attn = model.model.layers[0].self_attn
-    out, _, (k, v) = attn(hidden_states=x, past_key_value=None if pair is None else pair[0], use_cache=True)
-    assert out.shape == x.shape and k.shape == v.shape == (0, HEADS, rows, 128)
-    held = None if pair is None else KeptPair(*pair[0])
-    monkeypatch.setattr(attn, "layer_idx", 0)
-    out, _ = attn(hidden_states=x, position_ids=ids, past_key_values=held, position_embeddings=())
-    assert out.shape == x.shape
-
-
 @pytest.mark.parametrize("bsz", [1, 2])
 @pytest.mark.parametrize("form", ["misaligned", "strided", "part"])
 def test_forms_of_a_cache(model, form, bsz, monkeypatch):
