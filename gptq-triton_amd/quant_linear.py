@@ -120,8 +120,11 @@ class InverseOrder:
         self._kept = None  # (key, the permutations, the inverse)
 
     def of(self, *perms):
-        """The inverse of the permutation that all of `perms` are; None where they differ (looking at them synchronises, once), and
-        in a call that is being captured before the first one that is not."""
+        """The inverse of the permutation that all of `perms` are; None where they differ (looking at them synchronises, once),
+        in a call that is being captured before the first one that is not, and for a permutation that was worked out in
+        inference mode (it counts no versions, so a write to it would go unseen)."""
+        if any(p.is_inference() for p in perms):
+            return None
         key = tensor_key(*perms)
         if self._kept is None or self._kept[0] != key:
             if perms[0].is_cuda and torch.cuda.is_current_stream_capturing():

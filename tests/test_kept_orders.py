@@ -35,6 +35,37 @@ def test_a_permutation_lives_as_long_as_its_inverse_is_kept(which):
     assert old() is None                          # one permutation is kept, not all there were
 
 
+@pytest.mark.parametrize("which", ["context", "input"])
+def test_a_permutation_of_inference_mode_leaves_the_gather_to_the_projection(which):
+    """An act-order module works out its permutation in the first call; in inference mode that is a tensor without a version."""
+    attn, ways = attention()
+    q, order = ways[which]
+    with torch.inference_mode():
+        q._compact_perm = torch.randperm(K).int()
+        assert order() is None
+    assert order() is None
+
+
+@pytest.mark.gpu
+def test_act_order_model_in_inference_mode(monkeypatch):
+    """Permutations worked out in inference mode: the same logits as without it, where producers write in the sorted order."""
+    monkeypatch.setattr(G, "make_fused_mlp", lambda model: None)
+    models = [random_quant_model(hidden=1024, inter=2816, heads=8, layers=2, groupsize=128, seed=83, act_order=True) for _ in range(2)]
+    ids = torch.randint(0, 256, (2, 9), device="cuda")
+
+    def logits(model):
+        prompt, past = model(ids, use_cache=True)
+        step, _ = model(ids[:, :1], past_key_values=past, use_cache=True)
+        return prompt, step
+
+    with torch.inference_mode():
+        got = logits(models[0])
+    with torch.no_grad():
+        want = logits(models[1])
+    for g, w in zip(got, want):
+        assert (g - w).norm() <= 5e-3 * w.norm()  # (the same sums in fp32; fp16 roundings of two layers between them)
+
+
 @pytest.mark.gpu
 def test_first_call_of_an_act_order_block_inside_a_capture(monkeypatch):
     """Nothing is compared (a synchronisation) and nothing kept while a call is being captured: the block gathers for itself there."""
