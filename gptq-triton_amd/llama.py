@@ -81,7 +81,7 @@ class LlamaMLP(nn.Module):
         self.down_proj = nn.Linear(i, h, bias=False)
         self.up_proj = nn.Linear(h, i, bias=False)
         self._same_rows = InverseOrder()  # of gate's and up's permutation, where it is one
-        self._most_rows = None
+        self._most_rows = (None, 0)  # (sizes, rows): see _pair_rows
 
     def _pair(self, rows: int):
         """(groupsize, gate words and {scale, zero} words, up's, row permutation) where one launch can compute
@@ -107,9 +107,10 @@ class LlamaMLP(nn.Module):
         return self._same_rows.of(gate.row_permutation(), up.row_permutation())
 
     def _pair_rows(self, gate) -> int:
-        if self._most_rows is None:
-            self._most_rows = stream_rows(_lib.OP_MLP_GATEUP, gate.infeatures, gate.outfeatures, gate.groupsize)
-        return self._most_rows
+        sizes = gate.infeatures, gate.outfeatures, gate.groupsize
+        if self._most_rows[0] != sizes:
+            self._most_rows = sizes, stream_rows(_lib.OP_MLP_GATEUP, *sizes)
+        return self._most_rows[1]
 
     def forward(self, x, ordered: bool = False):
         # without make_fused_mlp the three projections stay modules of their own; on the GPU gate and up still are one

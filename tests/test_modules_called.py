@@ -67,12 +67,15 @@ def test_only_itself(how):
     assert only_itself(q, G.QuantLinear)
 
 
-def streamed_mlp(g_idx=False):
+def streamed_mlp(g_idx=False, mlp=None, **sizes):
     """An unfused MLP block whose gate and up look as in streaming order (no weights: nothing is launched)."""
-    mlp = LlamaMLP(tiny_config(**WIDE))
+    with torch.device("meta"):
+        made = LlamaMLP(tiny_config(**(sizes or WIDE)))
+    mlp = made if mlp is None else mlp
     for name in ("gate_proj", "up_proj", "down_proj"):
-        old = getattr(mlp, name)
-        q = G.QuantLinear(4, 128, old.in_features, old.out_features, bias=False, act_order=g_idx)
+        old = getattr(made, name)
+        with torch.device("meta"):
+            q = G.QuantLinear(4, 128, old.in_features, old.out_features, bias=False, act_order=g_idx)
         q._stream_meta, q._stream_rows = torch.zeros(1, dtype=torch.int32), 16
         q._compact_perm = torch.arange(old.in_features, dtype=torch.int32) if g_idx else None
         setattr(mlp, name, q)
@@ -92,6 +95,16 @@ def test_gate_and_up_are_one_launch_only_while_nothing_hangs_on_them(name, how):
     assert mlp.input_order() is None and not mlp.norm_fusable(1)
     undo()
     assert mlp.input_order() is not None
+
+
+def test_the_pair_is_asked_for_the_projections_there_are():
+    """Projections put in the place of narrower ones: the rows the launch takes are those of the new ones."""
+    mlp = streamed_mlp()
+    assert mlp._pair(16) is not None
+    streamed_mlp(mlp=mlp, hidden_size=8192, num_attention_heads=64, intermediate_size=32768)
+    assert mlp._pair(3) is not None and mlp._pair(4) is None and mlp._pair(16) is None
+    streamed_mlp(mlp=mlp, **WIDE)
+    assert mlp._pair(16) is not None
 
 
 @pytest.mark.parametrize("how", HOWS)
