@@ -304,7 +304,7 @@ class GreedyDecoder:
         (The launch can fetch the embedding rows of the next step too, but a step starts from `tokens`, which the caller may
         write to between two steps or two replays of `graph`.)"""
         head = self.model.lm_head
-        return head_argmax_takes(self.bsz, head.weight) and head.bias is None
+        return head_argmax_takes(self.bsz, head.weight) and getattr(head, "bias", None) is None
 
     def _layers(self, h, position_ids, kv_offset, attend, end):
         """The decoder stack on hidden states h [B, S, hidden]; every residual add is fused with the RMSNorm that follows it.

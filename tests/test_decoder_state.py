@@ -113,6 +113,9 @@ def test_an_lm_head_replaced_later(monkeypatch):
     model.lm_head = torch.nn.Linear(64, 512, bias=False)
     dec._end_step(None, None, model.model.norm, x)
     assert len(launches) == 2
+    model.lm_head = torch.nn.Embedding(512, 64)         # (tied weights: a module that has no bias at all)
+    dec._end_step(None, None, model.model.norm, x)
+    assert len(launches) == 3
 
 
 @pytest.mark.gpu
