@@ -8,6 +8,7 @@ operator that needs it raises with it.  There is no CPU fallback.
 from __future__ import annotations
 
 import ctypes
+import threading
 from ctypes import POINTER, Structure, c_char_p, c_float, c_int, c_size_t, c_uint, c_void_p
 from pathlib import Path
 
@@ -167,25 +168,31 @@ def current_stream(device: torch.device):
 # alive, because captured graphs may still launch kernels that point into it.
 _workspaces: dict = {}
 _outgrown: list = []
+# Two threads on one stream make or outgrow it one after the other: the extension keeps bare addresses, and one that lost
+# the race would be freed behind its back.
+_workspace_lock = threading.RLock()
 _WS_BYTES = WS_HEAD_BYTES + 16 * 16 * 2 * 32768 * 4  # splitk 16, M 16, 2 matrices, 32768 columns
 
 
 def workspace(device: torch.device, need: int):
     key = (device.index if device.index is not None else torch.cuda.current_device(), current_stream(device))
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < need:
-        if ws is not None:
-            _outgrown.append(ws)
-        ws = torch.zeros(max(need, _WS_BYTES, 2 * ws.numel() if ws is not None else 0), dtype=torch.uint8, device=device)
-        _workspaces[key] = ws
-        host().set_workspace(*key, ws.data_ptr(), ws.numel())
+    with _workspace_lock:
+        ws = _workspaces.get(key)
+        if ws is None or ws.numel() < need:
+            if ws is not None:
+                _outgrown.append(ws)
+            ws = torch.zeros(max(need, _WS_BYTES, 2 * ws.numel() if ws is not None else 0), dtype=torch.uint8, device=device)
+            _workspaces[key] = ws
+            host().set_workspace(*key, ws.data_ptr(), ws.numel())
     return ws
 
 
 def _workspace_of_current_stream(index: int, need: int) -> None:
     """What the _host extension calls when it knows no workspace of `need` bytes for the stream it is about to launch on."""
-    ws = workspace(torch.device("cuda", index), need)
-    host().set_workspace(index, current_stream(ws.device), ws.data_ptr(), ws.numel())
+    device = torch.device("cuda", index)
+    with _workspace_lock:
+        ws = workspace(device, need)
+        host().set_workspace(index, current_stream(device), ws.data_ptr(), ws.numel())
 
 
 def exchange_errors() -> list:
