@@ -215,9 +215,10 @@ def make_quant_attn(model: nn.Module):
         setattr(parent, child, attn)
 
 
-def _readable(t: torch.Tensor) -> bool:
-    """Whether the attention kernel reads a cache tensor where it lies, and nobody wants a gradient of it."""
-    return t.is_contiguous() and t.data_ptr() % 16 == 0 and not (t.requires_grad and torch.is_grad_enabled())
+def _readable(t: torch.Tensor, q: torch.Tensor) -> bool:
+    """Whether the attention kernel for the queries q reads a cache tensor where it lies (it has no broadcasting), and nobody wants
+    a gradient of it."""
+    return t.shape[:2] == q.shape[:2] and t.is_contiguous() and t.data_ptr() % 16 == 0 and not (t.requires_grad and torch.is_grad_enabled())
 
 
 def _past_rows(t: torch.Tensor, shape, device) -> torch.Tensor:
@@ -452,7 +453,7 @@ def _forward_with_cache(self, hidden_states, attention_mask, position_ids, cache
     elif attention_mask is None and q_len > 1 and self.head_dim == 128 and k_all.is_contiguous() and v_all.is_contiguous():
         # (the kernel reads cache rows 0 .. kv_len - 1 where they lie, whatever the capacity behind them)
         return self.o_proj(prefill_attention(query_states, k_all, v_all, kv_len - q_len)), None
-    elif attention_mask is None and q_len == 1 and self.head_dim == 128 and _readable(k_all) and _readable(v_all) \
+    elif attention_mask is None and q_len == 1 and self.head_dim == 128 and _readable(k_all, query_states) and _readable(v_all, query_states) \
             and query_states.is_cuda and bsz * self.num_heads <= ATTENTION_MAX_HEADS:
         last = self.rope.positions(query_states.device, kv_len - 1, bsz, 1)
         order = self.context_order()

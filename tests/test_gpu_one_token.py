@@ -109,7 +109,7 @@ def test_nothing_is_kept_without_use_cache(model):
 
 
 @pytest.mark.parametrize("bsz", [1, 2])
-@pytest.mark.parametrize("form", ["misaligned", "strided", "part"])
+@pytest.mark.parametrize("form", ["misaligned", "strided", "part", "one for all", "one head for all"])
 def test_forms_of_a_cache(model, form, bsz, monkeypatch):
     """One token with a Cache that hands back its rows in other forms than a contiguous aligned tensor (those may take torch's
     attention, which rounds the probabilities to fp16: 2^-11 of a value each, and the result once more)."""
@@ -118,7 +118,9 @@ def test_forms_of_a_cache(model, form, bsz, monkeypatch):
     x = torch.randn((bsz, 1, 1024), device="cuda", generator=torch.Generator(device="cuda").manual_seed(6)).half()
     ids = torch.full((bsz, 1), PAST, dtype=torch.long, device="cuda")
     step = lambda cache: attn(hidden_states=x, position_ids=ids, past_key_values=cache, position_embeddings=())[0]
-    want, got = step(KeptPair(*pairs(bsz)[0])), step(KeptPair(*pairs(bsz)[0], form=FORMS[form]))
+    part = FORMS.get(form, lambda t: t[:, :1])
+    whole = lambda t: part(t).expand(t.shape).clone(memory_format=torch.contiguous_format)
+    want, got = step(KeptPair(*pairs(bsz)[0], form=whole)), step(KeptPair(*pairs(bsz)[0], form=part))
     assert (got - want).float().norm() <= 2 ** -9 * want.float().norm()
 
 
