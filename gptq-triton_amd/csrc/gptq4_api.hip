@@ -187,11 +187,17 @@ struct TiledChoice {
     size_t partial;
 };
 
-TiledChoice choose_tiled(int epi, int M, int n, int K, bool kernel_gathers, bool allow_streamed = true) {
+// Two kinds of plan can be ruled out, for a workspace that has no room for their partial sums: the tiled kernel's streamed
+// schedule and the mid-M kernel's plans by estimated time.
+struct Allowed {
+    bool streamed = true, one_round = true;
+};
+
+TiledChoice choose_tiled(int epi, int M, int n, int K, bool kernel_gathers, Allowed allow = {}) {
     TiledChoice c = {};
-    c.kp = kslice_plan(epi, M, n, K, kernel_gathers);
+    c.kp = kslice_plan(epi, M, n, K, kernel_gathers, allow.one_round);
     c.kslice = prefer_kslice(c.kp, epi, M, n, K);
-    c.gp = gemm_plan(epi, M, n, K, kernel_gathers, allow_streamed);
+    c.gp = gemm_plan(epi, M, n, K, kernel_gathers, allow.streamed);
     c.partial = c.kslice ? kslice_partial_bytes(epi, c.kp) : gemm_partial_bytes(c.gp);
     return c;
 }
@@ -208,11 +214,11 @@ struct ColumnParts {
     bool first_is_wide;  // part 0 runs wide unsplit tiles whatever its own plan would say
 };
 
-ColumnParts tiled_parts(int epi, int M, int N, int K, bool kernel_gathers) {
+ColumnParts tiled_parts(int epi, int M, int N, int K, bool kernel_gathers, bool one_round = true) {
     ColumnParts parts = {1, {0, 0}, {N, 0}, false};
     if (g_gemm_tuning.parts == 1 || g_gemm_tuning.mt != 0 || g_gemm_tuning.splitk != 0 || g_gemm_tuning.streamed == 2 || g_kslice_tuning.mode == 2)
         return parts;
-    const TiledChoice whole = choose_tiled(epi, M, N, K, kernel_gathers);
+    const TiledChoice whole = choose_tiled(epi, M, N, K, kernel_gathers, {true, one_round});
     if (whole.kslice || whole.gp.mt != 4 || whole.gp.splitk != 1 || whole.gp.streamed || whole.gp.tail_split > 1) return parts;
     const long cus = device_shape().cus;
     const int bnw = (epi == EPI_SILU_MUL) ? 128 : 256;  // output columns of a wide tile
@@ -234,7 +240,7 @@ ColumnParts tiled_parts(int epi, int M, int N, int K, bool kernel_gathers) {
     return parts;
 }
 
-TiledChoice choose_part(int epi, int M, int K, const ColumnParts &parts, int i, bool kernel_gathers, bool allow_streamed = true) {
+TiledChoice choose_part(int epi, int M, int K, const ColumnParts &parts, int i, bool kernel_gathers, Allowed allow = {}) {
     if (i == 0 && parts.first_is_wide) {
         TiledChoice c = {};
         c.kslice = false;
@@ -248,14 +254,15 @@ TiledChoice choose_part(int epi, int M, int K, const ColumnParts &parts, int i, 
         c.partial = 0;
         return c;
     }
-    return choose_tiled(epi, M, parts.cols[i], K, kernel_gathers, allow_streamed);
+    return choose_tiled(epi, M, parts.cols[i], K, kernel_gathers, allow);
 }
 
 // A call's whole plan.  Making one weighs up to a hundred launch shapes (5 - 20 us of host time, as much as a small call
 // takes on the GPU), so every thread keeps its last ones: 64 slots by the call's sizes, good for one set of tuning values.
 struct TiledPlan {
     int epi, M, N, K, cus;
-    bool kernel_gathers, allow_streamed;
+    bool kernel_gathers;
+    Allowed allow;
     unsigned generation;  // of the tuning values; 0: an empty slot
     ColumnParts parts;
     TiledChoice choice[2];
@@ -263,17 +270,17 @@ struct TiledPlan {
 };
 unsigned g_tuning_generation = 1;
 
-const TiledPlan &tiled_plan(int epi, int M, int N, int K, bool kernel_gathers, bool allow_streamed) {
+const TiledPlan &tiled_plan(int epi, int M, int N, int K, bool kernel_gathers, Allowed allow) {
     static thread_local TiledPlan kept[64];
     const int cus = device_shape().cus;
     TiledPlan &t = kept[((unsigned)M * 2654435761u ^ (unsigned)N * 40503u ^ (unsigned)K * 97u ^ (unsigned)epi * 7u) >> 7 & 63u];
     if (t.generation == g_tuning_generation && t.epi == epi && t.M == M && t.N == N && t.K == K && t.cus == cus &&
-        t.kernel_gathers == kernel_gathers && t.allow_streamed == allow_streamed)
+        t.kernel_gathers == kernel_gathers && t.allow.streamed == allow.streamed && t.allow.one_round == allow.one_round)
         return t;
-    t = TiledPlan{epi, M, N, K, cus, kernel_gathers, allow_streamed, g_tuning_generation, {}, {}, 0};
-    t.parts = tiled_parts(epi, M, N, K, kernel_gathers);
+    t = TiledPlan{epi, M, N, K, cus, kernel_gathers, allow, g_tuning_generation, {}, {}, 0};
+    t.parts = tiled_parts(epi, M, N, K, kernel_gathers, allow.one_round);
     for (int i = 0; i < t.parts.count; ++i) {
-        t.choice[i] = choose_part(epi, M, K, t.parts, i, kernel_gathers, allow_streamed);
+        t.choice[i] = choose_part(epi, M, K, t.parts, i, kernel_gathers, allow);
         if (t.choice[i].partial > t.partial) t.partial = t.choice[i].partial;
     }
     return t;
@@ -284,13 +291,22 @@ int run_tiled(int epi, MatmulArgs &a, void *workspace, size_t workspace_bytes, h
     // kernel can run too); else the tiled kernel gathers by itself
     const size_t rows_bytes = (size_t)a.M * a.K * sizeof(half_t);
     bool stage = a.perm != nullptr && !g_gemm_tuning.own_gather && rows_bytes <= ACT_ORDER_STAGE_MAX;
-    bool allow_streamed = true;
-    auto plan_all = [&]() { return tiled_plan(epi, a.M, a.N, a.K, a.perm != nullptr && !stage, allow_streamed); };
+    Allowed allow;
+    auto plan_all = [&]() { return tiled_plan(epi, a.M, a.N, a.K, a.perm != nullptr && !stage, allow); };
+    auto by_estimate = [](const TiledChoice &c) { return c.kslice && c.kp.one_round; };
     TiledPlan pl = plan_all();
+    // a plan by estimated time may share K more ways than the plan by scores, and so ask for more partial sums: a workspace without
+    // the room for them (less than gptq4_workspace_bytes(), or none) keeps to the plan by scores
+    const size_t scratch = pl.partial + (stage ? rows_bytes : 0);
+    if (scratch > 0 && (workspace == nullptr || workspace_bytes < GPTQ4_WS_HEAD_BYTES + scratch) &&
+        (by_estimate(pl.choice[0]) || (pl.parts.count > 1 && by_estimate(pl.choice[1])))) {
+        allow.one_round = false;
+        pl = plan_all();
+    }
     // the streamed schedule keeps 128 MiB of partial sums: without the room for them, the unstreamed plan
     if (pl.parts.count == 1 && !pl.choice[0].kslice && pl.choice[0].gp.streamed &&
         (workspace == nullptr || workspace_bytes < GPTQ4_WS_HEAD_BYTES + pl.partial + (stage ? rows_bytes : 0))) {
-        allow_streamed = false;
+        allow.streamed = false;
         pl = plan_all();
     }
     if (stage && (workspace == nullptr || workspace_bytes < GPTQ4_WS_HEAD_BYTES + pl.partial + rows_bytes)) {
@@ -418,9 +434,10 @@ void gptq4_set_tuning(int words, int depth, int splitk) {
     g_skinny_tuning.splitk = splitk > 0 ? splitk : 0;
 }
 
-// allow_streamed = false: the need of the same call planned without the tiled kernel's streamed schedule (a
-// measurement mode whose partial sums alone are 128 MiB)
-static size_t workspace_need(int op, int M, int K, int N, bool allow_streamed) {
+// least = true: the need of the same call planned for the least scratch it can do with - without the tiled kernel's streamed
+// schedule (a measurement mode whose partial sums alone are 128 MiB) and without the plans by estimated time
+static size_t workspace_need(int op, int M, int K, int N, bool least) {
+    const Allowed allow = {!least, !least};
     size_t bytes = GPTQ4_WS_HEAD_BYTES;
     const bool with_perm = (op & GPTQ4_OP_WITH_PERM) != 0;
     op &= ~GPTQ4_OP_WITH_PERM;
@@ -434,7 +451,7 @@ static size_t workspace_need(int op, int M, int K, int N, bool allow_streamed) {
         // (kept like the plans it is made of)
         struct Need {
             int op, M, K, N, cus;
-            bool allow_streamed;
+            bool least;
             unsigned generation;
             size_t need;
         };
@@ -443,28 +460,28 @@ static size_t workspace_need(int op, int M, int K, int N, bool allow_streamed) {
         Need &slot = kept[((unsigned)M * 2654435761u ^ (unsigned)N * 40503u ^ (unsigned)K * 97u ^ (unsigned)op * 7u) >> 7 & 63u];
         const size_t rows = with_perm && (size_t)M * K * 2 <= ACT_ORDER_STAGE_MAX ? (size_t)M * K * 2 : 0;  // gathered for an act-order call
         if (slot.generation == g_tuning_generation && slot.op == op && slot.M == M && slot.K == K && slot.N == N && slot.cus == cus &&
-            slot.allow_streamed == allow_streamed)
+            slot.least == least)
             return bytes + slot.need + rows;
         const int epi = (op == GPTQ4_OP_MLP_GATEUP) ? EPI_SILU_MUL : (op == GPTQ4_OP_QKV_ROTARY ? EPI_ROPE : EPI_PLAIN);
         // whichever kernel the current (automatic or forced) plans pick, with or without act-order, for the whole
         // matrix and for each of the column ranges a call may be cut into
-        size_t need = gemm_partial_bytes(gemm_plan(epi, M, N, K, false, allow_streamed));
-        const KslicePlan kp = kslice_plan(epi, M, N, K, false);
+        size_t need = gemm_partial_bytes(gemm_plan(epi, M, N, K, false, allow.streamed));
+        const KslicePlan kp = kslice_plan(epi, M, N, K, false, allow.one_round);
         if (kp.ok && kslice_partial_bytes(epi, kp) > need) need = kslice_partial_bytes(epi, kp);
-        const ColumnParts parts = tiled_parts(epi, M, N, K, false);
+        const ColumnParts parts = tiled_parts(epi, M, N, K, false, allow.one_round);
         for (int i = 0; i < parts.count; ++i) {
-            const TiledChoice c = choose_part(epi, M, K, parts, i, false, allow_streamed);
+            const TiledChoice c = choose_part(epi, M, K, parts, i, false, allow);
             if (c.partial > need) need = c.partial;
-            const KslicePlan pk = kslice_plan(epi, M, parts.cols[i], K, false);
+            const KslicePlan pk = kslice_plan(epi, M, parts.cols[i], K, false, allow.one_round);
             if (pk.ok && kslice_partial_bytes(epi, pk) > need) need = kslice_partial_bytes(epi, pk);
         }
-        slot = Need{op, M, K, N, cus, allow_streamed, g_tuning_generation, need};
+        slot = Need{op, M, K, N, cus, least, g_tuning_generation, need};
         bytes += need + rows;
     }
     return bytes;
 }
 
-size_t gptq4_workspace_bytes(int op, int M, int K, int N) { return workspace_need(op, M, K, N, true); }
+size_t gptq4_workspace_bytes(int op, int M, int K, int N) { return workspace_need(op, M, K, N, false); }
 
 int gptq4_column_parts(int op, int M, int K, int N, int *begin, int *cols) {
     op &= ~GPTQ4_OP_WITH_PERM;
@@ -567,9 +584,8 @@ int gptq4_matmul_static(const void *x, const int32_t *qweight, const int32_t *qz
     int g = groupsize;
     int rc = check_dims(K, N, &g);
     if (rc) return rc;
-    // what the same call would ask of a caller's workspace - planned without the streamed schedule of the tiled
-    // kernel, whose partial sums alone are 128 MiB - has to fit the static array
-    const size_t need = workspace_need(GPTQ4_OP_MATMUL, M, K, N, false);
+    // the least that the same call would ask of a caller's workspace has to fit the static array
+    const size_t need = workspace_need(GPTQ4_OP_MATMUL, M, K, N, true);
     if (need > (size_t)GPTQ4_STATIC_SCRATCH_BYTES) return -GPTQ4_E_STATIC_LIMIT;
     void *ws = nullptr;
     rc = static_scratch(&ws);

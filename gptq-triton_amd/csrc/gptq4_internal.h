@@ -153,7 +153,7 @@ struct KsliceTuning {
     int paired;      // rotary epilogue, tiles of 32 + 32 paired columns: 0 = automatic, 1 = always, 2 = never
 };
 extern KsliceTuning g_kslice_tuning;
-KslicePlan kslice_plan(int epi, int M, int N, int K, bool has_perm);
+KslicePlan kslice_plan(int epi, int M, int N, int K, bool has_perm, bool allow_one_round = true);
 size_t kslice_partial_bytes(int epi, const KslicePlan &plan);
 int launch_kslice(int epi, const MatmulArgs &a, const KslicePlan &plan, hipStream_t stream);
 

@@ -886,10 +886,10 @@ static KslicePlan one_round_plan(int epi, int M, int N, int K) {
     return best;
 }
 
-KslicePlan kslice_plan(int epi, int M, int N, int K, bool has_perm) {
+KslicePlan kslice_plan(int epi, int M, int N, int K, bool has_perm, bool allow_one_round) {
     const KsliceTuning &t = g_kslice_tuning;
     KslicePlan pl = rounds_plan(epi, M, N, K, has_perm);
-    if (t.mode != 1 || t.mt != 0 || t.splitk != 0 || t.wide != 0 || t.waves != 0 || t.paired != 0 || has_perm) return pl;
+    if (t.mode != 1 || t.mt != 0 || t.splitk != 0 || t.wide != 0 || t.waves != 0 || t.paired != 0 || has_perm || !allow_one_round) return pl;
     const KslicePlan one = one_round_plan(epi, M, N, K);
     if (!one.ok) return pl;
     // the plan by scores stays where the estimates do not tell the two apart (7 %: it may then be level with the tiled kernel's

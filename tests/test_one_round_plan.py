@@ -92,3 +92,48 @@ def test_automatic_plans_agree_with_the_decode_kernels(op, m, k, n, stream):
     ulp = torch.from_numpy(np.spacing(big).astype(np.float32)).cuda()
     worst = ((got.float() - want.float()).abs() - ulp - slack).max().item()
     assert worst <= 0.0, worst
+
+
+# (rows, inputs, outputs, act-order, bytes of workspace behind its head): the plan by scores fits, the one by estimated time does not
+TIGHT = [(70, 12672, 6400, False, 0), (84, 13696, 12800, False, 8 << 20), (76, 19456, 10240, False, 4 << 20), (191, 6912, 5632, True, 4 << 20)]
+
+
+def matmul_in(workspace, tensors, m, k, n):
+    """The library's return code of a call with that (address, bytes) of workspace."""
+    x, w, z, s, perm, y = tensors
+    stream = 0 if not torch.cuda.is_available() else torch.cuda.current_stream().cuda_stream
+    return _lib.load().gptq4_matmul(x, w, z, s, perm, None, y, m, k, n, 128, *workspace, stream)
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the addresses are not memory: without a GPU nothing is launched")
+def test_a_workspace_that_the_plan_by_scores_fits_is_enough():
+    fake = 4096
+    for m, k, n, act_order, extra in TIGHT:
+        rc = matmul_in((fake, _lib.WS_HEAD_BYTES + extra), (fake, fake, fake, fake, fake if act_order else None, fake), m, k, n)
+        assert rc > 0, (rc, m, k, n)                    # (HIP's: there is no device)
+    for m, k, n in [(646, 14720, 22784), (677, 17152, 22784), (711, 13184, 22784)]:
+        rc = _lib.load().gptq4_matmul_static(fake, fake, fake, fake, None, fake, m, k, n, 128, None)
+        assert rc > 0, (rc, m, k, n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,k,n,act_order,extra", TIGHT)
+def test_calls_with_a_tight_workspace(m, k, n, act_order, extra):
+    """As with all the workspace the library asks for, up to the order of the fp32 sums (see above)."""
+    from gptq_triton_amd import quant_linear as Q
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    words = lambda *s: torch.randint(-2 ** 31, 2 ** 31 - 1, s, dtype=torch.int32, device="cuda", generator=gen)
+    w, z = words(k // 8, n), words(k // 128, n // 8)
+    s = ((0.2 + 0.3 * torch.rand((k // 128, n), device="cuda", generator=gen)) / (4.6 * k ** 0.5)).half()
+    x = torch.randn((m, k), device="cuda", generator=gen).half()
+    perm = torch.randperm(k, device="cuda", generator=gen).int() if act_order else None
+    ws = torch.zeros(_lib.WS_HEAD_BYTES + extra, dtype=torch.uint8, device="cuda")
+    got = torch.empty((m, n), dtype=torch.float16, device="cuda")
+    rc = matmul_in((ws.data_ptr(), ws.numel()), (x.data_ptr(), w.data_ptr(), z.data_ptr(), s.data_ptr(), _lib.ptr(perm), got.data_ptr()), m, k, n)
+    assert rc == 0
+    want = Q.matmul4(128, x, w, s, z, perm=perm)
+    ordered = x if perm is None else x[:, perm.long()]
+    slack = 2 * k * 2.0 ** -24 * (ordered.abs().float() @ Q.dequantize(w, z, s, 128).abs().float())
+    ulp = torch.from_numpy(np.spacing(torch.maximum(got.abs(), want.abs()).cpu().numpy()).astype(np.float32)).cuda()
+    assert ((got.float() - want.float()).abs() - ulp - slack).max().item() <= 0.0
+    assert int(ws[:_lib.WS_HEAD_BYTES].view(torch.int32).abs().sum()) == 0
