@@ -397,6 +397,8 @@ class GreedyDecoder:
     @torch.no_grad()
     def decode(self, steps: int, use_graph: bool = False) -> torch.Tensor:
         """`steps` more greedy tokens after prefill -> [B, steps]."""
+        if steps < 0:
+            raise RuntimeError(f"decode of {steps} steps")
         # where the sequences stand is read back: the kernels move `position` on, also in a step that is interrupted on the host
         # and in a replay of `graph` by the caller, and the caller may write to it
         stand = self.position.flatten().tolist()

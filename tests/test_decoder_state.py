@@ -72,6 +72,14 @@ def test_decode_goes_on_from_where_the_kernels_left_the_sequences(monkeypatch, m
     assert torch.equal(dec.decode(CAPACITY - 12), want(13, CAPACITY - 12))
 
 
+def test_decode_of_no_and_of_fewer_steps(monkeypatch):
+    dec = decoder_of_known_tokens(monkeypatch)
+    assert dec.decode(0).shape == (2, 0)
+    with pytest.raises(RuntimeError):
+        dec.decode(-1)
+    assert torch.equal(dec.decode(2), want(6, 2))
+
+
 def test_decode_of_sequences_at_different_places(monkeypatch):
     dec = decoder_of_known_tokens(monkeypatch)
     dec.position.copy_(torch.tensor([[4], [9]]))
