@@ -120,7 +120,7 @@ class InverseOrder:
         self._kept = None  # (key, the permutations, the inverse)
 
     def of(self, *perms):
-        """The inverse of the permutation that all of `perms` are; None where they differ (looking at them synchronises, once),
+        """The inverse of the permutation that all of `perms` are; None where they differ (working it out synchronises, once),
         in a call that is being captured before the first one that is not, and for a permutation that was worked out in
         inference mode (it counts no versions, so a write to it would go unseen)."""
         if any(p.is_inference() for p in perms):
@@ -129,8 +129,10 @@ class InverseOrder:
         if self._kept is None or self._kept[0] != key:
             if perms[0].is_cuda and torch.cuda.is_current_stream_capturing():
                 return None
-            same = all(torch.equal(perms[0], p) for p in perms[1:])
-            self._kept = (key, perms, inverse_permutation(perms[0]) if same else None)
+            inverse = inverse_permutation(perms[0]) if all(torch.equal(perms[0], p) for p in perms[1:]) else None
+            if inverse is not None and inverse.is_cuda:
+                torch.cuda.current_stream(inverse.device).synchronize()  # (the next call may come on another stream)
+            self._kept = (key, perms, inverse)
         return self._kept[2]
 
 

@@ -91,3 +91,21 @@ def test_first_call_of_an_act_order_block_inside_a_capture(monkeypatch):
         assert (out - want).norm() <= 2e-3 * want.norm()   # (separate launches for gate and up: SiLU and product on rounded values)
         assert torch.equal(att, want_att)
         assert torch.equal(layer.mlp(x), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("which", ["context", "input"])
+def test_another_stream_may_ask_next(which):
+    """The stream that works an inverse out is busy: the next call, on another one, is given what is filled already."""
+    attn, ways = attention()
+    q, order = ways[which]
+    q._compact_perm = torch.randperm(K, device="cuda").int()
+    torch.cuda.synchronize()
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(first):
+        torch.cuda._sleep(10_000_000)
+        order()
+    with torch.cuda.stream(second):
+        got = order().clone()
+    torch.cuda.synchronize()
+    assert torch.equal(got, inverse_permutation(q._compact_perm))
