@@ -20,7 +20,7 @@ import torch.nn as nn
 from . import _lib
 from .decoder_ops import (ATTENTION_MAX_HEADS, NORM_MAX_ROWS, check_norm_args, contiguous_delta, decode_attention, extend_attention,
                           norm_fusable, norm_fusion_pays, prefill_attention)
-from .quant_linear import QuantLinear, _check_device_tensors, _check_matmul_args, InverseOrder, only_itself
+from .quant_linear import QuantLinear, _check_device_tensors, _check_matmul_args, InverseOrder, child, only_itself
 
 
 @dataclass
@@ -267,7 +267,7 @@ class QuantLlamaAttention(nn.Module):
             need = max(kv_offset, 0) + hidden_states.shape[1]
         cos, sin = self.rope.get(hidden_states.device, max(need, self.max_position_embeddings))
         rows = hidden_states.shape[0] * hidden_states.shape[1]
-        qkv = self.qkv_proj
+        qkv = child(self, 'qkv_proj')
         sw = qkv.stream_weights(rows)
         if sw is not None and (norm is None or rows <= NORM_MAX_ROWS):
             return qkv_rotary_stream(qkv.groupsize, hidden_states, sw[0], sw[1], position_ids, cos, sin, self.num_heads,
@@ -281,13 +281,14 @@ class QuantLlamaAttention(nn.Module):
         it in the order of its sorted rows (int32 [hidden], the inverse of o_proj's permutation), or
         None without act-order and where o_proj is to be called as a module (only_itself).
         decode_attention(out_index=...) writes in that order."""
-        perm = self.o_proj.row_permutation() if only_itself(self.o_proj, QuantLinear) else None
+        o = child(self, 'o_proj')
+        perm = o.row_permutation() if only_itself(o, QuantLinear) else None
         return None if perm is None else self._context_order.of(perm)
 
     def input_order(self):
         """The same for the input of the fused QKV projection: rms_norm / add_rms_norm(out_index=...) write in
         that order, and project_qkv(ordered=True) then runs without a gather.  None without act-order."""
-        perm = self.qkv_proj.row_permutation()
+        perm = child(self, 'qkv_proj').row_permutation()
         return None if perm is None else self._input_order.of(perm)
 
     def attend_one(self, hidden_states: torch.Tensor, position_ids: torch.Tensor, past_key_value, norm=None, ordered: bool = False):
@@ -307,7 +308,8 @@ class QuantLlamaAttention(nn.Module):
 
     def project_out(self, context: torch.Tensor, ordered: bool = False) -> torch.Tensor:
         """o_proj(context); ordered: the context already is in the order of context_order()."""
-        return self.o_proj.multiply(context, ordered=True) if ordered else self.o_proj(context)
+        o = child(self, 'o_proj')
+        return o.multiply(context, ordered=ordered) if ordered or only_itself(o, QuantLinear) else o(context)
 
     def norm_fusable(self, rows: int) -> bool:
         """Whether project_qkv(norm=...) is the faster way for this many rows."""
@@ -352,7 +354,7 @@ class QuantLlamaAttention(nn.Module):
                 else torch.arange(past_len, kv_seq_len, device=hidden_states.device).unsqueeze(0)
 
         # (a past that is part of a gradient's graph stays in it by the copies below)
-        traced = past_key_value is not None and torch.is_grad_enabled() and any(t.requires_grad for t in past_key_value)
+        traced = past_key_value is not None and (past_key_value[0].requires_grad or past_key_value[1].requires_grad) and torch.is_grad_enabled()
         if q_len == 1 and attention_mask is None and not output_attentions and self.head_dim == 128 and hidden_states.is_cuda \
                 and bsz * self.num_heads <= ATTENTION_MAX_HEADS and not traced:
             context, pair = self.attend_one(hidden_states, position_ids, past_key_value, ordered=ordered)

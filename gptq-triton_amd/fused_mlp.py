@@ -14,7 +14,7 @@ import torch.nn as nn
 
 from . import _lib
 from .decoder_ops import NORM_MAX_ROWS, check_norm_args, contiguous_delta, norm_fusable, norm_fusion_pays
-from .quant_linear import (InverseOrder, QuantLinear, _check_device_tensors, _check_matmul_args, held, matmul4, stream_pack, stream_rows, stream_unpack,
+from .quant_linear import (InverseOrder, QuantLinear, _check_device_tensors, _check_matmul_args, child, held, matmul4, stream_pack, stream_rows, stream_unpack,
                            tensor_key)
 
 
@@ -308,7 +308,7 @@ class QuantLlamaMLP(nn.Module):
     def forward(self, x: torch.Tensor, ordered: bool = False) -> torch.Tensor:
         if self._stream_ready(x):
             mid = llama_mlp_4_stream(self.groupsize, x, *self._stream_words(), None if ordered else held(self, '_compact_rows'))
-            return self.down_proj.multiply(mid, ordered=True)  # the columns of gate and up are laid out in the order down_proj reads
+            return child(self, 'down_proj').multiply(mid, ordered=True)  # the columns of gate and up are laid out in the order down_proj reads
         w, perm, down_q = self._chained_weights()
         return self._down(llama_mlp_4(self.groupsize, x, *w, None if ordered else perm), down_q)
 
@@ -322,7 +322,7 @@ class QuantLlamaMLP(nn.Module):
         """(h + delta, forward(RMSNorm(h + delta))): the residual add and the norm run inside the gate/up launch."""
         if self._stream_ready(h) and h.numel() // self.infeatures <= NORM_MAX_ROWS:
             s, mid = llama_mlp_4_stream(self.groupsize, h, *self._stream_words(), held(self, '_compact_rows'), norm=(delta, norm_weight, eps))
-            return s, self.down_proj.multiply(mid, ordered=True)
+            return s, child(self, 'down_proj').multiply(mid, ordered=True)
         w, perm, down_q = self._chained_weights()
         s, mid = norm_llama_mlp_4(self.groupsize, h, delta, norm_weight, eps, *w, perm)
         return s, self._down(mid, down_q)

@@ -22,7 +22,7 @@ from .decoder_ops import (NORM_MAX_HIDDEN, add_rms_norm, decode_attention, greed
                           norm_fusion_pays, prefill_attention, rms_norm)
 from .fused_attention import KV_AT_POSITION, LlamaConfigLite, QuantLlamaAttention
 from .fused_mlp import QuantLlamaMLP, llama_mlp_4_stream
-from .quant_linear import InverseOrder, QuantLinear, only_itself, stream_rows
+from .quant_linear import InverseOrder, QuantLinear, child, only_itself, stream_rows
 
 # the rows the decode kernels built on the streaming-order weight layout take (more rows: the mid-M and tiled kernels)
 STREAM_BATCH = 16
@@ -86,7 +86,7 @@ class LlamaMLP(nn.Module):
     def _pair(self, rows: int):
         """(groupsize, gate words and {scale, zero} words, up's, row permutation) where one launch can compute
         silu(gate) * up from the two modules' own tensors in streaming order, else None."""
-        gate, up = self.gate_proj, self.up_proj
+        gate, up = child(self, 'gate_proj'), child(self, 'up_proj')
         if not (only_itself(gate, QuantLinear) and only_itself(up, QuantLinear)):
             return None
         g, u = gate.stream_weights(rows), up.stream_weights(rows)
@@ -100,7 +100,7 @@ class LlamaMLP(nn.Module):
     def input_order(self):
         """As QuantLlamaMLP.input_order: None without act-order, where gate and up each have an order of their own, and where
         this block, gate or up is to be called as a module (only_itself)."""
-        gate, up = self.gate_proj, self.up_proj
+        gate, up = child(self, 'gate_proj'), child(self, 'up_proj')
         if not (only_itself(self, LlamaMLP) and only_itself(gate, QuantLinear) and only_itself(up, QuantLinear)) \
                 or gate.g_idx is None or up.g_idx is None:
             return None
@@ -118,7 +118,7 @@ class LlamaMLP(nn.Module):
         pair = self._pair(x.numel() // max(x.shape[-1], 1)) if x.is_cuda else None
         if pair is not None:
             groupsize, gw, gm, uw, um, perm = pair
-            return self.down_proj(llama_mlp_4_stream(groupsize, x, gw, gm, uw, um, None if ordered else perm))
+            return child(self, 'down_proj')(llama_mlp_4_stream(groupsize, x, gw, gm, uw, um, None if ordered else perm))
         if ordered:
             return self.down_proj(torch.nn.functional.silu(self.gate_proj.multiply(x, ordered=True)) * self.up_proj.multiply(x, ordered=True))
         return self.down_proj(torch.nn.functional.silu(self.gate_proj(x)) * self.up_proj(x))
@@ -133,7 +133,7 @@ class LlamaMLP(nn.Module):
         """(h + delta, forward(RMSNorm(h + delta))) with the residual add and the norm inside the gate/up launch."""
         groupsize, gw, gm, uw, um, perm = self._pair(h.numel() // h.shape[-1])
         s, mid = llama_mlp_4_stream(groupsize, h, gw, gm, uw, um, perm, norm=(delta, norm_weight, eps))
-        return s, self.down_proj(mid)
+        return s, child(self, 'down_proj')(mid)
 
 
 class LlamaDecoderLayer(nn.Module):
@@ -156,10 +156,11 @@ class LlamaDecoderLayer(nn.Module):
 
     def only_themselves(self) -> bool:
         """Whether the layer and the blocks it calls are this package's own and nothing else would run with them."""
-        attn, mlp = self.self_attn, self.mlp
+        attn, mlp = child(self, 'self_attn'), child(self, 'mlp')
         return only_itself(self, LlamaDecoderLayer) and only_itself(attn, QuantLlamaAttention) \
             and only_itself(mlp, QuantLlamaMLP if type(mlp) is QuantLlamaMLP else LlamaMLP) \
-            and only_itself(self.input_layernorm, LlamaRMSNorm) and only_itself(self.post_attention_layernorm, LlamaRMSNorm)
+            and only_itself(child(self, 'input_layernorm'), LlamaRMSNorm) \
+            and only_itself(child(self, 'post_attention_layernorm'), LlamaRMSNorm)
 
 
 class LlamaModel(nn.Module):
@@ -228,11 +229,12 @@ class LlamaForCausalLM(nn.Module):
         presents = []
         delta = None
         for i, layer in enumerate(layers):
-            attn, n1, n2 = layer.self_attn, layer.input_layernorm, layer.post_attention_layernorm
+            attn, mlp = child(layer, 'self_attn'), child(layer, 'mlp')
+            n1, n2 = child(layer, 'input_layernorm'), child(layer, 'post_attention_layernorm')
             past = None if past_key_values is None else past_key_values[i]
             if inside:
                 context, present, h = attn.attend_one(h, position_ids, past, norm=(delta, n1.weight, n1.variance_epsilon))
-                h, delta = layer.mlp.forward_normed(h, attn.project_out(*context), n2.weight, n2.variance_epsilon)
+                h, delta = mlp.forward_normed(h, attn.project_out(*context), n2.weight, n2.variance_epsilon)
             else:
                 order = order_of(attn)
                 if delta is None:
@@ -241,9 +243,9 @@ class LlamaForCausalLM(nn.Module):
                     h, x = add_rms_norm(h, delta, n1.weight, n1.variance_epsilon, out_index=order)
                 out, _, present = attn(hidden_states=x, position_ids=position_ids, past_key_value=past, use_cache=use_cache, causal=True,
                                        ordered=order is not None)
-                order = order_of(layer.mlp)
+                order = order_of(mlp)
                 h, x = add_rms_norm(h, out, n2.weight, n2.variance_epsilon, out_index=order)
-                delta = layer.mlp(x, ordered=True) if order is not None else layer.mlp(x)
+                delta = mlp(x, ordered=True) if order is not None else mlp(x)
             presents.append(present if use_cache else None)
             del present  # (without use_cache a layer's pair is given back before the next one's is made)
         norm = self.model.norm

@@ -40,6 +40,12 @@ def held(m: nn.Module, name: str):
     return own[name] if name in own else getattr(m, name)
 
 
+def child(m: nn.Module, name: str):
+    """m.<name> of what usually is a submodule, without that half microsecond either; it may be held as something else."""
+    own = m._modules
+    return own[name] if name in own else getattr(m, name)
+
+
 def _check_matmul_args(a: torch.Tensor, qweight: torch.Tensor, groupsize: int):
     # the reference's host-side contract (quant_linear.py:244-257)
     assert a.shape[-1] == qweight.shape[0] * 8, "A must be a multiple of 8 in the last dimension"

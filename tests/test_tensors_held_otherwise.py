@@ -4,7 +4,7 @@ import torch
 import torch.nn as nn
 
 import gptq_triton_amd as G
-from gptq_triton_amd.quant_linear import compact_act_order
+from gptq_triton_amd.quant_linear import child, compact_act_order
 from test_gpu_stream import random_quant_model
 
 
@@ -67,3 +67,12 @@ def test_the_same_results(form, layout, act_order):
         form(m)
     for a, b in zip(run(), want):
         assert torch.equal(a, b)
+
+
+def test_submodules_are_found_where_they_are_held():
+    m, sub = nn.Module(), nn.Identity()
+    m.registered = sub
+    object.__setattr__(m, "plain", sub)
+    assert child(m, "registered") is sub and child(m, "plain") is sub
+    with pytest.raises(AttributeError):
+        child(m, "none")
