@@ -52,6 +52,33 @@ constexpr uint64_t S_MARK = 1ull << 32;
         int hgroups, int hbpg, uint32_t hgroup_magic
 #define STREAM_HOT_ARGS(a) (a).m[0].w, (a).m[0].meta, (a).m[1].w, (a).m[1].meta, (a).q, (a).r, (a).nb, (a).nb_magic, (a).groups, (a).batches_per_group, (a).group_magic
 
+// A SIMD issues from its oldest wave first.  Decoding a unit takes as long as its bytes do (about 115 vector instructions per
+// KiB and matrix), so of two waves with the same number of units the older one ran through at full speed and the younger one was
+// left with a third of its units and an idle partner (stamps of a LLaMA-7B gate/up launch, one row: waves 0 - 3 done at 8.9 us,
+// waves 4 - 7 at 11.1).  Two waves to a SIMD take the first place in turns, a ring of units each; four are ranked by what they
+// have left, in quarters of their own range (in turns they were 2 % slower).  One row, us, before / after: 7B gate/up 12.1 / 11.7,
+// QKV 8.5 / 8.2, o_proj 4.46 / 4.35, down_proj (sixteen waves) 7.8 / 7.4; 13B gate/up at 8 rows 20.3 / 19.1, at 16 rows 22.9 / 21.6.
+// Raising the younger half for good (12.0 us) only swaps the roles; waves of two or three units are left alone (3072 x 3072: 4.94 us,
+// 5.10 with turns).
+template <int NW>
+__device__ __forceinline__ void share_simd(int wave, int turn, int left, int n) {
+    if (NW == 8) {
+        if ((turn + (wave >> 2)) & 1)
+            __builtin_amdgcn_s_setprio(1);
+        else
+            __builtin_amdgcn_s_setprio(0);
+    } else {
+        if (4 * left >= 3 * n)
+            __builtin_amdgcn_s_setprio(3);
+        else if (2 * left >= n)
+            __builtin_amdgcn_s_setprio(2);
+        else if (4 * left >= n)
+            __builtin_amdgcn_s_setprio(1);
+        else
+            __builtin_amdgcn_s_setprio(0);
+    }
+}
+
 template <int NV>
 struct SUnit {
     u32x4_t w[NV];      // the lane's four packed words of the unit, per matrix
@@ -319,6 +346,7 @@ __global__ __launch_bounds__(64 * NW) void gptq4_stream_kernel(STREAM_HOT_PARAMS
     // ---- the loop: loads past the end of the range are switched off through their offset, not branched around, so
     //      that the compiler's counts of loads in flight stay exact
     for (int i = 0; i < n; i += DEPTH) {
+        if (n > 3) share_simd<NW>(wave, i / DEPTH, n - 1 - i, n);
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
             if (i + d < n) compute(ring[d]);
@@ -598,6 +626,7 @@ __global__ __launch_bounds__(64 * NW) void gptq4_stream_tall_kernel(STREAM_HOT_P
     };
 
     for (int i = 0; i < n; i += DEPTH) {
+        if (n > 3) share_simd<NW>(wave, i / DEPTH, n - 1 - i, n);
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
             if (i + d < n) compute(ring[d]);
@@ -863,7 +892,7 @@ uint32_t smagic(int d) { return d > 1 ? (uint32_t)(0x100000000ull / (unsigned)d 
 
 StreamTuning g_stream_tuning = {0, 0};
 
-static StreamPlan stream_plan_with(int epi, int M, int N, int K, bool norm, int strips, bool tall);
+static StreamPlan stream_plan_with(int epi, int M, int N, int K, bool norm, int strips, bool tall, int waves = 0);
 
 StreamPlan stream_plan(int epi, int M, int N, int K, bool norm) {
     // 5 .. 16 rows: a unit is the 128 input rows of TWO adjacent tiles, so that the rows' chunks - twice the bytes of a
@@ -883,12 +912,15 @@ StreamPlan stream_plan(int epi, int M, int N, int K, bool norm) {
         const bool longer = two.q >= 40 || (epi == EPI_PLAIN && two.nb >= 12 && two.q >= two.nb);
         if (two.ok && (mode == 2 || (longer && (epi != EPI_SILU_MUL || M >= 9)))) return two;
     }
-    const StreamPlan pl = stream_plan_with(epi, M, N, K, norm, 1, M > STREAM_MAX_M);
+    StreamPlan pl = stream_plan_with(epi, M, N, K, norm, 1, M > STREAM_MAX_M);
+    // (the partial sums of sixteen waves, two matrices each, may not fit beside three or four long rows)
+    if (!pl.ok && epi != EPI_PLAIN && pl.waves == 16 && !g_stream_tuning.waves) pl = stream_plan_with(epi, M, N, K, norm, 1, false, 8);
     // rows that with all of K do not fit the LDS (four of more than about 18000 values) are fetched with the units
     return !pl.ok && !pl.tall && !norm ? stream_plan_with(epi, M, N, K, norm, 1, true) : pl;
 }
 
-static StreamPlan stream_plan_with(int epi, int M, int N, int K, bool norm, int strips, bool tall) {
+// waves: 0 = by the rule below
+static StreamPlan stream_plan_with(int epi, int M, int N, int K, bool norm, int strips, bool tall, int waves) {
     StreamPlan pl = {};
     const int tuned_depth = g_stream_tuning.depth % 10;
     pl.depth = tuned_depth ? tuned_depth : 2;
@@ -902,18 +934,26 @@ static StreamPlan stream_plan_with(int epi, int M, int N, int K, bool norm, int 
     if (pl.workgroups < 1) return pl;
     pl.q = (int)(units / pl.workgroups);
     pl.r = (int)(units % pl.workgroups);
-    // Launch shape, from sweeps at LLaMA-7B shapes with the weights coming from HBM (one row): two units in flight per
-    // wave; eight waves per workgroup, sixteen for a plain projection with long ranges (down_proj: 8.1 against 8.6 us),
-    // where a wave of eight would walk through a dozen units one after the other.
-    pl.waves = g_stream_tuning.waves ? g_stream_tuning.waves : ((nv == 1 && pl.q >= 48) ? 16 : 8);
-    if (!g_stream_tuning.waves && pl.nb < pl.waves) pl.waves = 8;
-    if (pl.waves == 16 && pl.depth > 2) pl.depth = 2;
+    // Launch shape, from a sweep of waves x units in flight over the projections of hidden sizes 1024 to 8192, 1 to 4 rows, with
+    // the weights from HBM (us, eight waves of two units / of three / sixteen of one / of two).  Eight of two, but
+    //   plain, q >= 64: sixteen of two   4096 x 12288 at 1 row (q 96) 8.2 / 7.5 / 8.7 / 7.7, 11008 x 4096 (86) 8.2 / 7.9 / 8.1 / 7.3, 13824 x
+    //                                    5120 (135) 11.9 / 11.2 / 11.7 / 9.8, 6656 x 6656 at 2 rows (84) 9.5 / 8.9 / 9.3 / 8.1
+    //   plain, 40 <= q < 64: of three    5120 x 5120 (50) 6.4 / 6.1 / 6.8 / 6.9, 8192 x 3072 (48) 6.5 / 6.2 / 6.9 / 7.0 (at 2 to 4 rows level);
+    //                                    below: 4096 x 4096 (32) 4.6 / 4.7 / 5.0 / 5.2
+    //   two matrices, 3 and 4 rows, q >= 40: sixteen of one, where the LDS reads of a unit are the longer part
+    //                                    4096 QKV at 4 rows (48) 8.9 / 9.3 / 8.4 / 9.5, 5120 QKV (75) 11.7 / 12.0 / 11.2 / 11.5, gate/up 12.4 /
+    //                                    12.8 / 12.2 / 12.4; below: 3072 QKV (27) 7.5 / 8.3 / 7.7 / 8.6; at 1 and 2 rows level or slower
+    // (and only where eight waves have a thread for every output element of a range: sixteen take no call that eight do not)
     pl.pieces = (pl.q + 1 + pl.nb - 1) / pl.nb + 1;
+    const bool many = pl.nb >= 16 && (nv == 1 ? pl.q >= 64 : M >= 3 && M <= STREAM_MAX_M && pl.q >= 40 && pl.pieces * M * 16 <= 512);
+    pl.waves = g_stream_tuning.waves ? g_stream_tuning.waves : waves ? waves : many ? 16 : 8;
+    if (!tuned_depth) pl.depth = pl.waves == 16 && nv == 2 ? 1 : pl.waves == 8 && nv == 1 && pl.q >= 40 ? 3 : 2;
+    if (pl.waves == 16 && pl.depth > 2) pl.depth = 2;
     if (tall) {
         // the A operand comes from memory with every unit, LDS holds the waves' partial sums (1 KiB per wave, matrix and
         // tile) and the rotary table rows of the tokens
         pl.tall = true;
-        if (pl.depth > 2) pl.depth = 2;
+        pl.depth = tuned_depth ? (tuned_depth > 2 ? 2 : tuned_depth) : 2;
         // eight waves for every shape here (LLaMA-7B down_proj at 16 rows: 11.2 us against 11.7 with sixteen)
         if (!g_stream_tuning.waves) pl.waves = 8;
         pl.xrow = 0;
