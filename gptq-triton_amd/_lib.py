@@ -22,6 +22,7 @@ WS_HEAD_BYTES = WS_COUNTER_BYTES + (16 << 20)  # GPTQ4_WS_HEAD_BYTES: counters +
 WS_ERROR_WORD = 1                     # GPTQ4_WS_ERROR_WORD
 STATIC_SCRATCH_BYTES = WS_HEAD_BYTES + (8 << 20)  # GPTQ4_STATIC_SCRATCH_BYTES: what gptq4_matmul_static holds per GPU
 OP_MATMUL, OP_MLP_GATEUP, OP_QKV_ROTARY, OP_DECODE_ATTENTION = 0, 1, 2, 3
+OP_WITH_NORM = 0x200  # or-ed to the selector of gptq4_stream_rows: the call passes a norm weight
 OP_WITH_PERM = 0x100  # or-ed to a matmul selector in gptq4_workspace_bytes: the call passes `perm`
 
 IN_ROWS, IN_NORM_ROWS, IN_PREV, IN_NORM_PREV = 0, 1, 2, 3     # gptq4_phase_t.input

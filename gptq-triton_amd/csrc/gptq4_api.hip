@@ -918,12 +918,18 @@ static int stream_norm(StreamArgs &a, const void *delta, const void *norm_weight
 }
 
 int gptq4_stream_rows(int op, int K, int N, int groupsize) {
-    op &= ~GPTQ4_OP_WITH_PERM;
+    const bool norm = (op & GPTQ4_OP_WITH_NORM) != 0;
+    op &= ~(GPTQ4_OP_WITH_PERM | GPTQ4_OP_WITH_NORM);
     if (op < GPTQ4_OP_MATMUL || op > GPTQ4_OP_QKV_ROTARY) return 0;
     int g = groupsize;
     if (check_dims(K, N, &g)) return 0;
     const int epi = (op == GPTQ4_OP_MLP_GATEUP) ? EPI_SILU_MUL : (op == GPTQ4_OP_QKV_ROTARY ? EPI_ROPE : EPI_PLAIN);
     int rows = 0;
+    if (norm) {
+        if (epi == EPI_PLAIN || K > NORM_MAX_H) return 0;
+        while (rows < NORM_MAX_M && stream_plan(epi, rows + 1, N, K, true).ok) ++rows;
+        return rows;
+    }
     for (int m = 1; m <= STREAM_TALL_MAX_M; ++m)
         if (stream_plan(epi, m, N, K, false).ok) rows = m;
     return rows;

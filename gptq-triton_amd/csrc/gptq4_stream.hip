@@ -130,14 +130,13 @@ __global__ __launch_bounds__(64 * NW) void gptq4_stream_kernel(STREAM_HOT_PARAMS
     const __amdgpu_buffer_rsrc_t rs_x = srsrc(p.x, (uint32_t)M * K * 2u);
     constexpr int XPRE = 2;
     u32x4_t xv[XPRE];
-    NormLoads<NORM ? NORM : 1> nl;
+    constexpr int NG = NW / 4;  // rows are normalised by four waves each
+    NormRowLoads<NORM ? NORM : 1, NG> nl;
     if (NORM) {
-        if (wave < 4) {
-            if (p.nrm_delta != nullptr)
-                norm_issue_row0<true>(p.x, p.nrm_delta, p.nrm_weight, K, tid, nl);
-            else
-                norm_issue_row0<false>(p.x, p.x, p.nrm_weight, K, tid, nl);
-        }
+        if (p.nrm_delta != nullptr)
+            norm_issue_rows<true>(p.x, p.nrm_delta, p.nrm_weight, M, K, wave >> 2, tid & 255, nl);
+        else
+            norm_issue_rows<false>(p.x, p.x, p.nrm_weight, M, K, wave >> 2, tid & 255, nl);
     } else if (!PERM) {
 #pragma unroll
         for (int u = 0; u < XPRE; ++u) {
@@ -241,19 +240,19 @@ __global__ __launch_bounds__(64 * NW) void gptq4_stream_kernel(STREAM_HOT_PARAMS
     };
     if (NORM) {
         half_t *const sums = (wg == 0) ? p.nrm_sum_out : nullptr;
-        if (!PERM) {
-            // the normalised chunks go straight into the k order of the decoded weights
-            auto put = [&](int row, int c, uint4 v) { xs[row * p.xrow + c] = pair_order_u4(v); };
-            if (p.nrm_delta != nullptr)
-                norm_rows_put<true>(p.x, p.nrm_delta, p.nrm_weight, sums, put, norm_part, M, K, p.nrm_eps, tid, nl, wave < 4);
-            else
-                norm_rows_put<false>(p.x, p.x, p.nrm_weight, nullptr, put, norm_part, M, K, p.nrm_eps, tid, nl, wave < 4);
-        } else {
-            uint4 *const xn = smem + p.nat_off;  // [M][chunks], natural order: the gather reads single values of it
-            if (p.nrm_delta != nullptr)
-                norm_rows_to_lds<true>(p.x, p.nrm_delta, p.nrm_weight, sums, xn, norm_part, M, K, p.nrm_eps, tid, nl, wave < 4);
-            else
-                norm_rows_to_lds<false>(p.x, p.x, p.nrm_weight, nullptr, xn, norm_part, M, K, p.nrm_eps, tid, nl, wave < 4);
+        uint4 *const xn = smem + p.nat_off;  // PERM: [M][chunks], natural order: the gather reads single values of it
+        auto put = [&](int row, int c, uint4 v) {
+            if (PERM)
+                xn[row * chunks + c] = v;
+            else  // straight into the k order of the decoded weights
+                xs[row * p.xrow + c] = pair_order_u4(v);
+        };
+        if (p.nrm_delta != nullptr)
+            norm_put_rows<true>(sums, put, norm_part, M, K, p.nrm_eps, wave >> 2, tid & 255, nl);
+        else
+            norm_put_rows<false>(nullptr, put, norm_part, M, K, p.nrm_eps, wave >> 2, tid & 255, nl);
+        if (PERM) {
+            __syncthreads();
             for (int ch = tid; ch < M * chunks; ch += NT) gather_x(reinterpret_cast<const uint16_t *>(xn), ch);
         }
     } else if (!PERM) {
@@ -415,8 +414,9 @@ __global__ __launch_bounds__(64 * NW) void gptq4_stream_kernel(STREAM_HOT_PARAMS
             split_row(ra, e_row, bb, ss);
             float o1 = s[0], o2 = s[NV - 1];
             if (rope_which < 2) {
-                o1 = s[0] * rope_cs - s[NV - 1] * rope_sn;
-                o2 = s[NV - 1] * rope_cs + s[0] * rope_sn;
+                // (which product goes into the fused addition is fixed here: left to the compiler, the variants chose differently)
+                o1 = __builtin_fmaf(s[0], rope_cs, -(s[NV - 1] * rope_sn));
+                o2 = __builtin_fmaf(s[NV - 1], rope_cs, s[0] * rope_sn);
             }
             half_t *dst;
             size_t off;

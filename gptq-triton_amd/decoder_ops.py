@@ -13,9 +13,10 @@ from . import _lib
 
 # limits of the matmul kernels that normalise their own input (gptq4_norm_qkv_rotary, gptq4_norm_mlp_gateup)
 NORM_MAX_ROWS, NORM_MAX_HIDDEN = 4, 8192
-# up to how many rows the decoder uses them: one row costs 1.3-1.4 us on top of the plain projection against
-# a 4.7 us norm launch; two rows about as much as the launch, three and four more (every workgroup
-# normalises every row)
+# up to how many rows the decoder uses them on weights in checkpoint order: one row costs 1.3-1.4 us on top of the plain
+# projection against a 2.8 us norm launch; two rows about as much as the launch, three and four more (every workgroup
+# normalises every row, one after the other).  In streaming order (norm_fusion_pays: streamed) the rows are normalised side
+# by side: 0.2 / 0.6 / 1.1 / 1.5 us for 1 / 2 / 3 / 4 rows of 4096, 0.6 / 0.8 / 1.8 / 2.2 of 5120
 NORM_PAYS_ROWS = 1
 # GPTQ4_NORM_FUSION=0 in the environment keeps the norms as launches of their own (for A/B timing)
 NORM_FUSION = os.environ.get("GPTQ4_NORM_FUSION", "1") != "0"
@@ -26,9 +27,12 @@ def norm_fusable(rows: int, hidden: int) -> bool:
     return 0 < rows <= NORM_MAX_ROWS and hidden <= NORM_MAX_HIDDEN and hidden % 8 == 0
 
 
-def norm_fusion_pays(rows: int, hidden: int) -> bool:
-    """Whether it is also the faster way (what the decoder asks)."""
-    return NORM_FUSION and rows <= NORM_PAYS_ROWS and norm_fusable(rows, hidden)
+def norm_fusion_pays(rows: int, hidden: int, streamed=None) -> bool:
+    """Whether it is also the faster way (what the decoder asks).  streamed(): the rows that the launch on streaming-order
+    weights normalises, 0 in checkpoint order."""
+    if not (NORM_FUSION and norm_fusable(rows, hidden)):
+        return False
+    return rows <= NORM_PAYS_ROWS or (NORM_PAYS_ROWS > 0 and streamed is not None and rows <= streamed())
 
 
 def check_norm_args(h: torch.Tensor, delta, weight: torch.Tensor):

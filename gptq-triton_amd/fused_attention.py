@@ -20,7 +20,7 @@ import torch.nn as nn
 from . import _lib
 from .decoder_ops import (ATTENTION_MAX_HEADS, NORM_MAX_ROWS, check_norm_args, contiguous_delta, decode_attention, extend_attention,
                           norm_fusable, norm_fusion_pays, prefill_attention)
-from .quant_linear import QuantLinear, _check_device_tensors, _check_matmul_args, InverseOrder, child, only_itself
+from .quant_linear import QuantLinear, _check_device_tensors, _check_matmul_args, InverseOrder, child, only_itself, stream_norm_rows
 
 
 @dataclass
@@ -313,7 +313,11 @@ class QuantLlamaAttention(nn.Module):
 
     def norm_fusable(self, rows: int) -> bool:
         """Whether project_qkv(norm=...) is the faster way for this many rows."""
-        return norm_fusion_pays(rows, self.hidden_size)
+        return norm_fusion_pays(rows, self.hidden_size, self._streamed_norm_rows)
+
+    def _streamed_norm_rows(self) -> int:
+        qkv = child(self, 'qkv_proj')
+        return 0 if qkv.stream_weights() is None else stream_norm_rows(_lib.OP_QKV_ROTARY, qkv.infeatures, qkv.outfeatures, qkv.groupsize)
 
     def forward(
         self,

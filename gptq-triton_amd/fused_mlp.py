@@ -14,7 +14,7 @@ import torch.nn as nn
 
 from . import _lib
 from .decoder_ops import NORM_MAX_ROWS, check_norm_args, contiguous_delta, norm_fusable, norm_fusion_pays
-from .quant_linear import (InverseOrder, QuantLinear, _check_device_tensors, _check_matmul_args, child, held, matmul4, stream_pack, stream_rows, stream_unpack,
+from .quant_linear import (InverseOrder, QuantLinear, _check_device_tensors, _check_matmul_args, child, held, matmul4, stream_norm_rows, stream_pack, stream_rows, stream_unpack,
                            tensor_key)
 
 
@@ -316,7 +316,12 @@ class QuantLlamaMLP(nn.Module):
 
     def norm_fusable(self, rows: int) -> bool:
         """Whether forward_normed is the faster way for this many rows."""
-        return norm_fusion_pays(rows, self.infeatures)
+        return norm_fusion_pays(rows, self.infeatures, self._streamed_norm_rows)
+
+    def _streamed_norm_rows(self) -> int:
+        if held(self, '_gate_meta') is None:
+            return 0
+        return min(self._stream_rows, stream_norm_rows(_lib.OP_MLP_GATEUP, self.infeatures, held(self, 'gate_proj_qweight').shape[1], self.groupsize))
 
     def forward_normed(self, h: torch.Tensor, delta: Optional[torch.Tensor], norm_weight: torch.Tensor, eps: float):
         """(h + delta, forward(RMSNorm(h + delta))): the residual add and the norm run inside the gate/up launch."""

@@ -22,7 +22,7 @@ from .decoder_ops import (NORM_MAX_HIDDEN, add_rms_norm, decode_attention, greed
                           norm_fusion_pays, prefill_attention, rms_norm)
 from .fused_attention import KV_AT_POSITION, LlamaConfigLite, QuantLlamaAttention
 from .fused_mlp import QuantLlamaMLP, llama_mlp_4_stream
-from .quant_linear import InverseOrder, QuantLinear, child, only_itself, stream_rows
+from .quant_linear import InverseOrder, QuantLinear, child, only_itself, stream_norm_rows, stream_rows
 
 # the rows the decode kernels built on the streaming-order weight layout take (more rows: the mid-M and tiled kernels)
 STREAM_BATCH = 16
@@ -127,7 +127,9 @@ class LlamaMLP(nn.Module):
 
     def norm_fusable(self, rows: int) -> bool:
         """Whether forward_normed is the faster way for this many rows."""
-        return only_itself(self, LlamaMLP) and self._pair(rows) is not None and norm_fusion_pays(rows, self.gate_proj.infeatures)
+        gate = child(self, 'gate_proj')
+        return only_itself(self, LlamaMLP) and self._pair(rows) is not None and norm_fusion_pays(
+            rows, gate.infeatures, lambda: stream_norm_rows(_lib.OP_MLP_GATEUP, gate.infeatures, gate.outfeatures, gate.groupsize))
 
     def forward_normed(self, h, delta, norm_weight, eps):
         """(h + delta, forward(RMSNorm(h + delta))) with the residual add and the norm inside the gate/up launch."""

@@ -73,6 +73,7 @@ extern "C" {
 #define GPTQ4_OP_QKV_ROTARY 2
 #define GPTQ4_OP_DECODE_ATTENTION 3 /* M = B * H, K = kv_capacity, N unused */
 #define GPTQ4_OP_WITH_PERM 0x100    /* or-ed to a matmul selector: the call will pass `perm` */
+#define GPTQ4_OP_WITH_NORM 0x200    /* or-ed to the selector of gptq4_stream_rows(): the call will pass `norm_weight` */
 
 int gptq4_abi_version(void);
 const char *gptq4_strerror(int code);
@@ -283,7 +284,8 @@ int gptq4_prefill_attention(const void *q, const void *k_cache, const void *v_ca
 /* Most rows (M) the streaming-order entry points take for this operator and shape (at most 16); 0: the shape is not
  * supported (K below 1024, or partial sums that do not fit a CU's LDS).  Up to 4 rows the kernel keeps the rows in LDS;
  * from 5 rows on, and where the rows do not fit there, a variant fetches them with every block of weights.  `op` is a GPTQ4_OP_* matmul selector, N = I
- * for MLP_GATEUP, N = 3*H*D for QKV_ROTARY. */
+ * for MLP_GATEUP, N = 3*H*D for QKV_ROTARY.  With GPTQ4_OP_WITH_NORM: the rows (at most 4) whose residual add and norm the
+ * launch takes along. */
 int gptq4_stream_rows(int op, int K, int N, int groupsize);
 
 /* Checkpoint order -> streaming order and back.  smeta (and with it qzeros, scales) may be NULL: words only.
