@@ -808,7 +808,7 @@ int gptq4_extend_attention(const void *q, const void *past_k, const void *past_v
 static int head_argmax(HeadArgs &a, void *workspace, size_t workspace_bytes, void *stream) {
     if (!head_argmax_fits(a.B, a.K, a.V)) return -GPTQ4_E_SHAPE;
     if (workspace == nullptr || workspace_bytes < GPTQ4_WS_HEAD_BYTES + head_argmax_partial_bytes()) return -GPTQ4_E_WORKSPACE;
-    a.part = reinterpret_cast<float *>(reinterpret_cast<char *>(workspace) + GPTQ4_WS_HEAD_BYTES);
+    a.best = reinterpret_cast<uint64_t *>(reinterpret_cast<char *>(workspace) + GPTQ4_WS_HEAD_BYTES);
     a.counters = reinterpret_cast<int *>(workspace);
     return launch_head_argmax(a, reinterpret_cast<hipStream_t>(stream));
 }
@@ -825,6 +825,20 @@ int gptq4_lm_head_argmax(const void *x, const void *weight, int64_t *out, int B,
     a.K = K;
     a.V = V;
     return head_argmax(a, workspace, workspace_bytes, stream);
+}
+
+int gptq4_lm_head_logits(const void *x, const void *weight, void *out, int B, int K, int V, void *stream) {
+    if (!x || !weight || !out) return -GPTQ4_E_NULL;
+    if (!head_argmax_fits(B, K, V)) return -GPTQ4_E_SHAPE;
+    if (misaligned16(x) || misaligned16(weight) || (reinterpret_cast<uintptr_t>(out) & 1)) return -GPTQ4_E_ALIGN;
+    HeadArgs a = {};
+    a.x = reinterpret_cast<const half_t *>(x);
+    a.w = reinterpret_cast<const half_t *>(weight);
+    a.logits = reinterpret_cast<half_t *>(out);
+    a.B = B;
+    a.K = K;
+    a.V = V;
+    return launch_head_logits(a, reinterpret_cast<hipStream_t>(stream));
 }
 
 int gptq4_greedy_step_end(const void *x, const void *delta, const void *norm_weight, float eps, const void *weight, int B, int K, int V,

@@ -4,12 +4,17 @@
 // fp16 linear - and take the argmax of its output, generate.py.)
 //
 // A memory-bound stream over V x K x 2 bytes.  The rows of W are dealt to the workgroups in contiguous ranges and inside a
-// workgroup to its eight waves; a wave multiplies up to 16 of its rows at a time, as the A operand of
-// v_mfma_f32_16x16x32_f16 (lane (r, c): 16 bytes of row c), with the x rows as B out of LDS, so that one to sixteen
-// sequences cost the same: 8 KiB of W per wave are in flight while the 8 KiB before are multiplied.  Rows are dealt evenly,
-// not in sixteens: lanes past a tile's rows load nothing.  Sums are rounded to fp16 as the linear layer's output would be;
-// the best (value, index) per x row is kept in registers - torch.argmax's choice among equal values and NaN -, the
-// workgroups' bests go through the workspace and the last workgroup to arrive picks the winners, one wave per x row.
+// workgroup to its eight waves; a wave takes four rows at a time, 256 contiguous bytes of each per load, as the A operand of
+// v_mfma_f32_4x4x4_16b_f16: sixteen independent products of four rows by four columns, block b on the sixteenth b of the load's
+// values, whose sums meet across the lanes at the end of the four rows.  The x rows, four to a product, are B out of LDS.  4 KiB
+// of W per wave are in flight while the 4 KiB before are multiplied (8 KiB: the same from 5120 columns on, 49.9 against 47.0 us at
+// 4096; 2 KiB: 58).  With sixteen rows to a product (v_mfma_f32_16x16x32_f16) a load touched 64 bytes of sixteen rows - half
+// lines, which the streaming hint then fetched twice (58.8 us with it, 53.6 without).  32000 x 4096 at 1 / 8 / 16 rows, from HBM:
+// 53.6 / 55.4 / 60.1 -> 47.0 / 49.3 / 58.5 us (5.6 TB/s; a plain read of as many bytes takes 40), x 5120 at 8 rows 65.7 -> 58.6.
+// Rows are dealt evenly, not in fours: lanes past a tile's rows load nothing.  Sums are rounded to fp16 as the linear layer's
+// output would be.  They are the result (LOGITS), or the best (value, index) per x row is kept in registers - torch.argmax's
+// choice among equal values and NaN -, the workgroups' bests go through the workspace, one 8-byte value each, and the last
+// workgroup to arrive picks the winners, one wave per x row (2 - 4 us of the launch).
 #include "../../include/gptq4.h"
 #include "gptq4_internal.h"
 #include "gptq4_norm.h"
@@ -17,9 +22,10 @@
 namespace {
 
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 h4_t __attribute__((ext_vector_type(4)));
 constexpr int HEAD_WAVES = 8;
 constexpr int HEAD_MAX_B = 16;
-constexpr int HEAD_STEPS = 8;  // matrix steps (32 values of every row) per group of loads
+constexpr int HEAD_STEPS = 4;  // loads of 256 bytes of four rows per group
 
 // torch.argmax's order: NaN above every number, the lower index among equal values.
 __device__ __forceinline__ bool better(float v, int i, float bv, int bi) {
@@ -27,26 +33,36 @@ __device__ __forceinline__ bool better(float v, int i, float bv, int bi) {
     return v > bv || (v == bv && i < bi);
 }
 
-// NORM: 0 x as it is, 1 its RMSNorm, 2 the RMSNorm of x + delta
-template <int NORM>
-__global__ __launch_bounds__(64 * HEAD_WAVES) void gptq4_head_argmax_kernel(HeadArgs p) {
-    // [B][K / 8 + 1] chunks of 16 bytes: rows a chunk apart cost 4 conflict cycles a read at 8 and at 16 rows (SQ_LDS_BANK_CONFLICT:
-    // 4096 of a CU's 95 k cycles for 32000 x 4096), rows a power of two apart would meet in one bank
+// Sum over the sixteen lanes of a wave that are equal modulo 4, in every lane, always in the same order.
+__device__ __forceinline__ float blocks_sum(float v) {
+    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x128, 0xF, 0xF, true));  // row_ror:8
+    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x124, 0xF, 0xF, true));  // row_ror:4
+    v += __shfl_xor(v, 16);
+    return v + __shfl_xor(v, 32);
+}
+
+// NORM: 0 x as it is, 1 its RMSNorm, 2 the RMSNorm of x + delta; NB: groups of four x rows; LOGITS: the sums themselves are
+// the result
+template <int NORM, int NB, bool LOGITS>
+__global__ __launch_bounds__(64 * HEAD_WAVES) void gptq4_head_kernel(HeadArgs p) {
+    // [B][p.pitch] chunks of 16 bytes.  Rows four chunks apart beyond their length: the sixteen lanes of a pass read 64 bytes of
+    // each of four rows, all banks once.
     extern __shared__ uint4 head_xs[];
     __shared__ float s_val[HEAD_WAVES][HEAD_MAX_B];
     __shared__ int s_idx[HEAD_WAVES][HEAD_MAX_B];
     __shared__ float s_part[4];
     __shared__ int s_last;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r = lane >> 4, c = lane & 15;
-    const int B = p.B, K = p.K, chunks = K >> 3, pitch = chunks + 1;
+    const int blk = lane >> 2, c = lane & 3;
+    const int B = p.B, K = p.K, chunks = K >> 3, pitch = p.pitch;
 
-    // this wave's rows, in ntile tiles of `step` rows (16 at most)
+    // this wave's rows, in ntile tiles of `step` rows (four at most)
     const int wg0 = blockIdx.x * p.rows_per_wg, wg1 = min(wg0 + p.rows_per_wg, p.V);
     const int per_wave = (p.rows_per_wg + HEAD_WAVES - 1) / HEAD_WAVES;
     const int r0 = wg0 + wave * per_wave, r1 = min(r0 + per_wave, wg1);
-    const int ntile = (per_wave + 15) / 16, step = (per_wave + ntile - 1) / ntile;
-    const int groups = K / (32 * HEAD_STEPS);
+    const int ntile = (per_wave + 3) / 4, step = (per_wave + ntile - 1) / ntile;
+    const int loads = K >> 7;  // of 256 bytes of every row
+    const int groups = (loads + HEAD_STEPS - 1) / HEAD_STEPS;
     // (rows of 4096 or 8192 values are a power of two apart: waves that all started at the beginning of their rows would ask
     // the same few memory channels at a time, so every wave starts at a group of its own and goes round)
     const int g_first = (int)((blockIdx.x * HEAD_WAVES + wave) * 7u % (unsigned)groups);
@@ -54,16 +70,17 @@ __global__ __launch_bounds__(64 * HEAD_WAVES) void gptq4_head_argmax_kernel(Head
     u32x4_t cur[HEAD_STEPS], nxt[HEAD_STEPS];
     auto fetch = [&](u32x4_t (&dst)[HEAD_STEPS], int row0, int g) {
         const int row = row0 + c;
-        // (a row past the tile: an offset the buffer rejects - zeros, no memory touched)
-        const uint32_t off = (c < step && row < r1) ? (uint32_t)row * (uint32_t)(K * 2) + 16u * r : 0x80000000u;
+        // (a row past the tile, and what is past the row in its last group: an offset the buffer rejects - zeros, no memory touched)
+        const uint32_t off = (c < step && row < r1) ? (uint32_t)row * (uint32_t)(K * 2) + 16u * blk : 0x80000000u;
 #pragma unroll
-        for (int j = 0; j < HEAD_STEPS; ++j) dst[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, off, (uint32_t)(g * HEAD_STEPS + j) * 64u, 0);
+        for (int j = 0; j < HEAD_STEPS; ++j)
+            dst[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, g * HEAD_STEPS + j < loads ? off : 0x80000000u, (uint32_t)(g * HEAD_STEPS + j) * 256u, 2);  // (streamed once)
     };
     if constexpr (NORM == 0) {
         fetch(cur, r0, g_first);
         for (int i = tid; i < B * chunks; i += 64 * HEAD_WAVES) {
             const int b = i / chunks;
-            head_xs[i + b] = reinterpret_cast<const uint4 *>(p.x)[i];
+            head_xs[i + b * (pitch - chunks)] = reinterpret_cast<const uint4 *>(p.x)[i];
         }
     } else {
         NormLoads<NORM_KEEP> row;
@@ -74,10 +91,17 @@ __global__ __launch_bounds__(64 * HEAD_WAVES) void gptq4_head_argmax_kernel(Head
     }
     __syncthreads();
 
-    const uint4 *const xb = head_xs + min(c, B - 1) * pitch + r;
-    float bv = -INFINITY;
-    int bi = 0x7fffffff;
-    f4_t acc = {0.f, 0.f, 0.f, 0.f};
+    const uint4 *xb[NB];
+    float bv[NB];
+    int bi[NB];
+    f4_t acc[NB];
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+        xb[n] = head_xs + min(4 * n + c, B - 1) * pitch + blk;
+        bv[n] = -INFINITY;
+        bi[n] = 0x7fffffff;
+        acc[n] = f4_t{0.f, 0.f, 0.f, 0.f};
+    }
     int row0 = r0, g = g_first, left = groups;
     for (int t = ntile * groups; t > 0; --t) {
         const bool tile_ends = left == 1;
@@ -85,46 +109,56 @@ __global__ __launch_bounds__(64 * HEAD_WAVES) void gptq4_head_argmax_kernel(Head
         left = tile_ends ? groups : left - 1;
         fetch(nxt, t > 1 ? row_n : r1, g_n);
 #pragma unroll
-        for (int j = 0; j < HEAD_STEPS; ++j)
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, cur[j]), __builtin_bit_cast(h8_t, xb[4 * (g * HEAD_STEPS + j)]), acc,
-                                                         0, 0, 0);
+        for (int j = 0; j < HEAD_STEPS; ++j) {
+            if (g * HEAD_STEPS + j >= loads) break;  // (nothing of x is there either)
+            const uint2 w[2] = {make_uint2(cur[j].x, cur[j].y), make_uint2(cur[j].z, cur[j].w)};
+#pragma unroll
+            for (int n = 0; n < NB; ++n) {
+                const uint4 xv = xb[n][16 * (g * HEAD_STEPS + j)];
+                acc[n] = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(h4_t, w[0]), __builtin_bit_cast(h4_t, make_uint2(xv.x, xv.y)), acc[n], 0, 0, 0);
+                acc[n] = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(h4_t, w[1]), __builtin_bit_cast(h4_t, make_uint2(xv.z, xv.w)), acc[n], 0, 0, 0);
+            }
+        }
         if (tile_ends) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int at = 4 * r + i, row = row0 + at;
-                const float v = (float)(half_t)acc[i];  // the linear layer's fp16 output
-                if (at < step && row < r1 && better(v, row, bv, bi)) bv = v, bi = row;
+            for (int n = 0; n < NB; ++n) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int row = row0 + i;
+                    const half_t h = (half_t)blocks_sum(acc[n][i]);  // the linear layer's fp16 output
+                    if constexpr (LOGITS) {
+                        if (blk == i && i < step && row < r1 && 4 * n + c < B) p.logits[(size_t)(4 * n + c) * p.V + row] = h;
+                    } else {
+                        if (i < step && row < r1 && better((float)h, row, bv[n], bi[n])) bv[n] = (float)h, bi[n] = row;
+                    }
+                }
+                acc[n] = f4_t{0.f, 0.f, 0.f, 0.f};
             }
-            acc = f4_t{0.f, 0.f, 0.f, 0.f};
         }
         row0 = row_n, g = g_n;
 #pragma unroll
         for (int j = 0; j < HEAD_STEPS; ++j) cur[j] = nxt[j];
     }
-    // lanes c, c + 16, c + 32, c + 48 hold bests of x row c
+    if constexpr (LOGITS) return;
+    if (lane < 4) {
 #pragma unroll
-    for (int o = 16; o <= 32; o <<= 1) {
-        const float ov = __shfl_xor(bv, o);
-        const int oi = __shfl_xor(bi, o);
-        if (better(ov, oi, bv, bi)) bv = ov, bi = oi;
-    }
-    if (lane < HEAD_MAX_B) {
-        s_val[wave][lane] = bv;
-        s_idx[wave][lane] = bi;
+        for (int n = 0; n < NB; ++n) {
+            s_val[wave][4 * n + lane] = bv[n];
+            s_idx[wave][4 * n + lane] = bi[n];
+        }
     }
     __syncthreads();
 
     // ---- the workgroup's best per x row -> workspace; the last workgroup to arrive reduces them
     const int nwg = gridDim.x;
     if (tid < B) {
-        bv = -INFINITY;
-        bi = 0x7fffffff;
+        float bv = -INFINITY;
+        int bi = 0x7fffffff;
 #pragma unroll
         for (int wv = 0; wv < HEAD_WAVES; ++wv)
             if (better(s_val[wv][tid], s_idx[wv][tid], bv, bi)) bv = s_val[wv][tid], bi = s_idx[wv][tid];
-        float *dst = p.part + ((size_t)blockIdx.x * HEAD_MAX_B + tid) * 2;
-        __hip_atomic_store(dst, bv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(reinterpret_cast<int *>(dst) + 1, bi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(p.best + (size_t)blockIdx.x * HEAD_MAX_B + tid, (uint64_t)__float_as_uint(bv) | (uint64_t)(uint32_t)bi << 32, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -136,13 +170,19 @@ __global__ __launch_bounds__(64 * HEAD_WAVES) void gptq4_head_argmax_kernel(Head
     if (!s_last) return;
     if (tid == 0) __hip_atomic_store(&p.counters[0], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (int b = wave; b < B; b += HEAD_WAVES) {
-        bv = -INFINITY;
-        bi = 0x7fffffff;
-        for (int i = lane; i < nwg; i += 64) {
-            const float *src = p.part + ((size_t)i * HEAD_MAX_B + b) * 2;
-            const float v = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const int at = __hip_atomic_load(reinterpret_cast<const int *>(src) + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (better(v, at, bv, bi)) bv = v, bi = at;
+        float bv = -INFINITY;
+        int bi = 0x7fffffff;
+        for (int i = lane; i < nwg; i += 256) {
+            uint64_t got[4];  // (together: a round trip each costs more than everything else here; past the last workgroup the last one again)
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                got[k] = __hip_atomic_load(p.best + (size_t)min(i + 64 * k, nwg - 1) * HEAD_MAX_B + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float v = __uint_as_float((uint32_t)got[k]);
+                const int at = (int)(got[k] >> 32);
+                if (better(v, at, bv, bi)) bv = v, bi = at;
+            }
         }
 #pragma unroll
         for (int o = 32; o >= 1; o >>= 1) {
@@ -166,24 +206,36 @@ __global__ __launch_bounds__(64 * HEAD_WAVES) void gptq4_head_argmax_kernel(Head
     }
 }
 
-template <int NORM>
-int launch_norm(HeadArgs &a, hipStream_t stream) {
+template <int NORM, int NB, bool LOGITS>
+int launch_kernel(HeadArgs &a, hipStream_t stream) {
     const int cus = device_shape().cus;
     const int nwg = a.V < cus ? a.V : cus;
     a.rows_per_wg = (a.V + nwg - 1) / nwg;
     const int grid = (a.V + a.rows_per_wg - 1) / a.rows_per_wg;
-    const size_t lds = (size_t)a.B * (a.K / 8 + 1) * 16;
+    a.pitch = a.K / 8 + 4;
+    if ((size_t)a.B * a.pitch * 16 > (size_t)HEAD_LDS_BYTES) a.pitch = a.K / 8 + 1;
+    const size_t lds = (size_t)a.B * a.pitch * 16;
     if (lds > 48 * 1024) {
         static LdsGrant grant;
-        if (const int rc = allow_lds(grant, reinterpret_cast<const void *>(&gptq4_head_argmax_kernel<NORM>), HEAD_LDS_BYTES)) return rc;
+        if (const int rc = allow_lds(grant, reinterpret_cast<const void *>(&gptq4_head_kernel<NORM, NB, LOGITS>), HEAD_LDS_BYTES)) return rc;
     }
-    hipLaunchKernelGGL((gptq4_head_argmax_kernel<NORM>), dim3((unsigned)grid), dim3(64 * HEAD_WAVES), lds, stream, a);
+    hipLaunchKernelGGL((gptq4_head_kernel<NORM, NB, LOGITS>), dim3((unsigned)grid), dim3(64 * HEAD_WAVES), lds, stream, a);
     return (int)hipGetLastError();
+}
+
+template <bool LOGITS>
+int launch_rows(HeadArgs &a, hipStream_t stream) {
+    switch ((a.B + 3) / 4) {
+        case 1: return launch_kernel<0, 1, LOGITS>(a, stream);
+        case 2: return launch_kernel<0, 2, LOGITS>(a, stream);
+        case 3: return launch_kernel<0, 3, LOGITS>(a, stream);
+        default: return launch_kernel<0, 4, LOGITS>(a, stream);
+    }
 }
 
 }  // namespace
 
-size_t head_argmax_partial_bytes() { return (size_t)device_shape().cus * HEAD_MAX_B * 2 * sizeof(float); }
+size_t head_argmax_partial_bytes() { return (size_t)device_shape().cus * HEAD_MAX_B * sizeof(uint64_t); }
 
 bool head_argmax_fits(int B, int K, int V) {
     return B >= 1 && B <= HEAD_MAX_B && V >= 1 && K >= 256 && (K % 256) == 0 && (size_t)V * K * 2 < 0x7FFFFFF0ull &&
@@ -191,6 +243,8 @@ bool head_argmax_fits(int B, int K, int V) {
 }
 
 int launch_head_argmax(HeadArgs &a, hipStream_t stream) {
-    if (a.nrm_weight == nullptr) return launch_norm<0>(a, stream);
-    return a.delta == nullptr ? launch_norm<1>(a, stream) : launch_norm<2>(a, stream);
+    if (a.nrm_weight == nullptr) return launch_rows<false>(a, stream);
+    return a.delta == nullptr ? launch_kernel<1, 1, false>(a, stream) : launch_kernel<2, 1, false>(a, stream);
 }
+
+int launch_head_logits(HeadArgs &a, hipStream_t stream) { return launch_rows<true>(a, stream); }

@@ -241,9 +241,11 @@ struct HeadArgs {
     const half_t *x;  // [B, K]
     const half_t *w;  // [V, K]
     long long *tokens;
-    float *part;
+    uint64_t *best;  // [workgroups][16]: (value, index) of the workgroup's best per x row
     int *counters;
     int B, K, V, rows_per_wg;
+    int pitch;         // 16-byte chunks from row to row of x in LDS
+    half_t *logits;    // [B, V] (launch_head_logits only)
     // a decoding loop's state (positions null: tokens only): positions[b] moves on by one, the token is stored at that place
     // of history [B, history_capacity] and (embed not null) its row of embed [V, K] goes to next_hidden [B, K]
     int *positions;
@@ -257,6 +259,7 @@ struct HeadArgs {
 };
 bool head_argmax_fits(int B, int K, int V);
 int launch_head_argmax(HeadArgs &a, hipStream_t stream);
+int launch_head_logits(HeadArgs &a, hipStream_t stream);
 int launch_attn_prefill(const half_t *q, const half_t *kc, const half_t *vc, half_t *out, int B, int H, int S, int capacity, int past,
                         float scale, hipStream_t stream);
 int launch_attn_decode(const half_t *q, const half_t *kc, const half_t *vc, const int *positions, half_t *out,

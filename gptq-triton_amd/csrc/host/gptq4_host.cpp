@@ -589,6 +589,26 @@ PyObject *lm_head_argmax(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
+// lm_head_logits(x, weight) -> fp16 logits, V in the place of x's last dimension
+PyObject *lm_head_logits(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    GPTQ4_TAKES(2)
+    Args a{v};
+    const at::Tensor *x = a.need(0), *w = a.need(1);
+    if (!a.fine || !is_rows(x) || x->size(-1) == 0 || !is_table(w, x->size(-1), x->device())) Py_RETURN_NONE;
+    const int64_t k = x->size(-1), b = x->numel() / k;
+    at::Tensor out = empty_rows(*x, w->size(0));
+    const hipStream_t stream = stream_of(x->device());
+    int rc;
+    {
+        NoGil unlocked;
+        rc = gptq4_lm_head_logits(data(x), data(w), out.data_ptr(), (int)b, (int)k, (int)w->size(0), stream);
+    }
+    if (rc) return failed(rc, "gptq4_lm_head_logits");
+    return THPVariable_Wrap(out);
+    END_HANDLE_TH_ERRORS
+}
+
 // greedy_step_end(x, delta, norm weight, eps, lm_head weight, tokens, positions, history, embedding, next hidden) -> True;
 // embedding and next hidden None: not fetched
 PyObject *greedy_step_end(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
@@ -668,6 +688,7 @@ PyMethodDef g_methods[] = {GPTQ4_METHOD(init),
                            GPTQ4_METHOD(decode_attention),
                            GPTQ4_METHOD(extend_attention),
                            GPTQ4_METHOD(lm_head_argmax),
+                           GPTQ4_METHOD(lm_head_logits),
                            GPTQ4_METHOD(greedy_step_end),
                            {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_host", "The package's calls of libgptq4 on torch tensors.", -1, g_methods, nullptr, nullptr, nullptr, nullptr};

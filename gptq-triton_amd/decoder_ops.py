@@ -124,6 +124,15 @@ def lm_head_argmax(x: torch.Tensor, weight: torch.Tensor, max_rows: int = HEAD_M
     return out
 
 
+def lm_head_logits(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """x @ weight.T for up to HEAD_MAX_ROWS rows of x fp16 [..., K] and an fp16 lm_head weight [V, K] (head_argmax_takes)."""
+    x = x.contiguous()
+    out = _lib.host().lm_head_logits(x if x.data_ptr() % 16 == 0 else x.clone(), weight)
+    if out is None:
+        raise _lib.refused("lm_head_logits")
+    return out
+
+
 def greedy_step_end(x, delta, norm_weight, eps, weight, tokens, positions, history, embed=None, next_hidden=None) -> None:
     """The end of a greedy decode step in one launch: tokens (int64) become the argmax of the logits, positions (int32) go up by
     one, the tokens are stored at those places of history (int64 [B, capacity]) and, if given, their rows of the embedding in

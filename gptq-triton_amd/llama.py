@@ -18,14 +18,15 @@ import torch
 import torch.nn as nn
 
 from . import _lib
-from .decoder_ops import (NORM_MAX_HIDDEN, add_rms_norm, decode_attention, greedy_step_end, head_argmax_takes, lm_head_argmax,
+from .decoder_ops import (NORM_MAX_HIDDEN, add_rms_norm, decode_attention, greedy_step_end, head_argmax_takes, lm_head_argmax, lm_head_logits,
                           norm_fusion_pays, prefill_attention, rms_norm)
 from .fused_attention import KV_AT_POSITION, LlamaConfigLite, QuantLlamaAttention
 from .fused_mlp import QuantLlamaMLP, llama_mlp_4_stream
-from .quant_linear import InverseOrder, QuantLinear, child, only_itself, stream_norm_rows, stream_rows
+from .quant_linear import InverseOrder, QuantLinear, child, only_itself, plain_module, stream_norm_rows, stream_rows
 
 # the rows the decode kernels built on the streaming-order weight layout take (more rows: the mid-M and tiled kernels)
 STREAM_BATCH = 16
+LINEAR_FORWARD = nn.Linear.forward  # torch's own
 
 
 def config_from_json(path) -> LlamaConfigLite:
@@ -206,7 +207,7 @@ class LlamaForCausalLM(nn.Module):
             h, presents = self._layers_fused(h, past_len, past_key_values, use_cache)
             if last_token_only:
                 h = h[:, -1:, :]
-            return self.lm_head(h), (presents if use_cache else None)
+            return self._logits(h), (presents if use_cache else None)
         position_ids = torch.arange(past_len, past_len + q_len, device=input_ids.device).unsqueeze(0)
         presents = []
         for i, layer in enumerate(self.model.layers):
@@ -219,6 +220,16 @@ class LlamaForCausalLM(nn.Module):
         if last_token_only:
             h = h[:, -1:, :]
         return self.lm_head(h), (presents if use_cache else None)
+
+    def _logits(self, h):
+        """lm_head(h); up to HEAD_MAX_ROWS rows in a launch that streams the weight once (two rows of 4096 through 32000 x 4096:
+        torch's product 69 us), where lm_head is torch's own linear layer and nothing else would run with it."""
+        head = self.lm_head
+        if type(head) is nn.Linear and plain_module(head) and nn.Linear.forward is LINEAR_FORWARD and head.bias is None \
+                and head.weight.device == h.device and head.weight.shape[1] == h.shape[-1] \
+                and head_argmax_takes(h.numel() // h.shape[-1], head.weight) and not torch.is_autocast_enabled(h.device.type):
+            return lm_head_logits(h, head.weight)
+        return head(h)
 
     def _layers_fused(self, h, past_len, past_key_values, use_cache):
         """The stack and the final norm with every residual add in the launch of the norm behind it, and with one token in all

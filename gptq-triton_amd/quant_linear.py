@@ -26,8 +26,11 @@ def only_itself(m, cls) -> bool:
     """Whether calling `m` runs the forward that `cls` came with and nothing else: no subclass, no hook on it or on all modules,
     no forward put in the place of the instance's or the class's.  What computes a module's result without calling it asks
     this first.  (cls.own_forward: the forward a class of this package was defined with.)"""
-    if type(m) is not cls or cls.forward is not cls.own_forward:
-        return False
+    return type(m) is cls and cls.forward is cls.own_forward and plain_module(m)
+
+
+def plain_module(m: nn.Module) -> bool:
+    """Whether calling `m` runs its class's forward and no hook."""
     d = m.__dict__
     return not (d['_forward_hooks'] or d['_forward_pre_hooks'] or d['_backward_hooks'] or d['_backward_pre_hooks'] or 'forward' in d
                 or _nn_module._global_forward_hooks or _nn_module._global_forward_pre_hooks

@@ -243,7 +243,11 @@ int gptq4_extend_attention(const void *q, const void *past_k, const void *past_v
 int gptq4_lm_head_argmax(const void *x, const void *weight, int64_t *out, int B, int K, int V, void *workspace,
                          size_t workspace_bytes, void *stream);
 
-/* The same launch also moves a decoding loop on to its next step: tokens[b] = the argmax; positions[b] (int32) goes up by
+/* The logits themselves: out fp16 [B, V] = x . weight^T for the same operands (fp32 sums, rounded to fp16 once).  No workspace.
+ * Replaces the lm_head call of a sampling loop (the reference leaves it to the dense linear layer of transformers). */
+int gptq4_lm_head_logits(const void *x, const void *weight, void *out, int B, int K, int V, void *stream);
+
+/* gptq4_lm_head_argmax's launch also moves a decoding loop on to its next step: tokens[b] = the argmax; positions[b] (int32) goes up by
  * one, tokens[b] is stored at that place of history int64 [B, history_capacity] (if it has room), and, with
  * embed and next_hidden (both or neither), its row of the embedding embed fp16 [V, K] is copied to next_hidden fp16 [B, K],
  * which may not be x or delta.  With norm_weight fp16 [K] (B == 1, K <= 8192) x is the residual stream and the logits are those of

@@ -156,3 +156,39 @@ def test_operands_off_the_16_byte_grid(b, which):
     w[best] = 0.05 * x[:, 0]   # row `best` wins by far: its logit is about 100 where the others' spread is about 1
     got = ops().lm_head_argmax(off_by_one(x) if which != "weight" else x, off_by_one(w) if which != "x" else w)
     assert torch.equal(got.view(-1), best)
+
+
+@pytest.mark.parametrize("b", [1, 2, 4, 5, 9, 16])
+@pytest.mark.parametrize("k,v", [(256, 1), (768, 3), (1280, 255), (4096, 1031), (4864, 2049)])
+def test_logits_against_float64(b, k, v):
+    """Rows that do not fill a tile, a wave or a workgroup, and row lengths that end within a group of loads.  Every logit is
+    within half an fp16 ulp plus the bound of k fp32 additions in any order of the exact sum."""
+    gen = torch.Generator(device="cuda").manual_seed(b + k + v)
+    x = torch.randn((b, 1, k), device="cuda", generator=gen).half()
+    w = 0.02 * torch.randn((v, k), device="cuda", generator=gen).half()
+    y = ops().lm_head_logits(x, w)
+    assert y.shape == (b, 1, v) and y.dtype == torch.float16
+    xd, wd = x.view(b, k).double().cpu(), w.double().cpu()
+    exact, size = xd @ wd.t(), xd.abs() @ wd.abs().t()
+    err = (y.view(b, v).double().cpu() - exact).abs()
+    assert bool((err <= exact.abs() * 2.0 ** -11 + size * k * 2.0 ** -24 + 2.0 ** -25).all()), float((err / size).max())
+    assert torch.equal(ops().lm_head_argmax(x, w).view(b), y.view(b, v).argmax(-1))   # the same sums
+
+
+def test_logits_of_a_model_with_a_hook_on_its_lm_head():
+    """forward() calls an lm_head that a hook hangs on, and gives torch's logits within an fp16 ulp where none does."""
+    from gptq_triton_amd.llama import LlamaForCausalLM
+    head = torch.nn.Linear(512, 300, bias=False).cuda().half()
+    model = LlamaForCausalLM.__new__(LlamaForCausalLM)
+    torch.nn.Module.__init__(model)
+    model.lm_head = head
+    h = torch.randn((3, 1, 512), device="cuda").half()
+    with torch.no_grad():
+        own, torchs = model._logits(h), head(h)
+        assert float((own.float() - torchs.float()).abs().max()) <= 2.0 ** -10 * float(torchs.abs().max())
+        calls = []
+        handle = head.register_forward_hook(lambda m, i, o: calls.append(1) or o + 1)
+        assert torch.equal(model._logits(h), torchs + 1) and calls
+        handle.remove()
+        head.bias = torch.nn.Parameter(torch.ones(300, device="cuda").half())
+        assert torch.equal(model._logits(h), head(h))
