@@ -913,8 +913,11 @@ StreamPlan stream_plan(int epi, int M, int N, int K, bool norm) {
         if (two.ok && (mode == 2 || (longer && (epi != EPI_SILU_MUL || M >= 9)))) return two;
     }
     StreamPlan pl = stream_plan_with(epi, M, N, K, norm, 1, M > STREAM_MAX_M);
-    // (the partial sums of sixteen waves, two matrices each, may not fit beside three or four long rows)
-    if (!pl.ok && epi != EPI_PLAIN && pl.waves == 16 && !g_stream_tuning.waves) pl = stream_plan_with(epi, M, N, K, norm, 1, false, 8);
+    // The partial sums of sixteen waves, two matrices each, may not fit beside three or four long rows.  Whether they do is asked
+    // with the norm inside wherever it can be (four rows of 8192 fit without it only): the call with it and the norm launch
+    // with the call behind it give the same bits.
+    if (epi != EPI_PLAIN && pl.waves == 16 && !g_stream_tuning.waves && !stream_plan_with(epi, M, N, K, norm || K <= NORM_MAX_H, 1, false).ok)
+        pl = stream_plan_with(epi, M, N, K, norm, 1, false, 8);
     // rows that with all of K do not fit the LDS (four of more than about 18000 values) are fetched with the units
     return !pl.ok && !pl.tall && !norm ? stream_plan_with(epi, M, N, K, norm, 1, true) : pl;
 }

@@ -444,6 +444,31 @@ def test_normalising_variants_equal_norm_launch_plus_plain_call(hidden, heads, i
     assert head_is_zero()
 
 
+@pytest.mark.parametrize("hidden,inter,g", [(1280, 768, 128), (2304, 5632, -1), (4352, 11520, 128), (6656, 17920, 512), (8192, 4096, 128)])
+@pytest.mark.parametrize("m", [1, 2, 3, 4])
+def test_rows_normalised_side_by_side(hidden, inter, g, m):
+    """Row lengths that end within a thread's chunks, the longest, and launches of eight and sixteen waves (two and four groups
+    that normalise): the residual sums keep their bits, the results are those of the norm launch and the plain call."""
+    G = gptq()
+    from gptq_triton_amd import _lib
+    from gptq_triton_amd.decoder_ops import add_rms_norm
+    from gptq_triton_amd.quant_linear import stream_norm_rows
+    gs = hidden if g == -1 else g
+    layers = [to_dev(O.make_layer(hidden, n, g, seed=1650 + i)) for i, n in enumerate((3 * hidden, inter, inter))]
+    (sq, mq), (sg, mg), (su, mu) = (G.stream_pack(D["qweight"], D["qzeros"], D["scales"], gs) for D in layers)
+    assert m <= stream_norm_rows(_lib.OP_QKV_ROTARY, hidden, 3 * hidden, gs) and m <= stream_norm_rows(_lib.OP_MLP_GATEUP, hidden, inter, gs)
+    h, d, w = (torch.from_numpy(t).cuda() for t in residual_inputs(m, hidden, seed=m + 71))
+    pos = torch.arange(m, dtype=torch.int32, device="cuda").view(m, 1) * 5 + 3
+    cos, sin = G.RotaryTable(128, 2048).get(torch.device("cuda"), 2048)
+    sums, x = add_rms_norm(h, d, w, 1e-6)
+    plain = G.qkv_rotary_stream(gs, x.view(m, 1, hidden), sq, mq, pos, cos, sin, hidden // 128)
+    *normed, s = G.qkv_rotary_stream(gs, h.view(m, 1, hidden), sq, mq, pos, cos, sin, hidden // 128, norm=(d.view(m, 1, hidden), w, 1e-6))
+    assert torch.equal(s.view(m, hidden), sums) and all(torch.equal(a, b) for a, b in zip(normed, plain))
+    s, mid = G.llama_mlp_4_stream(gs, h, sg, mg, su, mu, None, norm=(d, w, 1e-6))
+    assert torch.equal(s, sums) and torch.equal(mid, G.llama_mlp_4_stream(gs, x, sg, mg, su, mu, None))
+    assert head_is_zero()
+
+
 # ------------------------------------------------------------------ the exchange between workgroups
 def test_a_wait_that_runs_out_sets_the_error_word_and_the_kernel_still_ends():
     """Spin limit 0xFFFFFFFF, the library's hook for this test: a workgroup that finishes a strip shared with a lower
