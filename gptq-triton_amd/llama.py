@@ -225,10 +225,13 @@ class LlamaForCausalLM(nn.Module):
         """lm_head(h); up to HEAD_MAX_ROWS rows in a launch that streams the weight once (two rows of 4096 through 32000 x 4096:
         torch's product 69 us), where lm_head is torch's own linear layer and nothing else would run with it."""
         head = self.lm_head
-        if type(head) is nn.Linear and plain_module(head) and nn.Linear.forward is LINEAR_FORWARD and head.bias is None \
-                and head.weight.device == h.device and head.weight.shape[1] == h.shape[-1] \
-                and head_argmax_takes(h.numel() // h.shape[-1], head.weight) and not torch.is_autocast_enabled(h.device.type):
-            return lm_head_logits(h, head.weight)
+        if type(head) is nn.Linear and plain_module(head) and nn.Linear.forward is LINEAR_FORWARD and head.bias is None:
+            weight = head.weight
+            # (a tensor subclass may stand for other values than those at its address)
+            if type(weight) in (nn.Parameter, torch.Tensor) and weight.device == h.device and weight.dim() == 2 and weight.shape[0] > 0 \
+                    and weight.shape[1] == h.shape[-1] and head_argmax_takes(h.numel() // h.shape[-1], weight) \
+                    and not torch.is_autocast_enabled(h.device.type):
+                return lm_head_logits(h, weight)
         return head(h)
 
     def _layers_fused(self, h, past_len, past_key_values, use_cache):

@@ -175,6 +175,41 @@ def test_logits_against_float64(b, k, v):
     assert torch.equal(ops().lm_head_argmax(x, w).view(b), y.view(b, v).argmax(-1))   # the same sums
 
 
+@pytest.mark.parametrize("b", [1, 6])
+def test_subnormal_weights_count(b):
+    """fp16 weights below 2^-14 are values, not zeros, in the matrix products."""
+    gen = torch.Generator(device="cuda").manual_seed(b)
+    x = 64 * torch.randn((b, 1024), device="cuda", generator=gen).half()
+    w = (2.0 ** -17 * torch.randn((77, 1024), device="cuda", generator=gen)).half()
+    exact = x.double() @ w.double().t()
+    size = x.double().abs() @ w.double().abs().t()
+    assert bool(((ops().lm_head_logits(x, w).double() - exact).abs() <= exact.abs() * 2.0 ** -11 + size * 1024 * 2.0 ** -24 + 2.0 ** -25).all())
+
+
+def test_logits_of_a_weight_that_is_more_than_a_tensor():
+    """A weight of a tensor subclass, and a vocabulary of none, take torch's linear layer as before."""
+    from gptq_triton_amd.llama import LlamaForCausalLM
+
+    class Counted(torch.Tensor):
+        calls = 0
+
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            cls.calls += func is torch.nn.functional.linear
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+    model = LlamaForCausalLM.__new__(LlamaForCausalLM)
+    torch.nn.Module.__init__(model)
+    model.lm_head = torch.nn.Linear(512, 300, bias=False).cuda().half()
+    h = torch.randn((3, 1, 512), device="cuda").half()
+    with torch.no_grad():
+        model.lm_head.weight = torch.nn.Parameter(model.lm_head.weight.detach().as_subclass(Counted), requires_grad=False)
+        assert model._logits(h).shape == (3, 1, 300) and Counted.calls == 1
+        model.lm_head = torch.nn.Linear(512, 300, bias=False).cuda().half()
+        model.lm_head.weight = torch.nn.Parameter(torch.empty((0, 512), device="cuda", dtype=torch.float16))
+        assert model._logits(h).shape == (3, 1, 0)
+
+
 def test_logits_of_a_model_with_a_hook_on_its_lm_head():
     """forward() calls an lm_head that a hook hangs on, and gives torch's logits within an fp16 ulp where none does."""
     from gptq_triton_amd.llama import LlamaForCausalLM
