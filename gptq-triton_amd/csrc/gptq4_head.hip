@@ -9,8 +9,9 @@
 // values, whose sums meet across the lanes at the end of the four rows.  The x rows, four to a product, are B out of LDS.  4 KiB
 // of W per wave are in flight while the 4 KiB before are multiplied (8 KiB: the same from 5120 columns on, 49.9 against 47.0 us at
 // 4096; 2 KiB: 58).  With sixteen rows to a product (v_mfma_f32_16x16x32_f16) a load touched 64 bytes of sixteen rows - half
-// lines, which the streaming hint then fetched twice (58.8 us with it, 53.6 without).  32000 x 4096 at 1 / 8 / 16 rows, from HBM:
-// 53.6 / 55.4 / 60.1 -> 47.0 / 49.3 / 58.5 us (5.6 TB/s; a plain read of as many bytes takes 40), x 5120 at 8 rows 65.7 -> 58.6.
+// lines, which the streaming hint then fetched twice (58.8 us with it, 53.6 without).  With four, us, W from HBM, the sixteen's
+// time first (argmax): 32000 x 4096 at 1 / 8 / 16 rows 56.1 / 58.9 / 63.1 -> 45.9 / 47.9 / 48.8 (5.7 TB/s; a plain read of as many
+// bytes takes 40), x 1024 19.0 / 20.8 / 23.4 -> 16.4 / 18.0 / 21.0, x 256 11.3 / 12.2 / 15.1 -> 10.6 / 11.7 / 15.1.
 // Rows are dealt evenly, not in fours: lanes past a tile's rows load nothing.  Sums are rounded to fp16 as the linear layer's
 // output would be.  They are the result (LOGITS), or the best (value, index) per x row is kept in registers - torch.argmax's
 // choice among equal values and NaN -, the workgroups' bests go through the workspace, one 8-byte value each, and the last
@@ -27,10 +28,9 @@ constexpr int HEAD_WAVES = 8;
 constexpr int HEAD_MAX_B = 16;
 constexpr int HEAD_STEPS = 4;  // loads of 256 bytes of four rows per group
 
-// torch.argmax's order: NaN above every number, the lower index among equal values.
+// torch.argmax's order: NaN above every number, the lower index among equal values.  No branches: a wave's lanes differ in the outcome.
 __device__ __forceinline__ bool better(float v, int i, float bv, int bi) {
-    if (v != v || bv != bv) return v != v && (bv == bv || i < bi);
-    return v > bv || (v == bv && i < bi);
+    return (v > bv) | ((v == bv) & (i < bi)) | ((v != v) & ((bv == bv) | (i < bi)));
 }
 
 // Sum over the sixteen lanes of a wave that are equal modulo 4, in every lane, always in the same order.
@@ -64,7 +64,8 @@ __global__ __launch_bounds__(64 * HEAD_WAVES) void gptq4_head_kernel(HeadArgs p)
     const int loads = K >> 7;  // of 256 bytes of every row
     const int groups = (loads + HEAD_STEPS - 1) / HEAD_STEPS;
     // (rows of 4096 or 8192 values are a power of two apart: waves that all started at the beginning of their rows would ask
-    // the same few memory channels at a time, so every wave starts at a group of its own and goes round)
+    // the same few memory channels at a time, so every wave starts at a group of its own and goes round; where the groups are a
+    // multiple of seven the waves share one or two starting points: 3584 and 7168 columns, level with wave number % groups)
     const int g_first = (int)((blockIdx.x * HEAD_WAVES + wave) * 7u % (unsigned)groups);
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(p.w), 0, (int)0x7FFFFFF0, 0x00020000);
     u32x4_t cur[HEAD_STEPS], nxt[HEAD_STEPS];
@@ -120,17 +121,21 @@ __global__ __launch_bounds__(64 * HEAD_WAVES) void gptq4_head_kernel(HeadArgs p)
             }
         }
         if (tile_ends) {
+            // Every lane gets all four rows' sums and goes on with row blk % 4 of the tile: one comparison per x row, without
+            // branches.  (Four comparisons one after the other, each behind its sum's way across the lanes and behind branches,
+            // took 3.7 us of the launch for every four x rows at 32000 rows of W, whatever their length: x 1024 at 16 rows 29.9 us.)
+            const int at = blk & 3, row = row0 + at;
+            const bool mine = (at < step) & (row < r1);
 #pragma unroll
             for (int n = 0; n < NB; ++n) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int row = row0 + i;
-                    const half_t h = (half_t)blocks_sum(acc[n][i]);  // the linear layer's fp16 output
-                    if constexpr (LOGITS) {
-                        if (blk == i && i < step && row < r1 && 4 * n + c < B) p.logits[(size_t)(4 * n + c) * p.V + row] = h;
-                    } else {
-                        if (i < step && row < r1 && better((float)h, row, bv[n], bi[n])) bv[n] = (float)h, bi[n] = row;
-                    }
+                const float s[4] = {blocks_sum(acc[n][0]), blocks_sum(acc[n][1]), blocks_sum(acc[n][2]), blocks_sum(acc[n][3])};
+                const half_t h = (half_t)(at < 2 ? at == 0 ? s[0] : s[1] : at == 2 ? s[2] : s[3]);  // the linear layer's fp16 output
+                if constexpr (LOGITS) {
+                    if (mine & (blk < 4) & (4 * n + c < B)) p.logits[(size_t)(4 * n + c) * p.V + row] = h;
+                } else {
+                    const bool up = mine & better((float)h, row, bv[n], bi[n]);
+                    bv[n] = up ? (float)h : bv[n];
+                    bi[n] = up ? row : bi[n];
                 }
                 acc[n] = f4_t{0.f, 0.f, 0.f, 0.f};
             }
@@ -140,9 +145,18 @@ __global__ __launch_bounds__(64 * HEAD_WAVES) void gptq4_head_kernel(HeadArgs p)
         for (int j = 0; j < HEAD_STEPS; ++j) cur[j] = nxt[j];
     }
     if constexpr (LOGITS) return;
-    if (lane < 4) {
+    // lanes c, c + 4, c + 8, c + 12 hold the bests of four rows of every tile
 #pragma unroll
-        for (int n = 0; n < NB; ++n) {
+    for (int n = 0; n < NB; ++n) {
+#pragma unroll
+        for (int o = 4; o <= 8; o <<= 1) {
+            const float ov = __shfl_xor(bv[n], o);
+            const int oi = __shfl_xor(bi[n], o);
+            const bool up = better(ov, oi, bv[n], bi[n]);
+            bv[n] = up ? ov : bv[n];
+            bi[n] = up ? oi : bi[n];
+        }
+        if (lane < 4) {
             s_val[wave][4 * n + lane] = bv[n];
             s_idx[wave][4 * n + lane] = bi[n];
         }

@@ -140,6 +140,23 @@ def test_nan_and_infinite_logits(b, k, v):
     assert head_is_zero()
 
 
+@pytest.mark.parametrize("b", [1, 4, 6, 16])
+def test_equal_logits_side_by_side(b):
+    """The lowest index among equal logits and NaN wherever the equals lie: next to each other (rows of one product, which
+    different lanes compare), one wave or one workgroup apart."""
+    k, v = 512, 8192   # 32 rows a workgroup of 256, four a wave
+    gen = torch.Generator(device="cuda").manual_seed(b)
+    x = (0.5 + torch.rand((b, k), device="cuda", generator=gen)).half()
+    for first in (0, 1, 2, 3, 30, 4097):
+        for step in (1, 2, 3, 4, 32):
+            for value in (0.5, float("nan")):
+                w = (0.001 * torch.randn((v, k), device="cuda", generator=gen)).half()
+                w[first::step][:5] = value
+                assert ops().lm_head_argmax(x, w).tolist() == [first] * b, (first, step, value)
+    assert ops().lm_head_argmax(torch.zeros_like(x), w.nan_to_num()).tolist() == [0] * b   # all of them
+    assert head_is_zero()
+
+
 def off_by_one(t):
     flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:]
     return flat.copy_(t.flatten()).view(t.shape)
