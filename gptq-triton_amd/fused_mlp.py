@@ -14,8 +14,8 @@ import torch.nn as nn
 
 from . import _lib
 from .decoder_ops import NORM_MAX_ROWS, check_norm_args, contiguous_delta, norm_fusable, norm_fusion_pays
-from .quant_linear import (InverseOrder, QuantLinear, _check_device_tensors, _check_matmul_args, child, held, matmul4, stream_norm_rows, stream_pack, stream_rows, stream_unpack,
-                           tensor_key)
+from .quant_linear import (InverseOrder, QuantLinear, _check_device_tensors, _check_matmul_args, child, held, matmul4, only_itself, stream_norm_rows,
+                           stream_pack, stream_rows, stream_unpack, tensor_key)
 
 
 def llama_mlp_4(groupsize: int, a: torch.Tensor,
@@ -291,9 +291,11 @@ class QuantLlamaMLP(nn.Module):
 
     def input_order(self):
         """Where a producer should store each input feature so that x arrives in the order gate and up read it
-        (int32 [infeatures], the inverse of their shared permutation; None without act-order):
-        rms_norm / add_rms_norm(out_index=...) write in that order and forward(x, ordered=True) runs
-        without a gather."""
+        (int32 [infeatures], the inverse of their shared permutation; None without act-order and where this
+        block is to be called as a module, only_itself): rms_norm / add_rms_norm(out_index=...) write in that
+        order and forward(x, ordered=True) runs without a gather."""
+        if not only_itself(self, QuantLlamaMLP):
+            return None
         perm = self._compact_rows if (self._is_compact or self._gate_meta is not None) else self._chained_weights()[1]
         return None if perm is None else self._input_order.of(perm)
 
@@ -316,7 +318,7 @@ class QuantLlamaMLP(nn.Module):
 
     def norm_fusable(self, rows: int) -> bool:
         """Whether forward_normed is the faster way for this many rows."""
-        return norm_fusion_pays(rows, self.infeatures, self._streamed_norm_rows)
+        return only_itself(self, QuantLlamaMLP) and norm_fusion_pays(rows, self.infeatures, self._streamed_norm_rows)
 
     def _streamed_norm_rows(self) -> int:
         if held(self, '_gate_meta') is None:

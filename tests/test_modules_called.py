@@ -97,6 +97,23 @@ def test_gate_and_up_are_one_launch_only_while_nothing_hangs_on_them(name, how):
     assert mlp.input_order() is not None
 
 
+@pytest.mark.parametrize("how", HOWS)
+@pytest.mark.parametrize("act_order", [False, True])
+def test_a_fused_mlp_is_called_while_something_hangs_on_it(how, act_order):
+    """The decoder normalises inside the gate/up launch, and writes the norm in the order gate and up read, only where calling
+    the block would do nothing else."""
+    new = lambda k, n: G.QuantLinear(4, 128, k, n, bias=False, act_order=act_order)
+    mlp = G.QuantLlamaMLP(new(1024, 2816), new(2816, 1024), new(1024, 2816))
+    mlp._gate_meta, mlp._stream_rows = torch.zeros(1, dtype=torch.int32), 16   # (as in streaming order; nothing is launched)
+    mlp._compact_rows = torch.arange(1024, dtype=torch.int32) if act_order else None
+    fuses = lambda: [mlp.norm_fusable(rows) for rows in (1, 2, 4)]
+    assert all(fuses()) and (mlp.input_order() is not None) == act_order
+    undo = hang(mlp, how, [])
+    assert not any(fuses()) and mlp.input_order() is None
+    undo()
+    assert all(fuses())
+
+
 def test_the_pair_is_asked_for_the_projections_there_are():
     """Projections put in the place of narrower ones: the rows the launch takes are those of the new ones."""
     mlp = streamed_mlp()
@@ -151,6 +168,38 @@ def test_forward_runs_what_hangs_on_its_modules(monkeypatch, bsz, new, act_order
             assert len(calls) == 1, (where, how, len(calls))
             assert (got - want).norm() <= 0.02 * want.norm(), (where, how)
     assert torch.equal(run(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act_order", [False, True])
+@pytest.mark.parametrize("bsz", [1, 2, 4, 6])
+def test_greedy_decoder_runs_what_hangs_on_a_fused_mlp(monkeypatch, bsz, act_order):
+    """Once a step, with the block's own input and with what it makes of the output: the tokens are those of a decoder that calls
+    its blocks in any case."""
+    from gptq_triton_amd import decoder_ops
+    model = random_quant_model(hidden=1024, inter=2816, heads=8, layers=2, groupsize=128, seed=54, act_order=act_order)
+    ids = torch.randint(0, model.config.vocab_size, (bsz, 9), device="cuda", generator=torch.Generator(device="cuda").manual_seed(bsz))
+    mlp = model.model.layers[1].mlp
+
+    def tokens():
+        dec = G.GreedyDecoder(model, bsz, 32)
+        return torch.cat([dec.prefill(ids), dec.decode(5)], dim=1)
+
+    plain = tokens()
+    for how in HOWS:
+        calls = []
+        undo = hang(mlp, how, calls)
+        tokens()
+        undo()
+        assert len(calls) == 1 + 5, (how, len(calls))
+    turned = mlp.register_forward_hook(lambda m, args, out: -4 * out - args[0])
+    got = tokens()
+    with monkeypatch.context() as mp:
+        mp.setattr(decoder_ops, "NORM_PAYS_ROWS", 0)
+        want = tokens()
+    turned.remove()
+    assert torch.equal(got, want) and not torch.equal(got, plain)
+    assert torch.equal(tokens(), plain)
 
 
 @pytest.mark.gpu
