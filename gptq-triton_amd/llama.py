@@ -249,8 +249,8 @@ class LlamaForCausalLM(nn.Module):
             n1, n2 = child(layer, 'input_layernorm'), child(layer, 'post_attention_layernorm')
             past = None if past_key_values is None else past_key_values[i]
             if inside:
-                context, present, h = attn.attend_one(h, position_ids, past, norm=(delta, n1.weight, n1.variance_epsilon))
-                h, delta = mlp.forward_normed(h, attn.project_out(*context), n2.weight, n2.variance_epsilon)
+                context, present, h = attn.attend_one(h, position_ids, past, norm=(delta, norm_weight(n1), n1.variance_epsilon))
+                h, delta = mlp.forward_normed(h, attn.project_out(*context), norm_weight(n2), n2.variance_epsilon)
             else:
                 order = order_of(attn)
                 if delta is None:
@@ -278,6 +278,12 @@ class LlamaForCausalLM(nn.Module):
         first = dec.prefill(input_ids)
         rest = dec.decode(max_new_tokens - 1, use_graph=use_graph) if max_new_tokens > 1 else first[:, :0]
         return torch.cat([input_ids, first, rest], dim=1)
+
+
+def norm_weight(norm: nn.Module) -> torch.Tensor:
+    """A norm's weight as the launches that normalise their own input read it (a strided one is copied, as rms_norm does)."""
+    w = norm.weight
+    return w if w.is_contiguous() else w.contiguous()
 
 
 def order_of(block):
@@ -356,12 +362,13 @@ class GreedyDecoder:
         add and the RMSNorm of their own input (same bits as _layers' separate launches), so a
         layer is 5 launches instead of 7."""
         layers = self.model.model.layers
+        h = h.contiguous()  # (the projections that normalise their own input take no strides)
         delta = None
         for layer, (kc, vc) in zip(layers, self.caches):
             attn, n1, n2 = layer.self_attn, layer.input_layernorm, layer.post_attention_layernorm
             q, _, _, h = attn.project_qkv(h, position_ids, kv_out=(kc, vc), kv_offset=kv_offset,
-                                          norm=(delta, n1.weight, n1.variance_epsilon))
-            h, delta = layer.mlp.forward_normed(h, attn.project_out(*attend(q, kc, vc, attn)), n2.weight, n2.variance_epsilon)
+                                          norm=(delta, norm_weight(n1), n1.variance_epsilon))
+            h, delta = layer.mlp.forward_normed(h, attn.project_out(*attend(q, kc, vc, attn)), norm_weight(n2), n2.variance_epsilon)
         return end(h, delta, self.model.model.norm, None)
 
     def _last_tokens(self, h, delta, norm, x):
@@ -377,7 +384,7 @@ class GreedyDecoder:
             self.tokens.copy_(self._last_tokens(h, delta, norm, x))
             self.position.add_(1)
             return
-        w = norm.weight
+        w = norm_weight(norm)
         if x is None and self.bsz == 1 and w.numel() <= NORM_MAX_HIDDEN:
             x = h  # (the launch normalises its row itself)
         else:

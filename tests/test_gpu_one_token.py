@@ -145,3 +145,43 @@ def test_embedding_rows_with_a_stride(model):
     finally:
         hook.remove()
     assert torch.equal(got, want)
+
+
+def tokens_of(model, bsz):
+    dec = G.GreedyDecoder(model, bsz, 32, layout="keep")
+    return torch.cat([dec.prefill(torch.arange(3 * bsz, device="cuda").view(bsz, 3)), dec.decode(4)], dim=1)
+
+
+@pytest.mark.parametrize("layout", ["stream", "checkpoint"])
+@pytest.mark.parametrize("bsz", [1, 2, 4, 5])
+def test_a_decoder_of_embedding_rows_with_a_stride(model, bsz, layout):
+    G.set_layout(model, layout)
+    want = tokens_of(model, bsz)
+    hook = model.model.embed_tokens.register_forward_hook(lambda m, args, rows: torch.stack([rows, rows], -1)[..., 0])
+    try:
+        got = tokens_of(model, bsz)
+    finally:
+        hook.remove()
+        G.set_layout(model, "checkpoint")
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("where", ["input_layernorm", "post_attention_layernorm", "norm"])
+@pytest.mark.parametrize("bsz", [1, 2, 4, 5])
+def test_norm_weights_with_a_stride(model, bsz, where):
+    """Through forward() and through the greedy decoder, in streaming order."""
+    G.set_layout(model, "stream")
+    norm = model.model.norm if where == "norm" else getattr(model.model.layers[1], where)
+    plain = norm.weight
+    ids = torch.arange(bsz, device="cuda").view(bsz, 1)
+    weights = 1 + 0.1 * torch.randn(1024, device="cuda", generator=torch.Generator(device="cuda").manual_seed(3)).half()
+    try:
+        norm.weight = torch.nn.Parameter(weights, requires_grad=False)
+        want = model(ids, past_key_values=pairs(bsz))[0], tokens_of(model, bsz)
+        norm.weight = torch.nn.Parameter(torch.stack([weights, weights], -1)[:, 0], requires_grad=False)
+        assert not norm.weight.is_contiguous()
+        got = model(ids, past_key_values=pairs(bsz))[0], tokens_of(model, bsz)
+    finally:
+        norm.weight = plain
+        G.set_layout(model, "checkpoint")
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
