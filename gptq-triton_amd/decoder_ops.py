@@ -16,8 +16,17 @@ NORM_MAX_ROWS, NORM_MAX_HIDDEN = 4, 8192
 # up to how many rows the decoder uses them on weights in checkpoint order: one row costs 1.3-1.4 us on top of the plain
 # projection against a 2.8 us norm launch; two rows about as much as the launch, three and four more (every workgroup
 # normalises every row, one after the other).  In streaming order (norm_fusion_pays: streamed) the rows are normalised side
-# by side: 0.2 / 0.6 / 1.1 / 1.5 us for 1 / 2 / 3 / 4 rows of 4096, 0.6 / 0.8 / 1.8 / 2.2 of 5120
+# by side.  QKV and gate/up behind a norm launch / with the norm inside, weights from HBM, us:
+#   hidden          1024                 4096                   5120                   6656                   8192
+#   2 rows   7.5/6.3   6.9/5.7   10.9/9.0   14.5/12.2   14.7/12.6  19.5/16.9   20.3/17.7  27.8/24.8   25.5/22.9  37.8/34.8
+#   3 rows   7.6/6.7   7.2/6.1   11.7/9.9   14.9/13.0   13.7/12.6  19.2/18.0   19.6/18.0  27.9/26.4   24.5/23.0  38.2/36.5
+#   4 rows   7.8/7.2   7.3/6.6   11.8/10.5  14.9/13.6   14.0/13.4  19.6/18.6   19.9/19.0  28.1/27.2   25.5/23.5  38.7/36.6
+# With act-order every workgroup also gathers the normalised rows, where the norm launch stores them in the order that is read:
+#   3 rows   7.9/7.2   7.5/6.6   12.1/10.8  15.4/14.0   14.1/13.7  19.8/19.1   20.1/19.4  28.4/27.6   24.8/24.7  38.6/37.9
+#   4 rows   8.1/7.8   7.5/7.2   12.2/11.6  15.4/14.8   14.4/14.7  20.1/20.1   20.4/20.7  28.7/29.0   25.9/25.7  39.0/38.9
 NORM_PAYS_ROWS = 1
+# so four act-order rows take the norm along up to this hidden size (4352: 13.1/13.3  16.9/16.8, 7168: 21.7/22.3  31.6/31.1)
+NORM_PAYS_GATHERED = 4096
 # GPTQ4_NORM_FUSION=0 in the environment keeps the norms as launches of their own (for A/B timing)
 NORM_FUSION = os.environ.get("GPTQ4_NORM_FUSION", "1") != "0"
 
@@ -29,10 +38,13 @@ def norm_fusable(rows: int, hidden: int) -> bool:
 
 def norm_fusion_pays(rows: int, hidden: int, streamed=None) -> bool:
     """Whether it is also the faster way (what the decoder asks).  streamed(): the rows that the launch on streaming-order
-    weights normalises, 0 in checkpoint order."""
+    weights normalises, 0 in checkpoint order, and whether it gathers them afterwards (act-order)."""
     if not (NORM_FUSION and norm_fusable(rows, hidden)):
         return False
-    return rows <= NORM_PAYS_ROWS or (NORM_PAYS_ROWS > 0 and streamed is not None and rows <= streamed())
+    if rows <= NORM_PAYS_ROWS or NORM_PAYS_ROWS == 0 or streamed is None:
+        return rows <= NORM_PAYS_ROWS
+    most, gathers = streamed()
+    return rows <= most and not (gathers and rows == NORM_MAX_ROWS and hidden > NORM_PAYS_GATHERED)
 
 
 def check_norm_args(h: torch.Tensor, delta, weight: torch.Tensor):

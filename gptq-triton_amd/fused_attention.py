@@ -315,9 +315,12 @@ class QuantLlamaAttention(nn.Module):
         """Whether project_qkv(norm=...) is the faster way for this many rows."""
         return norm_fusion_pays(rows, self.hidden_size, self._streamed_norm_rows)
 
-    def _streamed_norm_rows(self) -> int:
+    def _streamed_norm_rows(self):
         qkv = child(self, 'qkv_proj')
-        return 0 if qkv.stream_weights() is None else stream_norm_rows(_lib.OP_QKV_ROTARY, qkv.infeatures, qkv.outfeatures, qkv.groupsize)
+        sw = qkv.stream_weights()
+        if sw is None:
+            return 0, False
+        return stream_norm_rows(_lib.OP_QKV_ROTARY, qkv.infeatures, qkv.outfeatures, qkv.groupsize), sw[2] is not None
 
     def forward(
         self,

@@ -320,10 +320,11 @@ class QuantLlamaMLP(nn.Module):
         """Whether forward_normed is the faster way for this many rows."""
         return only_itself(self, QuantLlamaMLP) and norm_fusion_pays(rows, self.infeatures, self._streamed_norm_rows)
 
-    def _streamed_norm_rows(self) -> int:
+    def _streamed_norm_rows(self):
         if held(self, '_gate_meta') is None:
-            return 0
-        return min(self._stream_rows, stream_norm_rows(_lib.OP_MLP_GATEUP, self.infeatures, held(self, 'gate_proj_qweight').shape[1], self.groupsize))
+            return 0, False
+        rows = stream_norm_rows(_lib.OP_MLP_GATEUP, self.infeatures, held(self, 'gate_proj_qweight').shape[1], self.groupsize)
+        return min(self._stream_rows, rows), held(self, '_compact_rows') is not None
 
     def forward_normed(self, h: torch.Tensor, delta: Optional[torch.Tensor], norm_weight: torch.Tensor, eps: float):
         """(h + delta, forward(RMSNorm(h + delta))): the residual add and the norm run inside the gate/up launch."""

@@ -129,8 +129,9 @@ class LlamaMLP(nn.Module):
     def norm_fusable(self, rows: int) -> bool:
         """Whether forward_normed is the faster way for this many rows."""
         gate = child(self, 'gate_proj')
-        return only_itself(self, LlamaMLP) and self._pair(rows) is not None and norm_fusion_pays(
-            rows, gate.infeatures, lambda: stream_norm_rows(_lib.OP_MLP_GATEUP, gate.infeatures, gate.outfeatures, gate.groupsize))
+        pair = self._pair(rows) if only_itself(self, LlamaMLP) else None
+        return pair is not None and norm_fusion_pays(rows, gate.infeatures, lambda: (
+            stream_norm_rows(_lib.OP_MLP_GATEUP, gate.infeatures, gate.outfeatures, gate.groupsize), pair[5] is not None))
 
     def forward_normed(self, h, delta, norm_weight, eps):
         """(h + delta, forward(RMSNorm(h + delta))) with the residual add and the norm inside the gate/up launch."""

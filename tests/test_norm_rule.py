@@ -1,0 +1,38 @@
+"""Which decode steps put the residual add and the RMSNorm into the projection's own launch."""
+import pytest
+import torch
+
+import gptq_triton_amd as G
+from gptq_triton_amd.llama import LlamaMLP
+
+
+def blocks(hidden, inter, act_order):
+    """The attention block and both MLP blocks as they stand in streaming order (nothing is launched)."""
+    def new(k, n):
+        layer = G.QuantLinear(4, 128, k, n, bias=False, act_order=act_order)
+        layer._stream_meta, layer._stream_rows = torch.zeros(1, dtype=torch.int32), 16
+        layer._compact_perm = torch.arange(k, dtype=torch.int32) if act_order else None
+        return layer
+
+    cfg = G.LlamaConfigLite()
+    cfg.hidden_size, cfg.intermediate_size, cfg.num_attention_heads = hidden, inter, hidden // 128
+    with torch.device("meta"):
+        attn = G.QuantLlamaAttention(cfg, new(hidden, 3 * hidden), new(hidden, hidden))
+        mlp = LlamaMLP(cfg)
+        mlp.gate_proj, mlp.up_proj, mlp.down_proj = new(hidden, inter), new(hidden, inter), new(inter, hidden)
+        plain = [G.QuantLinear(4, 128, k, n, bias=False, act_order=False) for k, n in ((hidden, inter), (inter, hidden), (hidden, inter))]
+        fused = G.QuantLlamaMLP(*plain)
+    fused._gate_meta, fused._stream_rows = torch.zeros(1, dtype=torch.int32), 16
+    if act_order:
+        order = torch.arange(hidden, dtype=torch.int32)
+        fused.g_idx = fused._compact_rows = mlp.gate_proj._compact_perm = mlp.up_proj._compact_perm = order
+    return attn, mlp, fused
+
+
+@pytest.mark.parametrize("act_order", [False, True])
+@pytest.mark.parametrize("hidden,inter", [(1024, 2816), (4096, 11008), (4352, 11776), (6656, 17920), (8192, 22016)])
+def test_rows_that_take_the_norm_along(hidden, inter, act_order):
+    """Up to four; three with act-order and rows that every workgroup would gather for longer than a norm launch takes."""
+    most = 3 if act_order and hidden > 4096 else 4
+    for block in blocks(hidden, inter, act_order):
+        assert [block.norm_fusable(rows) for rows in range(6)] == [0 < rows <= most for rows in range(6)], type(block)
