@@ -644,6 +644,20 @@ PyObject *greedy_step_end(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
+// stream_rows(selector, K, N, groupsize) -> gptq4_stream_rows()
+PyObject *stream_rows(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    GPTQ4_TAKES(4)
+    Args a{v};
+    const long op = a.integer(0), k = a.integer(1), n = a.integer(2), g = a.integer(3);
+    if (!a.fine || op != (int)op || k != (int)k || n != (int)n || g != (int)g) {
+        PyErr_SetString(PyExc_TypeError, "stream_rows takes four integers of 32 bits");
+        return nullptr;
+    }
+    return PyLong_FromLong(gptq4_stream_rows((int)op, (int)k, (int)n, (int)g));
+    END_HANDLE_TH_ERRORS
+}
+
 // set_workspace(device index, stream handle, address, bytes): what _lib.workspace() made for that stream
 PyObject *set_workspace(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
@@ -676,6 +690,7 @@ PyObject *init(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
 #define GPTQ4_METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr}
 PyMethodDef g_methods[] = {GPTQ4_METHOD(init),
                            GPTQ4_METHOD(set_workspace),
+                           GPTQ4_METHOD(stream_rows),
                            GPTQ4_METHOD(matmul),
                            GPTQ4_METHOD(stream_matmul),
                            GPTQ4_METHOD(mlp_gateup),

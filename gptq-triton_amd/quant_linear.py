@@ -11,7 +11,6 @@ re-laid-out once, at first use, so each group's rows are contiguous (see
 """
 from __future__ import annotations
 
-import functools
 import math
 from typing import Optional
 
@@ -181,10 +180,9 @@ def sort_rows(qweight: torch.Tensor, perm: torch.Tensor) -> torch.Tensor:
 
 def stream_rows(op: int, k: int, n: int, groupsize: int) -> int:
     """Most rows the streaming-order kernels take for this operator and shape (0: the shape is not supported)."""
-    return int(_lib.load().gptq4_stream_rows(op, k, n, groupsize))
+    return _lib.host().stream_rows(op, k, n, groupsize)
 
 
-@functools.lru_cache(maxsize=256)
 def stream_norm_rows(op: int, k: int, n: int, groupsize: int) -> int:
     """Most rows such a launch takes with the residual add and the RMSNorm of its input inside."""
     return stream_rows(op | _lib.OP_WITH_NORM, k, n, groupsize)

@@ -36,3 +36,18 @@ def test_rows_that_take_the_norm_along(hidden, inter, act_order):
     most = 3 if act_order and hidden > 4096 else 4
     for block in blocks(hidden, inter, act_order):
         assert [block.norm_fusable(rows) for rows in range(6)] == [0 < rows <= most for rows in range(6)], type(block)
+
+
+def test_rows_follow_the_tuning_of_the_launches():
+    """The rows a launch normalises are asked for under the launch shape of the moment: sixteen waves with two matrices leave less
+    room for the rows."""
+    from gptq_triton_amd import _lib
+    from gptq_triton_amd.quant_linear import stream_norm_rows
+    shapes = [(op, k, n) for k in (1024, 4096, 6656, 8192) for op, n in ((_lib.OP_QKV_ROTARY, 3 * k), (_lib.OP_MLP_GATEUP, 4096))]
+    ask = lambda: [stream_norm_rows(op, k, n, 128) for op, k, n in shapes]
+    before = ask()
+    _lib.load().gptq4_set_stream_tuning(16, 1)
+    fresh = [_lib.load().gptq4_stream_rows(op | _lib.OP_WITH_NORM, k, n, 128) for op, k, n in shapes]
+    assert ask() == fresh != before
+    _lib.load().gptq4_set_stream_tuning(0, 0)
+    assert ask() == before
