@@ -244,3 +244,53 @@ def test_logits_of_a_model_with_a_hook_on_its_lm_head():
         handle.remove()
         head.bias = torch.nn.Parameter(torch.ones(300, device="cuda").half())
         assert torch.equal(model._logits(h), head(h))
+
+
+class Doubled(torch.nn.Linear):
+    def forward(self, x):
+        return 2 * super().forward(x)
+
+
+def hooked(head):
+    head.register_forward_hook(lambda m, args, out: out + 1)
+    return head
+
+
+def with_bias(head):
+    head.bias = torch.nn.Parameter(torch.ones(300, device="cuda").half())
+    return head
+
+
+def with_weight(change):
+    def made(head):
+        head.weight = torch.nn.Parameter(change(head.weight.detach()), requires_grad=False)
+        return head
+    return made
+
+
+HEADS = {"subclass": lambda head: Doubled(512, 300, bias=False).cuda().half(), "hook": hooked, "bias": with_bias,
+         "strided": with_weight(lambda w: w.t().contiguous().t()), "off the grid": with_weight(lambda w: off_by_one(w)),
+         "row length": with_weight(lambda w: w[:, :384].contiguous())}
+
+
+@pytest.mark.parametrize("rows", [1, 2, 7, 16, 17])
+@pytest.mark.parametrize("kind", [None, *HEADS])
+def test_which_lm_heads_the_kernel_computes(monkeypatch, kind, rows):
+    """Up to 16 rows of torch's own linear layer with nothing hung on it: the kernel, once.  Everything else: the module, whose
+    result comes back as it is."""
+    from gptq_triton_amd import llama
+    calls = []
+    real = llama.lm_head_logits
+    monkeypatch.setattr(llama, "lm_head_logits", lambda x, w: calls.append(1) or real(x, w))
+    model = llama.LlamaForCausalLM.__new__(llama.LlamaForCausalLM)
+    torch.nn.Module.__init__(model)
+    head = torch.nn.Linear(512, 300, bias=False).cuda().half()
+    model.lm_head = head if kind is None else HEADS[kind](head)
+    h = torch.randn((rows, 1, model.lm_head.weight.shape[1]), device="cuda").half()
+    with torch.no_grad():
+        got, want = model._logits(h), model.lm_head(h)
+    assert len(calls) == (kind is None and rows <= 16)
+    if calls:   # (either rounds its fp32 sums to fp16 once)
+        assert float((got.float() - want.float()).abs().max()) <= 2.0 ** -10 * float(want.abs().max())
+    else:
+        assert torch.equal(got, want)

@@ -273,7 +273,7 @@ def test_decoder_with_norm_in_matmul_gives_the_same_tokens(tmp_path, split_k_ker
     model = G.load_quant(str(tmp_path), device="cuda", fuse_mlp=True)
     torch.manual_seed(5)
     ids = torch.randint(0, cfg.vocab_size, (bsz, 9)).cuda()
-    monkeypatch.setattr(decoder_ops, "NORM_PAYS_ROWS", 4)   # by default only one-row steps take the 5-launch layer
+    monkeypatch.setattr(decoder_ops, "NORM_PAYS_ROWS", 4)   # in either layout (tests/test_norm_rule.py: what they take by default)
     calls = []
     real = model.model.layers[0].mlp.forward_normed.__func__
 

@@ -4,6 +4,7 @@ import torch
 
 import gptq_triton_amd as G
 from gptq_triton_amd.llama import LlamaMLP
+from test_gpu_stream import random_quant_model
 
 
 def blocks(hidden, inter, act_order):
@@ -51,3 +52,42 @@ def test_rows_follow_the_tuning_of_the_launches():
     assert ask() == fresh != before
     _lib.load().gptq4_set_stream_tuning(0, 0)
     assert ask() == before
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["stream", "checkpoint"])
+@pytest.mark.parametrize("act_order", [False, True])
+@pytest.mark.parametrize("fuse_mlp", [False, True])
+@pytest.mark.parametrize("bsz", [1, 2, 4, 5])
+def test_steps_take_the_norm_along_by_default(monkeypatch, bsz, fuse_mlp, act_order, layout):
+    """Decode steps and forward() of up to four sequences in streaming order, of one in checkpoint order where gate and up are
+    fused (unfused they are launches of their own there): tokens, logits and pairs are those of the layer with norm launches."""
+    from gptq_triton_amd import decoder_ops
+    if not fuse_mlp:
+        monkeypatch.setattr(G, "make_fused_mlp", lambda model: None)
+    model = random_quant_model(hidden=1024, inter=2816, heads=8, layers=2, groupsize=128, seed=71, act_order=act_order)
+    G.set_layout(model, layout)
+    ids = torch.randint(0, model.config.vocab_size, (bsz, 9), device="cuda", generator=torch.Generator(device="cuda").manual_seed(bsz))
+    _, past = model(ids[:, :8], use_cache=True)
+    taken = []
+    for block in {type(layer.mlp) for layer in model.model.layers}:
+        real = block.forward_normed
+        monkeypatch.setattr(block, "forward_normed", lambda self, *a, real=real: taken.append(1) or real(self, *a))
+
+    def step():
+        dec = G.GreedyDecoder(model, bsz, 32, layout="keep")
+        tokens = [dec.prefill(ids)]
+        del taken[:]
+        tokens.append(dec.decode(4))
+        decoded = len(taken)
+        del taken[:]
+        logits, pairs = model(ids[:, 8:], past_key_values=past, use_cache=True)
+        return decoded, len(taken), tokens + [logits] + [t for pair in pairs for t in pair]
+
+    inside = bsz <= 4 if layout == "stream" else bsz == 1 and fuse_mlp
+    decoded, forward, got = step()
+    assert (decoded, forward) == ((8, 2) if inside else (0, 0))
+    with monkeypatch.context() as mp:
+        mp.setattr(decoder_ops, "NORM_PAYS_ROWS", 0)
+        decoded, forward, want = step()
+    assert decoded == forward == 0 and all(torch.equal(a, b) for a, b in zip(got, want))
