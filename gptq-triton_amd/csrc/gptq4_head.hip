@@ -10,8 +10,10 @@
 // of W per wave are in flight while the 4 KiB before are multiplied (8 KiB: the same from 5120 columns on, 49.9 against 47.0 us at
 // 4096; 2 KiB: 58).  With sixteen rows to a product (v_mfma_f32_16x16x32_f16) a load touched 64 bytes of sixteen rows - half
 // lines, which the streaming hint then fetched twice (58.8 us with it, 53.6 without).  With four, us, W from HBM, the sixteen's
-// time first (argmax): 32000 x 4096 at 1 / 8 / 16 rows 56.1 / 58.9 / 63.1 -> 45.9 / 47.9 / 48.8 (5.7 TB/s; a plain read of as many
-// bytes takes 40), x 1024 19.0 / 20.8 / 23.4 -> 16.4 / 18.0 / 21.0, x 256 11.3 / 12.2 / 15.1 -> 10.6 / 11.7 / 15.1.
+// time first (argmax): 32000 x 4096 at 1 / 8 / 16 rows 59.6 / 60.9 / 66.1 -> 48.0 / 48.9 / 51.3 (5.5 TB/s; a plain read of as many
+// bytes takes 40), x 1024 19.7 / 21.4 / 24.4 -> 16.5 / 18.3 / 20.5, x 256 11.5 / 12.5 / 15.4 -> 10.3 / 11.5 / 13.7, and at the most rows
+// that fit the LDS x 5120 (15) 70.4 -> 60.6, x 6656 (12) 87.6 -> 73.1, x 8192 (9) 109.9 -> 89.0.  Rows of 256 values leave half of a
+// wave's loads empty, which shows where the vocabulary is long: 128256 x 256 19.1 / 20.0 / 23.0 -> 19.5 / 20.7 / 23.8.
 // Rows are dealt evenly, not in fours: lanes past a tile's rows load nothing.  Sums are rounded to fp16 as the linear layer's
 // output would be.  They are the result (LOGITS), or the best (value, index) per x row is kept in registers - torch.argmax's
 // choice among equal values and NaN -, the workgroups' bests go through the workspace, one 8-byte value each, and the last
@@ -33,12 +35,19 @@ __device__ __forceinline__ bool better(float v, int i, float bv, int bi) {
     return (v > bv) | ((v == bv) & (i < bi)) | ((v != v) & ((bv == bv) | (i < bi)));
 }
 
-// Sum over the sixteen lanes of a wave that are equal modulo 4, in every lane, always in the same order.
-__device__ __forceinline__ float blocks_sum(float v) {
-    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x128, 0xF, 0xF, true));  // row_ror:8
-    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x124, 0xF, 0xF, true));  // row_ror:4
-    v += __shfl_xor(v, 16);
-    return v + __shfl_xor(v, 32);
+// Sums over the sixteen lanes of a wave that are equal modulo 4, of four values at a time: lane l gets that of v[l / 16], always
+// summed in the same order.  Each exchange halves what is left to sum instead of giving every lane everything: eight
+// vector instructions where four sums in every lane take sixteen and eight reads through the LDS (argmax of 16 rows
+// through 128256 x 256 30.1 -> 23.8 us, 50304 x 1024 28.7 -> 27.3, 32000 x 4096 51.9 -> 51.3).
+__device__ __forceinline__ float blocks_sum(f4_t v) {
+    auto half = [](float a) { return __builtin_bit_cast(uint32_t, a); };
+    auto both = [](auto pair) { return __builtin_bit_cast(float, (uint32_t)pair[0]) + __builtin_bit_cast(float, (uint32_t)pair[1]); };
+    // (the upper half of the one against the lower half of the other, then the odd sixteens against the even ones)
+    const float s02 = both(__builtin_amdgcn_permlane32_swap(half(v[0]), half(v[2]), false, false));
+    const float s13 = both(__builtin_amdgcn_permlane32_swap(half(v[1]), half(v[3]), false, false));
+    float s = both(__builtin_amdgcn_permlane16_swap(half(s02), half(s13), false, false));
+    s += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, s), 0x128, 0xF, 0xF, true));        // row_ror:8
+    return s + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, s), 0x124, 0xF, 0xF, true));  // row_ror:4
 }
 
 // NORM: 0 x as it is, 1 its RMSNorm, 2 the RMSNorm of x + delta; NB: groups of four x rows; LOGITS: the sums themselves are
@@ -121,17 +130,16 @@ __global__ __launch_bounds__(64 * HEAD_WAVES) void gptq4_head_kernel(HeadArgs p)
             }
         }
         if (tile_ends) {
-            // Every lane gets all four rows' sums and goes on with row blk % 4 of the tile: one comparison per x row, without
-            // branches.  (Four comparisons one after the other, each behind its sum's way across the lanes and behind branches,
-            // took 3.7 us of the launch for every four x rows at 32000 rows of W, whatever their length: x 1024 at 16 rows 29.9 us.)
-            const int at = blk & 3, row = row0 + at;
+            // Every sixteen lanes go on with a row of the tile: one comparison per x row, without branches.  (Four comparisons one
+            // after the other, each behind its sum's way across the lanes and behind branches, took 3.7 us of the launch for every
+            // four x rows at 32000 rows of W, whatever their length: x 1024 at 16 rows 29.9 us.)
+            const int at = lane >> 4, row = row0 + at;
             const bool mine = (at < step) & (row < r1);
 #pragma unroll
             for (int n = 0; n < NB; ++n) {
-                const float s[4] = {blocks_sum(acc[n][0]), blocks_sum(acc[n][1]), blocks_sum(acc[n][2]), blocks_sum(acc[n][3])};
-                const half_t h = (half_t)(at < 2 ? at == 0 ? s[0] : s[1] : at == 2 ? s[2] : s[3]);  // the linear layer's fp16 output
+                const half_t h = (half_t)blocks_sum(acc[n]);  // the linear layer's fp16 output
                 if constexpr (LOGITS) {
-                    if (mine & (blk < 4) & (4 * n + c < B)) p.logits[(size_t)(4 * n + c) * p.V + row] = h;
+                    if (mine & ((lane & 12) == 0) & (4 * n + c < B)) p.logits[(size_t)(4 * n + c) * p.V + row] = h;
                 } else {
                     const bool up = mine & better((float)h, row, bv[n], bi[n]);
                     bv[n] = up ? (float)h : bv[n];
@@ -145,11 +153,11 @@ __global__ __launch_bounds__(64 * HEAD_WAVES) void gptq4_head_kernel(HeadArgs p)
         for (int j = 0; j < HEAD_STEPS; ++j) cur[j] = nxt[j];
     }
     if constexpr (LOGITS) return;
-    // lanes c, c + 4, c + 8, c + 12 hold the bests of four rows of every tile
+    // lanes c, c + 16, c + 32, c + 48 hold the bests of four rows of every tile
 #pragma unroll
     for (int n = 0; n < NB; ++n) {
 #pragma unroll
-        for (int o = 4; o <= 8; o <<= 1) {
+        for (int o = 16; o <= 32; o <<= 1) {
             const float ov = __shfl_xor(bv[n], o);
             const int oi = __shfl_xor(bi[n], o);
             const bool up = better(ov, oi, bv[n], bi[n]);
