@@ -121,6 +121,16 @@ def head_argmax_takes(rows: int, weight: torch.Tensor) -> bool:
         and rows * (k + 8) * 2 <= 160 * 1024 - 2048 and weight.numel() * 2 < 0x7FFFFFF0
 
 
+def head_logits_pays(rows: int, weight: torch.Tensor) -> bool:
+    """Whether lm_head_logits is the faster way to rows of logits.  Against torch's product, us, from HBM, at 1 / 8 / the most rows:
+    32000 x 1024 13.3 / 14.3 / 16.0 to 17.3 / 17.5 / 17.9, x 4096 46.1 / 45.9 / 47.6 to 62.6 / 61.4 / 61.3,
+    x 5120 54.9 / 54.3 / 56.9 to 66.2 / 63.7 / 64.2, x 6656 69.7 / 68.6 / 69.9 to 83.7 / 80.6 / 80.9, x 8192 84.5 / 84.8 / 85.4 to 99.1 / 97.4 / 97.3;
+    8192 x 2048 8.5 / 9.6 / 10.3 to 13.1 / 13.3 / 13.5, x 8192 25.3 / 26.8 / 27.1 to 31.4 / 30.5 / 30.3; 50304 x 1024 20.8 / 21.1 / 23.3 to 23.3 / 22.8 / 23.6.
+    Not with few of either: 4096 x 8192 16.2 / 17.7 / 18.0 to 16.1 / 16.3 / 16.3, 320 x 6656 10.0 / 11.5 / 12.3 to 8.1 / 8.2 / 8.2 (every
+    workgroup brings all of x into its LDS), 50304 x 768 18.5 / 18.8 / 20.8 to 19.4 / 19.1 / 19.7."""
+    return weight.shape[0] >= 8192 and weight.shape[1] >= 1024 and head_argmax_takes(rows, weight)
+
+
 def lm_head_argmax(x: torch.Tensor, weight: torch.Tensor, max_rows: int = HEAD_MAX_ROWS) -> torch.Tensor:
     """Greedy next tokens: argmax(x @ weight.T, -1) in one launch, for x fp16 [..., K] and an fp16 lm_head weight [V, K].
     Returns int64 of x's shape without the last dimension.  More than `max_rows` rows, and shapes the kernel does not take

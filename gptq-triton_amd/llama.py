@@ -18,8 +18,8 @@ import torch
 import torch.nn as nn
 
 from . import _lib
-from .decoder_ops import (NORM_MAX_HIDDEN, add_rms_norm, decode_attention, greedy_step_end, head_argmax_takes, lm_head_argmax, lm_head_logits,
-                          norm_fusion_pays, prefill_attention, rms_norm)
+from .decoder_ops import (NORM_MAX_HIDDEN, add_rms_norm, decode_attention, greedy_step_end, head_argmax_takes, head_logits_pays, lm_head_argmax,
+                          lm_head_logits, norm_fusion_pays, prefill_attention, rms_norm)
 from .fused_attention import KV_AT_POSITION, LlamaConfigLite, QuantLlamaAttention
 from .fused_mlp import QuantLlamaMLP, llama_mlp_4_stream
 from .quant_linear import InverseOrder, QuantLinear, child, only_itself, plain_module, stream_norm_rows, stream_rows
@@ -223,14 +223,14 @@ class LlamaForCausalLM(nn.Module):
         return self.lm_head(h), (presents if use_cache else None)
 
     def _logits(self, h):
-        """lm_head(h); up to HEAD_MAX_ROWS rows in a launch that streams the weight once (two rows of 4096 through 32000 x 4096:
-        torch's product 69 us), where lm_head is torch's own linear layer and nothing else would run with it."""
+        """lm_head(h); a few rows in a launch of this package's where that is faster (head_logits_pays), lm_head is torch's own linear
+        layer and nothing else would run with it."""
         head = self.lm_head
         if type(head) is nn.Linear and plain_module(head) and nn.Linear.forward is LINEAR_FORWARD and head.bias is None:
             weight = head.weight
             # (a tensor subclass may stand for other values than those at its address)
-            if type(weight) in (nn.Parameter, torch.Tensor) and weight.device == h.device and weight.dim() == 2 and weight.shape[0] > 0 \
-                    and weight.shape[1] == h.shape[-1] and head_argmax_takes(h.numel() // h.shape[-1], weight) \
+            if type(weight) in (nn.Parameter, torch.Tensor) and weight.device == h.device and weight.dim() == 2 \
+                    and weight.shape[1] == h.shape[-1] and head_logits_pays(h.numel() // h.shape[-1], weight) \
                     and not torch.is_autocast_enabled(h.device.type):
                 return lm_head_logits(h, weight)
         return head(h)

@@ -251,13 +251,17 @@ class Doubled(torch.nn.Linear):
         return 2 * super().forward(x)
 
 
+class Marked(torch.Tensor):
+    pass
+
+
 def hooked(head):
     head.register_forward_hook(lambda m, args, out: out + 1)
     return head
 
 
 def with_bias(head):
-    head.bias = torch.nn.Parameter(torch.ones(300, device="cuda").half())
+    head.bias = torch.nn.Parameter(torch.ones(8192, device="cuda").half())
     return head
 
 
@@ -268,23 +272,24 @@ def with_weight(change):
     return made
 
 
-HEADS = {"subclass": lambda head: Doubled(512, 300, bias=False).cuda().half(), "hook": hooked, "bias": with_bias,
-         "strided": with_weight(lambda w: w.t().contiguous().t()), "off the grid": with_weight(lambda w: off_by_one(w)),
-         "row length": with_weight(lambda w: w[:, :384].contiguous())}
+HEADS = {"subclass": lambda head: Doubled(1024, 8192, bias=False).cuda().half(), "hook": hooked, "bias": with_bias,
+         "weight of a subclass": with_weight(lambda w: w.as_subclass(Marked)), "strided": with_weight(lambda w: w.t().contiguous().t()), "off the grid": with_weight(lambda w: off_by_one(w)),
+         "row length": with_weight(lambda w: torch.cat([w, w[:, :128]], 1).contiguous()),
+         "fewer rows than pay": with_weight(lambda w: w[:8191].contiguous()), "shorter rows than pay": with_weight(lambda w: w[:, :768].contiguous())}
 
 
 @pytest.mark.parametrize("rows", [1, 2, 7, 16, 17])
 @pytest.mark.parametrize("kind", [None, *HEADS])
 def test_which_lm_heads_the_kernel_computes(monkeypatch, kind, rows):
-    """Up to 16 rows of torch's own linear layer with nothing hung on it: the kernel, once.  Everything else: the module, whose
-    result comes back as it is."""
+    """Up to 16 rows of torch's own linear layer with nothing hung on it and enough of a weight: the kernel, once.  Everything else:
+    the module, whose result comes back as it is."""
     from gptq_triton_amd import llama
     calls = []
     real = llama.lm_head_logits
     monkeypatch.setattr(llama, "lm_head_logits", lambda x, w: calls.append(1) or real(x, w))
     model = llama.LlamaForCausalLM.__new__(llama.LlamaForCausalLM)
     torch.nn.Module.__init__(model)
-    head = torch.nn.Linear(512, 300, bias=False).cuda().half()
+    head = torch.nn.Linear(1024, 8192, bias=False).cuda().half()
     model.lm_head = head if kind is None else HEADS[kind](head)
     h = torch.randn((rows, 1, model.lm_head.weight.shape[1]), device="cuda").half()
     with torch.no_grad():
