@@ -942,13 +942,18 @@ static StreamPlan stream_plan_with(int epi, int M, int N, int K, bool norm, int 
     //   plain, q >= 64: sixteen of two   4096 x 12288 at 1 row (q 96) 8.2 / 7.5 / 8.7 / 7.7, 11008 x 4096 (86) 8.2 / 7.9 / 8.1 / 7.3, 13824 x
     //                                    5120 (135) 11.9 / 11.2 / 11.7 / 9.8, 6656 x 6656 at 2 rows (84) 9.5 / 8.9 / 9.3 / 8.1
     //   plain, 40 <= q < 64: of three    5120 x 5120 (50) 6.4 / 6.1 / 6.8 / 6.9, 8192 x 3072 (48) 6.5 / 6.2 / 6.9 / 7.0 (at 2 to 4 rows level);
-    //                                    below: 4096 x 4096 (32) 4.6 / 4.7 / 5.0 / 5.2
+    //                                    below: 4096 x 4096 (32) 4.6 / 4.7 / 5.0 / 5.2.  From 52 units on the more rows and the longer the rows are the
+    //                                    longer eight waves take against sixteen of two (many_plain; of three / sixteen of two, 52 shapes, 1 to 4 rows):
+    //                                      3328 x 9216 (58) 6.6 / 6.9, 6.7 / 6.9, 7.3 / 7.0, 7.5 / 7.0     2560 x 12800 (62) 6.7 / 7.0, 6.9 / 7.0, 7.0 / 7.1, 7.6 / 7.1
+    //                                      8192 x 3584 (56) 6.6 / 7.2, 7.6 / 7.4, 7.9 / 7.7, 8.2 / 7.9     9216 x 3328 (58) 7.5 / 7.3, 7.9 / 7.5, 8.2 / 7.8, 8.5 / 8.0
+    //                                      13824 x 2048 (54) 7.5 / 7.1, 8.0 / 7.6, 8.6 / 8.0, 9.0 / 8.2    6144 x 4608 (54) 6.0 / 7.0, 6.7 / 7.1, 7.0 / 7.3, 7.1 / 7.6
     //   two matrices, 3 and 4 rows, q >= 40: sixteen of one, where the LDS reads of a unit are the longer part
     //                                    4096 QKV at 4 rows (48) 8.9 / 9.3 / 8.4 / 9.5, 5120 QKV (75) 11.7 / 12.0 / 11.2 / 11.5, gate/up 12.4 /
     //                                    12.8 / 12.2 / 12.4; below: 3072 QKV (27) 7.5 / 8.3 / 7.7 / 8.6; at 1 and 2 rows level or slower
     // (and only where eight waves have a thread for every output element of a range: sixteen take no call that eight do not)
     pl.pieces = (pl.q + 1 + pl.nb - 1) / pl.nb + 1;
-    const bool many = pl.nb >= 16 && (nv == 1 ? pl.q >= 64 : M >= 3 && M <= STREAM_MAX_M && pl.q >= 40 && pl.pieces * M * 16 <= 512);
+    const bool many_plain = pl.q >= 64 || (pl.q >= (pl.nb < 128 ? 52 : 48) && pl.nb >= 68) || (pl.q >= 55 && M >= 2 && pl.nb >= (M == 2 ? 36 : M == 3 ? 20 : 16));
+    const bool many = pl.nb >= 16 && (nv == 1 ? many_plain : M >= 3 && M <= STREAM_MAX_M && pl.q >= 40 && pl.pieces * M * 16 <= 512);
     pl.waves = g_stream_tuning.waves ? g_stream_tuning.waves : waves ? waves : many ? 16 : 8;
     if (!tuned_depth) pl.depth = pl.waves == 16 && nv == 2 ? 1 : pl.waves == 8 && nv == 1 && pl.q >= 40 ? 3 : 2;
     if (pl.waves == 16 && pl.depth > 2) pl.depth = 2;

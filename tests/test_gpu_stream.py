@@ -247,6 +247,19 @@ def test_matmul_in_every_launch_shape(waves, depth):
     assert head_is_zero()
 
 
+@pytest.mark.parametrize("k,n,rows", [(2048, 14336, (3, 4)), (3328, 9216, (2, 3)), (4608, 7168, (1, 2)), (8704, 3584, (1, 4)), (17152, 1536, (1, 3))])
+def test_matmul_where_eight_waves_end_and_sixteen_begin(k, n, rows):
+    """52 to 63 units to a workgroup: eight waves or sixteen by the number and the length of the rows."""
+    L = O.make_layer(k, n, -1, seed=1150 + n)
+    D = to_dev(L)
+    sw, meta = gptq().stream_pack(D["qweight"], D["qzeros"], D["scales"], k)
+    for m in rows:
+        x = O.make_x(m, k, seed=m + 3)
+        y = gptq().matmul4_stream(k, torch.from_numpy(x).cuda(), sw, meta)
+        assert_close(y.cpu().numpy(), O.quant_matmul_ref(x, L["qweight"], L["qzeros"], L["scales"], k), f"{k}x{n} M={m}")
+    assert head_is_zero()
+
+
 @pytest.mark.parametrize("mode", [10, 20])  # 5 .. 16 rows: one tile per unit of loads everywhere / two wherever they can run
 def test_rows_5_to_16_with_one_and_with_two_tiles_per_unit(mode):
     G = gptq()
