@@ -59,7 +59,10 @@ constexpr uint64_t S_MARK = 1ull << 32;
 // have left, in quarters of their own range (in turns they were 2 % slower).  One row, us, before / after: 7B gate/up 12.1 / 11.7,
 // QKV 8.5 / 8.2, o_proj 4.46 / 4.35, down_proj (sixteen waves) 7.8 / 7.4; 13B gate/up at 8 rows 20.3 / 19.1, at 16 rows 22.9 / 21.6.
 // Raising the younger half for good (12.0 us) only swaps the roles; waves of two or three units are left alone (3072 x 3072: 4.94 us,
-// 5.10 with turns).
+// 5.10 with turns).  So are eight waves of a plain projection whose range is shorter than a tile (every workgroup hands a part of
+// one on) and than 40 units, 56 from five rows on: there the turns gain at one length of range and lose at the next.  Without / with
+// them, 36 units to a workgroup (6144 x 3072) 5.6 / 5.8 us at 1 row, 6.6 / 6.8 at 5; 51 (8704 x 3072) 7.7 / 8.0 at 5 rows, 8.4 / 8.7 at 13; 42 (7168 x 3072)
+// 7.2 / 7.4 at 8; the other way 54 (9984 x 2816) 9.1 / 8.9 at 13, 47 (8704 x 2816) 7.7 / 7.6 at 5.
 template <int NW>
 __device__ __forceinline__ void share_simd(int wave, int turn, int left, int n) {
     if (NW == 8) {
@@ -345,7 +348,7 @@ __global__ __launch_bounds__(64 * NW) void gptq4_stream_kernel(STREAM_HOT_PARAMS
     // ---- the loop: loads past the end of the range are switched off through their offset, not branched around, so
     //      that the compiler's counts of loads in flight stay exact
     for (int i = 0; i < n; i += DEPTH) {
-        if (n > 3) share_simd<NW>(wave, i / DEPTH, n - 1 - i, n);
+        if (n > 3 && (NW > 8 || NV > 1 || hq >= nb || hq >= 40)) share_simd<NW>(wave, i / DEPTH, n - 1 - i, n);
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
             if (i + d < n) compute(ring[d]);
@@ -626,7 +629,7 @@ __global__ __launch_bounds__(64 * NW) void gptq4_stream_tall_kernel(STREAM_HOT_P
     };
 
     for (int i = 0; i < n; i += DEPTH) {
-        if (n > 3) share_simd<NW>(wave, i / DEPTH, n - 1 - i, n);
+        if (n > 3 && (NV2 > 1 || hq >= nb || hq >= 56)) share_simd<NW>(wave, i / DEPTH, n - 1 - i, n);
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
             if (i + d < n) compute(ring[d]);
