@@ -81,8 +81,7 @@ __device__ __forceinline__ void norm_issue_row0(const half_t *x, const half_t *d
 // null the sums x + delta are written there as well (one workgroup of the launch does that).
 // 256 threads, part = NORM_MAX_M * 4 floats of LDS.  Ends with a barrier.  In a workgroup of more than 256
 // threads all of them call it (the barriers are the workgroup's) and `active` is true for threads 0..255 only.
-// (`put(row, chunk, value)` places a normalised chunk: natural order into an LDS array for most callers, straight into
-// the k order of the decoded weights for the kernel that keeps its activations that way)
+// (`put(row, chunk, value)` places a normalised chunk)
 template <bool ADD, int KEEP, typename Put>
 __device__ __forceinline__ void norm_rows_put(const half_t *x, const half_t *delta, const half_t *w, half_t *sum_out, Put put,
                                               float *part, int M, int H, float eps, int tid, const NormLoads<KEEP> &r0,

@@ -236,8 +236,8 @@ class LlamaForCausalLM(nn.Module):
         return head(h)
 
     def _layers_fused(self, h, past_len, past_key_values, use_cache):
-        """The stack and the final norm with every residual add in the launch of the norm behind it, and with one token in all
-        both of them in the projection's launch."""
+        """The stack and the final norm with every residual add in the launch of the norm behind it, and with a
+        few tokens in all both of them in the projection's launch (norm_fusion_pays)."""
         layers = self.model.layers
         bsz, q_len, _ = h.shape
         position_ids = layers[0].self_attn.rope.positions(h.device, past_len, bsz, q_len)

@@ -243,7 +243,7 @@ int gptq4_extend_attention(const void *q, const void *past_k, const void *past_v
 int gptq4_lm_head_argmax(const void *x, const void *weight, int64_t *out, int B, int K, int V, void *workspace,
                          size_t workspace_bytes, void *stream);
 
-/* The logits themselves: out fp16 [B, V] = x . weight^T for the same operands (fp32 sums, rounded to fp16 once).  No workspace.
+/* The logits themselves: out fp16 [B, V] = x . weight^T for the same operands and the same limits of B, K and V (fp32 sums, rounded to fp16 once).  No workspace.
  * Replaces the lm_head call of a sampling loop (the reference leaves it to the dense linear layer of transformers). */
 int gptq4_lm_head_logits(const void *x, const void *weight, void *out, int B, int K, int V, void *stream);
 
