@@ -7,6 +7,7 @@
 #include "gptq4_internal.h"
 #include "gptq4_norm.h"
 
+#include <algorithm>
 #include <mutex>
 
 // Scratch memory of gptq4_matmul_static: arrival counters, then split-K partial sums, laid out like a
@@ -292,6 +293,7 @@ int run_tiled(int epi, MatmulArgs &a, void *workspace, size_t workspace_bytes, h
     const size_t rows_bytes = (size_t)a.M * a.K * sizeof(half_t);
     bool stage = a.perm != nullptr && !g_gemm_tuning.own_gather && rows_bytes <= ACT_ORDER_STAGE_MAX;
     Allowed allow;
+    allow.streamed = !a.stream_b;  // (the streamed schedule reads the checkpoint order only)
     auto plan_all = [&]() { return tiled_plan(epi, a.M, a.N, a.K, a.perm != nullptr && !stage, allow); };
     auto by_estimate = [](const TiledChoice &c) { return c.kslice && c.kp.one_round; };
     TiledPlan pl = plan_all();
@@ -465,7 +467,9 @@ static size_t workspace_need(int op, int M, int K, int N, bool least) {
         const int epi = (op == GPTQ4_OP_MLP_GATEUP) ? EPI_SILU_MUL : (op == GPTQ4_OP_QKV_ROTARY ? EPI_ROPE : EPI_PLAIN);
         // whichever kernel the current (automatic or forced) plans pick, with or without act-order, for the whole
         // matrix and for each of the column ranges a call may be cut into
-        size_t need = gemm_partial_bytes(gemm_plan(epi, M, N, K, false, allow.streamed));
+        // (also without the streamed schedule, which calls on streaming-order words never take)
+        size_t need = gemm_partial_bytes(gemm_plan(epi, M, N, K, false, false));
+        if (allow.streamed) need = std::max(need, gemm_partial_bytes(gemm_plan(epi, M, N, K, false, true)));
         const KslicePlan kp = kslice_plan(epi, M, N, K, false, allow.one_round);
         if (kp.ok && kslice_partial_bytes(epi, kp) > need) need = kslice_partial_bytes(epi, kp);
         const ColumnParts parts = tiled_parts(epi, M, N, K, false, allow.one_round);

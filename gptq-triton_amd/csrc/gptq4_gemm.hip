@@ -868,7 +868,7 @@ int launch_streamed(const MatmulArgs &a, int workgroups, hipStream_t stream) {
 
 template <int EPI>
 int launch_epi(const MatmulArgs &a, const GemmPlan &pl, hipStream_t stream) {
-    if (pl.streamed) return launch_streamed<EPI>(a, pl.streamed, stream);
+    if (pl.streamed) return a.stream_b ? (int)hipErrorInvalidValue : launch_streamed<EPI>(a, pl.streamed, stream);  // (run_tiled plans none for those)
     if (pl.tail_split > 1) return launch_one<EPI, 4>(a, pl.tail_first + (pl.tiles - pl.tail_first) * pl.tail_split, stream);
     return pl.mt == 4 ? launch_one<EPI, 4>(a, pl.tiles, stream) : launch_one<EPI, 2>(a, pl.tiles, stream);
 }

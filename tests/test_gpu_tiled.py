@@ -47,6 +47,24 @@ def test_tiled_matmul(forced_tiled, k, n, g, m):
         assert ok, max_abs
 
 
+@pytest.mark.parametrize("k,g", [(128, 128), (384, 128), (384, 384), (1152, 384), (1920, 640), (1664, 128)])
+@pytest.mark.parametrize("m", [17, 113, 129])
+def test_tiled_few_and_odd_k_tiles(forced_tiled, k, g, m):
+    """Both packed layouts where the loop of K tiles begins and ends: one pair, splits of an odd number, groups of six and ten
+    tiles, a last row tile of one row."""
+    n = 512
+    L = O.make_layer(k, n, g, seed=k + m)
+    x = O.make_x(m, k, seed=k + m + 1)
+    D = to_dev(L)
+    xd = torch.from_numpy(x).cuda()
+    ref = O.quant_matmul_ref(x, L["qweight"], L["qzeros"], L["scales"], g)
+    y = gptq().matmul4(g, xd, D["qweight"], D["scales"], D["qzeros"])
+    assert_close(y.cpu().numpy(), ref, f"tiled matmul K={k} g={g} M={m}")
+    sweight, smeta = gptq().quant_linear.stream_pack(D["qweight"], D["qzeros"], D["scales"], g)
+    y = gptq().quant_linear.matmul4_stream(g, xd, sweight, smeta)
+    assert_close(y.cpu().numpy(), ref, f"tiled matmul, streaming order, K={k} g={g} M={m}")
+
+
 @pytest.mark.parametrize("m", [40, 200])
 def test_tiled_gateup(forced_tiled, m):
     k, n, g = 1024, 1280, 128
