@@ -116,19 +116,47 @@ __device__ __forceinline__ ColDecodeNat make_col_decode_nat(uint32_t stored_zero
     return c;
 }
 
-// out = rows 0..7 of the word's 8-row block, in order.
-__device__ __forceinline__ h8_t decode_word_natural(uint32_t w, const ColDecodeNat &c) {
-    const h2_t unit = {(half_t)1.0f, (half_t)0.0625f};
-    const uint32_t magic = 0x64006400u;
+// The decode in four stages of four independent instructions each, for a caller that deals them out between other work.
+struct DecodeNat {
+    uint32_t u[4];
     h2_t p[4];
-    p[0] = as_h2(and_or_b32(__builtin_amdgcn_perm(w, w, 0x0c000c00u), 0x00F0000Fu, magic));
-    p[1] = as_h2(and_or_b32(__builtin_amdgcn_perm(w, w, 0x0c010c01u), 0x00F0000Fu, magic));
-    p[2] = as_h2(and_or_b32(__builtin_amdgcn_perm(w, w, 0x0c020c02u), 0x00F0000Fu, magic));
-    p[3] = as_h2(and_or_b32(__builtin_amdgcn_perm(w, w, 0x0c030c03u), 0x00F0000Fu, magic));
+    __device__ __forceinline__ void stage(int st, uint32_t w, const ColDecodeNat &c) {
+        const h2_t unit = {(half_t)1.0f, (half_t)0.0625f};
+        const uint32_t magic = 0x64006400u;
+        if (st == 0) {
+            u[0] = __builtin_amdgcn_perm(w, w, 0x0c000c00u);
+            u[1] = __builtin_amdgcn_perm(w, w, 0x0c010c01u);
+            u[2] = __builtin_amdgcn_perm(w, w, 0x0c020c02u);
+            u[3] = __builtin_amdgcn_perm(w, w, 0x0c030c03u);
+            return;
+        }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) p[j] = __builtin_elementwise_fma(p[j], unit, c.neg) * c.scale;
-    h8_t r = {p[0].x, p[0].y, p[1].x, p[1].y, p[2].x, p[2].y, p[3].x, p[3].y};
-    return r;
+        for (int j = 0; j < 4; ++j) {
+            if (st == 1) p[j] = as_h2(and_or_b32(u[j], 0x00F0000Fu, magic));
+            if (st == 2) p[j] = __builtin_elementwise_fma(p[j], unit, c.neg);
+            if (st == 3) p[j] = p[j] * c.scale;
+        }
+    }
+    // keeps the stage where it stands (the compiler sinks arithmetic towards its use, past the scheduling barriers)
+    __device__ __forceinline__ void pin(int st) {
+        if (st == 0) {
+            asm volatile("" : "+v"(u[0]), "+v"(u[1]), "+v"(u[2]), "+v"(u[3]));
+        } else {
+            uint32_t v[4] = {as_u32(p[0]), as_u32(p[1]), as_u32(p[2]), as_u32(p[3])};
+            asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+#pragma unroll
+            for (int j = 0; j < 4; ++j) p[j] = as_h2(v[j]);
+        }
+    }
+    __device__ __forceinline__ h8_t value() const { return (h8_t){p[0].x, p[0].y, p[1].x, p[1].y, p[2].x, p[2].y, p[3].x, p[3].y}; }
+};
+
+// rows 0..7 of the word's 8-row block, in order.
+__device__ __forceinline__ h8_t decode_word_natural(uint32_t w, const ColDecodeNat &c) {
+    DecodeNat d;
+#pragma unroll
+    for (int st = 0; st < 4; ++st) d.stage(st, w, c);
+    return d.value();
 }
 
 // 8 consecutive activations a0..a7 (natural order, as a uint4) -> pair order

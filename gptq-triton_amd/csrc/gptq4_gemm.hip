@@ -38,6 +38,8 @@
 // panels in its L2.
 #include "gptq4_internal.h"
 
+#include <type_traits>
+
 // Development aid, compiled out of the product build: per-workgroup stamps of the 100 MHz clock at the phase
 // boundaries of the kernel, written 32 MiB into the workspace (size it so).
 #ifdef GPTQ4_PHASE_TIMERS
@@ -315,29 +317,39 @@ __global__ __launch_bounds__(256, 2) void gptq4_gemm_kernel(MatmulArgs p) {
         }
     } else {
         // ---- plain path: activations go global -> LDS directly (no staging registers, so the
-        // loads of tile kt+1 are in flight under the MFMAs of tile kt).  A wave instruction
+        // loads of the next tiles are in flight under the MFMAs of tile kt).  A wave instruction
         // fills 64 consecutive 16-byte chunks = 8 rows x 8 chunks; chunk c of row r sits at
         // position c ^ ((r >> 1) & 7) of its row, which makes the 128-bit fragment reads
         // (16 lanes = 16 rows, one position each) conflict-free without padding.  The lane
         // picks the global chunk that belongs at its fixed LDS slot.
-        uint32_t a_goff[A_UNITS];
+        //
+        // A wave issues an instruction of any kind every five cycles, so the 32 cycles of an MFMA hide five others and no
+        // more.  The loop's instructions are therefore counted - 4 of the decode, half an LDS read, about one of everything
+        // else for every MFMA - and dealt to the MFMAs one by one (slot() below).  Hence also: addresses are scalars of the
+        // wave plus offsets of the lane that never change, the four LDS-direct loads of a tile share one LDS base (their
+        // distance is the instruction's own offset, which moves both addresses, so the lane's is that much smaller), and
+        // the group of a tile comes out of one multiplication.
+        uint32_t a_off[A_UNITS];
 #pragma unroll
         for (int u = 0; u < A_UNITS; ++u) {
-            const int slot = (u * NW + wave) * 64 + lane;
+            const int slot = (wave * A_UNITS + u) * 64 + lane;
             const int row = slot >> 3;
             const int c = (slot & 7) ^ ((row >> 1) & 7);
-            a_goff[u] = (uint32_t)min(row, M - 1 - m0) * (uint32_t)K + 8u * c;
+            // (8 rows are 2048 bytes at least; rows from M on are not read: an offset out of the buffer's range loads zeros)
+            a_off[u] = row < M - m0 ? (uint32_t)row * (uint32_t)K * 2u + 16u * c - 1024u * u : 0xFFFFF000u;
         }
         // Buffer-addressed form of the LDS-direct load: unlike the flat/global form the compiler
         // counts it in order with the other vector-memory loads, so its waits for the packed
         // words stay exact while activation tiles are in flight.
         const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
             (void *)a_base, 0, (int)((uint32_t)min(BM, M - m0) * (uint32_t)K * 2u), 0x00020000);
+        static_assert(A_UNITS == 4, "the loads below name the units");
         auto dma_a = [&](half_t *dst, int kt) {
-#pragma unroll
-            for (int u = 0; u < A_UNITS; ++u)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, (__attribute__((address_space(3))) void *)(dst + (u * NW + wave) * 512),
-                                                         16, (int)(a_goff[u] * 2u), kt * (BK * 2), 0, 0);
+            auto *const lds = (__attribute__((address_space(3))) void *)(dst + wave * (A_UNITS * 512));
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, lds, 16, (int)a_off[0], kt * (BK * 2), 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, lds, 16, (int)a_off[1], kt * (BK * 2), 1024, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, lds, 16, (int)a_off[2], kt * (BK * 2), 2048, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, lds, 16, (int)a_off[3], kt * (BK * 2), 3072, 0);
             asm volatile("" ::: "memory");  // the loads that follow stay behind these
         };
         const int sw = (l32 >> 1) & 7;  // (row >> 1) & 7 for every row this lane reads (rows = 32*j + l32)
@@ -348,20 +360,29 @@ __global__ __launch_bounds__(256, 2) void gptq4_gemm_kernel(MatmulArgs p) {
         // (SB: slot [par][2 * m + t] holds, for column t, the words of steps 2 * m and 2 * m + 1; both are refilled during
         // step 2 * m + 1, when the later of the two has been decoded)
         uint2 b2[2][4];
-        const uint32_t *sbptr = nullptr, *sb_meta = nullptr;
+        const int strip_bytes = (K >> 7) * 1024, groups = K / p.groupsize;
+        int sb_lane[2][2];  // SB: the wave's columns are four strips; [m][t]
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sb_lane[i >> 1][i & 1] = (l32 >> 3) * strip_bytes + (2 * l32 & 15) * 16 + 8 * lhi + 256 * (i >> 1) + 16 * (i & 1);
+        const int sb_meta_lane = (l32 >> 3) * groups * 64 + (2 * l32 & 15) * 4;
+        __amdgpu_buffer_rsrc_t sb_rsrc, sb_meta_rsrc;
         if constexpr (SB) {
-            sbptr = p.w[mat].qweight + ((size_t)(ncol >> 4) * (size_t)(K >> 7)) * 256 + (ncol & 15) * 4 + 2 * lhi;
-            sb_meta = p.w[mat].qzeros + (size_t)(ncol >> 4) * (size_t)(K / p.groupsize) * 16 + (ncol & 15);  // (the meta words travel in the qzeros field)
+            sb_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(p.w[mat].qweight + (size_t)(nw0 >> 4) * (size_t)(K >> 7) * 256), 0, 4 * strip_bytes, 0x00020000);
+            // (the meta words travel in the qzeros field)
+            sb_meta_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(p.w[mat].qzeros + (size_t)(nw0 >> 4) * (size_t)groups * 16), 0, 4 * groups * 64, 0x00020000);
         }
-        auto load_b2 = [&](int par, int kt, int ks) {
+        // checkpoint order: the lane's offset behind the first row of a step, its scales and its word of zero points
+        const int wlane = (lhi * N + 2 * l32) * 4, slane = 4 * l32, zlane = (l32 >> 2) * 4;
+        auto load_b2 = [&](int par, int tile, int ks) {
             if constexpr (SB) {
                 if (ks & 1) {
-                    const uint32_t *src = sbptr + ((size_t)(2 * min(kt, nk - 1) + (ks >> 1))) * 64;
-                    b2[par][ks - 1] = *reinterpret_cast<const uint2 *>(src);
-                    b2[par][ks] = *reinterpret_cast<const uint2 *>(src + 4);
+                    b2[par][ks - 1] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(sb_rsrc, sb_lane[ks >> 1][0], tile * 512, 0));
+                    b2[par][ks] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(sb_rsrc, sb_lane[ks >> 1][1], tile * 512, 0));
                 }
             } else {
-                b2[par][ks] = *reinterpret_cast<const uint2 *>(bptr + ((size_t)min(kt, nk - 1) * (BK / 8) + 2 * ks) * N);
+                // (the tile's eight rows, whose first is found in 64 bits)
+                const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc((void *)(p.w[mat].qweight + nw0 + (uint64_t)(uint32_t)tile * (uint32_t)(8 * N)), 0, (8 * N - nw0) * 4, 0x00020000);
+                b2[par][ks] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rows, wlane, 2 * ks * N * 4, 0));
             }
         };
         // the packed word of column t for step `step` of the tile of parity par
@@ -373,114 +394,125 @@ __global__ __launch_bounds__(256, 2) void gptq4_gemm_kernel(MatmulArgs p) {
                 return t ? b2[par][step].y : b2[par][step].x;
             }
         };
-        dma_a(As0, k_begin);
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) load_b2(0, k_begin, ks);
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) load_b2(1, k_begin + 1, ks);
-        // Scale and zero words run two tiles ahead as well: slot [par] is loaded at the top of a
+        // Scale and zero words run two tiles ahead as well: slot [par] is loaded in the last step of a
         // tile of parity par with the group of the tile two on, and turned into the decode
-        // constants of that tile during the last step of the tile in between.  The group of
-        // the look-ahead tile is tracked by counting, like the current one.
+        // constants of that tile during the last step of the tile in between.
         uint32_t g_s[2], g_z[2];
-        int group2 = group, left2 = left_in_group;
-        auto load_group2 = [&](int par) {
-            const int g = min(group2, last_group);
+        const uint32_t group_magic = p.tile_group_magic;  // (group = tile / (groupsize / 64): exact for every tile)
+        const int group_shift = p.tile_group_shift;
+        auto load_group2 = [&](int par, int tile) {
+            const uint32_t g = __umulhi((uint32_t)tile, group_magic) >> group_shift;
             if constexpr (SB) {
                 // {scale | zero << 16} of the lane's two columns: neighbours in the strip's row of the group
-                const uint2 m2 = *reinterpret_cast<const uint2 *>(sb_meta + (size_t)g * 16);
+                const uint2 m2 = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(sb_meta_rsrc, sb_meta_lane, (int)g * 64, 0));
                 g_s[par] = m2.x;
                 g_z[par] = m2.y;
             } else {
-                g_s[par] = *reinterpret_cast<const uint32_t *>(sc + (size_t)g * N);
-                g_z[par] = qz[(size_t)g * (N >> 3)];
-            }
-            if (left2 == 1) {
-                ++group2;
-                left2 = tiles_per_group;
-            } else {
-                --left2;
+                const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc((void *)(p.w[mat].scales + nw0 + (uint64_t)g * (uint32_t)N), 0, (N - nw0) * 2, 0x00020000);
+                const __amdgpu_buffer_rsrc_t zr = __builtin_amdgcn_make_buffer_rsrc((void *)(p.w[mat].qzeros + (nw0 >> 3) + (uint64_t)g * (uint32_t)(N >> 3)), 0, (N - nw0) >> 1, 0x00020000);
+                g_s[par] = __builtin_amdgcn_raw_buffer_load_b32(sr, slane, 0, 0);
+                g_z[par] = __builtin_amdgcn_raw_buffer_load_b32(zr, zlane, 0, 0);
             }
         };
         // the activation fragments come out of LDS in natural k order, so the weights are
         // decoded in natural order too
         ColDecodeNat cn[2];
-        auto make_cn = [&](int par) {
+        auto make_cn = [&](int par, int t) {
             if constexpr (SB) {
-                cn[0] = make_col_decode_nat((g_s[par] >> 16) & 0xFu, g_s[par]);
-                cn[1] = make_col_decode_nat((g_z[par] >> 16) & 0xFu, g_z[par]);
+                const uint32_t m = t ? g_z[par] : g_s[par];
+                cn[t] = make_col_decode_nat((m >> 16) & 0xFu, m);
             } else {
-                const uint32_t z2 = g_z[par] >> (((2 * l32) & 7) * 4);
-                cn[0] = make_col_decode_nat(z2 & 0xFu, g_s[par]);
-                cn[1] = make_col_decode_nat((z2 >> 4) & 0xFu, g_s[par] >> 16);
+                cn[t] = make_col_decode_nat((g_z[par] >> (((2 * l32) & 7) * 4 + 4 * t)) & 0xFu, t ? g_s[par] >> 16 : g_s[par]);
             }
         };
-        load_group2(0);  // group of tile k_begin
-        make_cn(0);
-        load_group2(1);  // group of tile k_begin + 1, made into constants at the end of tile k_begin
-        h8_t bf[2];
-        bf[0] = decode_word_natural(word_of(0, 0, 0), cn[0]);
-        bf[1] = decode_word_natural(word_of(0, 0, 1), cn[1]);
-
-        // one K tile (of parity `par` counted from k_begin) from buffer `cur`, while the next
-        // tile streams into `nxt`
-        auto k_tile = [&](const half_t *cur, half_t *nxt, int kt, int par) {
-            // Every wave has issued at least 4 vector-memory loads after its LDS-direct loads
-            // of this tile (the scale/zero words and the packed words of 4 K steps), and
-            // loads complete in order: at most 4 outstanding means the tile has landed.
-            // (tests/test_wait_counts.py counts the loads behind the tile's in the compiled code of every variant.)
-            asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            dma_a(nxt, min(kt + 1, nk - 1));
-            load_group2(par);
-            // fragments of K step ks+1 are read from LDS before the MFMAs of step ks are issued
-            h8_t araw[MT];
-            auto read_a = [&](int ks) {
+        // (in the order of the loop: a wait of the compiler's in the loop holds for the first pass too)
+        const int second = min(k_begin + 1, nk - 1);
+        dma_a(As0, k_begin);
+        load_group2(0, k_begin);
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) {
-                    const int row = wm * (32 * MT) + mt * 32 + l32;
-                    const int chunk = SB ? 4 * (ks >> 1) + 2 * lhi + (ks & 1) : 2 * ks + lhi;
-                    araw[mt] = *reinterpret_cast<const h8_t *>(cur + row * BK + 8 * (chunk ^ sw));
-                }
-            };
-            read_a(0);
+        for (int ks = 0; ks < 4; ++ks) load_b2(0, k_begin, ks);
+        dma_a(As1, second);
+        load_group2(1, second);  // made into constants at the end of tile k_begin
 #pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-                h8_t af[MT];
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt) {
-                    af[mt] = araw[mt];
-                }
-                if (ks < 3) read_a(ks + 1);
-                if (ks == 3) make_cn(par ^ 1);
-                load_b2(par, kt + 2, ks);  // this step's words were decoded during the previous step
-                __builtin_amdgcn_sched_barrier(0);  // keep the loads above the MFMAs that hide them
-                // words of the next step (step 0 of the next tile when ks == 3)
-                const uint32_t next0 = (ks < 3) ? word_of(par, ks + 1, 0) : word_of(par ^ 1, 0, 0);
-                const uint32_t next1 = (ks < 3) ? word_of(par, ks + 1, 1) : word_of(par ^ 1, 0, 1);
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt) acc[mt][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mt], bf[0], acc[mt][0], 0, 0, 0);
-                bf[0] = decode_word_natural(next0, cn[0]);
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt) acc[mt][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mt], bf[1], acc[mt][1], 0, 0, 0);
-                bf[1] = decode_word_natural(next1, cn[1]);
-                // The decode of the next step's words (32 VALU instructions) spread between this step's MFMAs, three
-                // after each of the wide tile's eight (six after each of the narrow tile's four), instead of four MFMAs
-                // back to back and the decode behind them: 1 - 4 % (LLaMA-7B down_proj at 2048 rows 184 -> 177 us,
-                // o_proj 76.8 -> 74.5, gate/up 353 -> 347; narrow tile: 13B o_proj at 640 rows 57.4 -> 53.8 with six,
-                // 30B o_proj at 512 rows 70.5 -> 65.8).
-#pragma unroll
-                for (int i = 0; i < 2 * MT; ++i) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, MT == 4 ? 3 : 6, 0);
-                }
-            }
-        };
+        for (int ks = 0; ks < 4; ++ks) load_b2(1, second, ks);
         // the first two blocks of the rotary tables: older than every load the waits below count, so landed
         // long before the epilogue
         if (need_tab) {
             dma_table(0, 0);
             dma_table(1, 1);
         }
+        h8_t bf[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            make_cn(0, t);
+            bf[t] = decode_word_natural(word_of(0, 0, t), cn[t]);
+        }
+        // fragment mt of K step ks of the tile in `src`
+        auto read_a = [&](const half_t *src, int ks, int mt) {
+            const int row = wm * (32 * MT) + mt * 32 + l32;
+            const int chunk = SB ? 4 * (ks >> 1) + 2 * lhi + (ks & 1) : 2 * ks + lhi;
+            return *reinterpret_cast<const h8_t *>(src + row * BK + 8 * (chunk ^ sw));
+        };
+        // (more than four loads follow those of the first tile)
+        asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        h8_t ahead[MT];  // fragments of the step to come
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) ahead[mt] = read_a(As0, 0, mt);
+
+        // One K tile (of parity `par` counted from k_begin) out of buffer `cur`: four steps of 2 * MT slots, each an MFMA with
+        // its share of what has to be done for the step to come - a fragment read from LDS in each of the first MT slots (all
+        // four at once would stand in the LDS' queue behind the other waves'), the two words decoded a stage of four independent
+        // instructions at a time.  What a tile needs of the next one is done during its last step: the next tile has landed in
+        // `nxt` for every wave (wait, barrier), its first fragments are read, and - every wave has its own last fragments of
+        // `cur` by then - the tile two on is requested into `cur`.  With the wait and the barrier between the tiles, four reads in
+        // front of a step's MFMAs and the rest where the compiler put it, a K tile of the wide tile (1024 cycles of MFMAs a wave)
+        // took 1530 cycles, two waves to a SIMD 2840 for both; now 1335 and 2510.  The clock gives a part of that back (the chip is
+        // at its power limit): 2048 x 6656 x 17920 387 -> 370 us, 2048 x 4096 x 12288 166 -> 158, 7B gate/up at 2048 rows
+        // 302 -> 288, 2048 x 11008 x 4096 155 -> 146, 2000 x 4096 x 4096 60.1 -> 57.0, 800 x 5120 x 15360 124 -> 119.
+        // (final: a last tile that nothing follows, where the loop ends on one - the tiles go in pairs)
+        auto k_tile = [&](half_t *cur, const half_t *nxt, int kt, int par, auto final) {
+            constexpr bool FINAL = decltype(final)::value;
+            const int tile2 = min(kt + 2, nk - 1);
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) {
+                h8_t af[MT], bnext[2];
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) af[mt] = ahead[mt];
+                DecodeNat dec;
+                if (ks < 3 || FINAL) __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), once for the step's fragments
+                __builtin_amdgcn_sched_barrier(0);
+                if (ks == 3 && !FINAL) {
+                    // Every wave has issued at least 4 vector-memory loads after its LDS-direct loads
+                    // of the next tile (the scale/zero words and the packed words of 4 K steps), and
+                    // loads complete in order: at most 4 outstanding means the tile has landed.
+                    // (tests/test_wait_counts.py counts the loads behind the tile's in the compiled code of every variant.)
+                    asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                }
+#pragma unroll
+                for (int i = 0; i < 2 * MT; ++i) {
+                    const int t = i / MT, mt = i % MT;
+                    acc[mt][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mt], bf[t], acc[mt][t], 0, 0, 0);
+                    if (t == 0 && (ks < 3 || !FINAL)) ahead[mt] = ks < 3 ? read_a(cur, ks + 1, mt) : read_a(nxt, 0, mt);
+                    if (t == 1 && ks == 3 && !FINAL) {
+                        if (mt == 0) dma_a(cur, tile2);
+                        if (mt == MT - 2) load_group2(par, tile2);
+                    }
+                    if (i == 2 * MT - 1 && !FINAL) load_b2(par, tile2, ks);  // (this step's words were decoded during the previous step)
+#pragma unroll
+                    for (int d = 0; d < 4 / MT && (ks < 3 || !FINAL); ++d) {
+                        // words of the next step (step 0 of the next tile when ks == 3)
+                        const int st = (4 / MT) * mt + d;
+                        if (ks == 3 && st == 0) make_cn(par ^ 1, t);
+                        dec.stage(st, ks < 3 ? word_of(par, ks + 1, t) : word_of(par ^ 1, 0, t), cn[t]);
+                        if (ks == 3 && st >= 2) dec.pin(st);
+                        if (st == 3) bnext[t] = dec.value();
+                    }
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // the MFMA first
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (ks < 3 || !FINAL) bf[0] = bnext[0], bf[1] = bnext[1];
+            }
+        };
         // pairs of tiles without a branch between them (a join there would make the compiler
         // move packed words that are still in flight, and wait for them), then the odd one
         GM_STAMP(1);
@@ -490,10 +522,10 @@ __global__ __launch_bounds__(256, 2) void gptq4_gemm_kernel(MatmulArgs p) {
 #endif
         int kt = k_begin;
         for (; kt + 1 < nk; kt += 2) {
-            k_tile(As0, As1, kt, 0);
-            k_tile(As1, As0, kt + 1, 1);
+            k_tile(As0, As1, kt, 0, std::false_type{});
+            k_tile(As1, As0, kt + 1, 1, std::false_type{});
         }
-        if (kt < nk) k_tile(As0, As1, kt, 0);
+        if (kt < nk) k_tile(As0, As1, kt, 0, std::true_type{});
         // all LDS-direct loads have landed and every wave is done reading before the
         // epilogues reuse the buffers
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -998,7 +1030,15 @@ size_t gemm_partial_bytes(const GemmPlan &pl) {
     return pl.splitk > 1 ? (size_t)pl.tiles * pl.splitk * (pl.mt * 32 * 256) * sizeof(float) : 0;
 }
 
-int launch_gemm(int epi, const MatmulArgs &a, const GemmPlan &pl, hipStream_t stream) {
+int launch_gemm(int epi, MatmulArgs &a, const GemmPlan &pl, hipStream_t stream) {
+    // K tile -> group: t / d = umulhi(t, magic) >> shift with 2^shift < d <= 2^(shift + 1), d = K tiles of a group (2 and more);
+    // magic = floor(2^(32 + shift) / d) + 1 is at most 2^32 - 1 unless d is 2^(shift + 1), where 2^31 divides exactly
+    const unsigned d = (unsigned)(a.groupsize / 64);
+    int shift = 0;
+    while ((2u << shift) < d) ++shift;
+    const uint64_t whole = 1ull << (32 + shift);
+    a.tile_group_magic = (uint32_t)(whole % d == 0 ? whole / d : whole / d + 1);
+    a.tile_group_shift = shift;
     switch (epi) {
         case EPI_PLAIN: return launch_epi<EPI_PLAIN>(a, pl, stream);
         case EPI_SILU_MUL: return launch_epi<EPI_SILU_MUL>(a, pl, stream);

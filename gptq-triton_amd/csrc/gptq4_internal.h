@@ -54,6 +54,8 @@ struct MatmulArgs {
     int m_shift;
     int nb;
     uint32_t nb_magic, q_magic, q1_magic;
+    uint32_t tile_group_magic;  // tiled kernel: K tile (64 k) -> group, umulhi(tile, magic) >> shift
+    int tile_group_shift;
     int lds_wave_chunks;  // 16-byte chunks of LDS per wave
     int x_chunks_max;     // chunks of the largest x slice: (slot_q + 1) << (4 + m_shift)
     int max_contrib;      // partial-sum slots per tile
@@ -129,7 +131,8 @@ extern GemmTuning g_gemm_tuning;
 GemmPlan gemm_plan(int epi, int M, int N, int K, bool has_perm = false, bool allow_streamed = true);
 size_t gemm_partial_bytes(const GemmPlan &plan);
 // Tiled matrix-core GEMM for any M.  Returns hipError_t.
-int launch_gemm(int epi, const MatmulArgs &a, const GemmPlan &plan, hipStream_t stream);
+// (fills in a's reciprocal of the group's K tiles)
+int launch_gemm(int epi, MatmulArgs &a, const GemmPlan &plan, hipStream_t stream);
 
 // Launch shape of the mid-M kernel (K split across the waves of a workgroup).
 struct KslicePlan {
