@@ -1031,14 +1031,7 @@ size_t gemm_partial_bytes(const GemmPlan &pl) {
 }
 
 int launch_gemm(int epi, MatmulArgs &a, const GemmPlan &pl, hipStream_t stream) {
-    // K tile -> group: t / d = umulhi(t, magic) >> shift with 2^shift < d <= 2^(shift + 1), d = K tiles of a group (2 and more);
-    // magic = floor(2^(32 + shift) / d) + 1 is at most 2^32 - 1 unless d is 2^(shift + 1), where 2^31 divides exactly
-    const unsigned d = (unsigned)(a.groupsize / 64);
-    int shift = 0;
-    while ((2u << shift) < d) ++shift;
-    const uint64_t whole = 1ull << (32 + shift);
-    a.tile_group_magic = (uint32_t)(whole % d == 0 ? whole / d : whole / d + 1);
-    a.tile_group_shift = shift;
+    set_tile_group(a);
     switch (epi) {
         case EPI_PLAIN: return launch_epi<EPI_PLAIN>(a, pl, stream);
         case EPI_SILU_MUL: return launch_epi<EPI_SILU_MUL>(a, pl, stream);

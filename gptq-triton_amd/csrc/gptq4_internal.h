@@ -54,7 +54,7 @@ struct MatmulArgs {
     int m_shift;
     int nb;
     uint32_t nb_magic, q_magic, q1_magic;
-    uint32_t tile_group_magic;  // tiled kernel: K tile (64 k) -> group, umulhi(tile, magic) >> shift
+    uint32_t tile_group_magic;  // tiled and mid-M kernel: K tile (64 k) -> group, umulhi(tile, magic) >> shift
     int tile_group_shift;
     int lds_wave_chunks;  // 16-byte chunks of LDS per wave
     int x_chunks_max;     // chunks of the largest x slice: (slot_q + 1) << (4 + m_shift)
@@ -130,8 +130,18 @@ extern GemmTuning g_gemm_tuning;
 // the call must not plan the streamed schedule (its partial sums would not fit the caller's scratch memory)
 GemmPlan gemm_plan(int epi, int M, int N, int K, bool has_perm = false, bool allow_streamed = true);
 size_t gemm_partial_bytes(const GemmPlan &plan);
+// The reciprocal of the group's K tiles (launch_gemm and launch_kslice fill it in).
+inline void set_tile_group(MatmulArgs &a) {
+    // K tile -> group: t / d = umulhi(t, magic) >> shift with 2^shift < d <= 2^(shift + 1), d = K tiles of a group (2 and more);
+    // magic = floor(2^(32 + shift) / d) + 1 is at most 2^32 - 1 unless d is 2^(shift + 1), where 2^31 divides exactly
+    const unsigned d = (unsigned)(a.groupsize / 64);
+    int shift = 0;
+    while ((2u << shift) < d) ++shift;
+    const uint64_t whole = 1ull << (32 + shift);
+    a.tile_group_magic = (uint32_t)(whole % d == 0 ? whole / d : whole / d + 1);
+    a.tile_group_shift = shift;
+}
 // Tiled matrix-core GEMM for any M.  Returns hipError_t.
-// (fills in a's reciprocal of the group's K tiles)
 int launch_gemm(int epi, MatmulArgs &a, const GemmPlan &plan, hipStream_t stream);
 
 // Launch shape of the mid-M kernel (K split across the waves of a workgroup).
@@ -158,7 +168,7 @@ struct KsliceTuning {
 extern KsliceTuning g_kslice_tuning;
 KslicePlan kslice_plan(int epi, int M, int N, int K, bool has_perm, bool allow_one_round = true);
 size_t kslice_partial_bytes(int epi, const KslicePlan &plan);
-int launch_kslice(int epi, const MatmulArgs &a, const KslicePlan &plan, hipStream_t stream);
+int launch_kslice(int epi, MatmulArgs &a, const KslicePlan &plan, hipStream_t stream);
 
 // ---- Streaming-order layout (gptq4_stream.hip) ------------------------------------------------------------------
 // One quantised projection in streaming order: per strip of 16 output columns and per unit of 128 input rows one

@@ -23,6 +23,8 @@
 // chip; the partial sums exchanged are the workgroup's already reduced tile.
 #include "gptq4_internal.h"
 
+#include <type_traits>
+
 // Development aid, compiled out of the product build: per-workgroup stamps of the 100 MHz clock at the
 // phase boundaries of the kernel, written 32 MiB into the workspace (size it so).
 #ifdef GPTQ4_PHASE_TIMERS
@@ -130,30 +132,6 @@ __global__ __launch_bounds__(64 * KS, MT > 2 || (KS == 8 && (MT == 2 || (EPI != 
     // block j of the wave tile: matrix j at the strip's columns (SiLU*mul), or columns
     // 64*j .. 64*j + 63 of the head (rotary); the lane's 2 columns of it (PAIRED: ncol and ncol + 64)
     const int ncol = PAIRED ? n0 + l32 : n0 + 2 * l32;
-    // (for rotary the second block is a constant offset from the first: no second set of pointers)
-    constexpr int NPTR = (EPI == EPI_SILU_MUL) ? 2 : 1;
-    const uint32_t *bptr_[NPTR];
-    const uint32_t *qz_[NPTR];
-    const half_t *sc_[NPTR];
-#pragma unroll
-    for (int j = 0; j < NPTR; ++j) {
-        bptr_[j] = p.w[j].qweight + (size_t)lhi * N + ncol;  // row lhi of K tile 0
-        qz_[j] = p.w[j].qzeros + (ncol >> 3);
-        sc_[j] = p.w[j].scales + ncol;
-    }
-    auto bptr = [&](int j) { return ADJ ? bptr_[0] + 64 * j : bptr_[j < NPTR ? j : 0]; };
-    // SB: word offset of the lane's rows 2 * lhi, 2 * lhi + 1 of chunk 0 of column ncol, and of its {scale, zero} word of
-    // group 0; 64 columns on are four strips on
-    const uint32_t sb_strip = (uint32_t)(K >> 7) * 256u;            // words of a strip
-    const uint32_t sb_groups16 = (uint32_t)(K / p.groupsize) * 16u;  // {scale, zero} words of a strip
-    const uint32_t sb_off = (uint32_t)(ncol >> 4) * sb_strip + (uint32_t)(ncol & 15) * 4u + 2u * lhi;
-    const uint32_t sb_moff = (uint32_t)(ncol >> 4) * sb_groups16 + (uint32_t)(ncol & 15);
-    auto sb_words = [&](int j) { return p.w[(EPI == EPI_SILU_MUL) ? j : 0].qweight + ((ADJ && j) ? 4 * sb_strip : 0u); };
-    auto sb_meta = [&](int j) { return p.w[(EPI == EPI_SILU_MUL) ? j : 0].qzeros + ((ADJ && j) ? 4 * sb_groups16 : 0u); };
-    auto qz = [&](int j) { return ADJ ? qz_[0] + 8 * j : qz_[j < NPTR ? j : 0]; };
-    auto sc = [&](int j) { return ADJ ? sc_[0] + 64 * j : sc_[j < NPTR ? j : 0]; };
-    const int tiles_per_group = p.groupsize / BK;
-    const int last_group = K / p.groupsize - 1;
 
     f16_t acc[NB][MT][2];
 #pragma unroll
@@ -178,68 +156,82 @@ __global__ __launch_bounds__(64 * KS, MT > 2 || (KS == 8 && (MT == 2 || (EPI != 
         // which makes the 128-bit fragment reads conflict-free without padding.  Rows of a
         // unit are 8u + lane / 8, so the swizzle term is (lane >> 4) for even u and that ^ 4
         // for odd u: two per-lane offsets, everything else is a scalar offset.
-        const int valid = min(BM, M - m0);
-        const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-            (void *)(p.x + (size_t)m0 * K), 0, (int)((uint32_t)valid * (uint32_t)K * 2u), 0x00020000);
-        const int r8 = lane >> 3, c8 = lane & 7;
-        const int voff_even = (r8 * K + 8 * (c8 ^ (r8 >> 1))) * 2;
-        const int voff_odd = (r8 * K + 8 * (c8 ^ (r8 >> 1) ^ 4)) * 2;
-        const bool full = (valid == BM);
-        auto dma_a = [&](half_t *dst, int kt) {
-            if (full) {
+        // Four units share an LDS base: their distance is the instruction's own offset, which moves both addresses, so the
+        // lane's is that much smaller (8 rows are 4096 bytes at least).  Rows from M on are not read: an offset out of the
+        // buffer's range loads zeros, and a tile that does not exist is one of an empty buffer - no memory is touched for what
+        // is requested ahead of a wave's last tile.
+        uint32_t a_off[4];
 #pragma unroll
-                for (int u = 0; u < A_UNITS; ++u)
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, (__attribute__((address_space(3))) void *)(dst + u * 512), 16,
-                                                             (u & 1) ? voff_odd : voff_even, (8 * u * K + kt * BK) * 2, 0, 0);
-            } else {
-                // last row tile: rows beyond M load row M-1 instead (the scalar offset is not
-                // covered by the buffer's range check, so the row has to be clamped per lane)
-#pragma unroll
-                for (int u = 0; u < A_UNITS; ++u) {
-                    const int row = min(8 * u + r8, valid - 1);
-                    const int chunk = c8 ^ (r8 >> 1) ^ ((u & 1) ? 4 : 0);
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, (__attribute__((address_space(3))) void *)(dst + u * 512), 16,
-                                                             (row * K + 8 * chunk) * 2, kt * (BK * 2), 0, 0);
-                }
+        for (int u = 0; u < 4; ++u) {
+            const int row = 8 * u + (lane >> 3);
+            const int c = (lane & 7) ^ ((row >> 1) & 7);
+            a_off[u] = (uint32_t)row * (uint32_t)K * 2u + 16u * c - 1024u * u;
+        }
+        auto dma_a = [&](half_t *dst, int tile, int u) {
+            const int rows = tile < nk ? min(32, max(M - m0 - 8 * (u & ~3), 0)) : 0;
+            const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+                (void *)(p.x + (size_t)(m0 + 8 * (u & ~3)) * K), 0, (int)((uint32_t)rows * (uint32_t)K * 2u), 0x00020000);
+            auto *const lds = (__attribute__((address_space(3))) void *)(dst + (u & ~3) * 512);
+            switch (u & 3) {
+                case 0: __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, lds, 16, (int)a_off[0], tile * (BK * 2), 0, 0); break;
+                case 1: __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, lds, 16, (int)a_off[1], tile * (BK * 2), 1024, 0); break;
+                case 2: __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, lds, 16, (int)a_off[2], tile * (BK * 2), 2048, 0); break;
+                default: __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, lds, 16, (int)a_off[3], tile * (BK * 2), 3072, 0); break;
             }
-            asm volatile("" ::: "memory");  // the loads that follow stay behind these
+            if (u == A_UNITS - 1) asm volatile("" ::: "memory");  // the loads that follow stay behind these
         };
         const int sw = (l32 >> 1) & 7;  // (row >> 1) & 7 for every row this lane reads (rows = 32*j + l32)
 
         // Packed words of two K tiles: slot [par][ks] holds step ks of a tile of parity par.  It
         // is decoded during step ks - 1 and refilled during step ks - once its old contents
         // are dead, so the load can land in place - with the same step two tiles on.
-        uint2 b2[NB][2][4];
         // (SB: slot [par][2 * m + t] holds, for column t, the words of steps 2 * m and 2 * m + 1; both are refilled during step
         // 2 * m + 1)
-        auto load_b2 = [&](int par, int kt, int ks) {
+        // Addresses are scalars of the wave plus offsets of the lane that never change, as in the tiled kernel.
+        uint2 b2[NB][2][4];
+        constexpr int NMAT = (EPI == EPI_SILU_MUL) ? 2 : 1;
+        const int strip_bytes = (K >> 7) * 1024, groups = K / p.groupsize;
+        // SB: the strips of the wave's columns from its first one on; columns 64 further are four strips further
+        const int sb_lane = PAIRED ? (l32 >> 4) * strip_bytes + (l32 & 15) * 16 + 8 * lhi : (l32 >> 3) * strip_bytes + (2 * l32 & 15) * 16 + 8 * lhi;
+        const int sb_meta_lane = PAIRED ? (l32 >> 4) * groups * 64 + (l32 & 15) * 4 : (l32 >> 3) * groups * 64 + (2 * l32 & 15) * 4;
+        constexpr int STRIPS = PAIRED ? 6 : ADJ ? 8 : 4;
+        const uint32_t *sb_words[NMAT];
+        __amdgpu_buffer_rsrc_t sb_meta_rsrc[NMAT];
+        if constexpr (SB) {
+#pragma unroll
+            for (int j = 0; j < NMAT; ++j) {
+                sb_words[j] = p.w[j].qweight + (size_t)(n0 >> 4) * (size_t)(K >> 7) * 256;
+                sb_meta_rsrc[j] = __builtin_amdgcn_make_buffer_rsrc((void *)(p.w[j].qzeros + (size_t)(n0 >> 4) * (size_t)groups * 16), 0, STRIPS * groups * 64, 0x00020000);
+            }
+        }
+        // checkpoint order: the lane's offset behind the first row of a step, its scales and its word of zero points
+        const int wlane = PAIRED ? (lhi * N + l32) * 4 : (lhi * N + 2 * l32) * 4;
+        const int slane = PAIRED ? 2 * l32 : 4 * l32, zlane = PAIRED ? (l32 >> 3) * 4 : (l32 >> 2) * 4;
+        auto load_b2 = [&](int par, int tile, int ks) {
             if constexpr (SB) {
                 if (ks & 1) {
-                    const uint32_t off = sb_off + (uint32_t)(2 * min(kt, nk - 1) + (ks >> 1)) * 64u;
 #pragma unroll
                     for (int j = 0; j < NB; ++j) {
-                        const uint32_t *src = sb_words(j) + off;
-                        b2[j][par][ks - 1] = *reinterpret_cast<const uint2 *>(src);
-                        b2[j][par][ks] = *reinterpret_cast<const uint2 *>(src + (PAIRED ? 4 * sb_strip : 4u));
+                        const int at = tile * 512 + ((ADJ && j) ? 4 * strip_bytes : 0), m = 256 * (ks >> 1);
+                        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)sb_words[j < NMAT ? j : 0], 0, tile < nk ? STRIPS * strip_bytes : 0, 0x00020000);
+                        b2[j][par][ks - 1] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(r, sb_lane + m, at, 0));
+                        b2[j][par][ks] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(r, sb_lane + m + (PAIRED ? 0 : 16), at + (PAIRED ? 4 * strip_bytes : 0), 0));
                     }
                 }
-                return;
-            }
-            const size_t off = ((size_t)min(kt, nk - 1) * (BK / 8) + 2 * ks) * N;
-            if constexpr (PAIRED) {
-                b2[0][par][ks].x = bptr_[0][off];
-                b2[0][par][ks].y = bptr_[0][off + 64];
             } else {
 #pragma unroll
-                for (int j = 0; j < NB; ++j) b2[j][par][ks] = *reinterpret_cast<const uint2 *>(bptr(j) + off);
+                for (int j = 0; j < NB; ++j) {
+                    // (the tile's eight rows, whose first is found in 64 bits)
+                    const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc((void *)(p.w[j < NMAT ? j : 0].qweight + n0 + (uint64_t)(uint32_t)tile * (uint32_t)(8 * N)), 0, tile < nk ? (8 * N - n0) * 4 : 0, 0x00020000);
+                    if constexpr (PAIRED) {
+                        b2[j][par][ks].x = __builtin_amdgcn_raw_buffer_load_b32(rows, wlane, 2 * ks * N * 4, 0);
+                        b2[j][par][ks].y = __builtin_amdgcn_raw_buffer_load_b32(rows, wlane + 256, 2 * ks * N * 4, 0);
+                    } else {
+                        b2[j][par][ks] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rows, wlane + ((ADJ && j) ? 256 : 0), 2 * ks * N * 4, 0));
+                    }
+                }
             }
         };
-        // Scale and zero words two tiles ahead as well; the group of the look-ahead tile is
-        // tracked by counting.
-        int group2 = k_begin / tiles_per_group;
-        int left2 = tiles_per_group - (k_begin - group2 * tiles_per_group);
-        uint32_t g_s[NB][2], g_z[NB][2];
-        uint32_t g_s_hi[2], g_z_hi[2];  // PAIRED: scale and zero word of the lane's second column
         auto word_of = [&](int j, int par, int step, int t) -> uint32_t {
             if constexpr (SB) {
                 const uint2 w = b2[j][par][(step & ~1) + t];
@@ -248,131 +240,149 @@ __global__ __launch_bounds__(64 * KS, MT > 2 || (KS == 8 && (MT == 2 || (EPI != 
                 return t ? b2[j][par][step].y : b2[j][par][step].x;
             }
         };
-        auto load_group2 = [&](int par) {
-            const int g = min(group2, last_group);
-            if constexpr (SB) {
-                // {scale | zero << 16} of the lane's two columns of each block, in g_s and g_z
+        // Scale and zero words run two tiles ahead as well: slot [par] is loaded in the last step of a tile of parity par and
+        // made into the decode constants of the tile two on during the last step of the tile in between.
+        uint32_t g_s[NB][2], g_z[NB][2];
+        uint32_t g_s_hi[2], g_z_hi[2];  // PAIRED: scale and zero word of the lane's second column
+        const uint32_t group_magic = p.tile_group_magic;  // (group = tile / (groupsize / 64): exact for every tile)
+        const int group_shift = p.tile_group_shift;
+        auto load_group2 = [&](int par, int tile) {
+            const uint32_t g = __umulhi((uint32_t)min(tile, nk - 1), group_magic) >> group_shift;
 #pragma unroll
-                for (int j = 0; j < NB; ++j) {
-                    const uint32_t *src = sb_meta(j) + sb_moff + (uint32_t)g * 16u;
+            for (int j = 0; j < NB; ++j) {
+                const int mat = j < NMAT ? j : 0;
+                if constexpr (SB) {
+                    // {scale | zero << 16} of the lane's two columns of each block, in g_s and g_z
+                    const int at = (int)g * 64 + ((ADJ && j) ? 4 * groups * 64 : 0);
                     if constexpr (PAIRED) {
-                        g_s[j][par] = src[0];
-                        g_z[j][par] = src[4 * sb_groups16];
+                        g_s[j][par] = __builtin_amdgcn_raw_buffer_load_b32(sb_meta_rsrc[mat], sb_meta_lane, at, 0);
+                        g_z[j][par] = __builtin_amdgcn_raw_buffer_load_b32(sb_meta_rsrc[mat], sb_meta_lane, at + 4 * groups * 64, 0);
                     } else {
-                        const uint2 m2 = *reinterpret_cast<const uint2 *>(src);
+                        const uint2 m2 = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(sb_meta_rsrc[mat], sb_meta_lane, at, 0));
                         g_s[j][par] = m2.x;
                         g_z[j][par] = m2.y;
                     }
+                } else {
+                    const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc((void *)(p.w[mat].scales + n0 + (uint64_t)g * (uint32_t)N), 0, (N - n0) * 2, 0x00020000);
+                    const __amdgpu_buffer_rsrc_t zr = __builtin_amdgcn_make_buffer_rsrc((void *)(p.w[mat].qzeros + (n0 >> 3) + (uint64_t)g * (uint32_t)(N >> 3)), 0, (N - n0) >> 1, 0x00020000);
+                    if constexpr (PAIRED) {
+                        g_s[j][par] = __builtin_amdgcn_raw_buffer_load_b16(sr, slane, 0, 0);
+                        g_s_hi[par] = __builtin_amdgcn_raw_buffer_load_b16(sr, slane + 128, 0, 0);
+                        g_z[j][par] = __builtin_amdgcn_raw_buffer_load_b32(zr, zlane, 0, 0);
+                        g_z_hi[par] = __builtin_amdgcn_raw_buffer_load_b32(zr, zlane + 32, 0, 0);
+                    } else {
+                        g_s[j][par] = __builtin_amdgcn_raw_buffer_load_b32(sr, slane + ((ADJ && j) ? 128 : 0), 0, 0);
+                        g_z[j][par] = __builtin_amdgcn_raw_buffer_load_b32(zr, zlane + ((ADJ && j) ? 32 : 0), 0, 0);
+                    }
                 }
-            } else if constexpr (PAIRED) {
-                const uint16_t *const sp = reinterpret_cast<const uint16_t *>(sc_[0] + (size_t)g * N);
-                g_s[0][par] = sp[0];
-                g_s_hi[par] = sp[64];
-                g_z[0][par] = qz_[0][(size_t)g * (N >> 3)];
-                g_z_hi[par] = qz_[0][(size_t)g * (N >> 3) + 8];
-            } else {
-#pragma unroll
-                for (int j = 0; j < NB; ++j) {
-                    g_s[j][par] = *reinterpret_cast<const uint32_t *>(sc(j) + (size_t)g * N);
-                    g_z[j][par] = qz(j)[(size_t)g * (N >> 3)];
-                }
-            }
-            if (left2 == 1) {
-                ++group2;
-                left2 = tiles_per_group;
-            } else {
-                --left2;
             }
         };
         ColDecodeNat cn[NB][2];
-        auto make_cn = [&](int par) {
+        auto make_cn = [&](int par, int j, int t) {
             if constexpr (SB) {
-#pragma unroll
-                for (int j = 0; j < NB; ++j) {
-                    cn[j][0] = make_col_decode_nat((g_s[j][par] >> 16) & 0xFu, g_s[j][par]);
-                    cn[j][1] = make_col_decode_nat((g_z[j][par] >> 16) & 0xFu, g_z[j][par]);
-                }
-                return;
-            }
-            if constexpr (PAIRED) {
-                const int sh = (l32 & 7) * 4;
-                cn[0][0] = make_col_decode_nat((g_z[0][par] >> sh) & 0xFu, g_s[0][par]);
-                cn[0][1] = make_col_decode_nat((g_z_hi[par] >> sh) & 0xFu, g_s_hi[par]);
-                return;
-            }
-#pragma unroll
-            for (int j = 0; j < NB; ++j) {
-                const uint32_t z2 = g_z[j][par] >> (((2 * l32) & 7) * 4);
-                cn[j][0] = make_col_decode_nat(z2 & 0xFu, g_s[j][par]);
-                cn[j][1] = make_col_decode_nat((z2 >> 4) & 0xFu, g_s[j][par] >> 16);
+                const uint32_t m = t ? g_z[j][par] : g_s[j][par];
+                cn[j][t] = make_col_decode_nat((m >> 16) & 0xFu, m);
+            } else if constexpr (PAIRED) {
+                cn[j][t] = make_col_decode_nat(((t ? g_z_hi[par] : g_z[j][par]) >> ((l32 & 7) * 4)) & 0xFu, t ? g_s_hi[par] : g_s[j][par]);
+            } else {
+                cn[j][t] = make_col_decode_nat((g_z[j][par] >> (((2 * l32) & 7) * 4 + 4 * t)) & 0xFu, t ? g_s[j][par] >> 16 : g_s[j][par]);
             }
         };
 
-        dma_a(buf0, k_begin);
+        const int second = k_begin + 1;
+#pragma unroll
+        for (int u = 0; u < A_UNITS; ++u) dma_a(buf0, k_begin, u);
+        load_group2(0, k_begin);
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) load_b2(0, k_begin, ks);
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) load_b2(1, k_begin + 1, ks);
-        load_group2(0);  // group of tile k_begin
-        make_cn(0);
-        load_group2(1);  // group of tile k_begin + 1, made into constants at the end of tile k_begin
+        for (int u = 0; u < A_UNITS; ++u) dma_a(buf1, second, u);
+        load_group2(1, second);  // made into constants at the end of tile k_begin
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) load_b2(1, second, ks);
         h8_t bf[NB][2];
 #pragma unroll
-        for (int j = 0; j < NB; ++j) {
-            bf[j][0] = decode_word_natural(word_of(j, 0, 0, 0), cn[j][0]);
-            bf[j][1] = decode_word_natural(word_of(j, 0, 0, 1), cn[j][1]);
-        }
-
-        // one K tile (of parity `par` counted from k_begin) from buffer `cur`, while the next
-        // tile streams into `nxt`
-        auto k_tile = [&](const half_t *cur, half_t *nxt, int kt, int par) {
-            // Loads complete in order and this wave issued 4 * NB packed-word loads after the
-            // scale/zero words that followed its LDS-direct loads of this tile: at most that
-            // many outstanding means the tile has landed.  It is this wave's own tile: no barrier.
-            // (tests/test_wait_counts.py counts the loads behind the tile's in the compiled code of every variant.)
-            // (lgkmcnt: the fragment reads of the tile before are done before its buffer is requested again.)
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(4 * NB * ((PAIRED && !SB) ? 2 : 1)) : "memory");
-            dma_a(nxt, min(kt + 1, nk - 1));
-            load_group2(par);
-            h8_t araw[MT];
-            auto read_a = [&](int ks) {
+        for (int j = 0; j < NB; ++j)
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-                    araw[mt] = *reinterpret_cast<const h8_t *>(cur + (mt * 32 + l32) * BK +
-                                                               8 * ((SB ? 4 * (ks >> 1) + 2 * lhi + (ks & 1) : 2 * ks + lhi) ^ sw));
-            };
-            read_a(0);
+            for (int t = 0; t < 2; ++t) {
+                make_cn(0, j, t);
+                bf[j][t] = decode_word_natural(word_of(j, 0, 0, t), cn[j][t]);
+            }
+        // fragment mt of K step ks of the tile in `src`
+        auto read_a = [&](const half_t *src, int ks, int mt) {
+            return *reinterpret_cast<const h8_t *>(src + (mt * 32 + l32) * BK + 8 * ((SB ? 4 * (ks >> 1) + 2 * lhi + (ks & 1) : 2 * ks + lhi) ^ sw));
+        };
+        // (the first tile's packed words and the whole second tile's loads follow the first tile's; it is this wave's own tile: no barrier)
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 * NB + A_UNITS) : "memory");
+        h8_t ahead[MT];  // fragments of the step to come
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) ahead[mt] = read_a(buf0, 0, mt);
+
+        // One K tile (of parity `par` counted from k_begin) out of buffer `cur`: four steps of 2 * NB * MT slots, each an MFMA
+        // with its share of what has to be done for the step to come, as in the tiled kernel.  With the wait, the requests and
+        // the fragment reads of a tile in front of its products and addresses of 64 bits per lane, a K tile of 64 rows x 64
+        // columns took four waves 0.88 us on 64 CUs and 1.04 on all 256, eight waves (twice the work) 1.57 and 1.96; now 0.70 and
+        // 0.86, 1.34 and 1.78, and 1.10 -> 0.95 for 96 rows: what is left is the rows' way through the CU (some 60 GB/s each, four
+        // waves or eight) beside ~190 instructions a wave.  Calls of 17 .. 700 rows: 4096 x 4096 at 320 rows 23.5 -> 19.3 us,
+        // 5120 x 5120 at 200 rows 28.0 -> 22.3 (both of four waves), 11008 x 4096 at 700 rows 79.3 -> 73.5; on average 3 %.
+        // (final: a last tile that nothing follows, where the loop ends on one - the tiles go in pairs)
+        auto k_tile = [&](half_t *cur, const half_t *nxt, int kt, int par, auto final) {
+            constexpr bool FINAL = decltype(final)::value;
+            constexpr int SLOTS = 2 * NB * MT;
+            const int tile2 = kt + 2;
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) {
-                h8_t af[MT];
+                const bool next = ks < 3 || !FINAL;  // a step follows
+                h8_t af[MT], bnext[NB][2];
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) af[mt] = araw[mt];
-                if (ks < 3) read_a(ks + 1);
-                if (ks == 3) make_cn(par ^ 1);
-                load_b2(par, kt + 2, ks);           // this step's words were decoded during the previous step
-                __builtin_amdgcn_sched_barrier(0);  // keep the loads above the MFMAs that hide them
+                for (int mt = 0; mt < MT; ++mt) af[mt] = ahead[mt];
+                DecodeNat dec;
+                if (ks < 3 || FINAL) __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), once for the step's fragments
+                __builtin_amdgcn_sched_barrier(0);
+                // Loads complete in order, and behind the LDS-direct loads of the next tile this wave issued scale/zero words and
+                // the packed words of four K steps: at most that many outstanding means the tile has landed.
+                // (tests/test_wait_counts.py counts the loads behind the tile's in the compiled code of every variant.)
+                if (ks == 3 && !FINAL) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(4 * NB * ((PAIRED && !SB) ? 2 : 1)) : "memory");
 #pragma unroll
-                for (int j = 0; j < NB; ++j) {
-                    const uint32_t next0 = (ks < 3) ? word_of(j, par, ks + 1, 0) : word_of(j, par ^ 1, 0, 0);
-                    const uint32_t next1 = (ks < 3) ? word_of(j, par, ks + 1, 1) : word_of(j, par ^ 1, 0, 1);
+                for (int i = 0; i < SLOTS; ++i) {
+                    const int j = i / (2 * MT), t = (i / MT) & 1, mt = i % MT;
+                    acc[j][mt][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mt], bf[j][t], acc[j][mt][t], 0, 0, 0);
+                    if (i < MT && next) ahead[i] = ks < 3 ? read_a(cur, ks + 1, i) : read_a(nxt, 0, i);
+                    if (ks == 3 && !FINAL) {
+                        // (all of this wave's reads of `cur` are done)
 #pragma unroll
-                    for (int mt = 0; mt < MT; ++mt)
-                        acc[j][mt][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mt], bf[j][0], acc[j][mt][0], 0, 0, 0);
-                    bf[j][0] = decode_word_natural(next0, cn[j][0]);
+                        for (int u = i * A_UNITS / SLOTS; u < (i + 1) * A_UNITS / SLOTS; ++u) dma_a(cur, tile2, u);
+                        if (i == SLOTS - 1) load_group2(par, tile2);
+                    }
+                    if (i == SLOTS - 1 && !FINAL) load_b2(par, tile2, ks);  // (this step's words were decoded during the previous step)
+                    if (next) {
+                        // words of the next step (step 0 of the next tile when ks == 3), a stage of four instructions at a time
 #pragma unroll
-                    for (int mt = 0; mt < MT; ++mt)
-                        acc[j][mt][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mt], bf[j][1], acc[j][mt][1], 0, 0, 0);
-                    bf[j][1] = decode_word_natural(next1, cn[j][1]);
+                        for (int st = 4 * mt / MT; st < 4 * (mt + 1) / MT; ++st) {
+                            if (ks == 3 && st == 0) make_cn(par ^ 1, j, t);
+                            dec.stage(st, ks < 3 ? word_of(j, par, ks + 1, t) : word_of(j, par ^ 1, 0, t), cn[j][t]);
+                            if (ks == 3 && st >= 2) dec.pin(st);
+                            if (st == 3) bnext[j][t] = dec.value();
+                        }
+                    }
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // the MFMA first
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (next) {
+#pragma unroll
+                    for (int j = 0; j < NB; ++j) bf[j][0] = bnext[j][0], bf[j][1] = bnext[j][1];
                 }
             }
         };
         KS_STAMP(1);
+        // pairs of tiles without a branch between them (a join there would make the compiler move packed words that are still
+        // in flight, and wait for them), then the odd one
         int kt = k_begin;
         for (; kt + 1 < nk; kt += 2) {
-            k_tile(buf0, buf1, kt, 0);
-            k_tile(buf1, buf0, kt + 1, 1);
+            k_tile(buf0, buf1, kt, 0, std::false_type{});
+            k_tile(buf1, buf0, kt + 1, 1, std::false_type{});
         }
-        if (kt < nk) k_tile(buf0, buf1, kt, 0);
+        if (kt < nk) k_tile(buf0, buf1, kt, 0, std::true_type{});
     }
     // every LDS-direct load has landed and every wave is done reading before the tiles are
     // reused for the exchange
@@ -910,7 +920,8 @@ size_t kslice_partial_bytes(int epi, const KslicePlan &pl) {
     return pl.splitk > 1 ? (size_t)pl.tiles * pl.splitk * pl.mt * nset * 32 * 64 * sizeof(float) : 0;
 }
 
-int launch_kslice(int epi, const MatmulArgs &a, const KslicePlan &pl, hipStream_t stream) {
+int launch_kslice(int epi, MatmulArgs &a, const KslicePlan &pl, hipStream_t stream) {
+    set_tile_group(a);
     switch (epi) {
         case EPI_PLAIN: return launch_epi<EPI_PLAIN>(a, pl, stream);
         case EPI_SILU_MUL: return launch_epi<EPI_SILU_MUL>(a, pl, stream);
