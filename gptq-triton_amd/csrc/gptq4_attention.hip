@@ -19,6 +19,8 @@
 #include "../../include/gptq4.h"
 #include "gptq4_internal.h"
 
+#include <type_traits>
+
 namespace {
 
 typedef float f16x_t __attribute__((ext_vector_type(16)));
@@ -28,11 +30,19 @@ constexpr size_t FA_LDS_BYTES = (size_t)2 * (FA_K_BUF + FA_V_BUF) * 16;  // 71,6
 constexpr int FA_GROUP = 4;  // heads of an XCD worked on together when it has many (1 MiB of keys and values each at 2048 tokens; 4 MiB of L2)
 
 // (fmaxf makes the compiler quiet possible signalling NaNs first, one more instruction per operand; the scores are
-// matrix-core outputs or -inf)
+// matrix-core outputs or -inf.  The compiler does not count the cycles between a matrix product and an asm statement that
+// reads its result, and the hardware does not wait: 18 and more have to lie between them where this is used.)
 __device__ __forceinline__ float max3(float a, float b, float c) {
     float r;
     asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
     return r;
+}
+
+// The larger of the lane's value and that of the lane 32 on, in both.
+__device__ __forceinline__ float max_of_halves(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
+    const uint32_t own = r[0], other = r[1];  // (variables: of the vector's elements themselves the compiler casts the first one twice)
+    return fmaxf(__builtin_bit_cast(float, own), __builtin_bit_cast(float, other));
 }
 
 __device__ __forceinline__ int key_slot(int key) {  // position of a key of a 64-key block in V^T's row
@@ -52,7 +62,7 @@ __global__ __launch_bounds__(256, 2) void gptq4_attn_prefill_kernel(const half_t
     uint4 *const v_s = fa_smem + 2 * FA_K_BUF;   // 2 x 128 x 9 chunks
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = lane >> 5, c32 = lane & 31;
     // Workgroup id -> (head, query block).  Consecutive ids go to the eight XCDs in turn, each with an L2 of its own:
     // id % 8 picks the XCD and all query blocks of a head are given to one XCD (head % 8, for the heads up to the last
@@ -121,94 +131,101 @@ __global__ __launch_bounds__(256, 2) void gptq4_attn_prefill_kernel(const half_t
     //      slot order too - and writes, per dimension, one dword {key 2p, key 2p + 1}: half a wave fills 128 bytes of a row.
     // (buffer loads: rows from kv_len on come back as zeros - they are masked.  The block's offset is part of the lane
     // offset: the range check does not see a scalar offset)
-    const __amdgpu_buffer_rsrc_t k_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(kb), 0, (int)((uint32_t)kv_len * 256u), 0x00020000);
-    const __amdgpu_buffer_rsrc_t v_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(vb), 0, (int)((uint32_t)kv_len * 256u), 0x00020000);
+    const int kv_bytes = (int)((uint32_t)kv_len * 256u);
     const uint32_t k_voff = (uint32_t)(tid >> 4) * 256u + (uint32_t)(tid & 15) * 16u;  // + 16 keys per n
     const uint32_t v_voff = (uint32_t)(2 * (tid & 31)) * 256u + (uint32_t)(tid >> 5) * 16u;  // + 1 key per kk, + 8 chunks per n
     u32x4_t kr[4], vr[2][2];
-#define FETCH_K(blk)                                                                                                      \
-    _Pragma("unroll") for (int n = 0; n < 4; ++n)                                                                         \
-        kr[n] = __builtin_amdgcn_raw_buffer_load_b128(k_rs, k_voff + 16u * 256u * n + (uint32_t)(blk) * (64u * 256u), 0, 0);
-#define FETCH_V(blk)                                                                                                      \
-    _Pragma("unroll") for (int n = 0; n < 2; ++n) _Pragma("unroll") for (int kk = 0; kk < 2; ++kk)                        \
-        vr[n][kk] = __builtin_amdgcn_raw_buffer_load_b128(v_rs, v_voff + 256u * kk + 128u * n + (uint32_t)(blk) * (64u * 256u), 0, 0);
+    // (a block beyond the last one is asked of an empty buffer: zeros without a trip to memory)
+    auto fetch_k = [&](int blk, int n) {
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(kb), 0, blk < nblk ? kv_bytes : 0, 0x00020000);
+        return __builtin_amdgcn_raw_buffer_load_b128(rs, k_voff + 16u * 256u * n + (uint32_t)blk * (64u * 256u), 0, 0);
+    };
+    auto fetch_v = [&](int blk, int n, int kk) {
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(vb), 0, blk < nblk ? kv_bytes : 0, 0x00020000);
+        return __builtin_amdgcn_raw_buffer_load_b128(rs, v_voff + 256u * kk + 128u * n + (uint32_t)blk * (64u * 256u), 0, 0);
+    };
+#define FETCH_K(blk) _Pragma("unroll") for (int n = 0; n < 4; ++n) kr[n] = fetch_k(blk, n);
+#define FETCH_V(blk) \
+    _Pragma("unroll") for (int n = 0; n < 2; ++n) _Pragma("unroll") for (int kk = 0; kk < 2; ++kk) vr[n][kk] = fetch_v(blk, n, kk);
     const int vslot = key_slot(2 * (tid & 31));  // even: the pair's dword
     uint4 *const k_put = k_s + (tid >> 4) * 17 + (tid & 15);                                          // + 16 rows per n
     uint32_t *const v_put = reinterpret_cast<uint32_t *>(v_s) + (8 * (tid >> 5)) * 36 + (vslot >> 1);  // + 36 dwords per dim
-    auto stage_k = [&](int buf) {
-#pragma unroll
-        for (int n = 0; n < 4; ++n) k_put[buf * FA_K_BUF + n * (16 * 17)] = __builtin_bit_cast(uint4, kr[n]);
+    auto stage_k = [&](int buf, int n) { k_put[buf * FA_K_BUF + n * (16 * 17)] = __builtin_bit_cast(uint4, kr[n]); };
+    auto stage_v = [&](int buf, int part) {  // an eighth of it: word part % 4 of chunk part / 4
+        const int n = part >> 2, w = part & 3;
+        const uint32_t lo = vr[n][0][w], hi = vr[n][1][w];
+        // halves 2 * w and 2 * w + 1 of the two keys
+        uint32_t *const at = v_put + buf * (FA_V_BUF * 4) + (64 * n + 2 * w) * 36;
+        at[0] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+        at[36] = __builtin_amdgcn_perm(hi, lo, 0x07060302u);
     };
-    auto stage_v = [&](int buf) {
-#pragma unroll
-        for (int n = 0; n < 2; ++n)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const uint32_t lo = vr[n][0][e >> 1], hi = vr[n][1][e >> 1];
-                // halves e of the two keys: bytes (0, 1) or (2, 3) of each word
-                const uint32_t w = (e & 1) ? __builtin_amdgcn_perm(hi, lo, 0x07060302u) : __builtin_amdgcn_perm(hi, lo, 0x05040100u);
-                v_put[buf * (FA_V_BUF * 4) + (64 * n + e) * 36] = w;
-            }
-    };
-    // ---- S^T = K Q^T for the two half blocks of 32 keys of the block in K buffer `buf`
-    auto scores = [&](int buf, f16x_t(&s)[2]) {
-        const uint4 *const kt = k_s + buf * FA_K_BUF + c32 * 17 + h;  // the lane's key row of a half block, chunk h
-#pragma unroll
-        for (int rb = 0; rb < 2; ++rb) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) s[rb][i] = 0.f;
-#pragma unroll
-            for (int ks = 0; ks < 8; ++ks) {
-                const h8_t a = __builtin_bit_cast(h8_t, kt[rb * (32 * 17) + 2 * ks]);
-                s[rb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qf[ks], s[rb], 0, 0, 0);
-            }
-        }
-    };
-
-    // ---- The order of work.  K is staged two blocks ahead of the block whose probabilities are being made and V one, in two
-    //      buffers each, with one barrier per block: in step i the wave takes the scores of block i, made in step i - 1,
-    //      issues the products for the scores of block i + 1, and turns block i's scores into probabilities while the matrix
-    //      cores work on those; then O^T += V^T P^T for block i.  Step i writes K block i + 2 over block i (last read in
-    //      step i - 1) and V block i + 1 over block i - 1.
+    // ---- The order of work.  A wave issues an instruction every five cycles and a product takes 32, so a step's some 330
+    //      instructions (32 products, 32 LDS reads, 32 exponentials) bound a wave that is alone on its SIMD, and what it waits
+    //      for in between comes on top: they are dealt to the products one by one.  Left to the compiler (fragments read one
+    //      product ahead, exponentials in front of the products that take them, the accumulators rescaled behind a branch) a
+    //      block of 64 keys took 1.45 us, now 1.2: 32 heads x 2000 tokens 60 -> 53 us, 8 x 2048 45 -> 39.5, 52 x 2000 103 -> 94,
+    //      8 x 52 x 2048 629 -> 590, 32 x 128 behind 1000 28.2 -> 25.3.
+    //      K is staged two blocks ahead of the block whose probabilities are being made and V one, in
+    //      two buffers each, with one barrier per block: step i issues the products for the scores of block i + 1 with the
+    //      probabilities of block i between them, then O^T += V^T P^T for block i with the maximum of block i + 1's scores and
+    //      the staging between those.  Step i writes K block i + 2 over block i (last read in step i - 1) and V block
+    //      i + 1 over block i - 1, and asks for K block i + 3 and V block i + 2 (beyond the last block: of an empty buffer).
     {
         FETCH_K(0)
         FETCH_V(0)
         u32x4_t k1[4];  // (block 1 of K asked for together with block 0: one round trip to memory before the first product)
         if (nblk > 1) {
 #pragma unroll
-            for (int n = 0; n < 4; ++n) k1[n] = __builtin_amdgcn_raw_buffer_load_b128(k_rs, k_voff + 16u * 256u * n + 64u * 256u, 0, 0);
+            for (int n = 0; n < 4; ++n) k1[n] = fetch_k(1, n);
         }
-        stage_k(0);
-        stage_v(0);
+#pragma unroll
+        for (int n = 0; n < 4; ++n) stage_k(0, n);
+#pragma unroll
+        for (int n = 0; n < 8; ++n) stage_v(0, n);
         if (nblk > 1) {
 #pragma unroll
             for (int n = 0; n < 4; ++n) k_put[FA_K_BUF + n * (16 * 17)] = __builtin_bit_cast(uint4, k1[n]);
+            FETCH_K(2)
             FETCH_V(1)
-            if (nblk > 2) {
-                FETCH_K(2)
-            }
         }
     }
-    __syncthreads();
+    const uint4 *const k_get = k_s + c32 * 17 + h;  // the lane's key row of a half block, chunk h
+    const uint4 *const v_get = v_s + c32 * 9 + h;   // the lane's dim row of a block of 32, chunk h
+    // operand A of product n of a step: K block i + 1 (0 .. 15, the two half blocks of 32 keys in turn), V block i (16 .. 31,
+    // four blocks of 32 dims to a step of 16 keys)
+    auto fragment = [&](int buf, int n) {
+        return __builtin_bit_cast(h8_t, n < 16 ? k_get[(buf ^ 1) * FA_K_BUF + (n & 1) * (32 * 17) + 2 * (n >> 1)]
+                                               : v_get[buf * FA_V_BUF + (n & 3) * (32 * 9) + 2 * ((n - 16) >> 2)]);
+    };
     f16x_t sa[2], sb[2];
-    scores(0, sa);
-    auto step = [&](int blk, f16x_t(&s)[2], f16x_t(&sn)[2]) {
-        const int buf = blk & 1;
-        __syncthreads();  // K block blk + 1 and V block blk are in their buffers; the buffers written below have been read
-        if (blk + 1 < nblk) {
-            stage_v(buf ^ 1);
-            if (blk + 2 < nblk) {
-                FETCH_V(blk + 2)
-                stage_k(buf);
-                if (blk + 3 < nblk) {
-                    FETCH_K(blk + 3)
-                }
-            }
+    auto block_max = [&](const f16x_t(&s)[2]) {
+        float mx = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mx = max3(mx, s[0][i], s[1][i]);
+        return mx;
+    };
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < 16; ++n) {
+        if (n < 2) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) sa[n & 1][i] = 0.f;
         }
-        const uint4 *const vt = v_s + buf * FA_V_BUF + c32 * 9 + h;  // the lane's dim row of a block of 32, chunk h
+        sa[n & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fragment(1, n), qf[n >> 1], sa[n & 1], 0, 0, 0);
+    }
+    float mx = -INFINITY;  // of the lane's scores of the block to come (not by max3: the products have only just been issued)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, fmaxf(sa[0][i], sa[1][i]));
+    constexpr int AHEAD = 4;   // LDS reads in flight ahead of the products
+    // (last: the workgroup's last block, which no other's scores and no staging follow)
+    auto step = [&](int blk, auto parity, auto last, f16x_t(&s)[2], f16x_t(&sn)[2]) {
+        constexpr int buf = decltype(parity)::value;
+        constexpr bool LAST = decltype(last)::value;
+        __syncthreads();  // K block blk + 1 and V block blk are in their buffers; the buffers written below have been read
         const int key0 = blk * 64;
-        if (key0 > my_last) return;  // nothing in this block is visible to the wave (it still takes part in the staging)
-
+        h8_t ring[AHEAD];
+#pragma unroll
+        for (int n = 0; n < AHEAD; ++n) ring[n] = fragment(buf, LAST ? 16 + n : n);
         // ---- masking (only a block that reaches past the wave's first query's last key)
         if (key0 + 63 > my_first) {
             asm volatile("" ::: "memory");  // (keeps this a branch: turned into selects the masking would run for every block)
@@ -218,67 +235,119 @@ __global__ __launch_bounds__(256, 2) void gptq4_attn_prefill_kernel(const half_t
 #pragma unroll
                 for (int i = 0; i < 16; ++i)
                     if (32 * rb + 8 * (i >> 2) + (i & 3) > limit) s[rb][i] = -INFINITY;
+            mx = block_max(s);
         }
-        // ---- the next block's scores (whatever the buffer holds after the last block: nobody reads them), then the
-        //      running maximum and the probabilities of this one; the accumulators are rescaled only when some lane's
-        //      maximum moved
+        const float m_new = fmaxf(m, max_of_halves(mx) * scale_log2e);  // (the scale is positive: the maximum commutes with it)
+        const float m_use = (m_new == -INFINITY) ? 0.f : m_new;  // (a query beyond S in a clamped row: nothing visible yet)
+        const float corr = __builtin_amdgcn_exp2f(m - m_use);
+        m = m_new;
+        float sum = 0.f;
+        const h2_t ones = {(_Float16)1.0f, (_Float16)1.0f};
+        uint32_t pf[4][4];
+        // Probabilities 2 * p and 2 * p + 1 of the lane's 32 in three stages, a slot apart so that none waits for the one before
+        // (the row sum takes them as the product takes them: rounded to fp16, two per instruction).  The empty asm statements
+        // keep them where they stand: the compiler sinks arithmetic towards its use, past the scheduling barriers.
+        auto probability = [&](int p, int stage) {
+            if (p < 0 || p > 15) return;
+            const int rb = p >> 3, i = 2 * (p & 7);
+            float x = s[rb][i], y = s[rb][i + 1];
+            if (stage == 0) x = __builtin_fmaf(x, scale_log2e, -m_use), y = __builtin_fmaf(y, scale_log2e, -m_use);
+            if (stage == 1) x = __builtin_amdgcn_exp2f(x), y = __builtin_amdgcn_exp2f(y);
+            if (stage == 2) {
+                const h2_t pp = {(_Float16)x, (_Float16)y};
+                sum = __builtin_amdgcn_fdot2(pp, ones, sum, false);
+                pf[p >> 2][p & 3] = as_u32(pp);
+                asm volatile("" : "+v"(pf[p >> 2][p & 3]), "+v"(sum));
+                return;
+            }
+            asm volatile("" : "+v"(x), "+v"(y));
+            s[rb][i] = x, s[rb][i + 1] = y;
+        };
+        // slot n of the step's 32: pair p's stages in slots 3 * p / 2, + 1 and + 2 (the products of its 16 keys are in slots
+        // 16 + 4 * (p / 4) and on)
+        auto probabilities = [&](int n) {
+#pragma unroll
+            for (int stage = 0; stage < 3; ++stage) {
+                const int at = n - stage;
+                if (at >= 0 && at % 3 != 2) probability(2 * (at / 3) + at % 3, stage);
+            }
+        };
         // (ahead of the other workgroup's wave on this SIMD while that one is staging or waiting at its barrier: 656 -> 622 us
         // at 416 heads, 84.6 -> 80.1 at 40)
         __builtin_amdgcn_s_setprio(1);
-        scores(buf ^ 1, sn);
-        float mx = -INFINITY;
+        l *= corr;
+        // The next block's scores, and the accumulators brought to the new maximum on the way.  (Some lane's maximum moves in
+        // most blocks of a sequence: behind a branch these 64 instructions took 380 of 2700 cycles a block on average.  An
+        // older maximum kept until it is 2^8 too small saves most of them too, but the largest probability is then no longer an
+        // exact 1: 2 - 6 % further from 64 bits.)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) mx = max3(mx, s[0][i], s[1][i]);
-        mx = fmaxf(mx, __shfl_xor(mx, 32)) * scale_log2e;  // (the scale is positive: the maximum commutes with it)
-        const float m_new = fmaxf(m, mx);
-        const float m_use = (m_new == -INFINITY) ? 0.f : m_new;  // (a query beyond S in a clamped row: nothing visible yet)
-        float sum = 0.f;
-        const h2_t ones = {(_Float16)1.0f, (_Float16)1.0f};
-        h8_t pf[2][2];
+        for (int n = 0; n < 16; ++n) {
+            if constexpr (!LAST) {
+                if (n < 2) {
 #pragma unroll
-        for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-            for (int u = 0; u < 2; ++u)
-#pragma unroll
-                for (int t = 0; t < 8; t += 2) {
-                    // (the row sum takes the probabilities as the product takes them: rounded to fp16, two per instruction)
-                    h2_t pp;
-                    pp.x = (_Float16)__builtin_amdgcn_exp2f(__builtin_fmaf(s[rb][8 * u + t], scale_log2e, -m_use));
-                    pp.y = (_Float16)__builtin_amdgcn_exp2f(__builtin_fmaf(s[rb][8 * u + t + 1], scale_log2e, -m_use));
-                    sum = __builtin_amdgcn_fdot2(pp, ones, sum, false);
-                    pf[rb][u][t] = pp.x;
-                    pf[rb][u][t + 1] = pp.y;
+                    for (int i = 0; i < 16; ++i) sn[n & 1][i] = 0.f;
                 }
-        if (__any(m_new != m)) {
-            const float corr = __builtin_amdgcn_exp2f(m - m_use);
-            l *= corr;
+                sn[n & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ring[n % AHEAD], qf[n >> 1], sn[n & 1], 0, 0, 0);
+                ring[n % AHEAD] = fragment(buf, n + AHEAD);
+            }
+            probabilities(n);
 #pragma unroll
-            for (int db = 0; db < 4; ++db)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) o[db][i] *= corr;
-            m = m_new;
+            for (int i = 0; i < 4; ++i) o[n >> 2][4 * (n & 3) + i] *= corr;
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // the product first
+            __builtin_amdgcn_sched_barrier(0);
         }
+        float mx2 = -INFINITY;  // (two in turns: neither waits for the other)
+        mx = -INFINITY;
+#pragma unroll
+        for (int n = 0; n < 16; ++n) {
+            const h8_t pv = __builtin_bit_cast(h8_t, (u32x4_t){pf[n >> 2][0], pf[n >> 2][1], pf[n >> 2][2], pf[n >> 2][3]});
+            o[n & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ring[n % AHEAD], pv, o[n & 3], 0, 0, 0);
+            if (n + AHEAD < 16) ring[n % AHEAD] = fragment(buf, 16 + n + AHEAD);
+            probabilities(16 + n);
+            if (LAST) {
+            } else if (n < 4) {
+                stage_k(buf, n);
+                kr[n] = fetch_k(blk + 3, n);
+            } else if (n < 12) {
+                stage_v(buf ^ 1, n - 4);
+                if (n == 7 || n == 11) vr[n >> 3][0] = fetch_v(blk + 2, n >> 3, 0), vr[n >> 3][1] = fetch_v(blk + 2, n >> 3, 1);
+            }
+            // (eight products and more behind those that made the scores)
+            if (!LAST && n >= 8) {
+                mx = max3(mx, sn[0][2 * n - 16], sn[1][2 * n - 16]);
+                mx2 = max3(mx2, sn[0][2 * n - 15], sn[1][2 * n - 15]);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        mx = fmaxf(mx, mx2);
         l += sum;
-        // ---- O^T += V^T P^T: per step of 16 keys four independent products (the four blocks of 32 dims), the V^T
-        //      fragments of the next step requested before this step's products are issued
-        h8_t va[2][4];
-        auto read_v = [&](int st, int slot) {
-#pragma unroll
-            for (int db = 0; db < 4; ++db) va[slot][db] = __builtin_bit_cast(h8_t, vt[db * (32 * 9) + 2 * st]);
-        };
-        read_v(0, 0);
-#pragma unroll
-        for (int st = 0; st < 4; ++st) {
-            if (st < 3) read_v(st + 1, (st + 1) & 1);
-#pragma unroll
-            for (int db = 0; db < 4; ++db)
-                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[st & 1][db], pf[st >> 1][st & 1], o[db], 0, 0, 0);
-        }
         __builtin_amdgcn_s_setprio(0);
     };
-    for (int blk = 0; blk < nblk; blk += 2) {
-        step(blk, sa, sb);
-        if (blk + 1 < nblk) step(blk + 1, sb, sa);
+    using even = std::integral_constant<int, 0>;
+    using odd = std::integral_constant<int, 1>;
+    const int mine = (my_last >> 6) + 1;  // blocks that the wave sees a key of
+    const int followed = min(mine, nblk - 1);
+    for (int blk = 0; blk < followed; blk += 2) {
+        step(blk, even{}, std::false_type{}, sa, sb);
+        if (blk + 1 < followed) step(blk + 1, odd{}, std::false_type{}, sb, sa);
+    }
+    if (mine == nblk) {
+        if (followed & 1)
+            step(followed, odd{}, std::true_type{}, sb, sa);
+        else
+            step(followed, even{}, std::true_type{}, sa, sb);
+    }
+    for (int blk = mine; blk < nblk; ++blk) {  // (the workgroup's others: the wave only takes part in the staging)
+        __syncthreads();
+        if (blk + 1 < nblk) {
+#pragma unroll
+            for (int n = 0; n < 4; ++n) stage_k(blk & 1, n);
+#pragma unroll
+            for (int n = 0; n < 8; ++n) stage_v((blk & 1) ^ 1, n);
+            FETCH_K(blk + 3)
+            FETCH_V(blk + 2)
+        }
     }
 
     // ---- out[b, s, head * 128 + d] = O[s, d] / l: lane (h, q) holds dims 32 * db + 8 * i + 4 * h + j of its query
