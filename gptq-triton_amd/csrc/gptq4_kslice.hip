@@ -279,13 +279,17 @@ __global__ __launch_bounds__(64 * KS, MT > 2 || (KS == 8 && (MT == 2 || (EPI != 
         };
         ColDecodeNat cn[NB][2];
         auto make_cn = [&](int par, int j, int t) {
+            // (the empty asm statements keep the arithmetic here: the compiler otherwise does it, and waits for the words, where they
+            // are loaded, a tile earlier)
+            uint32_t scale = (t && PAIRED && !SB) ? g_s_hi[par] : (t && SB) ? g_z[j][par] : g_s[j][par];
+            asm volatile("" : "+v"(scale));
             if constexpr (SB) {
-                const uint32_t m = t ? g_z[j][par] : g_s[j][par];
-                cn[j][t] = make_col_decode_nat((m >> 16) & 0xFu, m);
-            } else if constexpr (PAIRED) {
-                cn[j][t] = make_col_decode_nat(((t ? g_z_hi[par] : g_z[j][par]) >> ((l32 & 7) * 4)) & 0xFu, t ? g_s_hi[par] : g_s[j][par]);
+                cn[j][t] = make_col_decode_nat((scale >> 16) & 0xFu, scale);
             } else {
-                cn[j][t] = make_col_decode_nat((g_z[j][par] >> (((2 * l32) & 7) * 4 + 4 * t)) & 0xFu, t ? g_s[j][par] >> 16 : g_s[j][par]);
+                uint32_t zeros = (t && PAIRED) ? g_z_hi[par] : g_z[j][par];
+                asm volatile("" : "+v"(zeros));
+                cn[j][t] = PAIRED ? make_col_decode_nat((zeros >> ((l32 & 7) * 4)) & 0xFu, scale)
+                                  : make_col_decode_nat((zeros >> (((2 * l32) & 7) * 4 + 4 * t)) & 0xFu, t ? scale >> 16 : scale);
             }
         };
 
