@@ -328,7 +328,8 @@ __global__ __launch_bounds__(64 * KS, MT > 2 || (KS == 8 && (MT == 2 || (EPI != 
         // columns took four waves 0.88 us on 64 CUs and 1.04 on all 256, eight waves (twice the work) 1.57 and 1.96; now 0.70 and
         // 0.86, 1.34 and 1.78, and 1.10 -> 0.95 for 96 rows: what is left is the rows' way through the CU (some 60 GB/s each, four
         // waves or eight) beside ~190 instructions a wave.  Calls of 17 .. 700 rows: 4096 x 4096 at 320 rows 23.5 -> 19.3 us,
-        // 5120 x 5120 at 200 rows 28.0 -> 22.3 (both of four waves), 11008 x 4096 at 700 rows 79.3 -> 73.5; on average 3 %.
+        // 5120 x 5120 at 200 rows 28.0 -> 22.3 (both of four waves), 11008 x 4096 at 700 rows 79.3 -> 73.5; 1818 random calls of either
+        // layout on average 5 %.
         // (final: a last tile that nothing follows, where the loop ends on one - the tiles go in pairs)
         auto k_tile = [&](half_t *cur, const half_t *nxt, int kt, int par, auto final) {
             constexpr bool FINAL = decltype(final)::value;
