@@ -276,3 +276,28 @@ def test_tile_counts_just_above_a_whole_number_of_rounds_share_their_last_strips
     ws = L_.workspace(torch.device("cuda", torch.cuda.current_device()), 0)
     torch.cuda.synchronize()
     assert int(ws[:L_.WS_HEAD_BYTES].view(torch.int32).abs().sum()) == 0
+
+
+@pytest.mark.parametrize("config", [(1, 1), (2, 1), (12, 1), (102, 1), (201, 1), (202, 1), (3, 1), (13, 1), (202, 2)], ids=lambda c: "mt%d_s%d" % c)
+@pytest.mark.parametrize("k,g", [(1920, 384), (1280, 640), (2176, 128), (2304, 1152)])
+def test_midm_tiles_of_a_wave_and_groups(config, k, g):
+    """One to nine K tiles to a wave (an odd last one, and tiles requested past the last), groups of a number of K tiles that is no
+    power of two, rows of a block that does not exist."""
+    from gptq_triton_amd import _lib
+    from gptq_triton_amd import quant_linear as Q
+    lib = _lib.load()
+    n, m = 256, 67
+    L = O.make_layer(k, n, g, seed=k + g)
+    x = O.make_x(m, k, seed=k)
+    D = to_dev(L)
+    xd = torch.from_numpy(x).cuda()
+    lib.gptq4_set_midm_tuning(2, *config)
+    try:
+        y = gptq().matmul4(g, xd, D["qweight"], D["scales"], D["qzeros"])
+        packed = Q.stream_pack(D["qweight"], D["qzeros"], D["scales"], g)
+        streamed = Q.matmul4_stream(g, xd, *packed)
+    finally:
+        lib.gptq4_set_midm_tuning(1, 0, 0)
+    ref = O.quant_matmul_ref(x, L["qweight"], L["qzeros"], L["scales"], g)
+    assert_close(y.cpu().numpy(), ref, f"mid-M matmul K={k} g={g}")
+    assert_close(streamed.cpu().numpy(), ref, f"mid-M matmul, streaming order, K={k} g={g}")

@@ -83,3 +83,14 @@ def test_argument_errors():
     with pytest.raises(RuntimeError):
         ops().prefill_attention(torch.zeros(1, 1, 4, 128, dtype=torch.float16), torch.zeros(1, 1, 4, 128, dtype=torch.float16),
                                 torch.zeros(1, 1, 4, 128, dtype=torch.float16))
+
+
+@pytest.mark.parametrize("past", [0, 31, 32, 33, 63])
+@pytest.mark.parametrize("s", [1, 32, 63, 64, 96, 128, 160, 193])
+def test_blocks_at_the_end_of_a_workgroup(past, s):
+    """The last block of a workgroup makes no scores for another, and a wave takes part in the staging of up to two blocks behind
+    the last one it sees a key of (past % 64 = 32: the first 32 queries end two blocks before the last 32).  Wide scores: a
+    maximum that is not the block's own would overflow the probabilities."""
+    q, k, v = make(1, 2, s, past + s, seed=100 * s + past, scale=2.5)
+    out = ops().prefill_attention(torch.from_numpy(q).cuda(), torch.from_numpy(k).cuda(), torch.from_numpy(v).cuda(), past)
+    close(out.cpu().numpy(), O.prefill_attention_ref(q, k, v, past), f"S={s} past={past}")
