@@ -45,6 +45,12 @@ __device__ __forceinline__ float max_of_halves(float v) {
     return fmaxf(__builtin_bit_cast(float, own), __builtin_bit_cast(float, other));
 }
 
+// a * b, rounded by itself: not made one instruction with an addition that takes it.
+__device__ __forceinline__ float product(float a, float b) {
+#pragma clang fp contract(off)
+    return a * b;
+}
+
 __device__ __forceinline__ int key_slot(int key) {  // position of a key of a 64-key block in V^T's row
     const int o = key & 15;
     return (key & ~15) | (o < 4 ? o : o < 8 ? o + 4 : o < 12 ? o - 4 : o);
@@ -275,7 +281,7 @@ __global__ __launch_bounds__(256, 2) void gptq4_attn_prefill_kernel(const half_t
         // (ahead of the other workgroup's wave on this SIMD while that one is staging or waiting at its barrier: 656 -> 622 us
         // at 416 heads, 84.6 -> 80.1 at 40)
         __builtin_amdgcn_s_setprio(1);
-        l *= corr;
+        l = product(l, corr);  // (`sum` is added behind it: with one rounding for both, a result in some 10^4 is another fp16 value)
         // The next block's scores, and the accumulators brought to the new maximum on the way.  (Some lane's maximum moves in
         // most blocks of a sequence: behind a branch these 64 instructions took 380 of 2700 cycles a block on average.  An
         // older maximum kept until it is 2^8 too small saves most of them too, but the largest probability is then no longer an
