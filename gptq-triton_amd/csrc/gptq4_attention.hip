@@ -30,8 +30,9 @@ constexpr size_t FA_LDS_BYTES = (size_t)2 * (FA_K_BUF + FA_V_BUF) * 16;  // 71,6
 constexpr int FA_GROUP = 4;  // heads of an XCD worked on together when it has many (1 MiB of keys and values each at 2048 tokens; 4 MiB of L2)
 
 // (fmaxf makes the compiler quiet possible signalling NaNs first, one more instruction per operand; the scores are
-// matrix-core outputs or -inf.  The compiler does not count the cycles between a matrix product and an asm statement that
-// reads its result, and the hardware does not wait: 18 and more have to lie between them where this is used.)
+// matrix-core outputs or -inf.  Not on results of a matrix product that nothing has waited for: the compiler does not count
+// the cycles between a product and an asm statement that reads its result, and the hardware does not wait.  Every chain of
+// them begins with the fmaxf of a result of each product, in front of which the compiler puts the cycles they still need.)
 __device__ __forceinline__ float max3(float a, float b, float c) {
     float r;
     asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
@@ -205,9 +206,9 @@ __global__ __launch_bounds__(256, 2) void gptq4_attn_prefill_kernel(const half_t
     };
     f16x_t sa[2], sb[2];
     auto block_max = [&](const f16x_t(&s)[2]) {
-        float mx = -INFINITY;
+        float mx = fmaxf(s[0][0], s[1][0]);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) mx = max3(mx, s[0][i], s[1][i]);
+        for (int i = 1; i < 16; ++i) mx = max3(mx, s[0][i], s[1][i]);
         return mx;
     };
     __syncthreads();
@@ -219,9 +220,7 @@ __global__ __launch_bounds__(256, 2) void gptq4_attn_prefill_kernel(const half_t
         }
         sa[n & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fragment(1, n), qf[n >> 1], sa[n & 1], 0, 0, 0);
     }
-    float mx = -INFINITY;  // of the lane's scores of the block to come (not by max3: the products have only just been issued)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, fmaxf(sa[0][i], sa[1][i]));
+    float mx = block_max(sa);  // of the lane's scores of the block to come
     constexpr int AHEAD = 4;   // LDS reads in flight ahead of the products
     // (last: the workgroup's last block, which no other's scores and no staging follow)
     auto step = [&](int blk, auto parity, auto last, f16x_t(&s)[2], f16x_t(&sn)[2]) {
@@ -303,7 +302,6 @@ __global__ __launch_bounds__(256, 2) void gptq4_attn_prefill_kernel(const half_t
             __builtin_amdgcn_sched_barrier(0);
         }
         float mx2 = -INFINITY;  // (two in turns: neither waits for the other)
-        mx = -INFINITY;
 #pragma unroll
         for (int n = 0; n < 16; ++n) {
             const h8_t pv = __builtin_bit_cast(h8_t, (u32x4_t){pf[n >> 2][0], pf[n >> 2][1], pf[n >> 2][2], pf[n >> 2][3]});
@@ -318,8 +316,11 @@ __global__ __launch_bounds__(256, 2) void gptq4_attn_prefill_kernel(const half_t
                 stage_v(buf ^ 1, n - 4);
                 if (n == 7 || n == 11) vr[n >> 3][0] = fetch_v(blk + 2, n >> 3, 0), vr[n >> 3][1] = fetch_v(blk + 2, n >> 3, 1);
             }
-            // (eight products and more behind those that made the scores)
-            if (!LAST && n >= 8) {
+            if (!LAST && n == 8) {
+                mx = fmaxf(sn[0][0], sn[1][0]);
+                mx2 = max3(mx, sn[0][1], sn[1][1]);
+            }
+            if (!LAST && n > 8) {
                 mx = max3(mx, sn[0][2 * n - 16], sn[1][2 * n - 16]);
                 mx2 = max3(mx2, sn[0][2 * n - 15], sn[1][2 * n - 15]);
             }
