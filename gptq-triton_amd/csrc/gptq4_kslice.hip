@@ -112,6 +112,10 @@ __global__ __launch_bounds__(64 * KS, MT > 2 || (KS == 8 && (MT == 2 || (EPI != 
         } else if ((int)blockIdx.x < total) {
             split = 0, nsplit = 1, wg_begin = 0, wg_len = p.K / BK, xtile = 0;
         } else {
+            // (ahead of the whole tile of an older workgroup beside it while it multiplies, so that its sums are exchanged while
+            // that one still works: the waves of the older one are served first otherwise.  383 x 3840 x 3840 21.7 -> 19.8 us,
+            // 185 x 2560 x 7680 17.9 -> 16.4)
+            __builtin_amdgcn_s_setprio(1);
             const int s = p.tail_split, w = (int)blockIdx.x - total;
             xtile = w / s;
             split = w - xtile * s;
@@ -444,6 +448,7 @@ __global__ __launch_bounds__(64 * KS, MT > 2 || (KS == 8 && (MT == 2 || (EPI != 
     KS_STAMP(4);
     constexpr int NREG = NSET * 2 * IW;  // values per lane of an owner wave
     if (nsplit > 1) {
+        __builtin_amdgcn_s_setprio(0);  // (parts beside whole tiles, see above)
         // K split across workgroups as well: each publishes its reduced tile (agent-scope
         // atomics, no cache maintenance), the last one to arrive sums them in split order.
         __shared__ int s_is_last;
