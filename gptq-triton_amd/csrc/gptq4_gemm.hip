@@ -325,7 +325,7 @@ __global__ __launch_bounds__(256, 2) void gptq4_gemm_kernel(MatmulArgs p) {
         //
         // A wave issues an instruction of any kind every five cycles, so the 32 cycles of an MFMA hide five others and no
         // more.  The loop's instructions are therefore counted - 4 of the decode, half an LDS read, about one of everything
-        // else for every MFMA - and dealt to the MFMAs one by one (slot() below).  Hence also: addresses are scalars of the
+        // else for every MFMA - and dealt to the MFMAs one by one (k_tile() below).  Hence also: addresses are scalars of the
         // wave plus offsets of the lane that never change, the four LDS-direct loads of a tile share one LDS base (their
         // distance is the instruction's own offset, which moves both addresses, so the lane's is that much smaller), and
         // the group of a tile comes out of one multiplication.
@@ -344,14 +344,17 @@ __global__ __launch_bounds__(256, 2) void gptq4_gemm_kernel(MatmulArgs p) {
         const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
             (void *)a_base, 0, (int)((uint32_t)min(BM, M - m0) * (uint32_t)K * 2u), 0x00020000);
         static_assert(A_UNITS == 4, "the loads below name the units");
-        auto dma_a = [&](half_t *dst, int kt) {
+        auto dma_a = [&](half_t *dst, int kt, auto unit) {
+            constexpr int u = decltype(unit)::value;
             auto *const lds = (__attribute__((address_space(3))) void *)(dst + wave * (A_UNITS * 512));
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, lds, 16, (int)a_off[0], kt * (BK * 2), 0, 0);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, lds, 16, (int)a_off[1], kt * (BK * 2), 1024, 0);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, lds, 16, (int)a_off[2], kt * (BK * 2), 2048, 0);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, lds, 16, (int)a_off[3], kt * (BK * 2), 3072, 0);
-            asm volatile("" ::: "memory");  // the loads that follow stay behind these
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, lds, 16, (int)a_off[u], kt * (BK * 2), 1024 * u, 0);
+            if (u == A_UNITS - 1) asm volatile("" ::: "memory");  // the loads that follow stay behind these
         };
+        using U0 = std::integral_constant<int, 0>;
+        using U1 = std::integral_constant<int, 1>;
+        using U2 = std::integral_constant<int, 2>;
+        using U3 = std::integral_constant<int, 3>;
+        auto dma_tile = [&](half_t *dst, int kt) { dma_a(dst, kt, U0{}), dma_a(dst, kt, U1{}), dma_a(dst, kt, U2{}), dma_a(dst, kt, U3{}); };
         const int sw = (l32 >> 1) & 7;  // (row >> 1) & 7 for every row this lane reads (rows = 32*j + l32)
 
         // Packed words of two K tiles: slot [par][ks] holds step ks of a tile of parity par.  It
@@ -394,7 +397,7 @@ __global__ __launch_bounds__(256, 2) void gptq4_gemm_kernel(MatmulArgs p) {
                 return t ? b2[par][step].y : b2[par][step].x;
             }
         };
-        // Scale and zero words run two tiles ahead as well: slot [par] is loaded in the last step of a
+        // Scale and zero words run two tiles ahead as well: slot [par] is loaded in the first step of a
         // tile of parity par with the group of the tile two on, and turned into the decode
         // constants of that tile during the last step of the tile in between.
         uint32_t g_s[2], g_z[2];
@@ -418,20 +421,25 @@ __global__ __launch_bounds__(256, 2) void gptq4_gemm_kernel(MatmulArgs p) {
         // decoded in natural order too
         ColDecodeNat cn[2];
         auto make_cn = [&](int par, int t) {
+            // (the empty asm statements keep the arithmetic here: the compiler may otherwise do it, and wait for the words, where they
+            // are loaded)
+            uint32_t scale = (SB && t) ? g_z[par] : g_s[par];
+            asm volatile("" : "+v"(scale));
             if constexpr (SB) {
-                const uint32_t m = t ? g_z[par] : g_s[par];
-                cn[t] = make_col_decode_nat((m >> 16) & 0xFu, m);
+                cn[t] = make_col_decode_nat((scale >> 16) & 0xFu, scale);
             } else {
-                cn[t] = make_col_decode_nat((g_z[par] >> (((2 * l32) & 7) * 4 + 4 * t)) & 0xFu, t ? g_s[par] >> 16 : g_s[par]);
+                uint32_t zeros = g_z[par];
+                asm volatile("" : "+v"(zeros));
+                cn[t] = make_col_decode_nat((zeros >> (((2 * l32) & 7) * 4 + 4 * t)) & 0xFu, t ? scale >> 16 : scale);
             }
         };
         // (in the order of the loop: a wait of the compiler's in the loop holds for the first pass too)
         const int second = min(k_begin + 1, nk - 1);
-        dma_a(As0, k_begin);
+        dma_tile(As0, k_begin);
         load_group2(0, k_begin);
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) load_b2(0, k_begin, ks);
-        dma_a(As1, second);
+        dma_tile(As1, second);
         load_group2(1, second);  // made into constants at the end of tile k_begin
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) load_b2(1, second, ks);
@@ -482,21 +490,30 @@ __global__ __launch_bounds__(256, 2) void gptq4_gemm_kernel(MatmulArgs p) {
                 if (ks < 3 || FINAL) __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), once for the step's fragments
                 __builtin_amdgcn_sched_barrier(0);
                 if (ks == 3 && !FINAL) {
-                    // Every wave has issued at least 4 vector-memory loads after its LDS-direct loads
-                    // of the next tile (the scale/zero words and the packed words of 4 K steps), and
-                    // loads complete in order: at most 4 outstanding means the tile has landed.
+                    // Every wave has issued the packed words of 4 K steps and the scale/zero words (5 or 6 vector-memory
+                    // loads) after its LDS-direct loads of the next tile, and loads complete in order: at most that many
+                    // outstanding means the tile has landed.
                     // (tests/test_wait_counts.py counts the loads behind the tile's in the compiled code of every variant.)
-                    asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(SB ? 5 : 6) : "memory");
                 }
 #pragma unroll
                 for (int i = 0; i < 2 * MT; ++i) {
                     const int t = i / MT, mt = i % MT;
                     acc[mt][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mt], bf[t], acc[mt][t], 0, 0, 0);
                     if (t == 0 && (ks < 3 || !FINAL)) ahead[mt] = ks < 3 ? read_a(cur, ks + 1, mt) : read_a(nxt, 0, mt);
-                    if (t == 1 && ks == 3 && !FINAL) {
-                        if (mt == 0) dma_a(cur, tile2);
-                        if (mt == MT - 2) load_group2(par, tile2);
+                    if (ks == 3 && !FINAL) {
+                        // (as soon as the barrier allows: what is asked for here is waited for a tile later, and a workgroup that has
+                        // its CU to itself runs no faster than that comes.  From the middle of the step on, 341 x 3840 x 11264 in
+                        // streaming order took 48.2 us instead of 41.0.  One a slot 1 % faster than all four in the first
+                        // slot for streaming-order words, 4 % slower for checkpoint-order ones)
+                        if (i == 0) dma_a(cur, tile2, U0{});
+                        if (i == (SB ? MT / 4 : 0)) dma_a(cur, tile2, U1{});
+                        if (i == (SB ? 2 * MT / 4 : 0)) dma_a(cur, tile2, U2{});
+                        if (i == (SB ? 3 * MT / 4 : 0)) dma_a(cur, tile2, U3{});
                     }
+                    // (the slot was made into constants in the tile before: behind the wait of this tile's last step, so that it does
+                    // not wait for them)
+                    if (ks == 0 && i == 1 && !FINAL) load_group2(par, tile2);
                     if (i == 2 * MT - 1 && !FINAL) load_b2(par, tile2, ks);  // (this step's words were decoded during the previous step)
 #pragma unroll
                     for (int d = 0; d < 4 / MT && (ks < 3 || !FINAL); ++d) {
