@@ -157,10 +157,8 @@ __global__ __launch_bounds__(64 * KS, MT > 2 || (KS == 8 && (MT == 2 || (EPI != 
         half_t *const buf1 = As1 + wave * A_HALVES;
         // Activations global -> LDS directly.  One instruction fills 8 rows x 8 chunks of 16
         // bytes; the chunk that lands at position c of row r is global chunk c ^ ((r >> 1) & 7),
-        // which makes the 128-bit fragment reads conflict-free without padding.  Rows of a
-        // unit are 8u + lane / 8, so the swizzle term is (lane >> 4) for even u and that ^ 4
-        // for odd u: two per-lane offsets, everything else is a scalar offset.
-        // Four units share an LDS base: their distance is the instruction's own offset, which moves both addresses, so the
+        // which makes the 128-bit fragment reads conflict-free without padding.
+        // Four units share an LDS base and the lane's four offsets: their distance is the instruction's own offset, which moves both addresses, so the
         // lane's is that much smaller (8 rows are 4096 bytes at least).  Rows from M on are not read: an offset out of the
         // buffer's range loads zeros, and a tile that does not exist is one of an empty buffer - no memory is touched for what
         // is requested ahead of a wave's last tile.
@@ -244,10 +242,11 @@ __global__ __launch_bounds__(64 * KS, MT > 2 || (KS == 8 && (MT == 2 || (EPI != 
                 return t ? b2[j][par][step].y : b2[j][par][step].x;
             }
         };
-        // Scale and zero words run two tiles ahead as well: slot [par] is loaded in the last step of a tile of parity par and
+        // Scale and zero words run two tiles ahead as well: slot [par] is loaded in the first step of a tile of parity par and
         // made into the decode constants of the tile two on during the last step of the tile in between.
         uint32_t g_s[NB][2], g_z[NB][2];
-        uint32_t g_s_hi[2], g_z_hi[2];  // PAIRED: scale and zero word of the lane's second column
+        uint32_t g_z_hi[2];              // PAIRED: the zero word of the lane's second column,
+        uint16_t g_s16[2], g_s16_hi[2];  // and, checkpoint order, the scales of its two columns (widened at their use)
         const uint32_t group_magic = p.tile_group_magic;  // (group = tile / (groupsize / 64): exact for every tile)
         const int group_shift = p.tile_group_shift;
         auto load_group2 = [&](int par, int tile) {
@@ -270,8 +269,8 @@ __global__ __launch_bounds__(64 * KS, MT > 2 || (KS == 8 && (MT == 2 || (EPI != 
                     const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc((void *)(p.w[mat].scales + n0 + (uint64_t)g * (uint32_t)N), 0, (N - n0) * 2, 0x00020000);
                     const __amdgpu_buffer_rsrc_t zr = __builtin_amdgcn_make_buffer_rsrc((void *)(p.w[mat].qzeros + (n0 >> 3) + (uint64_t)g * (uint32_t)(N >> 3)), 0, (N - n0) >> 1, 0x00020000);
                     if constexpr (PAIRED) {
-                        g_s[j][par] = __builtin_amdgcn_raw_buffer_load_b16(sr, slane, 0, 0);
-                        g_s_hi[par] = __builtin_amdgcn_raw_buffer_load_b16(sr, slane + 128, 0, 0);
+                        g_s16[par] = __builtin_amdgcn_raw_buffer_load_b16(sr, slane, 0, 0);
+                        g_s16_hi[par] = __builtin_amdgcn_raw_buffer_load_b16(sr, slane + 128, 0, 0);
                         g_z[j][par] = __builtin_amdgcn_raw_buffer_load_b32(zr, zlane, 0, 0);
                         g_z_hi[par] = __builtin_amdgcn_raw_buffer_load_b32(zr, zlane + 32, 0, 0);
                     } else {
@@ -285,8 +284,15 @@ __global__ __launch_bounds__(64 * KS, MT > 2 || (KS == 8 && (MT == 2 || (EPI != 
         auto make_cn = [&](int par, int j, int t) {
             // (the empty asm statements keep the arithmetic here: the compiler otherwise does it, and waits for the words, where they
             // are loaded, a tile earlier)
-            uint32_t scale = (t && PAIRED && !SB) ? g_s_hi[par] : (t && SB) ? g_z[j][par] : g_s[j][par];
-            asm volatile("" : "+v"(scale));
+            uint32_t scale;
+            if constexpr (PAIRED && !SB) {
+                uint16_t half = t ? g_s16_hi[par] : g_s16[par];
+                asm volatile("" : "+v"(half));
+                scale = half;
+            } else {
+                scale = (SB && t) ? g_z[j][par] : g_s[j][par];
+                asm volatile("" : "+v"(scale));
+            }
             if constexpr (SB) {
                 cn[j][t] = make_col_decode_nat((scale >> 16) & 0xFu, scale);
             } else {
@@ -297,17 +303,18 @@ __global__ __launch_bounds__(64 * KS, MT > 2 || (KS == 8 && (MT == 2 || (EPI != 
             }
         };
 
+        // The second tile's rows are asked for when the first one's words are there: with 128 KiB of rows in front of them (eight
+        // waves, 64 rows) a wave waited 1.6 us for its first product instead of 1.2, which calls of two K tiles a wave do not make
+        // up for (833 x 1024 x 1024 7.86 -> 7.57 us, 170 x 1024 x 2816 7.92 -> 7.63).
         const int second = k_begin + 1;
 #pragma unroll
         for (int u = 0; u < A_UNITS; ++u) dma_a(buf0, k_begin, u);
         load_group2(0, k_begin);
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) load_b2(0, k_begin, ks);
+        constexpr int FIRST_STEPS = SB ? 2 : 4;  // (SB: the other two stand behind the rows, among the loads that the first wait in the loop counts)
 #pragma unroll
-        for (int u = 0; u < A_UNITS; ++u) dma_a(buf1, second, u);
-        load_group2(1, second);  // made into constants at the end of tile k_begin
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) load_b2(1, second, ks);
+        for (int ks = 0; ks < FIRST_STEPS; ++ks) load_b2(1, second, ks);
         h8_t bf[NB][2];
 #pragma unroll
         for (int j = 0; j < NB; ++j)
@@ -316,6 +323,12 @@ __global__ __launch_bounds__(64 * KS, MT > 2 || (KS == 8 && (MT == 2 || (EPI != 
                 make_cn(0, j, t);
                 bf[j][t] = decode_word_natural(word_of(j, 0, 0, t), cn[j][t]);
             }
+        asm volatile("" : "+v"(bf[0][0])::"memory");
+#pragma unroll
+        for (int u = 0; u < A_UNITS; ++u) dma_a(buf1, second, u);
+        load_group2(1, second);  // made into constants at the end of tile k_begin
+#pragma unroll
+        for (int ks = FIRST_STEPS; ks < 4; ++ks) load_b2(1, second, ks);
         // fragment mt of K step ks of the tile in `src`
         auto read_a = [&](const half_t *src, int ks, int mt) {
             return *reinterpret_cast<const h8_t *>(src + (mt * 32 + l32) * BK + 8 * ((SB ? 4 * (ks >> 1) + 2 * lhi + (ks & 1) : 2 * ks + lhi) ^ sw));
@@ -338,6 +351,9 @@ __global__ __launch_bounds__(64 * KS, MT > 2 || (KS == 8 && (MT == 2 || (EPI != 
         auto k_tile = [&](half_t *cur, const half_t *nxt, int kt, int par, auto final) {
             constexpr bool FINAL = decltype(final)::value;
             constexpr int SLOTS = 2 * NB * MT;
+            constexpr int ROW_SLOTS = (SLOTS + 3) / 4;  // slots of the last step in which rows are asked for
+            // packed words of four steps and scale/zero words: the loads behind those of a tile's rows
+            constexpr int BEHIND = SB ? (PAIRED ? 6 : 5 * NB) : 6 * NB * (PAIRED ? 2 : 1);
             const int tile2 = kt + 2;
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) {
@@ -348,22 +364,25 @@ __global__ __launch_bounds__(64 * KS, MT > 2 || (KS == 8 && (MT == 2 || (EPI != 
                 DecodeNat dec;
                 if (ks < 3 || FINAL) __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), once for the step's fragments
                 __builtin_amdgcn_sched_barrier(0);
-                // Loads complete in order, and behind the LDS-direct loads of the next tile this wave issued scale/zero words and
-                // the packed words of four K steps: at most that many outstanding means the tile has landed.
+                // Loads complete in order, and behind the LDS-direct loads of the next tile this wave issued the packed words of
+                // four K steps and scale/zero words: at most that many outstanding means the tile has landed.
                 // (tests/test_wait_counts.py counts the loads behind the tile's in the compiled code of every variant.)
-                if (ks == 3 && !FINAL) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(4 * NB * ((PAIRED && !SB) ? 2 : 1)) : "memory");
+                if (ks == 3 && !FINAL) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(BEHIND) : "memory");
 #pragma unroll
                 for (int i = 0; i < SLOTS; ++i) {
                     const int j = i / (2 * MT), t = (i / MT) & 1, mt = i % MT;
                     acc[j][mt][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mt], bf[j][t], acc[j][mt][t], 0, 0, 0);
                     if (i < MT && next) ahead[i] = ks < 3 ? read_a(cur, ks + 1, i) : read_a(nxt, 0, i);
                     if (ks == 3 && !FINAL) {
-                        // (all of this wave's reads of `cur` are done)
+                        // (all of this wave's reads of `cur` are done.  Asked for early: over the whole step, 65 rows of gate/up
+                        // 5120 x 13824 in checkpoint order took 37.1 us instead of 34.9)
 #pragma unroll
-                        for (int u = i * A_UNITS / SLOTS; u < (i + 1) * A_UNITS / SLOTS; ++u) dma_a(cur, tile2, u);
-                        if (i == SLOTS - 1) load_group2(par, tile2);
+                        for (int u = i * A_UNITS / ROW_SLOTS; u < (i + 1) * A_UNITS / ROW_SLOTS && u < A_UNITS; ++u) dma_a(cur, tile2, u);
                     }
-                    if (i == SLOTS - 1 && !FINAL) load_b2(par, tile2, ks);  // (this step's words were decoded during the previous step)
+                    // (this step's words were decoded during the previous step, the scale/zero slot made into constants in the tile
+                    // before; the last step's words stand behind the rows)
+                    if (i == (ks == 3 ? SLOTS - 1 : 0) && !FINAL) load_b2(par, tile2, ks);
+                    if (ks == 0 && i == 1 && !FINAL) load_group2(par, tile2);
                     if (next) {
                         // words of the next step (step 0 of the next tile when ks == 3), a stage of four instructions at a time
 #pragma unroll
