@@ -461,8 +461,8 @@ __global__ __launch_bounds__(256, 2) void gptq4_gemm_kernel(MatmulArgs p) {
             const int chunk = SB ? 4 * (ks >> 1) + 2 * lhi + (ks & 1) : 2 * ks + lhi;
             return *reinterpret_cast<const h8_t *>(src + row * BK + 8 * (chunk ^ sw));
         };
-        // (more than four loads follow those of the first tile)
-        asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        // (the first tile's words and the whole second tile's loads follow the first tile's)
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(SB ? 14 : 16) : "memory");
         h8_t ahead[MT];  // fragments of the step to come
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) ahead[mt] = read_a(As0, 0, mt);
