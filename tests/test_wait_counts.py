@@ -6,9 +6,10 @@ means the tile has landed only if the wave has issued at least N vector-memory i
 LDS-direct load.  N is written by hand next to the loads it counts (gptq4_gemm.hip, gptq4_kslice.hip); a compiler that
 merged, dropped or hoisted one of those loads above the LDS-direct loads would make the wait return early and the MFMAs
 read a tile that is still in flight - with results that are wrong only sometimes.  This test compiles the two files to
-gfx950 assembly and follows every path of every kernel variant from the kernel's entry and from each such wait to the
-next one: behind the first group of LDS-direct loads on the path (the tile that the next wait is for) it counts the
-vector-memory instructions, and the count must reach the N of the wait the path ends in.
+gfx950 assembly and follows every path of every kernel variant from the kernel's entry on, with the tiles requested on it
+(groups of LDS-direct loads) and the vector-memory instructions behind each.  A loop is entered with two tiles requested: the
+first such wait on a path is for the older one, every later wait for all that have been requested by then, and a tile's count
+must reach the N of the wait it is for (or of an earlier one).
 """
 import importlib.util
 import re
@@ -25,7 +26,6 @@ VMEM = re.compile(r"^(buffer|global|flat|scratch)_(load|store|atomic)")
 WAIT = re.compile(r"^s_waitcnt\b.*\bvmcnt\((\d+)\)")
 LABEL = re.compile(r"^(\.LBB\d+_\d+):")
 BRANCH = re.compile(r"^(s_c?branch\w*)\s+(\.LBB\d+_\d+)")
-CAP = 64  # counts beyond any wait's N are all the same
 
 
 def _build_flags():
@@ -61,43 +61,67 @@ def _kernels(asm: str):
         yield m.group(1), lines
 
 
+def _table_loads(text):
+    """Indices of the LDS-direct loads of the rotary tables (waited for with vmcnt(0), behind the loop): in the order they are
+    written, runs of them go through two buffers in turn, with no scalar offset."""
+    tables, run = set(), []
+    for i, l in enumerate(text + ["buffer_load_dword v0, v0, s[0:3], 0"]):
+        if not VMEM.match(l):
+            continue
+        if l.split()[-1] == "lds":
+            run.append(i)
+            continue
+        args = [[a.strip() for a in text[r].split(",")] for r in run]
+        if len({a[1] for a in args}) > 1 and all(a[2].split()[0] == "0" for a in args):
+            tables.update(run)
+        run = []
+    return tables
+
+
 def _paths_to_waits(lines):
-    """[(N, vector-memory instructions behind the first group of LDS-direct loads, index of the wait)] over all paths
-    from the entry and from every hand-written wait to the next hand-written wait."""
+    """[(N, vector-memory instructions behind a tile's LDS-direct loads, index of the wait)] over all paths from the entry, for
+    every hand-written wait and every tile it is for."""
     text = [l for l, _ in lines]
     label_at = {m.group(1): i for i, l in enumerate(text) if (m := LABEL.match(l))}
-    hand = {i: int(m.group(1)) for i, (l, inline) in enumerate(lines) if inline and (m := WAIT.match(l)) and int(m.group(1)) > 0}
+    waits = {i: int(m.group(1)) for i, l in enumerate(text) if (m := WAIT.match(l))}
+    hand = {i: n for i, n in waits.items() if lines[i][1] and n > 0}
+    if not hand:
+        return []
+    cap = max(hand.values()) + 1  # (counts beyond any wait's N are all the same)
+    tables = _table_loads(text)
     results, seen = [], set()
-    # state: (index, phase, count); phase 0 = no LDS-direct load yet, 1 = inside the first group, 2 = behind it
-    stack = [(0, 0, 0)] + [(w + 1, 0, 0) for w in hand]
+    # state: (index, counts behind the tiles requested and not yet known to have landed, inside a tile's loads, a wait has passed)
+    stack = [(0, (), False, False)]
     while stack:
-        i, phase, count = stack.pop()
+        i, behind, inside, later = stack.pop()
         while i < len(text):
-            if (i, phase, count) in seen:
+            if (i, behind, inside, later) in seen:
                 break
-            seen.add((i, phase, count))
+            seen.add((i, behind, inside, later))
             cur = text[i]
-            if i in hand:
-                if phase:
-                    results.append((hand[i], count, i))
-                break
+            if waits.get(i) == 0:  # everything has landed (of the source's own: a loop ends here, and another one may follow)
+                behind, inside, later = (), False, later and not lines[i][1]
+            elif i in hand and behind:
+                n = hand[i]
+                for count in behind if later else behind[:1]:
+                    results.append((n, count, i))
+                behind, inside, later = () if later else tuple(c for c in behind[1:] if c < n), False, True
             if VMEM.match(cur):
-                direct = cur.split()[-1] == "lds"
-                if direct and phase == 0:
-                    phase = 1
-                elif not direct and phase == 1:
-                    phase, count = 2, 1
-                elif phase == 2:
-                    count = min(count + 1, CAP)
+                if cur.split()[-1] == "lds" and i not in tables:
+                    if not inside:
+                        behind, inside = behind + (0,), True
+                    behind = tuple(min(c + 1, cap) for c in behind[:-1]) + (0,)
+                else:
+                    behind, inside = tuple(min(c + 1, cap) for c in behind), False
             if cur.startswith(("s_endpgm", "s_setpc")):
                 break
             b = BRANCH.match(cur)
             if b:
-                stack.append((label_at[b.group(2)], phase, count))
+                stack.append((label_at[b.group(2)], behind, inside, later))
                 if b.group(1) == "s_branch":
                     break
             i += 1
-    return results
+    return sorted(set(results))
 
 
 @pytest.fixture(scope="module")
@@ -144,3 +168,32 @@ def test_the_scan_sees_a_missing_load():
     assert sorted(_paths_to_waits(prog(3))) == [(4, 3, 7), (4, 5, 7)]
     # a wait of the compiler's own (not between the asm markers) is not a checkpoint
     assert _paths_to_waits([(l, False) for l, _ in prog(3)]) == []
+
+
+def test_the_scan_sees_a_missing_load_behind_the_second_tile_of_a_prologue():
+    """Two tiles requested before the loop, the next one behind the wait in the loop: the first wait in the loop is for the second."""
+    tile = [("buffer_load_dwordx4 v1, s[0:3], s4 offen lds", False)] * 2
+    words = lambda n: [("buffer_load_dwordx2 v[6:7], v8, s[8:11], s5 offen", False)] * n
+
+    def prog(behind_first, behind_second, in_loop):
+        return (tile + words(behind_first) + tile + words(behind_second) + [("s_waitcnt vmcnt(9)", True), (".LBB0_1:", False)] + words(in_loop - 1) +
+                [("s_waitcnt vmcnt(4) lgkmcnt(0)", True)] + tile + words(1) + [("s_cbranch_scc1 .LBB0_1", False), ("s_endpgm", False)])
+
+    def short(*counts):
+        return sorted({(n, behind) for n, behind, _ in _paths_to_waits(prog(*counts)) if behind < n})
+
+    assert short(5, 2, 4) == []
+    assert short(5, 0, 4) == [(4, 3), (9, 7)]  # the second tile's words requested in front of its rows
+    assert short(4, 2, 4) == [(9, 8)]
+    assert short(5, 2, 3) == [(4, 3)]
+    # a tile that an earlier wait has covered needs no other
+    assert short(5, 9, 2) == [(4, 2)] and (4, 10, 21) not in _paths_to_waits(prog(5, 9, 2))
+
+
+def test_table_loads_are_told_from_a_tiles():
+    """The rotary tables' loads behind the second tile are landed by the end of the loop only."""
+    tables = [("buffer_load_dwordx4 v1, s[12:15], 0 offen lds", False), ("buffer_load_dwordx4 v1, s[16:19], 0 offen lds", False)] * 2
+    tile = [("buffer_load_dwordx4 v1, s[0:3], 0 offen lds", False)] * 2
+    word = [("buffer_load_dwordx2 v[6:7], v8, s[8:11], s5 offen", False)]
+    body = tile + word * 3 + tables + [("s_waitcnt vmcnt(7)", True), ("s_waitcnt vmcnt(5)", True), ("s_waitcnt vmcnt(0)", True), ("s_endpgm", False)]
+    assert [r[:2] for r in _paths_to_waits(body)] == [(7, 7)]
