@@ -2,6 +2,8 @@
 every shape it accepts: row counts around its 32- and 64-row tiles and well past them, all
 three epilogues, bias, K split across workgroups as well, ragged last row tiles.
 Same bars as test_gpu_parity.py."""
+import functools
+
 import numpy as np
 import pytest
 import torch
@@ -301,3 +303,44 @@ def test_midm_tiles_of_a_wave_and_groups(config, k, g):
     ref = O.quant_matmul_ref(x, L["qweight"], L["qzeros"], L["scales"], g)
     assert_close(y.cpu().numpy(), ref, f"mid-M matmul K={k} g={g}")
     assert_close(streamed.cpu().numpy(), ref, f"mid-M matmul, streaming order, K={k} g={g}")
+
+
+@functools.lru_cache(maxsize=None)
+def fused_case(hidden, g, m):
+    """Inputs and float64 results of a gate/up pair and of a QKV projection with rotary."""
+    n, heads = 512, hidden // 128
+    gate, up, qkv = O.make_layer(hidden, n, g, seed=hidden), O.make_layer(hidden, n, g, seed=hidden + 1), O.make_layer(hidden, 3 * hidden, g, seed=hidden + 2)
+    x = O.make_x(m, hidden, seed=m)
+    pos = 5 + np.arange(m)[None, :]
+    trip = lambda L: (L["qweight"], L["qzeros"], L["scales"])
+    refs = (O.mlp_gateup_ref(x, trip(gate), trip(up), g),) + tuple(O.qkv_rotary_ref(x[None], *trip(qkv), g, pos, heads, 128, max_pos=2048))
+    return gate, up, qkv, x, pos, refs
+
+
+def check_fused(hidden, g, m, what):
+    """Both epilogues on two matrices or two column blocks, from either layout, against those."""
+    G = gptq()
+    gate, up, qkv, x, pos, refs = fused_case(hidden, g, m)
+    flat = [tuple(D[n] for n in ("qweight", "scales", "qzeros")) for D in map(to_dev, (gate, up, qkv))]
+    packed = [G.stream_pack(w, z, s, g) for w, s, z in flat]
+    xd, pd = torch.from_numpy(x).cuda(), torch.from_numpy(pos).cuda()
+    cos, sin = G.RotaryTable(128, 2048).get(xd.device, 2048)
+    for layout, gateup, rotary, (A, B, C) in (("checkpoint", G.llama_mlp_4, G.qkv_rotary, flat), ("streaming", G.llama_mlp_4_stream, G.qkv_rotary_stream, packed)):
+        got = (gateup(g, xd, *A, *B),) + tuple(rotary(g, xd[None], *C, pd, cos, sin, hidden // 128))
+        for name, y, ref in zip(("gate/up", "q", "k", "v"), got, refs):
+            assert_close(y.cpu().numpy(), ref, f"{what} {name}, {layout} order, K={hidden} g={g} M={m}")
+
+
+@pytest.mark.parametrize("config", [(c + w + mt, 1) for c in (1000, 2000) for w, mts in ((0, (1, 2, 3)), (100, (1, 2)), (200, (1, 2))) for mt in mts] + [(1002, 2), (2102, 2)],
+                         ids=lambda c: "mt%d_s%d" % c)
+@pytest.mark.parametrize("hidden,g", [(1280, 640), (1792, 896), (2304, 384)])
+def test_midm_fused_epilogues_tiles_of_a_wave_and_groups(config, hidden, g):
+    """Two, three, five, seven and nine K tiles to a wave of the gate/up, whole-head and paired rotary variants (their own second
+    matrix, second column block and 16-bit scales), groups of six, ten and fourteen K tiles, rows of a block that does not exist."""
+    from gptq_triton_amd import _lib
+    lib = _lib.load()
+    lib.gptq4_set_midm_tuning(2, *config)
+    try:
+        check_fused(hidden, g, 67, "mid-M")
+    finally:
+        lib.gptq4_set_midm_tuning(1, 0, 0)

@@ -382,3 +382,11 @@ def _gather_calls(lib, _lib, G, xd, x, m, k, n, g, heads, gate, up, qkv, Dg, Du,
                                   g_idx=qkv["g_idx"], max_pos=2048)
     for got, want, name in ((q, qr, "q"), (kk, kr, "k"), (vv, vr, "v")):
         assert_close(got.cpu().numpy(), want, f"in-kernel gather, {name} M={m}")
+
+
+@pytest.mark.parametrize("hidden,g", [(1280, 640), (1792, 896), (2304, 384)])
+def test_tiled_fused_epilogues_few_and_odd_k_tiles(forced_tiled, hidden, g):
+    """The gate/up and rotary epilogues from either layout where the loop of K tiles ends on an odd one, whole and split, and
+    groups of six, ten and fourteen K tiles."""
+    from test_gpu_midm import check_fused
+    check_fused(hidden, g, 67, "tiled")
