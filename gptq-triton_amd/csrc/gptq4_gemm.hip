@@ -474,9 +474,10 @@ __global__ __launch_bounds__(256, 2) void gptq4_gemm_kernel(MatmulArgs p) {
         // `nxt` for every wave (wait, barrier), its first fragments are read, and - every wave has its own last fragments of
         // `cur` by then - the tile two on is requested into `cur`.  With the wait and the barrier between the tiles, four reads in
         // front of a step's MFMAs and the rest where the compiler put it, a K tile of the wide tile (1024 cycles of MFMAs a wave)
-        // took 1530 cycles, two waves to a SIMD 2840 for both; now 1335 and 2510.  The clock gives a part of that back (the chip is
-        // at its power limit): 2048 x 6656 x 17920 387 -> 370 us, 2048 x 4096 x 12288 166 -> 158, 7B gate/up at 2048 rows
-        // 302 -> 288, 2048 x 11008 x 4096 155 -> 146, 2000 x 4096 x 4096 60.1 -> 57.0, 800 x 5120 x 15360 124 -> 119.
+        // took 1530 - 1590 cycles, two waves to a SIMD 2840 for both; now 1330 - 1370 and 2510.  The clock gives a part of that back (the
+        // chip is at its power limit).  Graph replays over rotating weights: 2048 x 6656 x 17920 430 -> 406 us, 2048 x 4096 x 12288
+        // 183 -> 175, 7B gate/up at 2048 rows 335 -> 315, 2048 x 11008 x 4096 167 -> 159, 2000 x 4096 x 4096 66.7 -> 63.3,
+        // 800 x 5120 x 15360 138 -> 128.
         // (final: a last tile that nothing follows, where the loop ends on one - the tiles go in pairs)
         auto k_tile = [&](half_t *cur, const half_t *nxt, int kt, int par, auto final) {
             constexpr bool FINAL = decltype(final)::value;

@@ -344,9 +344,9 @@ __global__ __launch_bounds__(64 * KS, MT > 2 || (KS == 8 && (MT == 2 || (EPI != 
         // the fragment reads of a tile in front of its products and addresses of 64 bits per lane, a K tile of 64 rows x 64
         // columns took four waves 0.88 us on 64 CUs and 1.04 on all 256, eight waves (twice the work) 1.57 and 1.96; now 0.70 and
         // 0.86, 1.34 and 1.78, and 1.10 -> 0.95 for 96 rows: what is left is the rows' way through the CU (some 60 GB/s each, four
-        // waves or eight) beside ~190 instructions a wave.  Calls of 17 .. 700 rows: 4096 x 4096 at 320 rows 23.5 -> 19.3 us,
-        // 5120 x 5120 at 200 rows 28.0 -> 22.3 (both of four waves), 11008 x 4096 at 700 rows 79.3 -> 73.5; 1818 random calls of either
-        // layout on average 5 %.
+        // waves or eight) beside ~190 instructions a wave.  Graph replays over rotating weights: 4096 x 4096 at 320 rows
+        // 23.3 -> 19.4 us, 5120 x 5120 at 200 rows 26.8 -> 21.6 (both of four waves), 11008 x 4096 at 700 rows 76.8 -> 71.5; slower by 2 - 4 %
+        // with K = 5120 and weights from HBM at some row counts from 32 to 125, where the streams of waves in step meet in few channels.
         // (final: a last tile that nothing follows, where the loop ends on one - the tiles go in pairs)
         auto k_tile = [&](half_t *cur, const half_t *nxt, int kt, int par, auto final) {
             constexpr bool FINAL = decltype(final)::value;
@@ -842,7 +842,9 @@ static KslicePlan rounds_plan(int epi, int M, int N, int K, bool has_perm) {
 // with steps = K tiles of the longest wave, `step` that of one workgroup or of two to a CU, `load` what the others' traffic
 // adds to a step, and the cost of splitting K across workgroups (the first split, then every further one).  One line per
 // kernel variant, in us, fitted to 3500 timings over 20 projections (K and N from 2048 to 19968) at 24 to 768 rows with the
-// weights from HBM: 3 - 7 % off per variant.  (Where it may decide: one_round_margin.)
+// weights from HBM - of the loop before its instructions were dealt to its MFMAs.  Against 5000 timings of the present one (31 projections,
+// K from 1024 to 17920, 17 to 768 rows, streaming order): 5 - 11 % off per variant, on average 8 % low (32-row tiles, eight waves) to 2 %
+// high (96-row tiles).  (Where it may decide: one_round_margin.)
 struct RoundCost {
     float t0, one, two, load, split, more;  // two = 0: one workgroup to a CU
 };
@@ -865,7 +867,8 @@ static double one_round_estimate(int epi, int K, const KslicePlan &pl, long cus)
            (pl.splitk > 1 ? c.split + c.more * (pl.splitk - 2) : 0.0);
 }
 
-// What the tiled kernel takes, whatever plan it chooses (us; fitted to the same timings, 10 % off; see one_round_margin).
+// What the tiled kernel takes, whatever plan it chooses (us; fitted to its loop before, too; against the present one 10 - 11 % off, on
+// average right for plain calls and 3 - 5 % high for the others; see one_round_margin).
 static double tiled_estimate(int epi, int M, int N, int K) {
     const double tiles = (double)((M + 127) / 128) * (N / (epi == EPI_SILU_MUL ? 128 : 256)) / device_shape().cus, nk = K / 64;
     const double t0 = epi == EPI_PLAIN ? 12.9 : epi == EPI_SILU_MUL ? 8.5 : 19.0;
@@ -876,7 +879,9 @@ static double tiled_estimate(int epi, int M, int N, int K) {
 
 // How far a launch of one round has to be ahead of the tiled kernel's estimate to be planned (0: never), so that the two
 // estimates' errors do not choose the slower one.  Both were fitted at 24 to 768 rows; against the plan by scores and the tiled
-// kernel they were then timed on 1800 calls outside the fit (17 to 8192 rows, K from 512 to 32768, N from 256 to 32000):
+// kernel they were then timed on 1800 calls outside the fit (17 to 8192 rows, K from 512 to 32768, N from 256 to 32000), with the
+// loops of that time (with the present ones the plan taken is 2.4 % behind the fastest of all timed, on average over 558 calls of 17 to
+// 768 rows, and more than 5 % behind for 92 of them, 25 % at most):
 //   up to 768 rows, 5 % ahead:     on average 11 % (plain, gate/up) and 20 % (rotary) faster; 11 of 871 calls slower, by 5 - 11 %
 //   769 .. 2048 rows, 15 % ahead:  on average 27 % and 29 % faster, 3 of 405 slower (12 % at most); at 5 % ahead 21 were, up to 24 %
 //   2049 .. 8192 rows, 30 % ahead: 40 of 99 calls still go there, 17 % faster, 1 slower; at 5 % ahead 17 were, up to 38 %
