@@ -346,7 +346,7 @@ __global__ __launch_bounds__(64 * KS, MT > 2 || (KS == 8 && (MT == 2 || (EPI != 
         // 0.86, 1.34 and 1.78, and 1.10 -> 0.95 for 96 rows: what is left is the rows' way through the CU (some 60 GB/s each, four
         // waves or eight) beside ~190 instructions a wave.  Graph replays over rotating weights: 4096 x 4096 at 320 rows
         // 23.3 -> 19.4 us, 5120 x 5120 at 200 rows 26.8 -> 21.6 (both of four waves), 11008 x 4096 at 700 rows 76.8 -> 71.5; slower by 2 - 4 %
-        // with K = 5120 and weights from HBM at some row counts from 32 to 125, where the streams of waves in step meet in few channels.
+        // with K = 5120 at some row counts from 32 to 125, where either loop waits for the weights from HBM (with warm ones 12 % faster).
         // (final: a last tile that nothing follows, where the loop ends on one - the tiles go in pairs)
         auto k_tile = [&](half_t *cur, const half_t *nxt, int kt, int par, auto final) {
             constexpr bool FINAL = decltype(final)::value;
